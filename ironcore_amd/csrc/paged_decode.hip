@@ -306,46 +306,44 @@ __global__ __launch_bounds__(NW *kWave) void paged_decode_kernel(const DecodeKP 
 
 constexpr int kReduceThreads = 256;
 
-// Combine the split-K partials of one pair (a KV head's query heads of one
-// sequence).  grid = (pairs per sequence / pairs per workgroup, n_seqs).  A pair's tiles in a row
-// are a contiguous run of a phase's tile sequence, so the shares that touched
-// it are first_tile / chunk .. last_tile / chunk and their partial ids follow.
-// With shared-prefix cohorts a sequence has two sources: its own row and its
-// cohort's row of the shared phase, where it owns `group` of the matrix
+// Where the split-K partials of one (sequence, pair) lie.  A pair's tiles in a
+// row are a contiguous run of a phase's tile sequence, so the shares that
+// touched it are first_tile / chunk .. last_tile / chunk and their partial ids
+// follow.  With shared-prefix cohorts a sequence has two sources: its own row
+// and its cohort's row of the shared phase, where it owns `group` of the matrix
 // columns of one wave of each unit.
-// Traffic is (hd+2)*4 bytes per partial, three orders of magnitude below the
-// K/V stream; what costs time here is the chain of dependent memory round
-// trips, so the prefix sums are fetched together and every thread fetches up
-// to four partials of its four output dims in one batch before it merges them
-// (a typical pair has two to four partials: two round trips in all).
-template <class E, int HD>
-__global__ __launch_bounds__(kReduceThreads) void paged_decode_reduce_kernel(const DecodeKP p) {
-  using T = typename E::type;
-  constexpr int QPH = HD / 4;  // 4-dim groups per head row
-  constexpr int UB = 4;        // partials fetched per batch
+struct PartialList {
+  int heads, head0;  // query heads of the pair
+  int n_tiles;       // tiles behind the row (0: no visible token)
+  int64_t n0, n_all;  // partials of source 0 (the cohort's row), of both
+  int64_t w_lo[2], slot0[2], mul[2], add[2];
+  int col0[2];
+  // Slot of partial i, column g: share w of a source left it in slot (w + slot0) * mul + add,
+  // column col0 + g.
+  __device__ __forceinline__ int64_t slot(int64_t i, int g, int cols) const {
+    const int src = i < n0 ? 0 : 1;
+    const int64_t w = src == 0 ? w_lo[0] + i : w_lo[1] + (i - n0);
+    return ((w + slot0[src]) * mul[src] + add[src]) * cols + col0[src] + g;
+  }
+};
+
+__device__ __forceinline__ PartialList partial_list(const DecodeKP &p, int seq, int pair_in_seq) {
+  PartialList r;
   const int COLS = p.gt;
-  // A pair keeps COLS * QPH threads busy; a workgroup takes as many pairs of
-  // its sequence as fit (8 for MHA at hd 128), each on its own slice of threads.
-  const int width = COLS * QPH < kReduceThreads ? COLS * QPH : kReduceThreads;
-  const int per_wg = kReduceThreads / width;
-  const int tid = threadIdx.x % width;
-  const int pair_in_seq = blockIdx.x * per_wg + threadIdx.x / width;
-  const int seq = blockIdx.y;
-  if (pair_in_seq >= p.pairs_per_seq || threadIdx.x >= per_wg * width) return;
   const int kvh = pair_in_seq / p.nsub;
   const bool cohorts = p.cohort_size > 1;
-  int heads, head0, cohort = 0, col_sh = 0, wave_sh = 0;
+  int cohort = 0, col_sh = 0, wave_sh = 0;
   if (!cohorts) {
     const int sub = pair_in_seq - kvh * p.nsub;
-    head0 = kvh * p.group + sub * COLS;
-    heads = (p.group - sub * COLS < COLS) ? p.group - sub * COLS : COLS;
+    r.head0 = kvh * p.group + sub * COLS;
+    r.heads = (p.group - sub * COLS < COLS) ? p.group - sub * COLS : COLS;
   } else {
     cohort = seq / p.cohort_size;
     const int u = seq - cohort * p.cohort_size;
     wave_sh = u / p.spw;                        // the wave of a unit that carries this member
     col_sh = (u - wave_sh * p.spw) * p.group;   // its first column there
-    head0 = kvh * p.group;
-    heads = p.group;
+    r.head0 = kvh * p.group;
+    r.heads = p.group;
   }
   const int cum_own = p.cum_blocks[seq];
   const int nb_own = p.cum_blocks[seq + 1] - cum_own;
@@ -356,79 +354,166 @@ __global__ __launch_bounds__(kReduceThreads) void paged_decode_reduce_kernel(con
     nb_sh = p.cum_shared[cohort + 1] - cum_sh;
     cum_sh_all = p.cum_shared[p.n_cohorts];
   }
-  T *orow = reinterpret_cast<T *>(p.out) + seq * p.out_stride_seq + (int64_t)head0 * HD;
-  if (nb_own + nb_sh == 0) {  // no visible token: zero rows
-    for (int o = tid; o < heads * HD; o += width) orow[o] = E::narrow(0.f);
-    return;
-  }
+  r.n_tiles = nb_own + nb_sh;
   // source 0: the cohort's row of the shared phase, source 1: the sequence's
-  // own row; an empty source gets an empty share range.  A share w of a source
-  // left its partial in slot (w + slot0) * mul + add, column col0 + g.
-  int64_t w_lo[2], w_hi[2], slot0[2], mul[2], add[2];
-  int col0[2];
+  // own row; an empty source gets an empty share range
+  int64_t n[2];
   {
     const int64_t chunk = chunk_tiles(p, (int64_t)cum_sh_all * p.pairs_per_seq, phase_units(p, 1));
     const int64_t first = (int64_t)cum_sh * p.pairs_per_seq + (int64_t)pair_in_seq * nb_sh;
-    w_lo[0] = first / chunk;
-    w_hi[0] = nb_sh > 0 ? (first + nb_sh - 1) / chunk : w_lo[0] - 1;
-    slot0[0] = (int64_t)cohort * p.pairs_per_seq + pair_in_seq;
-    mul[0] = (int64_t)1 << p.unit_shift;
-    add[0] = p.shared_slot0 + wave_sh;
-    col0[0] = col_sh;
+    r.w_lo[0] = first / chunk;
+    n[0] = nb_sh > 0 ? (first + nb_sh - 1) / chunk - r.w_lo[0] + 1 : 0;
+    r.slot0[0] = (int64_t)cohort * p.pairs_per_seq + pair_in_seq;
+    r.mul[0] = (int64_t)1 << p.unit_shift;
+    r.add[0] = p.shared_slot0 + wave_sh;
+    r.col0[0] = col_sh;
   }
   {
     const int64_t chunk = chunk_tiles(p, (int64_t)cum_all * p.pairs_per_seq, phase_units(p, 0));
     const int64_t first = (int64_t)cum_own * p.pairs_per_seq + (int64_t)pair_in_seq * nb_own;
-    w_lo[1] = first / chunk;
-    w_hi[1] = nb_own > 0 ? (first + nb_own - 1) / chunk : w_lo[1] - 1;
-    slot0[1] = (int64_t)seq * p.pairs_per_seq + pair_in_seq;
-    mul[1] = 1;
-    add[1] = 0;
-    col0[1] = 0;
+    r.w_lo[1] = first / chunk;
+    n[1] = nb_own > 0 ? (first + nb_own - 1) / chunk - r.w_lo[1] + 1 : 0;
+    r.slot0[1] = (int64_t)seq * p.pairs_per_seq + pair_in_seq;
+    r.mul[1] = 1;
+    r.add[1] = 0;
+    r.col0[1] = 0;
   }
-  // one wave covered all the sequence has for this pair and wrote the rows
-  if (nb_sh == 0 && w_lo[1] == w_hi[1]) return;
-  for (int o = tid; o < heads * QPH; o += width) {
-    const int g = o / QPH;
-    const int d = (o - g * QPH) * 4;
-    float m_run = kNegInf, l_run = 0.f;
-    float4 a_run = make_float4(0.f, 0.f, 0.f, 0.f);
-    // the partials of both sources as one list, fetched UB at a time: all loads of a batch are
-    // independent and in flight together, whichever source they come from
-    const int64_t n0 = w_hi[0] - w_lo[0] + 1, n_all = n0 + (w_hi[1] - w_lo[1] + 1);
-    for (int64_t ib = 0; ib < n_all; ib += UB) {
+  r.n0 = n[0];
+  r.n_all = n[0] + n[1];
+  return r;
+}
+
+// Four output dims of one head while partials are merged into them.
+struct Merged {
+  float m = kNegInf, l = 0.f;
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  __device__ __forceinline__ void add(float pm, float pl, const float4 &pa) {
+    if (pm == kNegInf) return;
+    const float m_new = fmaxf(m, pm);
+    const float keep = (m == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+    const float wt = __builtin_amdgcn_exp2f(pm - m_new);
+    l = __builtin_fmaf(pl, wt, l * keep);
+    a.x = __builtin_fmaf(pa.x, wt, a.x * keep);
+    a.y = __builtin_fmaf(pa.y, wt, a.y * keep);
+    a.z = __builtin_fmaf(pa.z, wt, a.z * keep);
+    a.w = __builtin_fmaf(pa.w, wt, a.w * keep);
+    m = m_new;
+  }
+  // Partials first, first + step, ... of head column g, dims d .. d+3: fetched four at a time, all
+  // loads of a batch independent and in flight together, whichever source they come from.
+  template <int HD>
+  __device__ __forceinline__ void add_all(const DecodeKP &p, const PartialList &pl, int64_t first, int64_t step, int g,
+                                          int d) {
+    constexpr int UB = 4;
+    for (int64_t ib = first; ib < pl.n_all; ib += UB * step) {
       float2 ml[UB];
       float4 av[UB];
 #pragma unroll
       for (int u = 0; u < UB; ++u) {
-        const int64_t i = ib + u < n_all ? ib + u : n_all - 1;
-        const int src = i < n0 ? 0 : 1;
-        const int64_t w = src == 0 ? w_lo[0] + i : w_lo[1] + (i - n0);
-        const int64_t slot = ((w + slot0[src]) * mul[src] + add[src]) * COLS + col0[src] + g;
+        const int64_t i = ib + u * step < pl.n_all ? ib + u * step : pl.n_all - 1;
+        const int64_t slot = pl.slot(i, g, p.gt);
         ml[u] = *reinterpret_cast<const float2 *>(p.part_ml + slot * 2);
         av[u] = *reinterpret_cast<const float4 *>(p.part_acc + slot * HD + d);
       }
 #pragma unroll
-      for (int u = 0; u < UB; ++u) {
-        if (ib + u >= n_all || ml[u].x == kNegInf) continue;
-        const float m_new = fmaxf(m_run, ml[u].x);
-        const float keep = (m_run == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
-        const float wt = __builtin_amdgcn_exp2f(ml[u].x - m_new);
-        l_run = __builtin_fmaf(ml[u].y, wt, l_run * keep);
-        a_run.x = __builtin_fmaf(av[u].x, wt, a_run.x * keep);
-        a_run.y = __builtin_fmaf(av[u].y, wt, a_run.y * keep);
-        a_run.z = __builtin_fmaf(av[u].z, wt, a_run.z * keep);
-        a_run.w = __builtin_fmaf(av[u].w, wt, a_run.w * keep);
-        m_run = m_new;
-      }
+      for (int u = 0; u < UB; ++u)
+        if (ib + u * step < pl.n_all) add(ml[u].x, ml[u].y, av[u]);
     }
-    const float inv = 1.f / l_run;
-    T *dst = orow + g * HD + d;
-    dst[0] = E::narrow(a_run.x * inv);
-    dst[1] = E::narrow(a_run.y * inv);
-    dst[2] = E::narrow(a_run.z * inv);
-    dst[3] = E::narrow(a_run.w * inv);
   }
+  template <class E>
+  __device__ __forceinline__ void write(typename E::type *dst) const {
+    const float inv = 1.f / l;
+    dst[0] = E::narrow(a.x * inv);
+    dst[1] = E::narrow(a.y * inv);
+    dst[2] = E::narrow(a.z * inv);
+    dst[3] = E::narrow(a.w * inv);
+  }
+};
+
+// Combine the split-K partials of one pair (a KV head's query heads of one
+// sequence).  grid = (pairs per sequence / pairs per workgroup, n_seqs).
+// Traffic is (hd+2)*4 bytes per partial, three orders of magnitude below the
+// K/V stream; what costs time here is the chain of dependent memory round
+// trips, so the prefix sums are fetched together and every thread fetches up
+// to four partials of its four output dims in one batch before it merges them
+// (a typical pair has two to four partials: two round trips in all).
+template <class E, int HD>
+__global__ __launch_bounds__(kReduceThreads) void paged_decode_reduce_kernel(const DecodeKP p) {
+  using T = typename E::type;
+  constexpr int QPH = HD / 4;  // 4-dim groups per head row
+  const int COLS = p.gt;
+  // A pair keeps COLS * QPH threads busy; a workgroup takes as many pairs of
+  // its sequence as fit (8 for MHA at hd 128), each on its own slice of threads.
+  const int width = COLS * QPH < kReduceThreads ? COLS * QPH : kReduceThreads;
+  const int per_wg = kReduceThreads / width;
+  const int tid = threadIdx.x % width;
+  const int pair_in_seq = blockIdx.x * per_wg + threadIdx.x / width;
+  const int seq = blockIdx.y;
+  if (pair_in_seq >= p.pairs_per_seq || threadIdx.x >= per_wg * width) return;
+  const PartialList pl = partial_list(p, seq, pair_in_seq);
+  T *orow = reinterpret_cast<T *>(p.out) + seq * p.out_stride_seq + (int64_t)pl.head0 * HD;
+  if (pl.n_tiles == 0) {  // no visible token: zero rows
+    for (int o = tid; o < pl.heads * HD; o += width) orow[o] = E::narrow(0.f);
+    return;
+  }
+  // one wave covered all the sequence has for this pair and wrote the rows
+  if (pl.n0 == 0 && pl.n_all == 1) return;
+  for (int o = tid; o < pl.heads * QPH; o += width) {
+    const int g = o / QPH;
+    const int d = (o - g * QPH) * 4;
+    Merged r;
+    r.add_all<HD>(p, pl, 0, 1, g, d);
+    r.write<E>(orow + g * HD + d);
+  }
+}
+
+// The same for batches of few, long rows, whose pairs are cut over many waves
+// (one sequence of 60 000 tokens: 112 partials per pair).  The kernel above
+// walks them one batch of four after the other, a round trip each; here a
+// workgroup belongs to ONE query head and its threads take the partials in
+// slices (16 at head dim 128), which are merged through LDS at the end.
+// grid = (hn, n_seqs).
+//
+// Measured, both launches of a call together, narrow / wide: 1 sequence of
+// 60 001 tokens (32 / 8 heads, fp16, 112 partials per pair) 68.1 / 46.4 us, 1 of
+// 4 096 (32 / 32 heads, 64 partials) 32.9 / 21.2 us, 4 of 8K-16K (32 / 8 heads,
+// 28 partials) 47.0 / 41.8 us, 16 of 500-1 000 (16 partials) 23.3 / 21.3 us, 32 of
+// 500-1 000 (8 partials, 1 024 workgroups) 29.5 / 31.4 us: hence the line at 12.
+constexpr int kWideReduceThreads = 512;
+constexpr int kWideReducePartials = 12;  // mean partials per pair from which this kernel is launched
+
+template <class E, int HD>
+__global__ __launch_bounds__(kWideReduceThreads) void paged_decode_wide_reduce_kernel(const DecodeKP p) {
+  using T = typename E::type;
+  constexpr int QPH = HD / 4;
+  constexpr int SLICES = kWideReduceThreads / QPH;
+  __shared__ __attribute__((aligned(16))) float s_acc[SLICES][HD];
+  __shared__ float2 s_ml[SLICES];
+  const int slice = threadIdx.x / QPH;
+  const int d = (threadIdx.x - slice * QPH) * 4;
+  const int seq = blockIdx.y;
+  const int head = blockIdx.x;
+  const int kvh = head / p.group;
+  const int in_group = head - kvh * p.group;
+  const int sub = p.cohort_size > 1 ? 0 : in_group / p.gt;
+  const PartialList pl = partial_list(p, seq, kvh * p.nsub + sub);
+  const int g = head - pl.head0;
+  T *orow = reinterpret_cast<T *>(p.out) + seq * p.out_stride_seq + (int64_t)head * HD;
+  if (pl.n_tiles == 0) {
+    for (int o = threadIdx.x; o < HD; o += kWideReduceThreads) orow[o] = E::narrow(0.f);
+    return;
+  }
+  if (pl.n0 == 0 && pl.n_all == 1) return;
+  Merged r;
+  r.add_all<HD>(p, pl, slice, SLICES, g, d);
+  *reinterpret_cast<float4 *>(&s_acc[slice][d]) = r.a;
+  if (d == 0) s_ml[slice] = make_float2(r.m, r.l);
+  __syncthreads();
+  if (slice != 0) return;
+#pragma unroll
+  for (int k = 1; k < SLICES; ++k)
+    r.add(s_ml[k].x, s_ml[k].y, *reinterpret_cast<const float4 *>(&s_acc[k][d]));
+  r.write<E>(orow + d);
 }
 
 // Waves of the main kernel that one GPU holds at once, per kernel variant.
@@ -446,6 +531,13 @@ int resident_workgroups() {
 
 template <class E, int HD>
 int launch_reduce(const DecodeKP &kp, hipStream_t stream) {
+  // Partials of a pair, when the rows are equally long: its share of the waves, one tile each at least.
+  const int64_t shares = kp.n_waves / ((int64_t)kp.n_seqs * kp.pairs_per_seq);
+  if ((shares < kp.max_ctx / 16 ? shares : kp.max_ctx / 16) >= kWideReducePartials) {
+    hipLaunchKernelGGL((paged_decode_wide_reduce_kernel<E, HD>), dim3(kp.hn, kp.n_seqs), dim3(kWideReduceThreads), 0,
+                       stream, kp);
+    return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
+  }
   const int width = kp.gt * (HD / 4) < kReduceThreads ? kp.gt * (HD / 4) : kReduceThreads;
   const int per_wg = kReduceThreads / width;  // pairs per workgroup, as the kernel derives it
   hipLaunchKernelGGL((paged_decode_reduce_kernel<E, HD>), dim3((kp.pairs_per_seq + per_wg - 1) / per_wg, kp.n_seqs),
