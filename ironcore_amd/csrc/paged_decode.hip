@@ -316,14 +316,10 @@ struct PartialList {
   int heads, head0;  // query heads of the pair
   int n_tiles;       // tiles behind the row (0: no visible token)
   int64_t n0, n_all;  // partials of source 0 (the cohort's row), of both
-  int64_t w_lo[2], slot0[2], mul[2], add[2];
-  int col0[2];
-  // Slot of partial i, column g: share w of a source left it in slot (w + slot0) * mul + add,
-  // column col0 + g.
-  __device__ __forceinline__ int64_t slot(int64_t i, int g, int cols) const {
-    const int src = i < n0 ? 0 : 1;
-    const int64_t w = src == 0 ? w_lo[0] + i : w_lo[1] + (i - n0);
-    return ((w + slot0[src]) * mul[src] + add[src]) * cols + col0[src] + g;
+  int64_t base0, base1, stride0, stride1;  // slot of a source's first partial (column 0 of the pair), and between two
+  // Slot of partial i, column g.
+  __device__ __forceinline__ int64_t slot(int64_t i, int g) const {
+    return g + (i < n0 ? base0 + i * stride0 : base1 + (i - n0) * stride1);
   }
 };
 
@@ -356,30 +352,30 @@ __device__ __forceinline__ PartialList partial_list(const DecodeKP &p, int seq, 
   }
   r.n_tiles = nb_own + nb_sh;
   // source 0: the cohort's row of the shared phase, source 1: the sequence's
-  // own row; an empty source gets an empty share range
-  int64_t n[2];
-  {
+  // own row; an empty source has no partials.  Share w of a source left its
+  // partial in slot (w + row and pair) of the own phase, resp. in the slots of
+  // its unit's waves from shared_slot0 on.
+  r.n0 = 0;
+  r.base0 = r.stride0 = 0;
+  if (nb_sh > 0) {
     const int64_t chunk = chunk_tiles(p, (int64_t)cum_sh_all * p.pairs_per_seq, phase_units(p, 1));
     const int64_t first = (int64_t)cum_sh * p.pairs_per_seq + (int64_t)pair_in_seq * nb_sh;
-    r.w_lo[0] = first / chunk;
-    n[0] = nb_sh > 0 ? (first + nb_sh - 1) / chunk - r.w_lo[0] + 1 : 0;
-    r.slot0[0] = (int64_t)cohort * p.pairs_per_seq + pair_in_seq;
-    r.mul[0] = (int64_t)1 << p.unit_shift;
-    r.add[0] = p.shared_slot0 + wave_sh;
-    r.col0[0] = col_sh;
+    const int64_t w_lo = first / chunk;
+    r.n0 = (first + nb_sh - 1) / chunk - w_lo + 1;
+    const int64_t unit_slot = w_lo + (int64_t)cohort * p.pairs_per_seq + pair_in_seq;
+    r.base0 = (p.shared_slot0 + (unit_slot << p.unit_shift) + wave_sh) * COLS + col_sh;
+    r.stride0 = (int64_t)COLS << p.unit_shift;
   }
-  {
+  r.n_all = r.n0;
+  r.base1 = 0;
+  r.stride1 = COLS;
+  if (nb_own > 0) {
     const int64_t chunk = chunk_tiles(p, (int64_t)cum_all * p.pairs_per_seq, phase_units(p, 0));
     const int64_t first = (int64_t)cum_own * p.pairs_per_seq + (int64_t)pair_in_seq * nb_own;
-    r.w_lo[1] = first / chunk;
-    n[1] = nb_own > 0 ? (first + nb_own - 1) / chunk - r.w_lo[1] + 1 : 0;
-    r.slot0[1] = (int64_t)seq * p.pairs_per_seq + pair_in_seq;
-    r.mul[1] = 1;
-    r.add[1] = 0;
-    r.col0[1] = 0;
+    const int64_t w_lo = first / chunk;
+    r.n_all += (first + nb_own - 1) / chunk - w_lo + 1;
+    r.base1 = (w_lo + (int64_t)seq * p.pairs_per_seq + pair_in_seq) * COLS;
   }
-  r.n0 = n[0];
-  r.n_all = n[0] + n[1];
   return r;
 }
 
@@ -411,7 +407,7 @@ struct Merged {
 #pragma unroll
       for (int u = 0; u < UB; ++u) {
         const int64_t i = ib + u * step < pl.n_all ? ib + u * step : pl.n_all - 1;
-        const int64_t slot = pl.slot(i, g, p.gt);
+        const int64_t slot = pl.slot(i, g);
         ml[u] = *reinterpret_cast<const float2 *>(p.part_ml + slot * 2);
         av[u] = *reinterpret_cast<const float4 *>(p.part_acc + slot * HD + d);
       }
