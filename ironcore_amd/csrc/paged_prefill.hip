@@ -56,38 +56,8 @@ using namespace prefill;
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
-typedef __attribute__((ext_vector_type(4))) short s16x4_t;
-typedef __attribute__((ext_vector_type(8))) short s16x8_t;
-
-
-// MFMA wrappers per element type: operands are 8 packed 16-bit values.
-struct MmaBf16 {
-  using T = __bf16;
-  static __device__ __forceinline__ f32x16_t mma(const Vec16 &a, const Vec16 &b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    return __builtin_bit_cast(uint32_t, v);
-  }
-};
-struct MmaF16 {
-  using T = _Float16;
-  static __device__ __forceinline__ f32x16_t mma(const Vec16 &a, const Vec16 &b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    f16x2_t v = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
-    return __builtin_bit_cast(uint32_t, v);
-  }
-};
-
 constexpr int kPrefillWaves = 8;
 constexpr int kPrefillThreads = kPrefillWaves * kWave;
-constexpr int kXcds = 8;
 constexpr int kBN = 64;                   // tokens per K/V tile
 constexpr int kBM = kPrefillWaves * 32;   // query rows per workgroup
 constexpr int kStageBuffers = 4;          // LDS buffers per pool: a tile is fetched three tiles ahead
@@ -119,8 +89,8 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   // resp. 4 * ((r / 2) % 2); none at head dim 32, where a row is one 64-byte group.
   __shared__ __attribute__((aligned(1024))) char s_k[NB][kBN * ROWB];
   __shared__ __attribute__((aligned(1024))) char s_v[NB][kBN * ROWB];
-  auto swz_k = [](int r) { return CPR == 16 ? (r & 15) : CPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); };
-  auto swz_v = [](int r) { return CPR == 16 ? ((r & 3) << 2) : CPR == 8 ? (((r >> 1) & 1) << 2) : 0; };
+  auto swz_k = [](int r) { return tile_swizzle_k<CPR>(r); };
+  auto swz_v = [](int r) { return tile_swizzle_v<CPR>(r); };
 
   // XCD-aware placement.  Workgroups are dealt to the 8 XCDs round-robin by
   // their linear id, and each XCD has its own L2.  All workgroups that read
@@ -136,35 +106,11 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   // Longest first: workgroups are dispatched in id order and differ in length
   // by the spread of context lengths (and, under the causal mask, by their
   // query tile), so early ids take the longest sequences and the last query
-  // tiles.  Sequences are ranked by context length on the fly (up to one per
-  // lane).
-  int seq = unit / p.gn;
-  const int kvh = unit - seq * p.gn;
-  const int n_seqs = p.n_units / p.gn;
-  int q_lo, L, C;
-  if (n_seqs <= kWave) {
-    // (the chunk bounds travel with the context lengths, one sequence per lane: the chosen
-    // sequence's come from its lane instead of a second round trip to memory)
-    const int ln = threadIdx.x & (kWave - 1);
-    const int mine = ln < n_seqs ? p.context_lens[ln] : -0x7fffffff;
-    const int lo_mine = ln < n_seqs ? p.cu_seqlens_q[ln] : 0;
-    const int hi_mine = ln < n_seqs ? p.cu_seqlens_q[ln + 1] : 0;
-    int rank = 0;
-    for (int j = 0; j < n_seqs; ++j) {
-      const int other = __builtin_amdgcn_readlane(mine, j);
-      rank += (other > mine || (other == mine && j < ln)) ? 1 : 0;
-    }
-    const uint64_t hit = __ballot(rank == seq && ln < n_seqs);
-    seq = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(hit | (1ull << 63)));
-    seq = seq < n_seqs ? seq : n_seqs - 1;
-    q_lo = __builtin_amdgcn_readlane(lo_mine, seq);
-    L = __builtin_amdgcn_readlane(mine, seq);
-    C = __builtin_amdgcn_readlane(hi_mine, seq) - q_lo;
-  } else {
-    q_lo = p.cu_seqlens_q[seq];
-    L = p.context_lens[seq];
-    C = p.cu_seqlens_q[seq + 1] - q_lo;
-  }
+  // tiles.
+  const int rank = unit / p.gn;
+  const int kvh = unit - rank * p.gn;
+  int seq, q_lo, L, C;
+  pick_sequence(p, rank, seq, q_lo, L, C);
   const int h = kvh * p.group + r / p.n_qtiles;
   const int q0 = (p.n_qtiles - 1 - r % p.n_qtiles) * kBM;
   const bool causal = !MASK && p.causal;
@@ -603,9 +549,11 @@ template <class M>
 int launch_mode(const PrefillKP &kp, const PrefillArgs &a, hipStream_t stream) {
   // A one-column block table means one block per sequence, of any length.
   const bool masked = a.mask != nullptr;
+  if (a.block_table_stride == 1 && !masked && prefill_takes_short(a)) return launch_paged_prefill_short(kp, a, stream);
   if (a.block_table_stride == 1)
     return masked ? launch_hd<M, true, true>(kp, a, stream) : launch_hd<M, true, false>(kp, a, stream);
   if (kp.block_size < 16 || kp.block_size % 16 != 0) return IC_ERR_UNSUPPORTED;  // whole 16-token groups
+  if (!masked && prefill_takes_short(a)) return launch_paged_prefill_short(kp, a, stream);
   return masked ? launch_hd<M, false, true>(kp, a, stream) : launch_hd<M, false, false>(kp, a, stream);
 }
 

@@ -1,0 +1,468 @@
+// Chunked prefill for 16-bit pools, the kernel for short work: chunks of a few
+// rows to a few hundred, and batches too small to fill the GPU with the
+// 256-row workgroups of paged_prefill.hip.
+//
+// Same contract and the same arithmetic per tile (K/V tiles of 64 tokens
+// straight into swizzled LDS, S^T = K Q^T and O^T += V^T P^T on
+// v_mfma_f32_32x32x16, lazy reference maximum).  What differs is the shape:
+//
+//  * A workgroup is 4 waves, each owning a WAVE BLOCK of 32 query rows of one
+//    head.  The blocks of a KV head's G query heads are numbered through
+//    (ceil(C / 32) per head), and a workgroup takes four neighbouring ones, so
+//    short chunks of several heads share a workgroup and its K/V tiles: 13 rows
+//    x 7 heads are two workgroups, not seven with 5 % of their rows in use.
+//  * Every wave stages a 16-row group of K AND of V of each tile, into two
+//    buffers (a third gained nothing); one barrier per tile.  64 KiB of LDS at head dim 128, 32 KiB at 64:
+//    two, resp. four, workgroups share a CU, and what the two-sided schedule of
+//    the long kernel arranges inside a workgroup (matrix work beside vector
+//    work, loads behind both) comes here from neighbours that are at other
+//    points of their sweeps, start and end included, which is most of a short
+//    sweep's life.
+//  * Grids that leave one workgroup to a CU run it with two groups of four waves
+//    (TG = 2) on the same query rows, which take the tiles in turn and merge
+//    their sums through LDS at the end: half the tiles one after the other.
+//
+// Bound by the latency of a tile (load, two products and a softmax in one wave's
+// instruction stream, about 1 us at head dim 128) at the sizes it is for; 80
+// sequences of 129 tokens, 12 heads of 64, without a cache: 24.1 -> 19.8 us; 9
+// prompts of 3-701 tokens, 28 / 4 heads of 128: 32.0 -> 24.3 us; 67 of 18 tokens,
+// 32 / 8 heads of 128: 41.1 -> 12.5 us (the long kernel -> this one).
+#include "prefill_common.h"
+#include "../../include/ironcore_paged.h"
+
+namespace ic {
+namespace prefill {
+
+namespace {
+
+constexpr int kShortWaves = 4;  // wave blocks per workgroup
+constexpr int kBN = 64;         // tokens per K/V tile
+
+constexpr int kShortBuffers = 2;  // LDS buffers per pool and tile group
+
+template <class M, int HD, bool SINGLE, int TG>
+__global__ __launch_bounds__(TG *kShortWaves *kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 2 : 4)))
+void paged_prefill_short_kernel(const PrefillKP p) {
+  using T = typename M::T;
+  constexpr int KS = HD / 16;      // k-steps of the QK contraction
+  constexpr int OB = HD / 32;      // 32-wide blocks of the output head dim
+  constexpr int TB = kBN / 32;     // 32-token blocks per tile
+  constexpr int CPR = HD / 8;      // 16-byte chunks per token row
+  constexpr int WR = kWave / CPR;  // token rows one load instruction of a wave covers
+  constexpr int NST = 16 / WR;     // loads per lane, pool and staged tile
+  constexpr int ROWB = HD * 2;
+
+  constexpr int NB = kShortBuffers;
+  constexpr int TILEB = kBN * ROWB;  // bytes of a tile in one pool
+
+  // [tile group][pool][buffer][tile]; after the sweep the second group hands its sums over in it
+  constexpr int kMergeBytes = TG > 1 ? kShortWaves * (OB * 16 + 2) * kWave * 4 : 0;
+  constexpr int kTileBytes = TG * 2 * NB * TILEB;
+  __shared__ __attribute__((aligned(1024))) char s_tiles[kTileBytes > kMergeBytes ? kTileBytes : kMergeBytes];
+
+  // XCD-aware placement as in the long kernel: the workgroups of one (sequence, KV head) unit get ids
+  // that differ by a multiple of 8.
+  const int per_unit = p.n_qtiles;  // workgroups per unit
+  const int slice = blockIdx.x / (kXcds * per_unit);
+  const int within = blockIdx.x - slice * (kXcds * per_unit);
+  const int unit = slice * kXcds + (within % kXcds);
+  if (unit >= p.n_units) return;
+  const int rank = unit / p.gn;
+  const int kvh = unit - rank * p.gn;
+  int seq, q_lo, L, C;
+  pick_sequence(p, rank, seq, q_lo, L, C);
+  const bool causal = p.causal;
+  if (L < 0) L = 0;
+  if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
+  const int n_blocks = (C + 31) >> 5;  // wave blocks per head
+  const int total = n_blocks * p.group;
+  // The last blocks (the longest sweeps) first; in the slices that share the CUs with the first ones when
+  // the whole grid is resident, last: a CU then holds a long and a short sweep, not two of the same length.
+  const int r = within / kXcds;
+  const int v0 = (slice < p.flip_slice ? per_unit - 1 - r : r) * kShortWaves;
+  if (v0 >= total) return;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((tid / kWave) % kShortWaves);
+  const int tg = TG > 1 ? __builtin_amdgcn_readfirstlane(tid / kWave / kShortWaves) : 0;  // tile group
+  char *const tiles_k = s_tiles + tg * 2 * NB * TILEB;
+  char *const tiles_v = tiles_k + NB * TILEB;
+  const int n = lane & 31;  // query column of this lane within the wave's 32-row block
+  const int hh = lane >> 5;  // which half of each k-step this lane feeds
+  const bool mine = v0 + wave < total;
+  const int v = mine ? v0 + wave : total - 1;
+  const int head = v / n_blocks;
+  const int row0 = (v - head * n_blocks) * 32;
+  const int h = kvh * p.group + head;
+  const int my_q = row0 + n;
+  if (L == 0) {  // query rows without any key (not under the causal rule): zero rows
+    if (mine && tg == 0 && my_q < C)
+#pragma unroll
+      for (int c = 0; c < HD / 16; ++c)
+        store16(p.out + ((q_lo + my_q) * p.out_stride_token + (int64_t)h * HD + (hh * (HD / 16) + c) * 8) * 2,
+                Vec16{{0u, 0u, 0u, 0u}});
+    return;
+  }
+  const int P = L - C;  // cached prefix (causal rule only)
+
+  const int qrow = my_q < C ? my_q : C - 1;
+  const int limit = causal ? P + qrow : L - 1;  // last key this query row may see
+  Vec16 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qf[ks] = load16(p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+
+  f32x16_t o[OB];
+  float m = kNegInf, l = 0.f;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[ob][i] = 0.f;
+
+  // tiles this wave's rows reach, and the most that any wave of the workgroup does: a workgroup whose
+  // blocks span two heads holds a head's last block
+  const int v_last = v0 + kShortWaves < total ? v0 + kShortWaves - 1 : total - 1;
+  const int last_row = v0 / n_blocks == v_last / n_blocks ? (v_last % n_blocks) * 32 + 32 : C;
+  int kv_end = causal ? P + last_row : L;
+  kv_end = kv_end < L ? kv_end : L;
+  const int n_tiles = __builtin_amdgcn_readfirstlane((kv_end + kBN - 1) / kBN);
+  int my_end = causal ? P + row0 + 32 : L;
+  my_end = my_end < kv_end ? my_end : kv_end;
+  const int my_tiles = mine ? (my_end + kBN - 1) / kBN : 0;
+
+  // ---- tile staging: memory -> LDS (see the long kernel: one table entry and one base address per
+  // 16-row group, fixed lane offsets, unconditional loads) -----------------------------------------
+  const int cc = lane % CPR;    // LDS slot (16-byte chunk of the row) this lane fills
+  const int rsub = lane / CPR;  // row within the rows one load covers
+  const int64_t head_bytes = (int64_t)kvh * p.stride_head * 2;
+  const uint32_t block_bytes = (uint32_t)(p.stride_block * 2);
+  const uint32_t token_bytes = (uint32_t)(p.stride_token * 2);
+  const int last_phys = (int)p.num_blocks - 1;
+  auto block_of = [&](int row) { return (int)__umulhi((uint32_t)row, p.block_magic); };
+  const int last_blk = SINGLE ? 0 : block_of(L - 1);
+  typedef const __attribute__((address_space(4))) int32_t *TablePtr;  // scalar (SMEM) loads
+  const TablePtr table_row = (TablePtr)(unsigned long long)(p.block_tables + (int64_t)seq * p.bt_stride);
+  uint32_t src_k[NST], src_v[NST];  // byte offset from the group's first row, less the load's instruction offset
+#pragma unroll
+  for (int i = 0; i < NST; ++i) {
+    const int r = i * WR + rsub;
+    src_k[i] = (uint32_t)((int64_t)r * p.stride_token * 2 + (cc ^ tile_swizzle_k<CPR>(r)) * 16) - i * WR * ROWB;
+    src_v[i] = (uint32_t)((int64_t)r * p.stride_token * 2 + (cc ^ tile_swizzle_v<CPR>(r)) * 16) - i * WR * ROWB;
+  }
+  const uint32_t lds_k = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)&s_tiles[0] + (uint32_t)(tg * 2 * NB * TILEB);
+  auto clamp_tile = [&](int tile) { return tile < n_tiles ? tile : n_tiles - 1; };
+  auto lookup = [&](int tile, int32_t &ent, int &rem) {
+    const int first = clamp_tile(tile) * kBN + 16 * wave;
+    int blk = SINGLE ? 0 : block_of(first);
+    rem = first - blk * p.block_size;
+    blk = blk < last_blk ? blk : last_blk;
+    ent = table_row[blk];
+  };
+  auto fetch = [&](int tile, int buf, int32_t ent, int rem) {
+    int phys = ent;
+    // A corrupt table entry must not become an out-of-pool address.
+    phys = phys < 0 ? 0 : phys;
+    phys = phys > last_phys ? last_phys : phys;
+    const uint32_t to = __builtin_amdgcn_readfirstlane(lds_k + (uint32_t)(buf * TILEB + 16 * wave * ROWB));
+    const uint64_t block = head_bytes + (uint64_t)(uint32_t)phys * block_bytes;
+    if (SINGLE) {
+      const int first = clamp_tile(tile) * kBN + 16 * wave;
+#pragma unroll
+      for (int pool = 0; pool < 2; ++pool) {
+        const char *base = (pool ? p.v_pool : p.k_pool) + block;
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+          const int r = i * WR + rsub;
+          int row = first + r;
+          row = row < L ? row : L - 1;
+          const int chunk = cc ^ (pool ? tile_swizzle_v<CPR>(r) : tile_swizzle_k<CPR>(r));
+          const char *src = base + (int64_t)row * p.stride_token * 2 + chunk * 16;
+          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                       :: "s"(to + pool * NB * TILEB + i * WR * ROWB), "v"(src) : "memory", "m0");
+        }
+      }
+    } else {
+      const uint64_t group = block + (uint32_t)rem * token_bytes;
+#pragma unroll
+      for (int pool = 0; pool < 2; ++pool) {
+        const char *base = (pool ? p.v_pool : p.k_pool) + group;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" :: "s"(to + pool * NB * TILEB) : "memory", "m0");
+#pragma unroll
+        for (int i = 0; i < NST; ++i)
+          asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2"
+                       :: "v"(pool ? src_v[i] : src_k[i]), "s"(base), "n"(i * WR * ROWB) : "memory", "m0");
+      }
+    }
+  };
+
+  // per-lane LDS offsets of the operand reads (the swizzles seen from the reading side)
+  const int k_lane = n * ROWB + ((hh ^ tile_swizzle_k<CPR>(n)) << 4);
+  const int vq = (lane & 15) >> 2;
+  const int v_lane = (4 * hh + vq) * ROWB + ((tile_swizzle_v<CPR>(vq) >> 2) << 6) + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+  const int mask_from = __builtin_amdgcn_readfirstlane(causal ? (P + row0 + 1) / kBN : L / kBN);
+
+  f32x16_t s[TB];      // S^T of the tile: (token, query n)
+  Vec16 pb[kBN / 16];  // its probabilities as MFMA B operands
+  auto scores = [&](int buf) {
+    const char *sk = tiles_k + buf * TILEB;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[tb][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) {
+        const Vec16 a = load16(sk + (k_lane ^ (ks * 32)) + tb * 32 * ROWB);
+        s[tb] = M::mma(a, qf[ks], s[tb]);
+      }
+    }
+    // operand reads run ahead of the MFMAs that use them (see the long kernel)
+    constexpr int kAhead = TB * KS < 6 ? TB * KS : 6;
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+#pragma unroll
+    for (int i = 0; i < TB * KS - kAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
+  };
+  auto softmax = [&](int tile) {
+    // s[tb][i] is (token tile*64 + tb*32 + 4*hh + 8*(i/4) + i%4, query n)
+    const int tok_base = tile * kBN + 4 * hh;
+    if (tile >= mask_from) {  // tiles that touch the causal diagonal (or the context end)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int tok = tok_base + tb * 32 + 8 * (i / 4) + (i & 3);
+          s[tb][i] = tok > limit ? kNegInf : s[tb][i];
+        }
+    }
+    float mx = kNegInf;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[tb][i]);
+    float mx_a, mx_b;
+    both_halves(mx, mx_a, mx_b);
+    mx = fmaxf(mx_a, mx_b) * p.scale_log2e;
+    if (__any(mx > m + kLazySlack)) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = (m == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[ob][i] *= alpha;
+    }
+    const float neg_ms = (m == kNegInf) ? 0.f : -m;
+    float ps = 0.f;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tb][i], p.scale_log2e, neg_ms));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tb][i + 1], p.scale_log2e, neg_ms));
+        ps += p0 + p1;
+        pb[2 * tb + i / 8].w[(i & 7) / 2] = M::pack2(p0, p1);
+      }
+    }
+    l += ps;
+  };
+  auto weighted_values = [&](int buf) {
+    const char *sv = tiles_v + buf * TILEB;
+#pragma unroll
+    for (int kk = 0; kk < kBN / 16; ++kk) {
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob) {
+        const char *at = sv + (v_lane ^ (ob * 64)) + kk * 16 * ROWB;
+        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t *)(at));
+        const s16x4_t hi =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t *)(at + 8 * ROWB));
+        const s16x8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[ob] = M::mma(__builtin_bit_cast(Vec16, both), pb[kk], o[ob]);
+      }
+    }
+    constexpr int kAheadV = 4;
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAheadV, 0);
+#pragma unroll
+    for (int i = 0; i < OB * (kBN / 16) - kAheadV; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAheadV, 0);
+  };
+
+  // ---- sweep: round i is this group's tile i * TG + tg, computed while the next NB - 1 are on their way ----
+  int32_t ent;
+  int rem;
+  const int rounds = (n_tiles + TG - 1) / TG;
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i) {
+    lookup(i * TG + tg, ent, rem);
+    fetch(i * TG + tg, i, ent, rem);
+  }
+  lookup((NB - 1) * TG + tg, ent, rem);
+  int buf = 0;
+  for (int i = 0; i < rounds; ++i) {
+    const int k = i * TG + tg;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * 2 * NST) : "memory");  // this wave's groups of tile k
+    // rows of a V tile past the context become zeros: their probabilities are zeros, but 0 x NaN is not,
+    // and unused pool slots may hold anything (only a sweep's last tile can reach past the context)
+    if (k == n_tiles - 1 && k * kBN + 16 * wave + 16 > L) {
+      char *at = tiles_v + buf * TILEB + 16 * wave * ROWB + lane * 16;
+      const int row = k * kBN + 16 * wave + rsub;
+#pragma unroll
+      for (int j = 0; j < NST; ++j)
+        if (row + j * WR >= L) store16(at + j * WR * ROWB, Vec16{{0u, 0u, 0u, 0u}});
+    }
+    __syncthreads();  // the round's tiles are whole, and nobody reads the buffer of the round before any more
+    // (unconditional, so that the wait above is exact: past the sweep the last tile is fetched again)
+    fetch(k + (NB - 1) * TG, buf == 0 ? NB - 1 : buf - 1, ent, rem);
+    lookup(k + NB * TG, ent, rem);
+    if (k < my_tiles) {
+      scores(buf);
+      softmax(k);
+      weighted_values(buf);
+    }
+    buf = buf + 1 < NB ? buf + 1 : 0;
+  }
+  // every load this wave issued must have landed before its LDS is given up
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  // ---- the second group's sums -----------------------------------------------------------
+  if constexpr (TG > 1) {
+    static_assert(TG == 2, "one hand-over");
+    float *slab = reinterpret_cast<float *>(s_tiles) + wave * (OB * 16 + 2) * kWave + lane;
+    __syncthreads();
+    if (tg == 1) {
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) slab[(ob * 16 + i) * kWave] = o[ob][i];
+      slab[OB * 16 * kWave] = m;
+      slab[(OB * 16 + 1) * kWave] = l;
+    }
+    __syncthreads();
+    if (tg == 1) return;
+    const float m1 = slab[OB * 16 * kWave], l1 = slab[(OB * 16 + 1) * kWave];
+    const float m_new = fmaxf(m, m1);
+    const float w0 = m == kNegInf ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+    const float w1 = m1 == kNegInf ? 0.f : __builtin_amdgcn_exp2f(m1 - m_new);
+    l = l * w0 + l1 * w1;
+#pragma unroll
+    for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[ob][i] = o[ob][i] * w0 + slab[(ob * 16 + i) * kWave] * w1;
+  }
+
+  // ---- normalise and store -------------------------------------------------------
+  float l_a, l_b;
+  both_halves(l, l_a, l_b);
+  const float lt = l_a + l_b;
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if (mine && my_q < C) {
+    T *orow = reinterpret_cast<T *>(p.out) + (q_lo + my_q) * p.out_stride_token + (int64_t)h * HD;
+#pragma unroll
+    for (int ob = 0; ob < OB; ++ob) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d = ob * 32 + 4 * hh + 8 * j;
+        uint2 w;
+        w.x = M::pack2(o[ob][4 * j] * inv, o[ob][4 * j + 1] * inv);
+        w.y = M::pack2(o[ob][4 * j + 2] * inv, o[ob][4 * j + 3] * inv);
+        *reinterpret_cast<uint2 *>(orow + d) = w;
+      }
+    }
+  }
+}
+
+template <class M, bool SINGLE, int TG>
+int launch_short_hd(const PrefillKP &kp, int hd, unsigned wgs, hipStream_t stream) {
+  const dim3 grid(wgs), block(TG * kShortWaves * kWave);
+  switch (hd) {
+    case 32:
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 32, SINGLE, TG>), grid, block, 0, stream, kp);
+      break;
+    case 64:
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 64, SINGLE, TG>), grid, block, 0, stream, kp);
+      break;
+    case 128:
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 128, SINGLE, TG>), grid, block, 0, stream, kp);
+      break;
+    default:
+      return IC_ERR_UNSUPPORTED;
+  }
+  return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
+}
+
+template <class M>
+int launch_short_type(const PrefillKP &kp, const PrefillArgs &a, unsigned wgs, bool split, hipStream_t stream) {
+  const bool single = a.block_table_stride == 1;
+  if (split)
+    return single ? launch_short_hd<M, true, 2>(kp, a.hd, wgs, stream) : launch_short_hd<M, false, 2>(kp, a.hd, wgs, stream);
+  return single ? launch_short_hd<M, true, 1>(kp, a.hd, wgs, stream) : launch_short_hd<M, false, 1>(kp, a.hd, wgs, stream);
+}
+
+}  // namespace
+
+// Which kernel a 16-bit call without a mask takes.  The host knows the longest chunk and, from the
+// block table, a bound on the contexts.  Times in us, 16 sequences, 32 query heads, head dim 128, this
+// kernel / the long one, by chunk length and cached prefix:
+//                     32 KV heads                            8 KV heads
+//   prefix      0       1 024     2 048      4 096       0      1 024     2 048      4 096
+//   chunk 128  18 / 25   70 / 79  119 / 130  220 / 228   15 / 22  46 / 63   78 / 99   160 / 182
+//         256  35 / 43  118 / 114 193 / 177  347 / 311   31 / 41  90 / 97  153 / 153  299 / 270
+//         384  52 / 71  168 / 178 270 / 290  484 / 507   49 / 66 136 / 161 226 / 251  432 / 450
+//         512  83 / 97  227 / 219 359 / 334  636 / 578   76 / 91 197 / 199 336 / 312  595 / 532
+//       1 024 239 / 268 485 / 485 740 / 710 1246 / 1165 217 / 265 450 / 477 698 / 689 1180 / 1118
+// The long kernel needs its 256 rows filled and long full sweeps (a prefix at least as long as the
+// chunk), where staging a tile once per 256 rows instead of 128 pays; sooner without grouped queries,
+// whose K/V the caches do not serve to several heads.  A grid that leaves the CUs one workgroup each is this
+// kernel's (with two tile groups, below: 2 sequences, chunks of 128 behind 4 096: 66 / 78 us, grouped 64 / 78)
+// unless it streams many ungrouped K/V rows, for which the long kernel keeps more bytes on their way (4
+// sequences behind 4 096 / 8 192: 84 / 81 and 164 / 149 us).  At head dim 64 and 32 (half the staged bytes per
+// row, four workgroups per CU) this one is within 4 % at worst (512 behind 4 096: 354 / 351) and up to a third
+// faster.
+namespace {
+int64_t short_workgroups_per_unit(const PrefillArgs &a) {
+  const int64_t blocks = (int64_t)((a.max_chunk_len + 31) / 32) * (a.hn / a.gn);
+  return (blocks + kShortWaves - 1) / kShortWaves;
+}
+int64_t context_bound(const PrefillArgs &a) { return a.block_table_stride * (int64_t)a.pool.block_size; }
+}  // namespace
+
+bool prefill_takes_short(const PrefillArgs &a) {
+  if (a.hd < 128) return true;
+  const int64_t ctx = context_bound(a);
+  const int64_t wgs = short_workgroups_per_unit(a) * a.n_seqs * a.gn;
+  if (wgs <= device_cu_count()) return a.hn > a.gn || wgs * ctx < 512 * 1024;
+  const int tiles = (a.max_chunk_len + 255) / 256;
+  const bool filled = (int64_t)a.max_chunk_len * 8 >= (int64_t)tiles * 256 * 7;
+  return !(filled && ctx >= 2 * (int64_t)a.max_chunk_len && ctx >= (a.hn > a.gn ? 2200 : 1250));
+}
+
+int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t stream) {
+  const int64_t per_unit = short_workgroups_per_unit(a);
+  const int64_t slices = (kp.n_units + kXcds - 1) / kXcds;
+  const int64_t wgs = slices * kXcds * per_unit;
+  if (wgs > 0x7fffffff) return IC_ERR_UNSUPPORTED;
+  kp.n_qtiles = (int)per_unit;
+  const int cus = device_cu_count();
+  kp.flip_slice = wgs > cus && wgs <= 2 * cus ? (int)(slices + 1) / 2 : 0x7fffffff;
+  // A grid that leaves the CUs one workgroup each: two groups of waves take the tiles in turn.  2 sequences,
+  // 32 heads of 128, chunks of 128 behind 512 / 1 024 / 4 096 cached tokens: 16.8 / 28.2 / 86.3 us with one
+  // group, 16.6 / 24.9 / 66.0 with two; behind nothing 7.8 / 10.0 (the hand-over), hence the second condition.
+  // At head dim 64 two such workgroups share a CU: 16 sequences, chunks of 128 behind 512 / 2 048 / 4 096:
+  // 22.6 / 69.6 / 137 with one group, 24.4 / 65.4 / 128 with two.
+  const int64_t ctx = context_bound(a);
+  const bool split = (wgs <= cus && ctx > 512) || (a.hd < 128 && wgs <= 2 * cus && ctx >= 2048);
+  return a.dtype == IC_DTYPE_BF16 ? launch_short_type<MmaBf16>(kp, a, (unsigned)wgs, split, stream)
+                                  : launch_short_type<MmaF16>(kp, a, (unsigned)wgs, split, stream);
+}
+
+}  // namespace prefill
+}  // namespace ic

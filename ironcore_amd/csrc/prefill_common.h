@@ -32,7 +32,8 @@ struct PrefillKP {
   int group;        // query heads per KV head
   int gn;           // KV heads
   int n_units;      // n_seqs * gn
-  int n_qtiles;     // query tiles per chunk (grid sizing)
+  int n_qtiles;     // query tiles per chunk (grid sizing); short kernel: workgroups per unit
+  int flip_slice;   // short kernel: first slice of units whose workgroups take their blocks shortest sweep first
   int causal;
   float scale_log2e;
   // General attention mask (MASK variant): byte (sequence i, head h, chunk row r, key j) at
@@ -66,8 +67,87 @@ __device__ __forceinline__ void both_halves(float x, float &a, float &b) {
   b = __builtin_bit_cast(float, r1);
 }
 
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+typedef __attribute__((ext_vector_type(8))) short s16x8_t;
+
+// MFMA wrappers per element type: operands are 8 packed 16-bit values.
+struct MmaBf16 {
+  using T = __bf16;
+  static __device__ __forceinline__ f32x16_t mma(const Vec16 &a, const Vec16 &b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+    return __builtin_bit_cast(uint32_t, v);
+  }
+};
+struct MmaF16 {
+  using T = _Float16;
+  static __device__ __forceinline__ f32x16_t mma(const Vec16 &a, const Vec16 &b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    f16x2_t v = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
+    return __builtin_bit_cast(uint32_t, v);
+  }
+};
+
+constexpr int kXcds = 8;
+
+// An LDS tile is unpadded [token][dim], CPR 16-byte chunks to a row, and chunk c
+// of row r lies in slot c ^ swizzle(r) of its row, so that the operand reads
+// stay free of bank conflicts: K is read as whole 16-byte chunks, 16 rows per
+// access, V by the transposing 8-byte reads, 4 rows x 64 bytes per access (one
+// 64-byte group is a whole row at head dim 32, which needs none).
+template <int CPR>
+__device__ __forceinline__ int tile_swizzle_k(int r) {
+  return CPR == 16 ? (r & 15) : CPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3);
+}
+template <int CPR>
+__device__ __forceinline__ int tile_swizzle_v(int r) {
+  return CPR == 16 ? ((r & 3) << 2) : CPR == 8 ? (((r >> 1) & 1) << 2) : 0;
+}
+
+// The sequence that is `rank`th by context length (longest first: workgroups
+// are dispatched in id order and should end together), its first query row,
+// context length and chunk length.  Up to one sequence per lane is ranked on
+// the fly; in longer batches rank r is simply sequence r.
+__device__ __forceinline__ void pick_sequence(const PrefillKP &p, int rank, int &seq, int &q_lo, int &L, int &C) {
+  seq = rank;
+  const int n_seqs = p.n_units / p.gn;
+  if (n_seqs <= kWave) {
+    // (the chunk bounds travel with the context lengths, one sequence per lane: the chosen
+    // sequence's come from its lane instead of a second round trip to memory)
+    const int ln = threadIdx.x & (kWave - 1);
+    const int mine = ln < n_seqs ? p.context_lens[ln] : -0x7fffffff;
+    const int lo_mine = ln < n_seqs ? p.cu_seqlens_q[ln] : 0;
+    const int hi_mine = ln < n_seqs ? p.cu_seqlens_q[ln + 1] : 0;
+    int above = 0;
+    for (int j = 0; j < n_seqs; ++j) {
+      const int other = __builtin_amdgcn_readlane(mine, j);
+      above += (other > mine || (other == mine && j < ln)) ? 1 : 0;
+    }
+    const uint64_t hit = __ballot(above == rank && ln < n_seqs);
+    seq = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(hit | (1ull << 63)));
+    seq = seq < n_seqs ? seq : n_seqs - 1;
+    q_lo = __builtin_amdgcn_readlane(lo_mine, seq);
+    L = __builtin_amdgcn_readlane(mine, seq);
+    C = __builtin_amdgcn_readlane(hi_mine, seq) - q_lo;
+  } else {
+    q_lo = p.cu_seqlens_q[seq];
+    L = p.context_lens[seq];
+    C = p.cu_seqlens_q[seq + 1] - q_lo;
+  }
+}
+
 constexpr float kLazySlack = 8.0f;  // log2 units
 
+// 16-bit pools, short work: the kernel of paged_prefill_short.hip, and whether a call is that.
+bool prefill_takes_short(const PrefillArgs &a);
+int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t stream);
 // fp32 pools: the kernel of paged_prefill_f32.hip (same parameters, same grid rules of its own).
 int launch_paged_prefill_f32(PrefillKP kp, const PrefillArgs &a, hipStream_t stream);
 
