@@ -7,12 +7,14 @@ missing every paged operation raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libironcore_paged.so"
+HOST_PATH = LIB_PATH.parent / "_host.so"
 
 IC_OK = 0
 IC_DTYPE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
@@ -130,6 +132,34 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native call path (csrc/host_binding.cpp): each of its functions does
+    the whole call for ordinary arguments, or returns None / False and leaves
+    them to the Python wrapper, which handles or refuses the rest."""
+    global _host
+    if _host is None:
+        if not HOST_PATH.exists():
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m ironcore_amd.build`")
+        load()
+        spec = importlib.util.spec_from_file_location("_host", HOST_PATH)
+        _host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_host)
+    return _host
+
+
+def here(t: torch.Tensor):
+    """(device index, stream) for a tensor on the current GPU, else None."""
+    if not t.is_cuda:
+        return None
+    device = t.get_device()
+    if device != torch._C._cuda_getDevice():
+        return None
+    return device, torch._C._cuda_getCurrentRawStream(device)
 
 
 def check(func: str, code: int) -> None:

@@ -3,7 +3,8 @@
     python -m ironcore_amd.build
 
 compiles every translation unit under ironcore_amd/csrc/ and links
-ironcore_amd/lib/libironcore_paged.so.  Cross-compiles without a GPU.
+ironcore_amd/lib/libironcore_paged.so, then the torch-side call path
+ironcore_amd/lib/_host.so.  Cross-compiles without a GPU.
 """
 from __future__ import annotations
 
@@ -18,6 +19,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB_DIR = PKG / "lib"
 LIB_PATH = LIB_DIR / "libironcore_paged.so"
+HOST_PATH = LIB_DIR / "_host.so"   # native call path (csrc/host_binding.cpp), links LIB_PATH
 OBJ_DIR = PKG / "build" / "obj"
 
 SOURCES = ["ic_api.hip", "kv_append.hip", "rope_kv_append.hip", "paged_decode.hip", "paged_decode_mfma.hip", "paged_prefill.hip",
@@ -81,13 +83,41 @@ def _compile(src: str, extra: list[str]) -> Path:
     return obj
 
 
+def _compile_host() -> Path:
+    """The torch-side call path: host code only, torch's headers, the system compiler."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    obj = OBJ_DIR / "host_binding.cpp.o"
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-DTORCH_EXTENSION_NAME=_host",
+           "-DTORCH_API_INCLUDE_EXTENSION_H", *(f"-I{p}" for p in includes), "-c", str(CSRC / "host_binding.cpp"),
+           "-o", str(obj)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on host_binding.cpp:\n{res.stdout}\n{res.stderr}")
+    return obj
+
+
+def _link_host(obj: Path) -> None:
+    from torch.utils import cpp_extension
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = ["g++", "-shared", str(obj), "-o", str(tmp), f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN",
+           *(f"-L{p}" for p in cpp_extension.library_paths()), "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = True, extra_flags: list[str] | None = None) -> Path:
     """Compile and link; returns the path of the shared library."""
     extra = list(extra_flags or [])
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as pool:
+        host = pool.submit(_compile_host)
         objs = list(pool.map(lambda s: _compile(s, extra), SOURCES))
+        host_obj = host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc",
            *map(str, objs), "-o", str(tmp)]
@@ -95,6 +125,7 @@ def build(verbose: bool = True, extra_flags: list[str] | None = None) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_host(host_obj)
     if verbose:
         print(f"built {LIB_PATH} ({LIB_PATH.stat().st_size} bytes)")
     return LIB_PATH

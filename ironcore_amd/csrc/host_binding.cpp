@@ -1,0 +1,187 @@
+// The call path of the attention layer and of the tensor-level wrappers, native:
+// shape checks, strides, output and workspace allocation and the C-ABI calls,
+// without the interpreter in between.  A cached decode step of a small model is
+// bound by this path (three launches of a few microseconds each behind 33 us of
+// Python on one core); the functions here leave 2-3 us of it.
+//
+// Each function handles the ordinary case completely, or does nothing and
+// returns None: the Python wrapper (paged_ops.py, layers/attention.py) then takes
+// its own path, which makes tensors contiguous, switches the device or names
+// what is wrong with the arguments.  Nothing is kept between calls: outputs and
+// workspaces come from torch's allocator, which orders their reuse on the stream
+// and serves a capturing stream from the graph's own pool.
+#include <torch/extension.h>
+
+#include "../../include/ironcore_paged.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = c10::optional<Tensor>;
+namespace py = pybind11;
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kBFloat16: return IC_DTYPE_BF16;
+    case at::kHalf: return IC_DTYPE_F16;
+    case at::kFloat: return IC_DTYPE_F32;
+    default: return -1;
+  }
+}
+
+bool on(const Tensor &t, int64_t device) { return t.is_cuda() && t.get_device() == device; }
+
+struct Pool {
+  int64_t nb, gn, bs, hd, sb, sh, st;
+  int dtype;
+  const void *k, *v;
+  bool ok = false;
+  Pool(const Tensor &kp, const Tensor &vp, int64_t device) {
+    if (kp.dim() != 4 || !on(kp, device) || !on(vp, device) || kp.scalar_type() != vp.scalar_type() ||
+        kp.sizes() != vp.sizes() || kp.strides() != vp.strides() || kp.stride(3) != 1)
+      return;
+    nb = kp.size(0), gn = kp.size(1), bs = kp.size(2), hd = kp.size(3);
+    sb = kp.stride(0), sh = kp.stride(1), st = kp.stride(2);
+    dtype = dtype_code(kp.scalar_type());
+    k = kp.data_ptr(), v = vp.data_ptr();
+    ok = dtype >= 0 && gn > 0;
+  }
+  bool attends() const { return hd == 32 || hd == 64 || hd == 128; }
+};
+
+bool index_vector(const Tensor &t, at::ScalarType type, int64_t n, int64_t device) {
+  return on(t, device) && t.scalar_type() == type && t.numel() == n && t.is_contiguous();
+}
+bool table(const Tensor &t, int64_t rows, int64_t device) {
+  return on(t, device) && t.scalar_type() == at::kInt && t.dim() == 2 && t.size(0) == rows && t.stride(1) == 1;
+}
+
+// [n, heads, hd] rows, heads contiguous within a row.
+bool rows3(const Tensor &t, int64_t heads, int64_t hd) {
+  return t.dim() == 3 && t.size(1) == heads && t.size(2) == hd && t.stride(2) == 1 && t.stride(1) == hd;
+}
+// [b, s, heads, hd] that is [b*s, heads, hd] rows at one stride.
+bool rows4(const Tensor &t, int64_t b, int64_t s, int64_t heads, int64_t hd) {
+  return t.dim() == 4 && t.size(0) == b && t.size(1) == s && t.size(2) == heads && t.size(3) == hd &&
+         t.stride(3) == 1 && t.stride(2) == hd && (b == 1 || t.stride(0) == s * t.stride(1));
+}
+int64_t row_stride4(const Tensor &t) { return t.size(1) > 1 ? t.stride(1) : t.stride(0); }
+
+bool append_rows(const void *k, const void *v, int64_t stride, const Pool &p, const Tensor &slots, int64_t n,
+                 void *stream) {
+  return ic_kv_append(k, v, stride, const_cast<void *>(p.k), const_cast<void *>(p.v), p.sb, p.sh, p.st,
+                      slots.data_ptr<int64_t>(), n, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream) == IC_OK;
+}
+
+struct Decode {
+  const Tensor &tables, &lens;
+  int64_t max_ctx, min_chunk, cohort;
+  const OptTensor &shared;
+  double scale;
+};
+
+bool decode_fits(const Pool &p, int64_t b, int64_t hn, const Decode &d, int64_t device) {
+  if (!p.attends() || hn % p.gn != 0 || b == 0 || !table(d.tables, b, device) ||
+      !index_vector(d.lens, at::kInt, b, device) || d.max_ctx > d.tables.size(1) * p.bs || d.cohort < 1)
+    return false;
+  return d.cohort == 1 ||
+         (d.shared.has_value() && index_vector(*d.shared, at::kInt, (b + d.cohort - 1) / d.cohort, device));
+}
+
+bool decode(const Tensor &out, const void *q, int64_t q_stride, const Pool &p, int64_t b, int64_t hn, const Decode &d,
+            void *stream) {
+  const size_t need = ic_paged_decode_shared_workspace_bytes((int)b, (int)hn, (int)p.gn, (int)p.hd, (int)d.cohort);
+  if (need == 0) return false;
+  const Tensor ws = at::empty({(int64_t)need}, out.options().dtype(at::kByte));
+  return ic_paged_decode_shared(out.data_ptr(), out.stride(0), q, q_stride, p.k, p.v, p.sb, p.sh, p.st,
+                                d.tables.data_ptr<int32_t>(), d.tables.stride(0), d.lens.data_ptr<int32_t>(), (int)b,
+                                (int)hn, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, (int)d.max_ctx, (float)d.scale,
+                                (int)d.min_chunk, (int)d.cohort,
+                                d.cohort > 1 ? d.shared->data_ptr<int32_t>() : nullptr, ws.data_ptr(), need, p.dtype,
+                                stream) == IC_OK;
+}
+
+// ---- tensor-level calls (paged_ops) ----------------------------------------------------------
+
+bool kv_append(const Tensor &k_new, const Tensor &v_new, const Tensor &k_pool, const Tensor &v_pool,
+               const Tensor &slots, int64_t device, int64_t stream) {
+  const Pool p(k_pool, v_pool, device);
+  if (!p.ok || !rows3(k_new, p.gn, p.hd) || !rows3(v_new, p.gn, p.hd) || k_new.size(0) != v_new.size(0) ||
+      k_new.stride(0) != v_new.stride(0) || k_new.scalar_type() != k_pool.scalar_type() ||
+      v_new.scalar_type() != k_pool.scalar_type() || !on(k_new, device) || !on(v_new, device) ||
+      !index_vector(slots, at::kLong, k_new.size(0), device))
+    return false;
+  return append_rows(k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), p, slots, k_new.size(0), (void *)stream);
+}
+
+OptTensor paged_decode(const Tensor &query, const Tensor &k_pool, const Tensor &v_pool, const Tensor &tables,
+                       const Tensor &lens, int64_t max_ctx, double scale, const OptTensor &out_given,
+                       int64_t min_chunk, int64_t cohort, const OptTensor &shared, int64_t device, int64_t stream) {
+  const Pool p(k_pool, v_pool, device);
+  if (!p.ok || query.dim() != 3 || !rows3(query, query.size(1), p.hd) || !on(query, device) ||
+      query.scalar_type() != k_pool.scalar_type())
+    return c10::nullopt;
+  const int64_t b = query.size(0), hn = query.size(1);
+  const Decode d{tables, lens, max_ctx, min_chunk, cohort, shared, scale};
+  if (!decode_fits(p, b, hn, d, device)) return c10::nullopt;
+  if (out_given.has_value() &&
+      (out_given->dim() != 2 || out_given->size(0) != b || out_given->size(1) != hn * p.hd ||
+       out_given->scalar_type() != query.scalar_type() || out_given->stride(1) != 1 || !on(*out_given, device)))
+    return c10::nullopt;
+  const Tensor out = out_given.has_value() ? *out_given : at::empty({b, hn * p.hd}, query.options());
+  if (!decode(out, query.data_ptr(), query.stride(0), p, b, hn, d, (void *)stream)) return c10::nullopt;
+  return out;
+}
+
+// ---- the layer -----------------------------------------------------------------------------
+
+// One cached decode step of a layer (sq == 1): append, then attend.  With rotary tables the query is
+// rotated into a tensor of its own and the keys on their way into the pool.
+OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
+                      const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
+                      int64_t max_ctx, double scale, int64_t cohort, const OptTensor &shared,
+                      const OptTensor &positions, const OptTensor &cos, const OptTensor &sin, int64_t device,
+                      int64_t stream) {
+  const Pool p(k_pool, v_pool, device);
+  if (!p.ok || query.dim() != 4) return c10::nullopt;
+  const int64_t b = query.size(0), hn = query.size(2);
+  const auto type = k_pool.scalar_type();
+  if (!rows4(query, b, 1, hn, p.hd) || !rows4(key, b, 1, p.gn, p.hd) || !rows4(value, b, 1, p.gn, p.hd) ||
+      row_stride4(key) != row_stride4(value) || query.scalar_type() != type || key.scalar_type() != type ||
+      value.scalar_type() != type || !on(query, device) || !on(key, device) || !on(value, device) ||
+      !index_vector(slots, at::kLong, b, device))
+    return c10::nullopt;
+  const Decode d{tables, lens, max_ctx, 0, cohort, shared, scale};
+  if (!decode_fits(p, b, hn, d, device)) return c10::nullopt;
+  const void *q = query.data_ptr();
+  int64_t q_stride = row_stride4(query);
+  Tensor rotated;
+  if (cos.has_value()) {
+    if (!positions.has_value() || !sin.has_value() || !index_vector(*positions, at::kInt, b, device) ||
+        cos->dim() != 2 || cos->size(1) != p.hd / 2 || cos->sizes() != sin->sizes() ||
+        !index_vector(*cos, at::kFloat, cos->numel(), device) || !index_vector(*sin, at::kFloat, cos->numel(), device))
+      return c10::nullopt;
+    rotated = query.clone(at::MemoryFormat::Contiguous);
+    q = rotated.data_ptr();
+    q_stride = hn * p.hd;
+    if (ic_rope_kv_append(rotated.data_ptr(), q_stride, (int)hn, key.data_ptr(), value.data_ptr(), row_stride4(key),
+                          const_cast<void *>(p.k), const_cast<void *>(p.v), p.sb, p.sh, p.st,
+                          slots.data_ptr<int64_t>(), positions->data_ptr<int32_t>(), cos->data_ptr<float>(),
+                          sin->data_ptr<float>(), cos->size(0), b, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype,
+                          (void *)stream) != IC_OK)
+      return c10::nullopt;
+  } else if (!append_rows(key.data_ptr(), value.data_ptr(), row_stride4(key), p, slots, b, (void *)stream)) {
+    return c10::nullopt;
+  }
+  const Tensor out = at::empty({b, 1, hn * p.hd}, query.options());
+  if (!decode(out, q, q_stride, p, b, hn, d, (void *)stream)) return c10::nullopt;
+  return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("kv_append", &kv_append);
+  m.def("paged_decode", &paged_decode);
+  m.def("decode_step", &decode_step);
+}

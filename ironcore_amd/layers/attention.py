@@ -37,7 +37,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from .. import paged_ops
+from .. import _lib, paged_ops
 from .module import BaseModule, get_model_dtype
 
 # The reference takes its flash branch only when this import worked
@@ -288,6 +288,18 @@ class Attention(BaseModule):
         if key.shape[1] != sq:
             raise ValueError("with a KV cache, key/value carry only the new tokens (sk == sq)")
         k_pool, v_pool = kv_cache
+        rows = getattr(meta, "chunk_rows", None)
+        here = _lib.here(query)
+        if here is not None and sq == 1 and rows is None:
+            rope = rotary_pos_emb
+            cohort = meta.cohort_size if query.dtype != torch.float32 else 1
+            out = _lib.host().decode_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
+                                          meta.slot_mapping, meta.max_context_len, 1.0 / self.scale_factor, cohort,
+                                          meta.cohort_shared_blocks if cohort > 1 else None, meta.positions,
+                                          None if rope is None else rope.cos_emb,
+                                          None if rope is None else rope.sin_emb, *here)
+            if out is not None:
+                return out
         if rotary_pos_emb is None:
             paged_ops.kv_append(key.reshape(b * sq, gn, hd), value.reshape(b * sq, gn, hd), k_pool, v_pool,
                                 meta.slot_mapping)
@@ -300,7 +312,6 @@ class Attention(BaseModule):
                                      rotary_pos_emb.cos_emb, rotary_pos_emb.sin_emb)
             query = rotated.view(b, sq, hn, hd)
         scale = 1.0 / self.scale_factor
-        rows = getattr(meta, "chunk_rows", None)
         if rows is not None:
             return self._ragged_chunks(query, k_pool, v_pool, meta, rows, scale)
         if sq == 1:

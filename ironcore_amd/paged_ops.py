@@ -87,6 +87,9 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_pool: torch.Tensor, v_
     """Copy rows ``k_new[t]``, ``v_new[t]`` (``[n, gn, hd]``) into pool slot
     ``slot_mapping[t]`` (= block*block_size + offset), bit for bit.  Negative
     slots are skipped."""
+    here = _lib.here(k_pool)
+    if here is not None and _lib.host().kv_append(k_new, v_new, k_pool, v_pool, slot_mapping, *here):
+        return
     lib = _lib.load()
     dev = _require_gpu(k_new, v_new, k_pool, v_pool, slot_mapping)
     nb, gn, bs, hd, sb, sh, st = _pool_strides(k_pool, v_pool)
@@ -188,6 +191,13 @@ def paged_decode(query: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor
     says how many leading block-table entries are the same pool block in all
     of its rows; those blocks are read once per cohort.  The result is the
     same as without cohorts."""
+    here = _lib.here(query)
+    if here is not None and key_mask is None:
+        got = _lib.host().paged_decode(query, k_pool, v_pool, block_tables, context_lens, int(max_context_len),
+                                       1.0 / math.sqrt(query.shape[-1]) if scale is None else scale, out,
+                                       min_chunk_tokens, int(cohort_size), cohort_shared_blocks, *here)
+        if got is not None:
+            return got
     lib = _lib.load()
     dev = _require_gpu(query, k_pool, v_pool, block_tables, context_lens)
     nb, gn, bs, hd, sb, sh, st = _pool_strides(k_pool, v_pool)

@@ -1,0 +1,83 @@
+"""The native call path (csrc/host_binding.cpp) against the Python one on the
+same arguments: same bits, and arguments that are not ordinary left to Python."""
+import pytest
+import torch
+
+from ironcore_amd import _lib, config as ic_config, paged_ops, workloads
+from ironcore_amd.layers import Attention, PagedAttentionMetadata, RotaryPositionalEmbedding
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(hn, gn, hd, precision):
+    return Attention(ic_config.MainConfig(
+        model=ic_config.ModelConfig(d_model=hn * hd, num_attention_heads=hn, num_attention_groups=gn, head_dim=hd,
+                                    dropout_attn=0.0, precision=precision),
+        trainer=ic_config.TrainerConfig(use_flash_attn=False))).eval()
+
+
+def _both(monkeypatch, call):
+    native = call()
+    monkeypatch.setattr(_lib, "here", lambda t: None)
+    plain = call()
+    monkeypatch.undo()
+    return native, plain
+
+
+@pytest.mark.parametrize("dtype,precision", [(torch.bfloat16, "bf16"), (torch.float32, "fp32")])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("strided", [False, True])
+def test_decode_step(gpu, monkeypatch, dtype, precision, rope, strided):
+    hn, gn, hd, b = 8, 2, 64, 5
+    wl = workloads.make_decode_workload(b, hn, gn, hd, 1, 300, dtype=dtype, seed=3).to(gpu)
+    last = wl.context_lens.long() - 1
+    slots = wl.block_tables.long().gather(1, (last // 16).unsqueeze(1)).squeeze(1) * 16 + last % 16
+    meta = PagedAttentionMetadata(block_tables=wl.block_tables, context_lens=wl.context_lens, slot_mapping=slots,
+                                  max_context_len=wl.max_context_len, positions=last.int())
+    g = torch.Generator(device=gpu).manual_seed(1)
+    kv = torch.randn(b, 1, 2 * gn * hd, generator=g, device=gpu).to(dtype)
+    key, value = (t.view(b, 1, gn, hd) for t in kv.chunk(2, dim=-1))     # as the model hands them over
+    query = torch.randn(b, 1, hn, hd, generator=g, device=gpu).to(dtype)
+    if strided:
+        query = torch.stack([query, query], dim=3)[..., 0, :]            # heads apart: Python makes it contiguous
+    emb = RotaryPositionalEmbedding(hd, max_seq_len=300).to(gpu) if rope else None
+    attn = _layer(hn, gn, hd, precision)
+    pools = [(wl.k_pool.clone(), wl.v_pool.clone()) for _ in range(2)]
+    left = list(pools)
+
+    def call():
+        return attn(query, key, value, kv_cache=left.pop(), attn_metadata=meta, rotary_pos_emb=emb)
+    native, plain = _both(monkeypatch, call)
+    assert native.shape == plain.shape == (b, 1, hn * hd) and torch.equal(native, plain)
+    assert torch.equal(pools[0][0], pools[1][0]) and torch.equal(pools[0][1], pools[1][1])
+
+
+def test_paged_decode_and_append(gpu, monkeypatch):
+    wl = workloads.make_grpo_workload(2, 4, 8, 2, 128, 64, 1, 90, seed=2).to(gpu)
+    shared = torch.full((2,), 4, dtype=torch.int32, device=gpu)
+    out = torch.empty(8, 8 * 128 + 64, dtype=torch.bfloat16, device=gpu)[:, :8 * 128]     # rows wider apart than long
+
+    def call():
+        return paged_ops.paged_decode(wl.query, wl.k_pool, wl.v_pool, wl.block_tables, wl.context_lens,
+                                      wl.max_context_len, out=out, cohort_size=4, cohort_shared_blocks=shared).clone()
+    native, plain = _both(monkeypatch, call)
+    assert torch.equal(native, plain)
+    k = torch.randn(3, 2, 128, device=gpu).bfloat16()
+    slots = torch.tensor([5, -1, 17], device=gpu)
+    pools = [torch.zeros_like(wl.k_pool) for _ in range(4)]
+    left = list(pools)
+    _both(monkeypatch, lambda: paged_ops.kv_append(k, k, left.pop(), left.pop(), slots))
+    assert torch.equal(pools[0], pools[2]) and torch.equal(pools[1], pools[3]) and pools[0].any()
+
+
+def test_what_is_not_ordinary_is_refused_by_name(gpu):
+    wl = workloads.make_decode_workload(2, 4, 2, 64, 20, 40, seed=1).to(gpu)
+    args = (wl.k_pool, wl.v_pool, wl.block_tables, wl.context_lens)
+    with pytest.raises(TypeError, match="share a dtype"):
+        paged_ops.paged_decode(wl.query.float(), *args, wl.max_context_len)
+    with pytest.raises(ValueError, match="exceeds what the block table"):
+        paged_ops.paged_decode(wl.query, *args, 10_000)
+    with pytest.raises(ValueError, match="context_lens"):
+        paged_ops.paged_decode(wl.query, *args[:3], wl.context_lens.long(), wl.max_context_len)
+    with pytest.raises(_lib.PagedLibraryError):
+        paged_ops.paged_decode(wl.query, *args, wl.max_context_len, min_chunk_tokens=24)
