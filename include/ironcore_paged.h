@@ -159,6 +159,22 @@ int ic_rope_kv_append(void *q, int64_t q_stride_token, int hn,
                       int64_t num_blocks, int dtype, void *stream);
 
 /*
+ * The same with the rotated query rows going to a buffer of their own (q_out,
+ * row stride q_out_stride_token) instead of over the query; q_out == q is the
+ * call above.
+ */
+int ic_rope_kv_append_to(void *q_out, int64_t q_out_stride_token,
+                         const void *q, int64_t q_stride_token, int hn,
+                         const void *k_new, const void *v_new, int64_t new_stride_token,
+                         void *k_pool, void *v_pool,
+                         int64_t pool_stride_block, int64_t pool_stride_head,
+                         int64_t pool_stride_token,
+                         const int64_t *slot_mapping, const int32_t *positions,
+                         const float *cos_table, const float *sin_table, int64_t table_rows,
+                         int64_t n_tokens, int gn, int hd, int block_size,
+                         int64_t num_blocks, int dtype, void *stream);
+
+/*
  * Workspace the decode entry point needs (block-count prefix sums and
  * split-K partials), in bytes, for a batch of n_seqs sequences with these
  * head counts.  Returns 0 for invalid arguments.
@@ -310,6 +326,53 @@ int ic_paged_prefill(void *out, int64_t out_stride_token,
                      int hn, int gn, int hd, int block_size,
                      int64_t num_blocks, float scale, int causal,
                      int dtype, void *stream);
+
+/*
+ * Chunked prefill by descriptor: ic_paged_prefill (same fields, same meaning)
+ * plus three forms of input that spare a caller passes over its tensors.
+ * Clear the struct first; a field left zero is the plain call's behaviour.
+ *
+ *   row_pitch        > 0: the chunks are padded, row r of sequence i is row
+ *                    i*row_pitch + r of q and out (cu_seqlens_q still gives the
+ *                    chunk lengths); output rows from a chunk's end to
+ *                    max_chunk_len are set to zero.  row_pitch >= max_chunk_len.
+ *   uniform_context  with context_lens, cu_seqlens_q and block_tables all NULL:
+ *                    equal sequences.  Every context has this many keys, every
+ *                    chunk max_chunk_len rows (row_pitch is required), and
+ *                    sequence i is pool block i (uniform_context <= block_size,
+ *                    any block size): a dense [b, s, gn, hd] tensor as a pool.
+ *   positions, cos_table, sin_table, table_rows
+ *                    positions != NULL: the query rows have NOT been rotated;
+ *                    row r of q is rotated as it is loaded, by table row
+ *                    positions[r], with the arithmetic and the rounding of
+ *                    ic_rope_kv_append.  The keys in the pool are rotated already.
+ */
+typedef struct ic_prefill_call {
+  void *out;
+  int64_t out_stride_token;
+  const void *q;
+  int64_t q_stride_token;
+  const void *k_pool;
+  const void *v_pool;
+  int64_t pool_stride_block, pool_stride_head, pool_stride_token;
+  const int32_t *block_tables;
+  int64_t block_table_stride;
+  const int32_t *context_lens;
+  const int32_t *cu_seqlens_q;
+  int n_seqs, max_chunk_len;
+  int hn, gn, hd, block_size;
+  int64_t num_blocks;
+  float scale;
+  int causal;
+  int dtype;
+  int uniform_context;
+  int64_t row_pitch;
+  const int32_t *positions;
+  const float *cos_table;
+  const float *sin_table;
+  int64_t table_rows;
+} ic_prefill_call;
+int ic_paged_prefill_ex(const ic_prefill_call *call, void *stream);
 
 /*
  * Chunked prefill under a general attention mask: ic_paged_prefill with the

@@ -41,6 +41,16 @@ SIGNATURES = {
         c_void_p, c_void_p, c_int64,            # cos_table, sin_table, table_rows
         c_int64, c_int, c_int, c_int,           # n_tokens, gn, hd, block_size
         c_int64, c_int, c_void_p]),             # num_blocks, dtype, stream
+    "ic_rope_kv_append_to": (c_int, [
+        c_void_p, c_int64,                      # q_out, q_out_stride_token
+        c_void_p, c_int64, c_int,               # q, q_stride_token, hn
+        c_void_p, c_void_p, c_int64,            # k_new, v_new, new_stride_token
+        c_void_p, c_void_p,                     # k_pool, v_pool
+        c_int64, c_int64, c_int64,              # pool strides
+        c_void_p, c_void_p,                     # slot_mapping, positions
+        c_void_p, c_void_p, c_int64,            # cos_table, sin_table, table_rows
+        c_int64, c_int, c_int, c_int,           # n_tokens, gn, hd, block_size
+        c_int64, c_int, c_void_p]),             # num_blocks, dtype, stream
     "ic_paged_decode_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "ic_paged_decode": (c_int, [
         c_void_p, c_int64, c_void_p, c_int64,   # out, out_stride, q, q_stride
@@ -80,6 +90,7 @@ SIGNATURES = {
         c_int, c_int, c_int, c_int,             # hn, gn, hd, block_size
         c_int64, c_float, c_int,                # num_blocks, scale, causal
         c_int, c_void_p]),                      # dtype, stream
+    "ic_paged_prefill_ex": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_paged_prefill_masked": (c_int, [
         c_void_p, c_int64, c_void_p, c_int64,   # out, out_stride, q, q_stride
         c_void_p, c_void_p,                     # k_pool, v_pool

@@ -135,6 +135,48 @@ OptTensor paged_decode(const Tensor &query, const Tensor &k_pool, const Tensor &
 
 // ---- the layer -----------------------------------------------------------------------------
 
+// Rotary tables and the table row of each of n tokens; `on` is false without rotary embeddings.
+struct Rope {
+  bool used = false, ok = true;
+  const int32_t *positions = nullptr;
+  const float *cos = nullptr, *sin = nullptr;
+  int64_t rows = 0;
+  Rope(const OptTensor &pos, const OptTensor &c, const OptTensor &s, int64_t n, int64_t hd, int64_t device) {
+    if (!c.has_value()) return;
+    used = true;
+    ok = pos.has_value() && s.has_value() && index_vector(*pos, at::kInt, n, device) && c->dim() == 2 &&
+         c->size(1) == hd / 2 && c->sizes() == s->sizes() && index_vector(*c, at::kFloat, c->numel(), device) &&
+         index_vector(*s, at::kFloat, c->numel(), device);
+    if (!ok) return;
+    positions = pos->data_ptr<int32_t>();
+    cos = c->data_ptr<float>(), sin = s->data_ptr<float>();
+    rows = c->size(0);
+  }
+};
+
+// The new rows of a layer call: query [b, s, hn, hd], key and value [b, s, gn, hd], a slot for each.
+struct NewRows {
+  int64_t b = 0, s = 0, hn = 0;
+  bool ok = false;
+  NewRows(const Tensor &query, const Tensor &key, const Tensor &value, const Pool &p, at::ScalarType type,
+          int64_t device) {
+    if (query.dim() != 4) return;
+    b = query.size(0), s = query.size(1), hn = query.size(2);
+    ok = rows4(query, b, s, hn, p.hd) && rows4(key, b, s, p.gn, p.hd) && rows4(value, b, s, p.gn, p.hd) &&
+         row_stride4(key) == row_stride4(value) && query.scalar_type() == type && key.scalar_type() == type &&
+         value.scalar_type() == type && on(query, device) && on(key, device) && on(value, device) && b * s > 0;
+  }
+};
+
+// Append with the keys rotated on their way; q_out == nullptr: the query is left alone.
+bool rope_append(const Tensor &key, const Tensor &value, const Pool &p, const Tensor &slots, const Rope &r, int64_t n,
+                 void *q_out, const void *q, int64_t q_stride, int64_t hn, void *stream) {
+  return ic_rope_kv_append_to(q_out, hn * p.hd, q_out ? q : nullptr, q_stride, (int)hn, key.data_ptr(),
+                              value.data_ptr(), row_stride4(key), const_cast<void *>(p.k), const_cast<void *>(p.v),
+                              p.sb, p.sh, p.st, slots.data_ptr<int64_t>(), r.positions, r.cos, r.sin, r.rows, n,
+                              (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream) == IC_OK;
+}
+
 // One cached decode step of a layer (sq == 1): append, then attend.  With rotary tables the query is
 // rotated into a tensor of its own and the keys on their way into the pool.
 OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
@@ -143,38 +185,92 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
                       const OptTensor &positions, const OptTensor &cos, const OptTensor &sin, int64_t device,
                       int64_t stream) {
   const Pool p(k_pool, v_pool, device);
-  if (!p.ok || query.dim() != 4) return c10::nullopt;
-  const int64_t b = query.size(0), hn = query.size(2);
-  const auto type = k_pool.scalar_type();
-  if (!rows4(query, b, 1, hn, p.hd) || !rows4(key, b, 1, p.gn, p.hd) || !rows4(value, b, 1, p.gn, p.hd) ||
-      row_stride4(key) != row_stride4(value) || query.scalar_type() != type || key.scalar_type() != type ||
-      value.scalar_type() != type || !on(query, device) || !on(key, device) || !on(value, device) ||
-      !index_vector(slots, at::kLong, b, device))
-    return c10::nullopt;
+  if (!p.ok) return c10::nullopt;
+  const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
+  if (!in.ok || in.s != 1 || !index_vector(slots, at::kLong, in.b, device)) return c10::nullopt;
   const Decode d{tables, lens, max_ctx, 0, cohort, shared, scale};
-  if (!decode_fits(p, b, hn, d, device)) return c10::nullopt;
+  const Rope rope(positions, cos, sin, in.b, p.hd, device);
+  if (!rope.ok || !decode_fits(p, in.b, in.hn, d, device)) return c10::nullopt;
   const void *q = query.data_ptr();
   int64_t q_stride = row_stride4(query);
   Tensor rotated;
-  if (cos.has_value()) {
-    if (!positions.has_value() || !sin.has_value() || !index_vector(*positions, at::kInt, b, device) ||
-        cos->dim() != 2 || cos->size(1) != p.hd / 2 || cos->sizes() != sin->sizes() ||
-        !index_vector(*cos, at::kFloat, cos->numel(), device) || !index_vector(*sin, at::kFloat, cos->numel(), device))
+  if (rope.used) {
+    rotated = at::empty({in.b, in.hn * p.hd}, query.options());
+    if (!rope_append(key, value, p, slots, rope, in.b, rotated.data_ptr(), q, q_stride, in.hn, (void *)stream))
       return c10::nullopt;
-    rotated = query.clone(at::MemoryFormat::Contiguous);
     q = rotated.data_ptr();
-    q_stride = hn * p.hd;
-    if (ic_rope_kv_append(rotated.data_ptr(), q_stride, (int)hn, key.data_ptr(), value.data_ptr(), row_stride4(key),
-                          const_cast<void *>(p.k), const_cast<void *>(p.v), p.sb, p.sh, p.st,
-                          slots.data_ptr<int64_t>(), positions->data_ptr<int32_t>(), cos->data_ptr<float>(),
-                          sin->data_ptr<float>(), cos->size(0), b, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype,
-                          (void *)stream) != IC_OK)
-      return c10::nullopt;
-  } else if (!append_rows(key.data_ptr(), value.data_ptr(), row_stride4(key), p, slots, b, (void *)stream)) {
+    q_stride = in.hn * p.hd;
+  } else if (!append_rows(key.data_ptr(), value.data_ptr(), row_stride4(key), p, slots, in.b, (void *)stream)) {
     return c10::nullopt;
   }
-  const Tensor out = at::empty({b, 1, hn * p.hd}, query.options());
-  if (!decode(out, q, q_stride, p, b, hn, d, (void *)stream)) return c10::nullopt;
+  const Tensor out = at::empty({in.b, 1, in.hn * p.hd}, query.options());
+  if (!decode(out, q, q_stride, p, in.b, in.hn, d, (void *)stream)) return c10::nullopt;
+  return out;
+}
+
+ic_prefill_call prefill_call(const Tensor &out, const Tensor &query, const Pool &p, int64_t b, int64_t s, int64_t hn,
+                             double scale, bool causal) {
+  ic_prefill_call c = {};
+  c.out = out.data_ptr();
+  c.out_stride_token = hn * p.hd;
+  c.q = query.data_ptr();
+  c.q_stride_token = row_stride4(query);
+  c.k_pool = p.k, c.v_pool = p.v;
+  c.pool_stride_block = p.sb, c.pool_stride_head = p.sh, c.pool_stride_token = p.st;
+  c.n_seqs = (int)b, c.max_chunk_len = (int)s;
+  c.hn = (int)hn, c.gn = (int)p.gn, c.hd = (int)p.hd;
+  c.block_size = (int)p.bs, c.num_blocks = p.nb;
+  c.scale = (float)scale, c.causal = causal, c.dtype = p.dtype;
+  c.row_pitch = s;
+  return c;
+}
+
+// A chunk of new tokens per sequence: append, then attend.  `bounds` int32 [b + 1] holds the chunks' bounds
+// when they are of unequal length (rows past a chunk's end are padding: slot -1, output zero), else the
+// bounds of equal chunks.  The query is rotated inside the attention kernel.
+OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
+                       const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
+                       const Tensor &bounds, double scale, const OptTensor &positions, const OptTensor &cos,
+                       const OptTensor &sin, int64_t device, int64_t stream) {
+  const Pool p(k_pool, v_pool, device);
+  if (!p.ok || !p.attends()) return c10::nullopt;
+  const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
+  if (!in.ok || in.hn % p.gn != 0 || !index_vector(slots, at::kLong, in.b * in.s, device) ||
+      !table(tables, in.b, device) || !index_vector(lens, at::kInt, in.b, device) ||
+      !index_vector(bounds, at::kInt, in.b + 1, device))
+    return c10::nullopt;
+  const Rope rope(positions, cos, sin, in.b * in.s, p.hd, device);
+  if (!rope.ok) return c10::nullopt;
+  if (rope.used ? !rope_append(key, value, p, slots, rope, in.b * in.s, nullptr, nullptr, 0, in.hn, (void *)stream)
+                : !append_rows(key.data_ptr(), value.data_ptr(), row_stride4(key), p, slots, in.b * in.s,
+                               (void *)stream))
+    return c10::nullopt;
+  const Tensor out = at::empty({in.b, in.s, in.hn * p.hd}, query.options());
+  ic_prefill_call c = prefill_call(out, query, p, in.b, in.s, in.hn, scale, true);
+  c.block_tables = tables.data_ptr<int32_t>();
+  c.block_table_stride = tables.stride(0);
+  c.context_lens = lens.data_ptr<int32_t>();
+  c.cu_seqlens_q = bounds.data_ptr<int32_t>();
+  c.positions = rope.positions;
+  c.cos_table = rope.cos, c.sin_table = rope.sin, c.table_rows = rope.rows;
+  if (ic_paged_prefill_ex(&c, (void *)stream) != IC_OK) return c10::nullopt;
+  return out;
+}
+
+// The dense call: query [b, sq, hn, hd] on key / value [b, sk, gn, hd], which the kernel walks as a pool of
+// one block per sequence, at whatever strides they have.
+OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, bool causal, double scale,
+                int64_t device, int64_t stream) {
+  if (query.dim() != 4 || key.dim() != 4 || key.size(1) == 0 || query.size(1) == 0) return c10::nullopt;
+  const Pool p(key.permute({0, 2, 1, 3}), value.permute({0, 2, 1, 3}), device);
+  const int64_t b = query.size(0), s = query.size(1), hn = query.size(2);
+  if (!p.ok || !p.attends() || p.nb != b || hn % p.gn != 0 || !rows4(query, b, s, hn, p.hd) || !on(query, device) ||
+      query.scalar_type() != key.scalar_type() || (b == 1 && p.sb < p.bs * p.st))
+    return c10::nullopt;
+  const Tensor out = at::empty({b, s, hn * p.hd}, query.options());
+  ic_prefill_call c = prefill_call(out, query, p, b, s, hn, scale, causal);
+  c.uniform_context = (int)p.bs;
+  if (ic_paged_prefill_ex(&c, (void *)stream) != IC_OK) return c10::nullopt;
   return out;
 }
 
@@ -184,4 +280,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append);
   m.def("paged_decode", &paged_decode);
   m.def("decode_step", &decode_step);
+  m.def("prefill_step", &prefill_step);
+  m.def("dense", &dense);
 }

@@ -137,53 +137,100 @@ int decode_checked(void *out, int64_t out_stride_seq, const void *q, int64_t q_s
   return ic::launch_paged_decode(a, static_cast<hipStream_t>(stream));
 }
 
-int prefill_checked(void *out, int64_t out_stride_token, const void *q, int64_t q_stride_token,
-                    const void *k_pool, const void *v_pool, int64_t pool_stride_block,
-                    int64_t pool_stride_head, int64_t pool_stride_token, const int32_t *block_tables,
-                    int64_t block_table_stride, const int32_t *context_lens, const int32_t *cu_seqlens_q,
-                    int n_seqs, int max_chunk_len, int hn, int gn, int hd, int block_size,
-                    int64_t num_blocks, float scale, int causal, const uint8_t *mask,
-                    int64_t mask_stride_seq, int64_t mask_stride_head, int64_t mask_stride_row,
-                    int64_t mask_keys, int dtype, void *stream) {
-  if (n_seqs < 0 || max_chunk_len < 0 || hn <= 0 || gn <= 0 || hn % gn != 0) return IC_ERR_BAD_SHAPE;
-  if (!dtype_ok(dtype)) return IC_ERR_UNSUPPORTED;
-  const int es = ic::elem_size(dtype);
-  if (int rc = check_pool(pool_stride_block, pool_stride_head, pool_stride_token, gn, hd, block_size,
-                          num_blocks, es))
+ic_prefill_call prefill_call(void *out, int64_t out_stride_token, const void *q, int64_t q_stride_token,
+                             const void *k_pool, const void *v_pool, int64_t pool_stride_block,
+                             int64_t pool_stride_head, int64_t pool_stride_token, const int32_t *block_tables,
+                             int64_t block_table_stride, const int32_t *context_lens, const int32_t *cu_seqlens_q,
+                             int n_seqs, int max_chunk_len, int hn, int gn, int hd, int block_size,
+                             int64_t num_blocks, float scale, int causal, int dtype) {
+  ic_prefill_call c = {};
+  c.out = out;
+  c.out_stride_token = out_stride_token;
+  c.q = q;
+  c.q_stride_token = q_stride_token;
+  c.k_pool = k_pool;
+  c.v_pool = v_pool;
+  c.pool_stride_block = pool_stride_block;
+  c.pool_stride_head = pool_stride_head;
+  c.pool_stride_token = pool_stride_token;
+  c.block_tables = block_tables;
+  c.block_table_stride = block_table_stride;
+  c.context_lens = context_lens;
+  c.cu_seqlens_q = cu_seqlens_q;
+  c.n_seqs = n_seqs;
+  c.max_chunk_len = max_chunk_len;
+  c.hn = hn;
+  c.gn = gn;
+  c.hd = hd;
+  c.block_size = block_size;
+  c.num_blocks = num_blocks;
+  c.scale = scale;
+  c.causal = causal;
+  c.dtype = dtype;
+  return c;
+}
+
+int prefill_checked(const ic_prefill_call &c, const uint8_t *mask, int64_t mask_stride_seq, int64_t mask_stride_head,
+                    int64_t mask_stride_row, int64_t mask_keys, void *stream) {
+  if (c.n_seqs < 0 || c.max_chunk_len < 0 || c.hn <= 0 || c.gn <= 0 || c.hn % c.gn != 0) return IC_ERR_BAD_SHAPE;
+  if (!dtype_ok(c.dtype)) return IC_ERR_UNSUPPORTED;
+  const int es = ic::elem_size(c.dtype);
+  if (int rc = check_pool(c.pool_stride_block, c.pool_stride_head, c.pool_stride_token, c.gn, c.hd, c.block_size,
+                          c.num_blocks, es))
     return rc;
-  if (n_seqs == 0 || max_chunk_len == 0) return IC_OK;
-  if (!out || !q || !k_pool || !v_pool || !block_tables || !context_lens || !cu_seqlens_q)
-    return IC_ERR_NULL_POINTER;
-  if (out_stride_token < (int64_t)hn * hd || q_stride_token < (int64_t)hn * hd) return IC_ERR_BAD_SHAPE;
-  if (block_table_stride <= 0) return IC_ERR_BAD_SHAPE;
-  if (!aligned16(q) || !aligned16(out) || !aligned16(k_pool) || !aligned16(v_pool) ||
-      !stride16(q_stride_token, es) || !stride16(out_stride_token, es))
+  if (c.n_seqs == 0 || c.max_chunk_len == 0) return IC_OK;
+  if (!c.out || !c.q || !c.k_pool || !c.v_pool) return IC_ERR_NULL_POINTER;
+  if (c.context_lens == nullptr) {  // equal sequences
+    if (c.block_tables != nullptr || c.cu_seqlens_q != nullptr) return IC_ERR_NULL_POINTER;
+    if (c.row_pitch < c.max_chunk_len || c.uniform_context < 0 || c.uniform_context > c.block_size ||
+        c.n_seqs > c.num_blocks)
+      return IC_ERR_BAD_SHAPE;
+  } else {
+    if (!c.block_tables || !c.cu_seqlens_q) return IC_ERR_NULL_POINTER;
+    if (c.block_table_stride <= 0 || c.row_pitch < 0 || (c.row_pitch > 0 && c.row_pitch < c.max_chunk_len))
+      return IC_ERR_BAD_SHAPE;
+  }
+  if (c.row_pitch > 0 && c.row_pitch * c.n_seqs > 0x7fffffff) return IC_ERR_UNSUPPORTED;
+  if (c.out_stride_token < (int64_t)c.hn * c.hd || c.q_stride_token < (int64_t)c.hn * c.hd) return IC_ERR_BAD_SHAPE;
+  if (!aligned16(c.q) || !aligned16(c.out) || !aligned16(c.k_pool) || !aligned16(c.v_pool) ||
+      !stride16(c.q_stride_token, es) || !stride16(c.out_stride_token, es))
     return IC_ERR_ALIGNMENT;
+  if (c.positions != nullptr) {
+    if (!c.cos_table || !c.sin_table) return IC_ERR_NULL_POINTER;
+    if (c.table_rows <= 0) return IC_ERR_BAD_SHAPE;
+    if (!aligned16(c.cos_table) || !aligned16(c.sin_table)) return IC_ERR_ALIGNMENT;
+  }
   ic::PrefillArgs a;
-  a.out = out;
-  a.out_stride_token = out_stride_token;
-  a.q = q;
-  a.q_stride_token = q_stride_token;
-  a.k_pool = k_pool;
-  a.v_pool = v_pool;
-  a.pool = {pool_stride_block, pool_stride_head, pool_stride_token, num_blocks, block_size};
-  a.block_tables = block_tables;
-  a.block_table_stride = block_table_stride;
-  a.context_lens = context_lens;
-  a.cu_seqlens_q = cu_seqlens_q;
-  a.n_seqs = n_seqs;
-  a.max_chunk_len = max_chunk_len;
-  a.hn = hn;
-  a.gn = gn;
-  a.hd = hd;
-  a.scale = scale;
-  a.causal = causal;
-  a.dtype = dtype;
+  a.out = c.out;
+  a.out_stride_token = c.out_stride_token;
+  a.q = c.q;
+  a.q_stride_token = c.q_stride_token;
+  a.k_pool = c.k_pool;
+  a.v_pool = c.v_pool;
+  a.pool = {c.pool_stride_block, c.pool_stride_head, c.pool_stride_token, c.num_blocks, c.block_size};
+  a.block_tables = c.block_tables;
+  a.block_table_stride = c.block_table_stride;
+  a.context_lens = c.context_lens;
+  a.cu_seqlens_q = c.cu_seqlens_q;
+  a.n_seqs = c.n_seqs;
+  a.max_chunk_len = c.max_chunk_len;
+  a.hn = c.hn;
+  a.gn = c.gn;
+  a.hd = c.hd;
+  a.scale = c.scale;
+  a.causal = c.causal;
+  a.dtype = c.dtype;
   a.mask = mask;
   a.mask_stride_seq = mask_stride_seq;
   a.mask_stride_head = mask_stride_head;
   a.mask_stride_row = mask_stride_row;
   a.mask_keys = mask_keys;
+  a.row_pitch = c.row_pitch;
+  a.uniform_context = c.uniform_context;
+  a.positions = c.positions;
+  a.cos_table = c.cos_table;
+  a.sin_table = c.sin_table;
+  a.table_rows = c.table_rows;
   return ic::launch_paged_prefill(a, static_cast<hipStream_t>(stream));
 }
 
@@ -266,7 +313,8 @@ int ic_kv_append(const void *k_new, const void *v_new, int64_t new_stride_token,
   return ic::launch_kv_append(a, static_cast<hipStream_t>(stream));
 }
 
-int ic_rope_kv_append(void *q, int64_t q_stride_token, int hn, const void *k_new, const void *v_new,
+int ic_rope_kv_append_to(void *q_out, int64_t q_out_stride_token, const void *q, int64_t q_stride_token, int hn,
+                         const void *k_new, const void *v_new,
                       int64_t new_stride_token, void *k_pool, void *v_pool, int64_t pool_stride_block,
                       int64_t pool_stride_head, int64_t pool_stride_token, const int64_t *slot_mapping,
                       const int32_t *positions, const float *cos_table, const float *sin_table,
@@ -288,8 +336,10 @@ int ic_rope_kv_append(void *q, int64_t q_stride_token, int hn, const void *k_new
   if (q == nullptr && !has_kv) return IC_ERR_NULL_POINTER;
   if (!aligned16(cos_table) || !aligned16(sin_table)) return IC_ERR_ALIGNMENT;
   if (q != nullptr) {
-    if (q_stride_token < (int64_t)hn * hd) return IC_ERR_BAD_SHAPE;
-    if (!aligned16(q) || !stride16(q_stride_token, es)) return IC_ERR_ALIGNMENT;
+    if (q_out == nullptr) return IC_ERR_NULL_POINTER;
+    if (q_stride_token < (int64_t)hn * hd || q_out_stride_token < (int64_t)hn * hd) return IC_ERR_BAD_SHAPE;
+    if (!aligned16(q) || !stride16(q_stride_token, es) || !aligned16(q_out) || !stride16(q_out_stride_token, es))
+      return IC_ERR_ALIGNMENT;
   }
   if (has_kv) {
     if (!k_new || !v_new || !k_pool || !v_pool || !slot_mapping) return IC_ERR_NULL_POINTER;
@@ -313,12 +363,26 @@ int ic_rope_kv_append(void *q, int64_t q_stride_token, int hn, const void *k_new
   a.append.dtype = dtype;
   a.q = q;
   a.q_stride_token = q_stride_token;
+  a.q_out = q_out;
+  a.q_out_stride_token = q_out_stride_token;
   a.hn = hn;
   a.positions = positions;
   a.cos_table = cos_table;
   a.sin_table = sin_table;
   a.table_rows = table_rows;
   return ic::launch_rope_kv_append(a, static_cast<hipStream_t>(stream));
+}
+
+int ic_rope_kv_append(void *q, int64_t q_stride_token, int hn, const void *k_new, const void *v_new,
+                      int64_t new_stride_token, void *k_pool, void *v_pool, int64_t pool_stride_block,
+                      int64_t pool_stride_head, int64_t pool_stride_token, const int64_t *slot_mapping,
+                      const int32_t *positions, const float *cos_table, const float *sin_table,
+                      int64_t table_rows, int64_t n_tokens, int gn, int hd, int block_size,
+                      int64_t num_blocks, int dtype, void *stream) {
+  return ic_rope_kv_append_to(q, q_stride_token, q, q_stride_token, hn, k_new, v_new, new_stride_token, k_pool, v_pool,
+                              pool_stride_block, pool_stride_head, pool_stride_token, slot_mapping, positions,
+                              cos_table, sin_table, table_rows, n_tokens, gn, hd, block_size, num_blocks, dtype,
+                              stream);
 }
 
 size_t ic_paged_decode_workspace_bytes(int n_seqs, int hn, int gn, int hd) {
@@ -389,6 +453,11 @@ int ic_paged_decode_static(void *out, int64_t out_stride_seq, const void *q, int
                         kStaticMaxWaves, dtype, stream);
 }
 
+int ic_paged_prefill_ex(const ic_prefill_call *call, void *stream) {
+  if (call == nullptr) return IC_ERR_NULL_POINTER;
+  return prefill_checked(*call, nullptr, 0, 0, 0, 0, stream);
+}
+
 int ic_paged_prefill(void *out, int64_t out_stride_token, const void *q, int64_t q_stride_token,
                      const void *k_pool, const void *v_pool, int64_t pool_stride_block,
                      int64_t pool_stride_head, int64_t pool_stride_token,
@@ -396,10 +465,13 @@ int ic_paged_prefill(void *out, int64_t out_stride_token, const void *q, int64_t
                      const int32_t *context_lens, const int32_t *cu_seqlens_q, int n_seqs,
                      int max_chunk_len, int hn, int gn, int hd, int block_size, int64_t num_blocks,
                      float scale, int causal, int dtype, void *stream) {
-  return prefill_checked(out, out_stride_token, q, q_stride_token, k_pool, v_pool, pool_stride_block,
-                         pool_stride_head, pool_stride_token, block_tables, block_table_stride,
-                         context_lens, cu_seqlens_q, n_seqs, max_chunk_len, hn, gn, hd, block_size,
-                         num_blocks, scale, causal, nullptr, 0, 0, 0, 0, dtype, stream);
+  const ic_prefill_call c = prefill_call(out, out_stride_token, q, q_stride_token, k_pool, v_pool, pool_stride_block,
+                                         pool_stride_head, pool_stride_token, block_tables, block_table_stride,
+                                         context_lens, cu_seqlens_q, n_seqs, max_chunk_len, hn, gn, hd, block_size,
+                                         num_blocks, scale, causal, dtype);
+  // (a null array is an error here: equal sequences are the descriptor call's)
+  if (n_seqs > 0 && max_chunk_len > 0 && (!block_tables || !context_lens || !cu_seqlens_q)) return IC_ERR_NULL_POINTER;
+  return prefill_checked(c, nullptr, 0, 0, 0, 0, stream);
 }
 
 int ic_paged_prefill_masked(void *out, int64_t out_stride_token, const void *q, int64_t q_stride_token,
@@ -415,11 +487,13 @@ int ic_paged_prefill_masked(void *out, int64_t out_stride_token, const void *q, 
   if (mask_stride_seq < 0 || mask_stride_head < 0 || mask_stride_row < 0 || mask_keys < 0) return IC_ERR_BAD_SHAPE;
   if (mask_stride_row != 0 && mask_stride_row < mask_keys) return IC_ERR_BAD_SHAPE;
   if (n_seqs > 0 && max_chunk_len > 0 && mask_keys < 1) return IC_ERR_BAD_SHAPE;  // a mask row holds a byte at least
-  return prefill_checked(out, out_stride_token, q, q_stride_token, k_pool, v_pool, pool_stride_block,
-                         pool_stride_head, pool_stride_token, block_tables, block_table_stride,
-                         context_lens, cu_seqlens_q, n_seqs, max_chunk_len, hn, gn, hd, block_size,
-                         num_blocks, scale, 0, mask, mask_stride_seq, mask_stride_head, mask_stride_row,
-                         mask_keys, dtype, stream);
+  const ic_prefill_call c = prefill_call(out, out_stride_token, q, q_stride_token, k_pool, v_pool, pool_stride_block,
+                                         pool_stride_head, pool_stride_token, block_tables, block_table_stride,
+                                         context_lens, cu_seqlens_q, n_seqs, max_chunk_len, hn, gn, hd, block_size,
+                                         num_blocks, scale, 0, dtype);
+  // (a null array is an error here: equal sequences are the descriptor call's)
+  if (n_seqs > 0 && max_chunk_len > 0 && (!block_tables || !context_lens || !cu_seqlens_q)) return IC_ERR_NULL_POINTER;
+  return prefill_checked(c, mask, mask_stride_seq, mask_stride_head, mask_stride_row, mask_keys, stream);
 }
 
 int ic_paged_decode_masked(void *out, int64_t out_stride_seq, const void *q, int64_t q_stride_seq,

@@ -34,8 +34,10 @@ struct AppendArgs {
 // may be null: rotate the query rows only) plus the query rows and the tables.
 struct RopeAppendArgs {
   AppendArgs append;
-  void *q;                 // [n_tokens, hn, hd] rotated in place, or nullptr
+  const void *q;           // [n_tokens, hn, hd], or nullptr
   int64_t q_stride_token;  // elements
+  void *q_out;             // rotated rows (q itself: in place)
+  int64_t q_out_stride_token;
   int hn;
   const int32_t *positions;  // [n_tokens] row of the tables each token uses
   const float *cos_table;    // [table_rows, hd / 2]
@@ -103,6 +105,18 @@ struct PrefillArgs {
   int64_t mask_stride_head = 0;
   int64_t mask_stride_row = 0;
   int64_t mask_keys = 0;  // keys a mask row covers; keys from there on are hidden
+  // Rows of sequence i start at i * row_pitch in q and out instead of cu_seqlens_q[i] (0 = packed rows);
+  // output rows from a chunk's end to max_chunk_len are zeroed.
+  int64_t row_pitch = 0;
+  // Equal sequences: context_lens, cu_seqlens_q and block_tables may be null; then every context has
+  // uniform_context keys, every chunk max_chunk_len rows, and sequence i is pool block i.
+  int uniform_context = 0;
+  // Rotary embedding of the query rows as they are loaded (nullptr = none): row r of q uses table row
+  // positions[r].
+  const int32_t *positions = nullptr;
+  const float *cos_table = nullptr;
+  const float *sin_table = nullptr;
+  int64_t table_rows = 0;
 };
 
 // Each returns IC_OK, IC_ERR_UNSUPPORTED (no kernel built for this

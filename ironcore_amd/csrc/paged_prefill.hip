@@ -116,6 +116,8 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   const bool causal = !MASK && p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
+  if (p.row_pitch > 0 && C < p.max_chunk)
+    zero_padding<HD, 2, kPrefillThreads>(p, q_lo, C, kvh * p.group, p.group, r, per_unit);
   if (q0 >= C) return;
   if (L == 0) {  // query rows without any key (not under the causal rule): zero rows
     const int rows = C - q0 < kBM ? C - q0 : kBM;
@@ -140,6 +142,12 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
     qf[ks] = load16(p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+  if (p.positions != nullptr) {
+    const int64_t trig = rope_row(p, q_lo + qrow) + hh * 4;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = rotate_chunk<typename M::E>(qf[ks], p.cos_table + trig + ks * 8, p.sin_table + trig + ks * 8);
+  }
 
   f32x16_t o[OB];
   float m = kNegInf, l = 0.f;
@@ -207,7 +215,7 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
     int blk = SINGLE ? 0 : block_of(first);
     rem = first - blk * p.block_size;
     blk = blk < last_blk ? blk : last_blk;
-    ent = table_row[blk];
+    ent = SINGLE && p.block_tables == nullptr ? seq : table_row[blk];
   };
   // Issue the loads of this wave's group of `tile` into the tile's LDS buffer.
   auto fetch_rows = [&](int tile, int32_t ent, int rem) {
@@ -549,8 +557,9 @@ template <class M>
 int launch_mode(const PrefillKP &kp, const PrefillArgs &a, hipStream_t stream) {
   // A one-column block table means one block per sequence, of any length.
   const bool masked = a.mask != nullptr;
-  if (a.block_table_stride == 1 && !masked && prefill_takes_short(a)) return launch_paged_prefill_short(kp, a, stream);
-  if (a.block_table_stride == 1)
+  const bool single = a.block_tables == nullptr || a.block_table_stride == 1;
+  if (single && !masked && prefill_takes_short(a)) return launch_paged_prefill_short(kp, a, stream);
+  if (single)
     return masked ? launch_hd<M, true, true>(kp, a, stream) : launch_hd<M, true, false>(kp, a, stream);
   if (kp.block_size < 16 || kp.block_size % 16 != 0) return IC_ERR_UNSUPPORTED;  // whole 16-token groups
   if (!masked && prefill_takes_short(a)) return launch_paged_prefill_short(kp, a, stream);
@@ -599,6 +608,14 @@ int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream) {
   kp.mask_stride_head = a.mask_stride_head;
   kp.mask_stride_row = a.mask_stride_row;
   kp.mask_keys = a.mask_keys > 0x7fffffff ? 0x7fffffff : (int)a.mask_keys;
+  kp.row_pitch = a.row_pitch;
+  kp.max_chunk = a.max_chunk_len;
+  kp.uniform_context = a.uniform_context;
+  kp.positions = a.positions;
+  kp.cos_table = a.cos_table;
+  kp.sin_table = a.sin_table;
+  kp.table_rows = a.table_rows > 0x7fffffff ? 0x7fffffff : (int)a.table_rows;
+  kp.half_hd = a.hd / 2;
   if ((int64_t)a.max_chunk_len >= (int64_t)65535 * 128 || a.hn > 65535 || a.n_seqs > 65535)
     return IC_ERR_UNSUPPORTED;
   // The 16-bit kernel addresses a block with 32-bit byte offsets (a block, and in a block table's

@@ -63,12 +63,16 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   const int h = blockIdx.x / p.n_qtiles;
   const int q0 = (p.n_qtiles - 1 - blockIdx.x % p.n_qtiles) * kF32BM;  // last query tiles (the longest) first
   const int kvh = h / p.group;
-  const int q_lo = p.cu_seqlens_q[seq];
-  int L = p.context_lens[seq];
-  int C = p.cu_seqlens_q[seq + 1] - q_lo;
+  const bool equal = p.context_lens == nullptr;  // equal sequences: nothing to look up
+  int q_lo = equal ? 0 : p.cu_seqlens_q[seq];
+  int L = equal ? p.uniform_context : p.context_lens[seq];
+  int C = equal ? p.max_chunk : p.cu_seqlens_q[seq + 1] - q_lo;
+  if (p.row_pitch > 0) q_lo = (int)(seq * p.row_pitch);
   const bool causal = !MASK && p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
+  if (p.row_pitch > 0 && C < p.max_chunk)
+    zero_padding<HD, 4, kF32Threads>(p, q_lo, C, h, 1, blockIdx.x % p.n_qtiles, p.n_qtiles);
   if (q0 >= C) return;
   const int tid = threadIdx.x;
   if (L == 0) {  // query rows without any key (not under the causal rule): zero rows
@@ -93,6 +97,13 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   for (int j = 0; j < NJ; ++j)
     qf[j] = *reinterpret_cast<const float4 *>(
         p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + 8 * j + 4 * hh) * 4);
+  if (p.positions != nullptr) {
+    const int64_t trig = rope_row(p, q_lo + qrow) + 2 * hh;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      qf[j] = __builtin_bit_cast(float4, rotate_chunk<F32>(__builtin_bit_cast(Vec16, qf[j]), p.cos_table + trig + 4 * j,
+                                                           p.sin_table + trig + 4 * j));
+  }
 
   f32x16_t o[OB];
   float m = kNegInf, l = 0.f;
@@ -123,7 +134,7 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
         blk = p.block_shift >= 0 ? tok >> p.block_shift : tok / p.block_size;
         within = tok - blk * p.block_size;
       }
-      int64_t phys = table_row[blk];
+      int64_t phys = SINGLE && p.block_tables == nullptr ? seq : table_row[blk];
       // A corrupt table entry must not become an out-of-pool address.
       phys = phys < 0 ? 0 : phys;
       phys = phys >= p.num_blocks ? p.num_blocks - 1 : phys;
@@ -287,7 +298,7 @@ int launch_paged_prefill_f32(PrefillKP kp, const PrefillArgs &a, hipStream_t str
   const dim3 grid((unsigned)wgs_x, (unsigned)a.n_seqs);
   const bool masked = a.mask != nullptr;
   // A one-column block table means one block per sequence, of any length.
-  if (a.block_table_stride == 1)
+  if (a.block_tables == nullptr || a.block_table_stride == 1)
     return masked ? launch_hd<true, true>(kp, a.hd, grid, stream) : launch_hd<true, false>(kp, a.hd, grid, stream);
   if (kp.block_size < 1) return IC_ERR_UNSUPPORTED;
   return masked ? launch_hd<false, true>(kp, a.hd, grid, stream) : launch_hd<false, false>(kp, a.hd, grid, stream);

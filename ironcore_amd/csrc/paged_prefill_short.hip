@@ -74,6 +74,8 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const bool causal = p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
+  if (p.row_pitch > 0 && C < p.max_chunk)
+    zero_padding<HD, 2, TG * kShortWaves * kWave>(p, q_lo, C, kvh * p.group, p.group, within / kXcds, per_unit);
   const int n_blocks = (C + 31) >> 5;  // wave blocks per head
   const int total = n_blocks * p.group;
   // The last blocks (the longest sweeps) first; in the slices that share the CUs with the first ones when
@@ -112,6 +114,12 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
     qf[ks] = load16(p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+  if (p.positions != nullptr) {
+    const int64_t trig = rope_row(p, q_lo + qrow) + hh * 4;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = rotate_chunk<typename M::E>(qf[ks], p.cos_table + trig + ks * 8, p.sin_table + trig + ks * 8);
+  }
 
   f32x16_t o[OB];
   float m = kNegInf, l = 0.f;
@@ -157,7 +165,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
     int blk = SINGLE ? 0 : block_of(first);
     rem = first - blk * p.block_size;
     blk = blk < last_blk ? blk : last_blk;
-    ent = table_row[blk];
+    ent = SINGLE && p.block_tables == nullptr ? seq : table_row[blk];
   };
   auto fetch = [&](int tile, int buf, int32_t ent, int rem) {
     int phys = ent;
@@ -401,7 +409,7 @@ int launch_short_hd(const PrefillKP &kp, int hd, unsigned wgs, hipStream_t strea
 
 template <class M>
 int launch_short_type(const PrefillKP &kp, const PrefillArgs &a, unsigned wgs, bool split, hipStream_t stream) {
-  const bool single = a.block_table_stride == 1;
+  const bool single = a.block_tables == nullptr || a.block_table_stride == 1;
   if (split)
     return single ? launch_short_hd<M, true, 2>(kp, a.hd, wgs, stream) : launch_short_hd<M, false, 2>(kp, a.hd, wgs, stream);
   return single ? launch_short_hd<M, true, 1>(kp, a.hd, wgs, stream) : launch_short_hd<M, false, 1>(kp, a.hd, wgs, stream);
@@ -432,7 +440,9 @@ int64_t short_workgroups_per_unit(const PrefillArgs &a) {
   const int64_t blocks = (int64_t)((a.max_chunk_len + 31) / 32) * (a.hn / a.gn);
   return (blocks + kShortWaves - 1) / kShortWaves;
 }
-int64_t context_bound(const PrefillArgs &a) { return a.block_table_stride * (int64_t)a.pool.block_size; }
+int64_t context_bound(const PrefillArgs &a) {
+  return a.context_lens == nullptr ? a.uniform_context : a.block_table_stride * (int64_t)a.pool.block_size;
+}
 }  // namespace
 
 bool prefill_takes_short(const PrefillArgs &a) {

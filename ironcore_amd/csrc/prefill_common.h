@@ -6,6 +6,7 @@
 
 #include "ic_device.h"
 #include "ic_internal.h"
+#include "rope_device.h"
 
 namespace ic {
 namespace prefill {
@@ -43,6 +44,14 @@ struct PrefillKP {
   int64_t mask_stride_head;
   int64_t mask_stride_row;
   int mask_keys;  // keys a mask row covers: keys from there on are hidden and never read
+  int64_t row_pitch;    // rows from one sequence's chunk to the next in q and out (0 = packed, cu_seqlens_q)
+  int max_chunk;        // longest chunk; with row_pitch, output rows from a chunk's end to here are zeroed
+  int uniform_context;  // context_lens == nullptr: keys of every context (every chunk has max_chunk rows)
+  const int32_t *positions;  // rotary embedding of the query rows (nullptr: none)
+  const float *cos_table;
+  const float *sin_table;
+  int table_rows;
+  int half_hd;
 };
 
 constexpr float kNegInf = -__builtin_huge_valf();
@@ -73,6 +82,7 @@ typedef __attribute__((ext_vector_type(8))) short s16x8_t;
 
 // MFMA wrappers per element type: operands are 8 packed 16-bit values.
 struct MmaBf16 {
+  using E = Bf16;
   using T = __bf16;
   static __device__ __forceinline__ f32x16_t mma(const Vec16 &a, const Vec16 &b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
@@ -84,6 +94,7 @@ struct MmaBf16 {
   }
 };
 struct MmaF16 {
+  using E = F16;
   using T = _Float16;
   static __device__ __forceinline__ f32x16_t mma(const Vec16 &a, const Vec16 &b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
@@ -114,9 +125,16 @@ __device__ __forceinline__ int tile_swizzle_v(int r) {
 // The sequence that is `rank`th by context length (longest first: workgroups
 // are dispatched in id order and should end together), its first query row,
 // context length and chunk length.  Up to one sequence per lane is ranked on
-// the fly; in longer batches rank r is simply sequence r.
+// the fly; in longer batches rank r is simply sequence r.  Equal sequences
+// (no context_lens) need no look at memory.
 __device__ __forceinline__ void pick_sequence(const PrefillKP &p, int rank, int &seq, int &q_lo, int &L, int &C) {
   seq = rank;
+  if (p.context_lens == nullptr) {
+    q_lo = (int)(seq * p.row_pitch);
+    L = p.uniform_context;
+    C = p.max_chunk;
+    return;
+  }
   const int n_seqs = p.n_units / p.gn;
   if (n_seqs <= kWave) {
     // (the chunk bounds travel with the context lengths, one sequence per lane: the chosen
@@ -141,6 +159,27 @@ __device__ __forceinline__ void pick_sequence(const PrefillKP &p, int rank, int 
     L = p.context_lens[seq];
     C = p.cu_seqlens_q[seq + 1] - q_lo;
   }
+  if (p.row_pitch > 0) q_lo = (int)(seq * p.row_pitch);
+}
+
+// Output rows C .. max_chunk-1 of a sequence, `heads` heads of HD elements from head0 on: zeros.  Share
+// `share` of `shares` takes every shares-th row.
+template <int HD, int ES, int THREADS>
+__device__ __forceinline__ void zero_padding(const PrefillKP &p, int64_t row0, int C, int head0, int heads, int share,
+                                             int shares) {
+  const int chunks = heads * (HD * ES / 16);
+  for (int r = C + share; r < p.max_chunk; r += shares) {
+    char *row = p.out + ((row0 + r) * p.out_stride_token + (int64_t)head0 * HD) * ES;
+    for (int c = threadIdx.x; c < chunks; c += THREADS) store16(row + c * 16, Vec16{{0u, 0u, 0u, 0u}});
+  }
+}
+
+// The rotary tables' row of query row `row` (clamped into them).
+__device__ __forceinline__ int64_t rope_row(const PrefillKP &p, int64_t row) {
+  int pos = p.positions[row];
+  pos = pos < 0 ? 0 : pos;
+  pos = pos >= p.table_rows ? p.table_rows - 1 : pos;
+  return (int64_t)pos * p.half_hd;
 }
 
 constexpr float kLazySlack = 8.0f;  // log2 units

@@ -24,8 +24,8 @@
 // K, V or Q.  Algorithmic traffic: K and V rows read once and written once,
 // Q rows read and written in place, 12 bytes of slot and position per token;
 // the table rows in use stay in cache.
-#include "ic_device.h"
 #include "ic_internal.h"
+#include "rope_device.h"
 #include "../../include/ironcore_paged.h"
 
 namespace ic {
@@ -35,7 +35,8 @@ namespace {
 constexpr int kRopeThreads = 256;
 
 struct RopeKP {
-  char *q;                // rotated in place, or nullptr
+  const char *q;          // or nullptr
+  char *q_out;            // where its rotated rows go (q itself: in place)
   const char *k_new;      // or nullptr: no K/V work
   const char *v_new;
   char *k_pool;
@@ -45,6 +46,7 @@ struct RopeKP {
   const float *cos_table;
   const float *sin_table;
   int64_t q_stride_bytes;
+  int64_t q_out_stride_bytes;
   int64_t new_stride_bytes;
   int64_t stride_block_bytes;
   int64_t stride_head_bytes;
@@ -58,64 +60,6 @@ struct RopeKP {
   int half_hd;
 };
 
-// Products and sums rounded one by one, as a sequence of separate torch ops
-// is.  Contraction is off for these operations: by default the compiler may
-// fuse a product into the following sum (one rounding instead of two), and
-// for fp16 inputs also the widening and the final narrowing.
-__device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s, float &o1, float &o2) {
-#pragma clang fp contract(off)
-  const float a = x1 * c;
-  const float b = x2 * s;
-  const float d = x1 * s;
-  const float e = x2 * c;
-  o1 = a - b;
-  o2 = d + e;
-}
-
-template <class E>
-__device__ __forceinline__ Vec16 rotate_chunk(const Vec16 &x, const float *cs, const float *sn);
-
-template <>
-__device__ __forceinline__ Vec16 rotate_chunk<F32>(const Vec16 &x, const float *cs, const float *sn) {
-  const float2 c = *reinterpret_cast<const float2 *>(cs);
-  const float2 s = *reinterpret_cast<const float2 *>(sn);
-  float o[4];
-  rotate_pair(__builtin_bit_cast(float, x.w[0]), __builtin_bit_cast(float, x.w[1]), c.x, s.x, o[0], o[1]);
-  rotate_pair(__builtin_bit_cast(float, x.w[2]), __builtin_bit_cast(float, x.w[3]), c.y, s.y, o[2], o[3]);
-  Vec16 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r.w[i] = __builtin_bit_cast(uint32_t, o[i]);
-  return r;
-}
-
-template <class E>
-__device__ __forceinline__ Vec16 rotate_chunk16(const Vec16 &x, const float *cs, const float *sn) {
-  using T = typename E::type;
-  const float4 c = *reinterpret_cast<const float4 *>(cs);
-  const float4 s = *reinterpret_cast<const float4 *>(sn);
-  const float cc[4] = {c.x, c.y, c.z, c.w};
-  const float ss[4] = {s.x, s.y, s.z, s.w};
-  float f[8];
-  E::widen(x, f);
-  Vec16 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float o1, o2;
-    rotate_pair(f[2 * i], f[2 * i + 1], cc[i], ss[i], o1, o2);
-    const T lo = E::narrow(o1), hi = E::narrow(o2);
-    r.w[i] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
-  }
-  return r;
-}
-template <>
-__device__ __forceinline__ Vec16 rotate_chunk<Bf16>(const Vec16 &x, const float *cs, const float *sn) {
-  return rotate_chunk16<Bf16>(x, cs, sn);
-}
-template <>
-__device__ __forceinline__ Vec16 rotate_chunk<F16>(const Vec16 &x, const float *cs, const float *sn) {
-  return rotate_chunk16<F16>(x, cs, sn);
-}
-
 template <class E>
 __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(const RopeKP p, int64_t t0) {
   constexpr int PAIRS = E::EPL / 2;  // pairs in one 16-byte chunk
@@ -128,9 +72,9 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(const Rope
   if (part == 2) {
     if (p.q == nullptr || c >= p.q_chunks) return;
     const int within = c % p.chunks_per_head;
-    char *at = p.q + t * p.q_stride_bytes + (int64_t)c * 16;
     const int64_t trig = pos * p.half_hd + within * PAIRS;
-    store16(at, rotate_chunk<E>(load16(at), p.cos_table + trig, p.sin_table + trig));
+    store16(p.q_out + t * p.q_out_stride_bytes + (int64_t)c * 16,
+            rotate_chunk<E>(load16(p.q + t * p.q_stride_bytes + (int64_t)c * 16), p.cos_table + trig, p.sin_table + trig));
     return;
   }
   if (p.k_new == nullptr || c >= p.kv_chunks) return;
@@ -170,7 +114,8 @@ int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream) {
   const AppendArgs &ap = a.append;
   const int es = elem_size(ap.dtype);
   RopeKP kp;
-  kp.q = (char *)a.q;
+  kp.q = (const char *)a.q;
+  kp.q_out = (char *)a.q_out;
   kp.k_new = (const char *)ap.k_new;
   kp.v_new = (const char *)ap.v_new;
   kp.k_pool = (char *)ap.k_pool;
@@ -180,6 +125,7 @@ int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream) {
   kp.cos_table = a.cos_table;
   kp.sin_table = a.sin_table;
   kp.q_stride_bytes = a.q_stride_token * es;
+  kp.q_out_stride_bytes = a.q_out_stride_token * es;
   kp.new_stride_bytes = ap.new_stride_token * es;
   kp.stride_block_bytes = ap.pool.stride_block * es;
   kp.stride_head_bytes = ap.pool.stride_head * es;

@@ -257,6 +257,11 @@ class Attention(BaseModule):
     def _dense_on_kernel_width(self, query, key, value, causal, mask):
         b, sq, hn, hd = query.shape
         sk, gn = key.shape[1], key.shape[2]
+        here = _lib.here(query)
+        if here is not None and mask is None:
+            out = _lib.host().dense(query, key, value, causal, 1.0 / self.scale_factor, *here)
+            if out is not None:
+                return out
         key, value = key.contiguous(), value.contiguous()
         # one pool block per sequence: [b, gn, sk, hd] view of the [b, sk, gn, hd] rows
         k_pool, v_pool = key.permute(0, 2, 1, 3), value.permute(0, 2, 1, 3)
@@ -298,6 +303,17 @@ class Attention(BaseModule):
                                           meta.cohort_shared_blocks if cohort > 1 else None, meta.positions,
                                           None if rope is None else rope.cos_emb,
                                           None if rope is None else rope.sin_emb, *here)
+            if out is not None:
+                return out
+        elif here is not None and (rows is None or meta.max_chunk_len == sq):
+            rope = rotary_pos_emb
+            bounds = meta.cu_seqlens_q
+            if bounds is None:
+                bounds = torch.arange(0, (b + 1) * sq, sq, dtype=torch.int32, device=query.device)
+            out = _lib.host().prefill_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
+                                           meta.slot_mapping, bounds, 1.0 / self.scale_factor, meta.positions,
+                                           None if rope is None else rope.cos_emb,
+                                           None if rope is None else rope.sin_emb, *here)
             if out is not None:
                 return out
         if rotary_pos_emb is None:

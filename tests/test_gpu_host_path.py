@@ -81,3 +81,61 @@ def test_what_is_not_ordinary_is_refused_by_name(gpu):
         paged_ops.paged_decode(wl.query, *args[:3], wl.context_lens.long(), wl.max_context_len)
     with pytest.raises(_lib.PagedLibraryError):
         paged_ops.paged_decode(wl.query, *args, wl.max_context_len, min_chunk_tokens=24)
+
+
+def _ragged(gpu, wl, dtype, block, seed):
+    """The layer's view of a prefill workload: padded [b, width] tensors and their metadata."""
+    b, width = len(wl.chunk_lens), wl.max_chunk_len
+    rows = torch.cat([torch.arange(c) + i * width for i, c in enumerate(wl.chunk_lens)])
+    slots = torch.full((b * width,), -1, dtype=torch.int64)
+    slots[rows] = wl.slot_mapping
+    positions = torch.zeros(b * width, dtype=torch.int32)
+    positions[rows] = torch.cat([torch.arange(p, p + c) for p, c in zip(wl.prefix_lens, wl.chunk_lens)]).int()
+    even = all(c == width for c in wl.chunk_lens)
+    meta = PagedAttentionMetadata(
+        block_tables=wl.block_tables.to(gpu), context_lens=wl.context_lens.to(gpu), slot_mapping=slots.to(gpu),
+        max_context_len=int(wl.context_lens.max()), cu_seqlens_q=None if even else wl.cu_seqlens_q.to(gpu),
+        positions=positions.to(gpu), chunk_rows=None if even else rows.to(gpu), max_chunk_len=width)
+    g = torch.Generator(device=gpu).manual_seed(seed)
+
+    def rand(heads):
+        return torch.randn(b, width, heads, wl.hd, generator=g, device=gpu).to(dtype)
+    return meta, rand(wl.hn), rand(wl.gn), rand(wl.gn)
+
+
+@pytest.mark.parametrize("dtype,precision", [(torch.bfloat16, "bf16"), (torch.float16, "fp16"), (torch.float32, "fp32")])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("hn,gn,hd,prefix,chunks", [
+    (6, 2, 64, (0, 90), (1, 70)), (4, 4, 128, (40, 40), (33, 33)), (7, 1, 128, (0, 0), (3, 200)),
+    (4, 4, 32, (0, 30), (0, 45)), (8, 8, 128, (1300, 1400), (250, 256))])   # the last: the long kernel's case
+def test_prefill_step(gpu, monkeypatch, dtype, precision, rope, hn, gn, hd, prefix, chunks):
+    """Padded rows read and written in place, the query rotated inside the
+    kernel: the same bits as packing, rotating and scattering around it."""
+    n = 20 if prefix[0] > 1000 else 4    # (enough workgroups that long sweeps leave the short kernel)
+    wl = workloads.make_prefill_workload(n, hn, gn, hd, *prefix, *chunks, dtype=dtype, seed=hn + hd)
+    meta, query, key, value = _ragged(gpu, wl, dtype, 16, 5)
+    emb = RotaryPositionalEmbedding(hd, max_seq_len=int(wl.context_lens.max())).to(gpu) if rope else None
+    attn = _layer(hn, gn, hd, precision)
+    pools = [(wl.k_pool.to(gpu), wl.v_pool.to(gpu)) for _ in range(2)]
+    left = list(pools)
+
+    def call():
+        return attn(query, key, value, kv_cache=left.pop(), attn_metadata=meta, rotary_pos_emb=emb)
+    native, plain = _both(monkeypatch, call)
+    assert torch.isfinite(native.float()).all() and torch.equal(native, plain)
+    assert torch.equal(pools[0][0], pools[1][0]) and torch.equal(pools[0][1], pools[1][1])
+
+
+@pytest.mark.parametrize("dtype,precision", [(torch.bfloat16, "bf16"), (torch.float32, "fp32")])
+@pytest.mark.parametrize("b,s,hn,gn,hd,masked", [(3, 70, 6, 2, 64, True), (1, 1, 4, 4, 128, False), (2, 129, 4, 1, 128, True),
+                                                  (70, 5, 2, 2, 32, True), (1, 2304, 2, 2, 128, False)])
+def test_dense_call(gpu, monkeypatch, dtype, precision, b, s, hn, gn, hd, masked):
+    """Equal sequences without tables, key and value as two halves of one projection."""
+    g = torch.Generator(device=gpu).manual_seed(s)
+    query = torch.randn(b, s, hn, hd, generator=g, device=gpu).to(dtype)
+    kv = torch.randn(b, s, 2 * gn * hd, generator=g, device=gpu).to(dtype)
+    key, value = (t.view(b, s, gn, hd) for t in kv.chunk(2, dim=-1))
+    mask = torch.ones(1, 1, s, s, device=gpu).tril() if masked else None
+    attn = _layer(hn, gn, hd, precision)
+    native, plain = _both(monkeypatch, lambda: attn(query, key, value, mask))
+    assert torch.equal(native, plain)
