@@ -328,6 +328,25 @@ int ic_paged_prefill(void *out, int64_t out_stride_token,
                      int dtype, void *stream);
 
 /*
+ * Packs a byte mask (nonzero = visible; strides in bytes, key stride 1) of
+ * n_seqs x heads planes of `rows` x `keys` for ic_paged_prefill_ex: one bit per key,
+ * the list of 64-key tiles each 128-row query tile has to visit, and two flags.
+ * It reads the mask once for all heads that share it and for every later call
+ * that uses it.  No counterpart in the reference, which adds its fill value to
+ * the whole score matrix (attention.py:115-117).
+ *
+ *   bits   uint64 [n_seqs*heads][ceil(rows/128)*4][ceil(keys/64)][32]
+ *   lists  int32 [n_seqs*heads][ceil(rows/128)][ceil(keys/64) + 1]
+ *   flags  int32 [2], set to nonzero by the caller; flags[0] is cleared when the
+ *          mask hides a key, flags[1] when it is not the causal pattern
+ *          (row r sees keys j <= (keys - rows) + r)
+ * At most 524 288 keys, 65 535 heads and sequences (else IC_ERR_UNSUPPORTED).
+ */
+int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row,
+                 int n_seqs, int heads, int rows, int keys,
+                 uint64_t *bits, int32_t *lists, int32_t *flags, void *stream);
+
+/*
  * Chunked prefill by descriptor: ic_paged_prefill (same fields, same meaning)
  * plus three forms of input that spare a caller passes over its tensors.
  * Clear the struct first; a field left zero is the plain call's behaviour.
@@ -346,6 +365,12 @@ int ic_paged_prefill(void *out, int64_t out_stride_token,
  *                    row r of q is rotated as it is loaded, by table row
  *                    positions[r], with the arithmetic and the rounding of
  *                    ic_rope_kv_append.  The keys in the pool are rotated already.
+ *   mask_bits, mask_lists, mask_plane_seq, mask_plane_head
+ *                    mask_bits != NULL: a general mask of max_chunk_len rows and
+ *                    uniform_context keys, packed by ic_mask_pack (equal sequences
+ *                    only, causal = 0); sequence i and head h use plane
+ *                    i*mask_plane_seq + h*mask_plane_head of it.  Semantics of
+ *                    ic_paged_prefill_masked.
  */
 typedef struct ic_prefill_call {
   void *out;
@@ -371,6 +396,9 @@ typedef struct ic_prefill_call {
   const float *cos_table;
   const float *sin_table;
   int64_t table_rows;
+  const uint64_t *mask_bits;
+  const int32_t *mask_lists;
+  int mask_plane_seq, mask_plane_head;
 } ic_prefill_call;
 int ic_paged_prefill_ex(const ic_prefill_call *call, void *stream);
 

@@ -90,6 +90,10 @@ SIGNATURES = {
         c_int, c_int, c_int, c_int,             # hn, gn, hd, block_size
         c_int64, c_float, c_int,                # num_blocks, scale, causal
         c_int, c_void_p]),                      # dtype, stream
+    "ic_mask_pack": (c_int, [
+        c_void_p, c_int64, c_int64, c_int64,    # mask, strides: seq, head, row
+        c_int, c_int, c_int, c_int,             # n_seqs, heads, rows, keys
+        c_void_p, c_void_p, c_void_p, c_void_p]),   # bits, lists, flags, stream
     "ic_paged_prefill_ex": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_paged_prefill_masked": (c_int, [
         c_void_p, c_int64, c_void_p, c_int64,   # out, out_stride, q, q_stride

@@ -257,10 +257,30 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
   return out;
 }
 
+// A byte mask [1 or b, 1 or hn, sq, sk] (nonzero = visible) packed for the prefill kernels: (bits, lists,
+// flags), see ic_mask_pack.  The flags are still on the device.
+c10::optional<std::tuple<Tensor, Tensor, Tensor>> pack_mask(const Tensor &mask, int64_t device, int64_t stream) {
+  if (mask.dim() != 4 || mask.scalar_type() != at::kByte || !on(mask, device) || mask.numel() == 0 ||
+      mask.stride(3) != 1)
+    return c10::nullopt;
+  const int64_t n = mask.size(0), heads = mask.size(1), rows = mask.size(2), keys = mask.size(3);
+  const int64_t qtiles = (rows + 127) / 128, tiles = (keys + 63) / 64;
+  const Tensor bits = at::empty({n * heads, qtiles * 4, tiles, 32}, mask.options().dtype(at::kLong));
+  const Tensor lists = at::empty({n * heads, qtiles, tiles + 1}, mask.options().dtype(at::kInt));
+  const Tensor flags = at::ones({2}, mask.options().dtype(at::kInt));
+  if (ic_mask_pack(mask.data_ptr<uint8_t>(), mask.stride(0), mask.stride(1), mask.stride(2), (int)n, (int)heads,
+                   (int)rows, (int)keys, reinterpret_cast<uint64_t *>(bits.data_ptr<int64_t>()),
+                   lists.data_ptr<int32_t>(), flags.data_ptr<int32_t>(), (void *)stream) != IC_OK)
+    return c10::nullopt;
+  return std::make_tuple(bits, lists, flags);
+}
+
 // The dense call: query [b, sq, hn, hd] on key / value [b, sk, gn, hd], which the kernel walks as a pool of
 // one block per sequence, at whatever strides they have.
-OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, bool causal, double scale,
-                int64_t device, int64_t stream) {
+// `bits`, `lists`: a packed mask of mask_seqs x mask_heads planes (1 or b, 1 or hn).
+OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, bool causal, const OptTensor &bits,
+                const OptTensor &lists, int64_t mask_seqs, int64_t mask_heads, double scale, int64_t device,
+                int64_t stream) {
   if (query.dim() != 4 || key.dim() != 4 || key.size(1) == 0 || query.size(1) == 0) return c10::nullopt;
   const Pool p(key.permute({0, 2, 1, 3}), value.permute({0, 2, 1, 3}), device);
   const int64_t b = query.size(0), s = query.size(1), hn = query.size(2);
@@ -270,6 +290,17 @@ OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, boo
   const Tensor out = at::empty({b, s, hn * p.hd}, query.options());
   ic_prefill_call c = prefill_call(out, query, p, b, s, hn, scale, causal);
   c.uniform_context = (int)p.bs;
+  if (bits.has_value()) {
+    const int64_t planes = mask_seqs * mask_heads, qtiles = (s + 127) / 128, tiles = (p.bs + 63) / 64;
+    if (causal || !lists.has_value() || (mask_seqs != 1 && mask_seqs != b) || (mask_heads != 1 && mask_heads != hn) ||
+        !index_vector(*bits, at::kLong, planes * qtiles * 4 * tiles * 32, device) ||
+        !index_vector(*lists, at::kInt, planes * qtiles * (tiles + 1), device))
+      return c10::nullopt;
+    c.mask_bits = reinterpret_cast<const uint64_t *>(bits->data_ptr<int64_t>());
+    c.mask_lists = lists->data_ptr<int32_t>();
+    c.mask_plane_head = mask_heads > 1 ? 1 : 0;
+    c.mask_plane_seq = mask_seqs > 1 ? (int)mask_heads : 0;
+  }
   if (ic_paged_prefill_ex(&c, (void *)stream) != IC_OK) return c10::nullopt;
   return out;
 }
@@ -282,4 +313,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_step", &decode_step);
   m.def("prefill_step", &prefill_step);
   m.def("dense", &dense);
+  m.def("pack_mask", &pack_mask);
 }

@@ -190,6 +190,11 @@ int prefill_checked(const ic_prefill_call &c, const uint8_t *mask, int64_t mask_
     if (c.block_table_stride <= 0 || c.row_pitch < 0 || (c.row_pitch > 0 && c.row_pitch < c.max_chunk_len))
       return IC_ERR_BAD_SHAPE;
   }
+  if (c.mask_bits != nullptr) {
+    if (c.mask_lists == nullptr) return IC_ERR_NULL_POINTER;
+    if (c.context_lens != nullptr || c.causal || mask != nullptr || c.mask_plane_seq < 0 || c.mask_plane_head < 0)
+      return IC_ERR_BAD_SHAPE;
+  }
   if (c.row_pitch > 0 && c.row_pitch * c.n_seqs > 0x7fffffff) return IC_ERR_UNSUPPORTED;
   if (c.out_stride_token < (int64_t)c.hn * c.hd || c.q_stride_token < (int64_t)c.hn * c.hd) return IC_ERR_BAD_SHAPE;
   if (!aligned16(c.q) || !aligned16(c.out) || !aligned16(c.k_pool) || !aligned16(c.v_pool) ||
@@ -231,6 +236,10 @@ int prefill_checked(const ic_prefill_call &c, const uint8_t *mask, int64_t mask_
   a.cos_table = c.cos_table;
   a.sin_table = c.sin_table;
   a.table_rows = c.table_rows;
+  a.mask_bits = c.mask_bits;
+  a.mask_lists = c.mask_lists;
+  a.mask_plane_seq = c.mask_plane_seq;
+  a.mask_plane_head = c.mask_plane_head;
   return ic::launch_paged_prefill(a, static_cast<hipStream_t>(stream));
 }
 
@@ -451,6 +460,16 @@ int ic_paged_decode_static(void *out, int64_t out_stride_seq, const void *q, int
                         context_lens, n_seqs, hn, gn, hd, block_size, num_blocks, max_context_len,
                         scale, min_chunk_tokens, 1, nullptr, ws, (size_t)IC_STATIC_SCRATCH_BYTES,
                         kStaticMaxWaves, dtype, stream);
+}
+
+int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,
+                 int heads, int rows, int keys, uint64_t *bits, int32_t *lists, int32_t *flags, void *stream) {
+  if (n_seqs < 0 || heads < 0 || rows < 0 || keys < 0 || stride_seq < 0 || stride_head < 0 || stride_row < 0)
+    return IC_ERR_BAD_SHAPE;
+  if (n_seqs == 0 || heads == 0 || rows == 0 || keys == 0) return IC_OK;
+  if (!mask || !bits || !lists || !flags) return IC_ERR_NULL_POINTER;
+  return ic::launch_mask_pack(mask, stride_seq, stride_head, stride_row, n_seqs, heads, rows, keys, bits, lists, flags,
+                              static_cast<hipStream_t>(stream));
 }
 
 int ic_paged_prefill_ex(const ic_prefill_call *call, void *stream) {

@@ -117,6 +117,12 @@ struct PrefillArgs {
   const float *cos_table = nullptr;
   const float *sin_table = nullptr;
   int64_t table_rows = 0;
+  // Packed mask (mask_pack.hip) of equal sequences: words and tile lists, one plane per sequence and head
+  // or one for all of them (the strides 0).
+  const uint64_t *mask_bits = nullptr;
+  const int32_t *mask_lists = nullptr;
+  int mask_plane_seq = 0;   // planes from one sequence to the next
+  int mask_plane_head = 0;  // ... from one head to the next
 };
 
 // Each returns IC_OK, IC_ERR_UNSUPPORTED (no kernel built for this
@@ -125,6 +131,9 @@ int launch_kv_append(const AppendArgs &a, hipStream_t stream);
 int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream);
 int launch_paged_decode(const DecodeArgs &a, hipStream_t stream);
 int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream);
+int launch_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,
+                     int heads, int rows, int keys, uint64_t *bits, int32_t *lists, int32_t *flags,
+                     hipStream_t stream);
 
 constexpr int kDefaultMinChunkTokens = 16;  // one tile: short batches spread over all waves
 // Upper bound on the waves of one decode launch (sizes the workspace): 8 waves

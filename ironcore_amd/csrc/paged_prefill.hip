@@ -558,7 +558,8 @@ int launch_mode(const PrefillKP &kp, const PrefillArgs &a, hipStream_t stream) {
   // A one-column block table means one block per sequence, of any length.
   const bool masked = a.mask != nullptr;
   const bool single = a.block_tables == nullptr || a.block_table_stride == 1;
-  if (single && !masked && prefill_takes_short(a)) return launch_paged_prefill_short(kp, a, stream);
+  if (single && !masked && (a.mask_bits != nullptr || prefill_takes_short(a)))
+    return launch_paged_prefill_short(kp, a, stream);
   if (single)
     return masked ? launch_hd<M, true, true>(kp, a, stream) : launch_hd<M, true, false>(kp, a, stream);
   if (kp.block_size < 16 || kp.block_size % 16 != 0) return IC_ERR_UNSUPPORTED;  // whole 16-token groups
@@ -616,6 +617,12 @@ int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream) {
   kp.sin_table = a.sin_table;
   kp.table_rows = a.table_rows > 0x7fffffff ? 0x7fffffff : (int)a.table_rows;
   kp.half_hd = a.hd / 2;
+  kp.mask_bits = a.mask_bits;
+  kp.mask_lists = a.mask_lists;
+  kp.mask_plane_seq = a.mask_plane_seq;
+  kp.mask_plane_head = a.mask_plane_head;
+  kp.mask_tiles = (a.uniform_context + 63) / 64;
+  kp.mask_qtiles = (a.max_chunk_len + 127) / 128;
   if ((int64_t)a.max_chunk_len >= (int64_t)65535 * 128 || a.hn > 65535 || a.n_seqs > 65535)
     return IC_ERR_UNSUPPORTED;
   // The 16-bit kernel addresses a block with 32-bit byte offsets (a block, and in a block table's

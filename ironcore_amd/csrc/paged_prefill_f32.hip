@@ -45,7 +45,8 @@ constexpr int kF32Threads = kF32Waves * kWave;
 constexpr int kF32BM = kF32Waves * 32;  // query rows per workgroup
 constexpr int kF32BN = 32;              // tokens per K/V tile
 
-template <int HD, bool SINGLE, bool MASK>
+// MASK: 0 the causal rule or none, 1 a byte mask, 2 a packed one (equal sequences).
+template <int HD, bool SINGLE, int MASK>
 __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const PrefillKP p) {
   constexpr int NJ = HD / 8;            // 16-byte operand groups of the QK contraction
   constexpr int OB = HD / 32;           // 32-wide blocks of the output head dim
@@ -68,7 +69,7 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   int L = equal ? p.uniform_context : p.context_lens[seq];
   int C = equal ? p.max_chunk : p.cu_seqlens_q[seq + 1] - q_lo;
   if (p.row_pitch > 0) q_lo = (int)(seq * p.row_pitch);
-  const bool causal = !MASK && p.causal;
+  const bool causal = MASK == 0 && p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
   if (p.row_pitch > 0 && C < p.max_chunk)
@@ -114,7 +115,10 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
 
   int kv_end = causal ? P + q0 + kF32BM : L;  // keys any row of this workgroup can see
   kv_end = kv_end < L ? kv_end : L;
-  const int n_tiles = (kv_end + kF32BN - 1) / kF32BN;
+  // (a packed mask's list is of 64-key tiles: two tiles of this kernel each)
+  MaskList list;
+  if constexpr (MASK == 2) list.open(p, seq, h, q0 / kF32BM, wave);
+  const int n_tiles = MASK == 2 ? 2 * list.count : (kv_end + kF32BN - 1) / kF32BN;
   int my_end = causal ? P + q0 + wave * 32 + 32 : L;
   my_end = my_end < kv_end ? my_end : kv_end;
   const int my_tiles = (my_end > 0 && q0 + wave * 32 < C) ? (my_end + kF32BN - 1) / kF32BN : 0;
@@ -124,7 +128,12 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   const int c4 = tid % F4R;  // its 16-byte piece of the row
   const int32_t *table_row = p.block_tables + (int64_t)seq * p.bt_stride;
   const int64_t head_off = (int64_t)kvh * p.stride_head + c4 * 4;
-  auto fetch = [&](int tile, Vec16 *kr, Vec16 *vr) {
+  // tile t of the sweep: its number, and under a packed mask the class of this wave's rows and the words
+  auto number = [&](int t) { return MASK == 2 ? 2 * MaskList::tile(list.entry(t >> 1)) + (t & 1) : t; };
+  uint32_t word = 0, word_next = 0;  // packed mask: this lane's row, tile t and t + 1
+  auto fetch = [&](int t, Vec16 *kr, Vec16 *vr) {
+    const int tile = number(t);
+    if constexpr (MASK == 2) word_next = reinterpret_cast<const uint32_t *>(list.words)[((tile >> 1) * 32 + n) * 2 + (tile & 1)];
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       int tok = tile * kF32BN + r0 + i * RP;
@@ -168,7 +177,7 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
     }
   };
   // ---- softmax of the tile's scores: s -> probabilities, m, l (and o when the reference moves) ----
-  auto softmax = [&](int tile) {
+  auto softmax = [&](int tile, int kind) {
     // s[i] is (token tile*32 + 4*hh + 8*(i/4) + i%4, query n)
     const int tok_base = tile * kF32BN + 4 * hh;
     const bool need_mask = causal ? (tile * kF32BN + kF32BN - 1 > P + q0 + wave * 32) : (tile * kF32BN + kF32BN > L);
@@ -179,7 +188,7 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
         s[i] = tok > limit ? kNegInf : s[i];
       }
     }
-    if constexpr (MASK) {  // keys the caller's mask hides from this lane's query row
+    if constexpr (MASK == 1) {  // keys the caller's mask hides from this lane's query row
       const uint8_t *mrow = p.mask + (int64_t)seq * p.mask_stride_seq + (int64_t)h * p.mask_stride_head +
                             (int64_t)qrow * p.mask_stride_row;
       // unconditional loads from an index clamped into the part of the row that exists and counts
@@ -195,6 +204,14 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
         const int tok = tok_base + 8 * (i / 4) + (i & 3);
         const bool hidden = (tok <= limit) & ((tok >= p.mask_keys) | (seen[i] == 0));
         s[i] = hidden ? kHiddenScore : s[i];
+      }
+    }
+    if (MASK == 2 && kind == 1) {
+      const uint32_t w = word >> (4 * hh);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const bool hidden = (w & (1u << (8 * (i / 4) + (i & 3)))) == 0;
+        s[i] = hidden ? fminf(s[i], kHiddenScore) : s[i];
       }
     }
     float mx = kNegInf;
@@ -241,10 +258,14 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   __syncthreads();
   for (int t = 0; t < n_tiles; ++t) {
     const bool more = t + 1 < n_tiles;  // the same for every wave of the workgroup
+    word = word_next;
     if (more) fetch(t + 1, kr, vr);
-    if (t < my_tiles) {
+    const int tile = number(t);
+    const int kind = MASK == 2 ? MaskList::kind(list.entry(t >> 1), wave) : 2;
+    // (the second half of a packed mask's last tile may lie past the context altogether)
+    if (MASK == 2 ? (kind != 0 && tile * kF32BN < L && q0 + wave * 32 < C) : t < my_tiles) {
       scores(t & 1);
-      softmax(t);
+      softmax(tile, kind);
       weighted_values(t & 1);
     }
     // buffer (t + 1) & 1 was last read for tile t - 1, before the barrier that ended that round
@@ -271,7 +292,7 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   }
 }
 
-template <bool SINGLE, bool MASK>
+template <bool SINGLE, int MASK>
 int launch_hd(const PrefillKP &kp, int hd, dim3 grid, hipStream_t stream) {
   switch (hd) {
     case 32:
@@ -297,11 +318,12 @@ int launch_paged_prefill_f32(PrefillKP kp, const PrefillArgs &a, hipStream_t str
   if (wgs_x > 0x7fffffff || a.n_seqs > 65535) return IC_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs_x, (unsigned)a.n_seqs);
   const bool masked = a.mask != nullptr;
+  if (a.mask_bits != nullptr) return launch_hd<true, 2>(kp, a.hd, grid, stream);
   // A one-column block table means one block per sequence, of any length.
   if (a.block_tables == nullptr || a.block_table_stride == 1)
-    return masked ? launch_hd<true, true>(kp, a.hd, grid, stream) : launch_hd<true, false>(kp, a.hd, grid, stream);
+    return masked ? launch_hd<true, 1>(kp, a.hd, grid, stream) : launch_hd<true, 0>(kp, a.hd, grid, stream);
   if (kp.block_size < 1) return IC_ERR_UNSUPPORTED;
-  return masked ? launch_hd<false, true>(kp, a.hd, grid, stream) : launch_hd<false, false>(kp, a.hd, grid, stream);
+  return masked ? launch_hd<false, 1>(kp, a.hd, grid, stream) : launch_hd<false, 0>(kp, a.hd, grid, stream);
 }
 
 }  // namespace prefill

@@ -22,6 +22,13 @@
 //    (TG = 2) on the same query rows, which take the tiles in turn and merge
 //    their sums through LDS at the end: half the tiles one after the other.
 //
+//  * PACKED: a general mask as mask_pack.hip leaves it.  The sweep visits the tiles
+//    of the query tile's list; a wave skips the ones its 32 rows do not see and
+//    applies the words (fetched with the tile, 256 bytes per wave) only where they
+//    are mixed.  2 x 1 024 tokens in packed documents, 16 heads of 64: 149 us with
+//    the byte mask of the long kernel (32 byte loads per lane and tile, every tile
+//    walked), 11.9 us here, launch to launch.
+//
 // Bound by the latency of a tile (load, two products and a softmax in one wave's
 // instruction stream, about 1 us at head dim 128) at the sizes it is for; 80
 // sequences of 129 tokens, 12 heads of 64, without a cache: 24.1 -> 19.8 us; 9
@@ -40,7 +47,7 @@ constexpr int kBN = 64;         // tokens per K/V tile
 
 constexpr int kShortBuffers = 2;  // LDS buffers per pool and tile group
 
-template <class M, int HD, bool SINGLE, int TG>
+template <class M, int HD, bool SINGLE, int TG, bool PACKED>
 __global__ __launch_bounds__(TG *kShortWaves *kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 2 : 4)))
 void paged_prefill_short_kernel(const PrefillKP p) {
   using T = typename M::T;
@@ -59,6 +66,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   constexpr int kMergeBytes = TG > 1 ? kShortWaves * (OB * 16 + 2) * kWave * 4 : 0;
   constexpr int kTileBytes = TG * 2 * NB * TILEB;
   __shared__ __attribute__((aligned(1024))) char s_tiles[kTileBytes > kMergeBytes ? kTileBytes : kMergeBytes];
+  __shared__ uint64_t s_words[PACKED ? TG * kShortWaves * NB * 32 : 1];  // packed mask: a wave's words of its tiles
 
   // XCD-aware placement as in the long kernel: the workgroups of one (sequence, KV head) unit get ids
   // that differ by a multiple of 8.
@@ -76,7 +84,8 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
   if (p.row_pitch > 0 && C < p.max_chunk)
     zero_padding<HD, 2, TG * kShortWaves * kWave>(p, q_lo, C, kvh * p.group, p.group, within / kXcds, per_unit);
-  const int n_blocks = (C + 31) >> 5;  // wave blocks per head
+  // wave blocks per head (a packed mask's lists belong to 128 rows of one head: four blocks, unused ones too)
+  const int n_blocks = PACKED ? ((C + 127) >> 7) * kShortWaves : (C + 31) >> 5;
   const int total = n_blocks * p.group;
   // The last blocks (the longest sweeps) first; in the slices that share the CUs with the first ones when
   // the whole grid is resident, last: a CU then holds a long and a short sweep, not two of the same length.
@@ -92,10 +101,10 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   char *const tiles_v = tiles_k + NB * TILEB;
   const int n = lane & 31;  // query column of this lane within the wave's 32-row block
   const int hh = lane >> 5;  // which half of each k-step this lane feeds
-  const bool mine = v0 + wave < total;
-  const int v = mine ? v0 + wave : total - 1;
+  const int v = v0 + wave < total ? v0 + wave : total - 1;
   const int head = v / n_blocks;
   const int row0 = (v - head * n_blocks) * 32;
+  const bool mine = v0 + wave < total && row0 < C;
   const int h = kvh * p.group + head;
   const int my_q = row0 + n;
   if (L == 0) {  // query rows without any key (not under the causal rule): zero rows
@@ -134,7 +143,9 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const int last_row = v0 / n_blocks == v_last / n_blocks ? (v_last % n_blocks) * 32 + 32 : C;
   int kv_end = causal ? P + last_row : L;
   kv_end = kv_end < L ? kv_end : L;
-  const int n_tiles = __builtin_amdgcn_readfirstlane((kv_end + kBN - 1) / kBN);
+  MaskList list;
+  if constexpr (PACKED) list.open(p, seq, h, row0 >> 7, wave);
+  const int n_tiles = PACKED ? list.count : __builtin_amdgcn_readfirstlane((kv_end + kBN - 1) / kBN);
   int my_end = causal ? P + row0 + 32 : L;
   my_end = my_end < kv_end ? my_end : kv_end;
   const int my_tiles = mine ? (my_end + kBN - 1) / kBN : 0;
@@ -159,30 +170,41 @@ void paged_prefill_short_kernel(const PrefillKP p) {
     src_v[i] = (uint32_t)((int64_t)r * p.stride_token * 2 + (cc ^ tile_swizzle_v<CPR>(r)) * 16) - i * WR * ROWB;
   }
   const uint32_t lds_k = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)&s_tiles[0] + (uint32_t)(tg * 2 * NB * TILEB);
-  auto clamp_tile = [&](int tile) { return tile < n_tiles ? tile : n_tiles - 1; };
-  auto lookup = [&](int tile, int32_t &ent, int &rem) {
-    const int first = clamp_tile(tile) * kBN + 16 * wave;
-    int blk = SINGLE ? 0 : block_of(first);
-    rem = first - blk * p.block_size;
-    blk = blk < last_blk ? blk : last_blk;
-    ent = SINGLE && p.block_tables == nullptr ? seq : table_row[blk];
+  // What round r visits: `tile` (with a packed mask the list's entry, the classes above the tile's number), the
+  // table entry of this wave's group and the group's first row within its block.
+  struct Stop {
+    int32_t tile, ent;
+    int rem;
   };
-  auto fetch = [&](int tile, int buf, int32_t ent, int rem) {
-    int phys = ent;
+  auto number = [](const Stop &st) { return PACKED ? MaskList::tile(st.tile) : st.tile; };
+  auto lookup = [&](int r) {
+    Stop st;
+    st.tile = PACKED ? list.entry(r) : r < n_tiles ? r : n_tiles - 1;
+    const int first = number(st) * kBN + 16 * wave;
+    int blk = SINGLE ? 0 : block_of(first);
+    st.rem = first - blk * p.block_size;
+    if (SINGLE) st.rem = first;
+    blk = blk < last_blk ? blk : last_blk;
+    st.ent = SINGLE && p.block_tables == nullptr ? seq : table_row[blk];
+    return st;
+  };
+  const uint32_t lds_words =
+      (uint32_t)(size_t)(__attribute__((address_space(3))) char *)&s_words[0] + (uint32_t)((tg * kShortWaves + wave) * NB * 256);
+  auto fetch = [&](const Stop &st, int buf) {
+    int phys = st.ent;
     // A corrupt table entry must not become an out-of-pool address.
     phys = phys < 0 ? 0 : phys;
     phys = phys > last_phys ? last_phys : phys;
     const uint32_t to = __builtin_amdgcn_readfirstlane(lds_k + (uint32_t)(buf * TILEB + 16 * wave * ROWB));
     const uint64_t block = head_bytes + (uint64_t)(uint32_t)phys * block_bytes;
     if (SINGLE) {
-      const int first = clamp_tile(tile) * kBN + 16 * wave;
 #pragma unroll
       for (int pool = 0; pool < 2; ++pool) {
         const char *base = (pool ? p.v_pool : p.k_pool) + block;
 #pragma unroll
         for (int i = 0; i < NST; ++i) {
           const int r = i * WR + rsub;
-          int row = first + r;
+          int row = st.rem + r;
           row = row < L ? row : L - 1;
           const int chunk = cc ^ (pool ? tile_swizzle_v<CPR>(r) : tile_swizzle_k<CPR>(r));
           const char *src = base + (int64_t)row * p.stride_token * 2 + chunk * 16;
@@ -191,7 +213,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
         }
       }
     } else {
-      const uint64_t group = block + (uint32_t)rem * token_bytes;
+      const uint64_t group = block + (uint32_t)st.rem * token_bytes;
 #pragma unroll
       for (int pool = 0; pool < 2; ++pool) {
         const char *base = (pool ? p.v_pool : p.k_pool) + group;
@@ -201,6 +223,11 @@ void paged_prefill_short_kernel(const PrefillKP p) {
           asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2"
                        :: "v"(pool ? src_v[i] : src_k[i]), "s"(base), "n"(i * WR * ROWB) : "memory", "m0");
       }
+    }
+    if constexpr (PACKED) {
+      const char *src = reinterpret_cast<const char *>(list.words) + (int64_t)number(st) * 256 + lane * 4;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                   :: "s"((uint32_t)__builtin_amdgcn_readfirstlane(lds_words + buf * 256)), "v"(src) : "memory", "m0");
     }
   };
 
@@ -236,7 +263,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
     }
     __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
   };
-  auto softmax = [&](int tile) {
+  auto softmax = [&](int tile, int kind, int buf) {
     // s[tb][i] is (token tile*64 + tb*32 + 4*hh + 8*(i/4) + i%4, query n)
     const int tok_base = tile * kBN + 4 * hh;
     if (tile >= mask_from) {  // tiles that touch the causal diagonal (or the context end)
@@ -247,6 +274,18 @@ void paged_prefill_short_kernel(const PrefillKP p) {
           const int tok = tok_base + tb * 32 + 8 * (i / 4) + (i & 3);
           s[tb][i] = tok > limit ? kNegInf : s[tb][i];
         }
+    }
+    if (PACKED && kind == 1) {  // keys the mask hides from this lane's row (beyond the context -inf stays)
+      const uint64_t word = s_words[((tg * kShortWaves + wave) * NB + buf) * 32 + n];
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) {
+        const uint32_t w = (uint32_t)(word >> (32 * tb)) >> (4 * hh);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const bool hidden = (w & (1u << (8 * (i / 4) + (i & 3)))) == 0;
+          s[tb][i] = hidden ? fminf(s[tb][i], kHiddenScore) : s[tb][i];
+        }
+      }
     }
     float mx = kNegInf;
 #pragma unroll
@@ -304,39 +343,36 @@ void paged_prefill_short_kernel(const PrefillKP p) {
     __builtin_amdgcn_sched_group_barrier(0x008, kAheadV, 0);
   };
 
-  // ---- sweep: round i is this group's tile i * TG + tg, computed while the next NB - 1 are on their way ----
-  int32_t ent;
-  int rem;
+  // ---- sweep: round i is this group's tile i * TG + tg, computed while the next one is on its way ----
+  static_assert(NB == 2, "the wait below is for every load in flight");
   const int rounds = (n_tiles + TG - 1) / TG;
-#pragma unroll
-  for (int i = 0; i < NB - 1; ++i) {
-    lookup(i * TG + tg, ent, rem);
-    fetch(i * TG + tg, i, ent, rem);
-  }
-  lookup((NB - 1) * TG + tg, ent, rem);
-  int buf = 0;
+  Stop now = lookup(tg);
+  fetch(now, 0);
+  Stop next = lookup(TG + tg);
   for (int i = 0; i < rounds; ++i) {
     const int k = i * TG + tg;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * 2 * NST) : "memory");  // this wave's groups of tile k
+    const int buf = i & 1;
+    const int tile = number(now);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's groups of the round's tile
     // rows of a V tile past the context become zeros: their probabilities are zeros, but 0 x NaN is not,
     // and unused pool slots may hold anything (only a sweep's last tile can reach past the context)
-    if (k == n_tiles - 1 && k * kBN + 16 * wave + 16 > L) {
+    if (tile * kBN + 16 * wave + 16 > L) {
       char *at = tiles_v + buf * TILEB + 16 * wave * ROWB + lane * 16;
-      const int row = k * kBN + 16 * wave + rsub;
+      const int row = tile * kBN + 16 * wave + rsub;
 #pragma unroll
       for (int j = 0; j < NST; ++j)
         if (row + j * WR >= L) store16(at + j * WR * ROWB, Vec16{{0u, 0u, 0u, 0u}});
     }
     __syncthreads();  // the round's tiles are whole, and nobody reads the buffer of the round before any more
-    // (unconditional, so that the wait above is exact: past the sweep the last tile is fetched again)
-    fetch(k + (NB - 1) * TG, buf == 0 ? NB - 1 : buf - 1, ent, rem);
-    lookup(k + NB * TG, ent, rem);
-    if (k < my_tiles) {
+    fetch(next, buf ^ 1);  // (past the sweep the last tile is fetched again: nobody reads it)
+    const int kind = PACKED ? MaskList::kind(now.tile, wave) : 2;
+    now = next;
+    next = lookup(k + 2 * TG);
+    if (PACKED ? (k < n_tiles && mine && kind != 0) : k < my_tiles) {
       scores(buf);
-      softmax(k);
+      softmax(tile, kind, buf);
       weighted_values(buf);
     }
-    buf = buf + 1 < NB ? buf + 1 : 0;
   }
   // every load this wave issued must have landed before its LDS is given up
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -388,18 +424,18 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   }
 }
 
-template <class M, bool SINGLE, int TG>
+template <class M, bool SINGLE, int TG, bool PACKED>
 int launch_short_hd(const PrefillKP &kp, int hd, unsigned wgs, hipStream_t stream) {
   const dim3 grid(wgs), block(TG * kShortWaves * kWave);
   switch (hd) {
     case 32:
-      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 32, SINGLE, TG>), grid, block, 0, stream, kp);
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 32, SINGLE, TG, PACKED>), grid, block, 0, stream, kp);
       break;
     case 64:
-      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 64, SINGLE, TG>), grid, block, 0, stream, kp);
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 64, SINGLE, TG, PACKED>), grid, block, 0, stream, kp);
       break;
     case 128:
-      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 128, SINGLE, TG>), grid, block, 0, stream, kp);
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 128, SINGLE, TG, PACKED>), grid, block, 0, stream, kp);
       break;
     default:
       return IC_ERR_UNSUPPORTED;
@@ -409,10 +445,14 @@ int launch_short_hd(const PrefillKP &kp, int hd, unsigned wgs, hipStream_t strea
 
 template <class M>
 int launch_short_type(const PrefillKP &kp, const PrefillArgs &a, unsigned wgs, bool split, hipStream_t stream) {
-  const bool single = a.block_tables == nullptr || a.block_table_stride == 1;
-  if (split)
-    return single ? launch_short_hd<M, true, 2>(kp, a.hd, wgs, stream) : launch_short_hd<M, false, 2>(kp, a.hd, wgs, stream);
-  return single ? launch_short_hd<M, true, 1>(kp, a.hd, wgs, stream) : launch_short_hd<M, false, 1>(kp, a.hd, wgs, stream);
+  if (a.mask_bits != nullptr)
+    return split ? launch_short_hd<M, true, 2, true>(kp, a.hd, wgs, stream)
+                 : launch_short_hd<M, true, 1, true>(kp, a.hd, wgs, stream);
+  if (a.block_tables == nullptr || a.block_table_stride == 1)
+    return split ? launch_short_hd<M, true, 2, false>(kp, a.hd, wgs, stream)
+                 : launch_short_hd<M, true, 1, false>(kp, a.hd, wgs, stream);
+  return split ? launch_short_hd<M, false, 2, false>(kp, a.hd, wgs, stream)
+               : launch_short_hd<M, false, 1, false>(kp, a.hd, wgs, stream);
 }
 
 }  // namespace
@@ -437,7 +477,8 @@ int launch_short_type(const PrefillKP &kp, const PrefillArgs &a, unsigned wgs, b
 // faster.
 namespace {
 int64_t short_workgroups_per_unit(const PrefillArgs &a) {
-  const int64_t blocks = (int64_t)((a.max_chunk_len + 31) / 32) * (a.hn / a.gn);
+  const int64_t per_head = a.mask_bits ? (int64_t)((a.max_chunk_len + 127) / 128) * kShortWaves : (a.max_chunk_len + 31) / 32;
+  const int64_t blocks = per_head * (a.hn / a.gn);
   return (blocks + kShortWaves - 1) / kShortWaves;
 }
 int64_t context_bound(const PrefillArgs &a) {

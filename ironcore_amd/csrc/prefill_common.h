@@ -52,6 +52,12 @@ struct PrefillKP {
   const float *sin_table;
   int table_rows;
   int half_hd;
+  const uint64_t *mask_bits;   // packed mask: see mask_pack.hip
+  const int32_t *mask_lists;
+  int mask_plane_seq;
+  int mask_plane_head;
+  int mask_tiles;    // 64-key tiles of a mask row
+  int mask_qtiles;   // 128-row query tiles of a plane
 };
 
 constexpr float kNegInf = -__builtin_huge_valf();
@@ -173,6 +179,24 @@ __device__ __forceinline__ void zero_padding(const PrefillKP &p, int64_t row0, i
     for (int c = threadIdx.x; c < chunks; c += THREADS) store16(row + c * 16, Vec16{{0u, 0u, 0u, 0u}});
   }
 }
+
+// The tiles a query tile visits under a packed mask: entry i (clamped to the last one) holds the tile and the
+// classes of the query tile's four 32-row groups.
+struct MaskList {
+  typedef const __attribute__((address_space(4))) int32_t *ScalarPtr;  // scalar (SMEM) loads
+  ScalarPtr at;
+  int count;
+  const uint64_t *words;  // of the wave's row group: [tile][32]
+  __device__ __forceinline__ void open(const PrefillKP &p, int seq, int head, int qtile, int group) {
+    const int64_t plane = (int64_t)seq * p.mask_plane_seq + (int64_t)head * p.mask_plane_head;
+    at = (ScalarPtr)(unsigned long long)(p.mask_lists + (plane * p.mask_qtiles + qtile) * (p.mask_tiles + 1));
+    count = at[0];
+    words = p.mask_bits + ((plane * p.mask_qtiles + qtile) * 4 + group) * p.mask_tiles * 32;
+  }
+  __device__ __forceinline__ int32_t entry(int i) const { return at[1 + (i < count ? i : count - 1)]; }
+  static __device__ __forceinline__ int tile(int32_t e) { return e & 0xffff; }
+  static __device__ __forceinline__ int kind(int32_t e, int group) { return (e >> (16 + 2 * group)) & 3; }
+};
 
 // The rotary tables' row of query row `row` (clamped into them).
 __device__ __forceinline__ int64_t rope_row(const PrefillKP &p, int64_t row) {

@@ -68,6 +68,22 @@ def _mask_version(mask):
 
 
 @dataclass
+class PackedMask:
+    """A general mask as the prefill kernels read it (``ic_mask_pack``): a bit
+    per key and the K/V tiles each query tile has to visit."""
+    bits: torch.Tensor    # int64 [planes, 4 * query tiles, key tiles, 32]
+    lists: torch.Tensor   # int32 [planes, query tiles, key tiles + 1]
+    shape: tuple          # of the byte mask: (1 or b, 1 or hn, sq, sk)
+
+    def bytes(self) -> torch.Tensor:
+        """The byte mask again (uint8), for a call the packed kernels do not take."""
+        n, heads, rows, keys = self.shape
+        words = self.bits.permute(0, 1, 3, 2).reshape(n * heads, -1, self.bits.shape[2], 1)
+        bit = (words >> torch.arange(64, device=words.device)) & 1
+        return bit.reshape(n, heads, bit.shape[1], -1)[:, :, :rows, :keys].to(torch.uint8).contiguous()
+
+
+@dataclass
 class PagedAttentionMetadata:
     """What one forward pass over a batch needs to know about the block KV
     cache (built by ``ironcore_amd.kv_cache.PagedKVCache.prepare``).
@@ -144,8 +160,9 @@ class Attention(BaseModule):
         to [b, hn, sq, sk], attention.py:115-117): ``("none", None)`` when every
         key is visible, ``("causal", None)`` for the lower-triangular pattern the
         reference model builds (ironcore/language_model.py:109-114,159; shifted
-        when sq < sk), else ``("general", bytes)`` with the mask as a uint8
-        ``[1 or b, 1 or hn, sq, sk]`` tensor for the masked kernels.
+        when sq < sk), else ``("general", data)``: the mask packed for the
+        prefill kernels, or (off the current GPU) as a uint8
+        ``[1 or b, 1 or hn, sq, sk]`` tensor.
 
         Telling the patterns apart needs a look at the values (one device
         synchronisation); the answer is remembered per mask TENSOR (identity
@@ -163,17 +180,34 @@ class Attention(BaseModule):
         if m.dim() != 4 or m.shape[-2:] != (sq, sk) or m.shape[0] not in (1, b) or m.shape[1] not in (1, hn):
             raise ValueError(f"attention_mask must be broadcastable to [{b}, {hn}, {sq}, {sk}], "
                              f"got {tuple(attention_mask.shape)}")
+        here = _lib.here(m)
+        if here is not None and sq > 0 and sk > 0:
+            as_bytes = m.view(torch.uint8) if m.dtype in (torch.bool, torch.uint8) else (m != 0).view(torch.uint8)
+            packed = _lib.host().pack_mask(as_bytes if as_bytes.stride(3) == 1 else as_bytes.contiguous(), *here)
+            if packed is not None:
+                flags = torch.stack(packed[2].unbind()).tolist()                     # the one synchronisation
+                if flags[0]:
+                    kind, data = "none", None
+                elif flags[1] and sq <= sk:
+                    kind, data = "causal", None
+                else:
+                    kind, data = "general", PackedMask(packed[0], packed[1], tuple(m.shape))
+                return self._remember_mask(attention_mask, version, (b, sq, sk, hn), kind, data)
         visible = m != 0
         i = torch.arange(sq, device=m.device).unsqueeze(1)
         j = torch.arange(sk, device=m.device).unsqueeze(0)
         want = j <= (sk - sq) + i
-        flags = torch.stack([visible.all(), (visible == want).all()]).tolist()   # the one synchronisation
+        flags = torch.stack([visible.all(), (visible == want).all()]).tolist()
         if flags[0]:
             kind, data = "none", None
         elif flags[1] and sq <= sk:
             kind, data = "causal", None
         else:
             kind, data = "general", visible.to(torch.uint8).contiguous()
+        return self._remember_mask(attention_mask, version, (b, sq, sk, hn), kind, data)
+
+    @staticmethod
+    def _remember_mask(attention_mask, version, shapes, kind, data):
         if version is not None:
             key = id(attention_mask)
             _MASK_CLASSES.pop(key, None)
@@ -183,7 +217,7 @@ class Attention(BaseModule):
             def forget(ref, key=key):
                 if key in _MASK_CLASSES and _MASK_CLASSES[key][0] is ref:
                     del _MASK_CLASSES[key]
-            _MASK_CLASSES[key] = (weakref.ref(attention_mask, forget), (version, b, sq, sk, hn), kind, data)
+            _MASK_CLASSES[key] = (weakref.ref(attention_mask, forget), (version, *shapes), kind, data)
         return kind, data
 
     # ------------------------------------------------------------------ forward
@@ -258,10 +292,15 @@ class Attention(BaseModule):
         b, sq, hn, hd = query.shape
         sk, gn = key.shape[1], key.shape[2]
         here = _lib.here(query)
-        if here is not None and mask is None:
-            out = _lib.host().dense(query, key, value, causal, 1.0 / self.scale_factor, *here)
+        packed = mask if isinstance(mask, PackedMask) else None
+        if here is not None and (mask is None or packed is not None):
+            bits, lists, planes = (packed.bits, packed.lists, packed.shape) if packed is not None else (None, None, (1, 1))
+            out = _lib.host().dense(query, key, value, causal, bits, lists, planes[0], planes[1],
+                                    1.0 / self.scale_factor, *here)
             if out is not None:
                 return out
+        if packed is not None:
+            mask = packed.bytes()
         key, value = key.contiguous(), value.contiguous()
         # one pool block per sequence: [b, gn, sk, hd] view of the [b, sk, gn, hd] rows
         k_pool, v_pool = key.permute(0, 2, 1, 3), value.permute(0, 2, 1, 3)
