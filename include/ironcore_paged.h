@@ -351,13 +351,13 @@ int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, i
  * plus three forms of input that spare a caller passes over its tensors.
  * Clear the struct first; a field left zero is the plain call's behaviour.
  *
- *   row_pitch        > 0: the chunks are padded, row r of sequence i is row
- *                    i*row_pitch + r of q and out (cu_seqlens_q still gives the
- *                    chunk lengths); output rows from a chunk's end to
- *                    max_chunk_len are set to zero.  row_pitch >= max_chunk_len.
+ *   rows, n_rows, q_rows
+ *                    rows != NULL: row i of the packed chunks (cu_seqlens_q) is row
+ *                    rows[i] of q and out, of q_rows rows; n_rows entries.  The other
+ *                    rows of out are left alone (ic_zero_unlisted_rows).
  *   uniform_context  with context_lens, cu_seqlens_q and block_tables all NULL:
  *                    equal sequences.  Every context has this many keys, every
- *                    chunk max_chunk_len rows (row_pitch is required), and
+ *                    chunk max_chunk_len rows, row_pitch >= max_chunk_len apart, and
  *                    sequence i is pool block i (uniform_context <= block_size,
  *                    any block size): a dense [b, s, gn, hd] tensor as a pool.
  *   positions, cos_table, sin_table, table_rows
@@ -392,6 +392,8 @@ typedef struct ic_prefill_call {
   int dtype;
   int uniform_context;
   int64_t row_pitch;
+  const int64_t *rows;
+  int64_t n_rows, q_rows;
   const int32_t *positions;
   const float *cos_table;
   const float *sin_table;
@@ -401,6 +403,16 @@ typedef struct ic_prefill_call {
   int mask_plane_seq, mask_plane_head;
 } ic_prefill_call;
 int ic_paged_prefill_ex(const ic_prefill_call *call, void *stream);
+
+/*
+ * Zeroes rows of a padded output [n_seqs * row_pitch rows of row_bytes, 16-byte
+ * aligned] ahead of a prefill call with `rows`: at least every row that is not
+ * among rows[0 .. n_rows-1].  (A row that is listed anywhere but at its sequence's
+ * start, entry bounds[i] + r for row i*row_pitch + r, may be zeroed too: the
+ * attention call writes it afterwards.)
+ */
+int ic_zero_unlisted_rows(void *out, int64_t out_stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
+                          const int32_t *bounds, int n_seqs, int row_pitch, void *stream);
 
 /*
  * Chunked prefill under a general attention mask: ic_paged_prefill with the

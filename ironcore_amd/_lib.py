@@ -95,6 +95,9 @@ SIGNATURES = {
         c_int, c_int, c_int, c_int,             # n_seqs, heads, rows, keys
         c_void_p, c_void_p, c_void_p, c_void_p]),   # bits, lists, flags, stream
     "ic_paged_prefill_ex": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
+    "ic_zero_unlisted_rows": (c_int, [
+        c_void_p, c_int64, c_int, c_void_p, c_int64,   # out, stride, row_bytes, rows, n_rows
+        c_void_p, c_int, c_int, c_void_p]),             # bounds, n_seqs, row_pitch, stream
     "ic_paged_prefill_masked": (c_int, [
         c_void_p, c_int64, c_void_p, c_int64,   # out, out_stride, q, q_stride
         c_void_p, c_void_p,                     # k_pool, v_pool

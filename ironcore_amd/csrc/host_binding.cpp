@@ -221,23 +221,24 @@ ic_prefill_call prefill_call(const Tensor &out, const Tensor &query, const Pool 
   c.hn = (int)hn, c.gn = (int)p.gn, c.hd = (int)p.hd;
   c.block_size = (int)p.bs, c.num_blocks = p.nb;
   c.scale = (float)scale, c.causal = causal, c.dtype = p.dtype;
-  c.row_pitch = s;
   return c;
 }
 
-// A chunk of new tokens per sequence: append, then attend.  `bounds` int32 [b + 1] holds the chunks' bounds
-// when they are of unequal length (rows past a chunk's end are padding: slot -1, output zero), else the
-// bounds of equal chunks.  The query is rotated inside the attention kernel.
+// A chunk of new tokens per sequence: append, then attend.  `bounds` int32 [b + 1] holds the bounds of the
+// packed chunks; chunks of unequal length come with the rows of the padded tensors they are (int64, any
+// placement), whose other rows are padding: slot -1, output zero.  The query is rotated inside the attention
+// kernel.
 OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
                        const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
-                       const Tensor &bounds, double scale, const OptTensor &positions, const OptTensor &cos,
+                       const Tensor &bounds, const OptTensor &rows, int64_t longest, double scale, const OptTensor &positions, const OptTensor &cos,
                        const OptTensor &sin, int64_t device, int64_t stream) {
   const Pool p(k_pool, v_pool, device);
   if (!p.ok || !p.attends()) return c10::nullopt;
   const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
   if (!in.ok || in.hn % p.gn != 0 || !index_vector(slots, at::kLong, in.b * in.s, device) ||
       !table(tables, in.b, device) || !index_vector(lens, at::kInt, in.b, device) ||
-      !index_vector(bounds, at::kInt, in.b + 1, device))
+      !index_vector(bounds, at::kInt, in.b + 1, device) || longest > in.s ||
+      (rows.has_value() && (rows->numel() == 0 || !index_vector(*rows, at::kLong, rows->numel(), device))))
     return c10::nullopt;
   const Rope rope(positions, cos, sin, in.b * in.s, p.hd, device);
   if (!rope.ok) return c10::nullopt;
@@ -246,7 +247,15 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
                                (void *)stream))
     return c10::nullopt;
   const Tensor out = at::empty({in.b, in.s, in.hn * p.hd}, query.options());
-  ic_prefill_call c = prefill_call(out, query, p, in.b, in.s, in.hn, scale, true);
+  ic_prefill_call c = prefill_call(out, query, p, in.b, longest, in.hn, scale, true);
+  if (rows.has_value()) {
+    c.rows = rows->data_ptr<int64_t>();
+    c.n_rows = rows->numel(), c.q_rows = in.b * in.s;
+    const int row_bytes = (int)(in.hn * p.hd * query.element_size());
+    if (ic_zero_unlisted_rows(c.out, row_bytes, row_bytes, c.rows, c.n_rows, bounds.data_ptr<int32_t>(), (int)in.b,
+                              (int)in.s, (void *)stream) != IC_OK)
+      return c10::nullopt;
+  }
   c.block_tables = tables.data_ptr<int32_t>();
   c.block_table_stride = tables.stride(0);
   c.context_lens = lens.data_ptr<int32_t>();
@@ -289,6 +298,7 @@ OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, boo
     return c10::nullopt;
   const Tensor out = at::empty({b, s, hn * p.hd}, query.options());
   ic_prefill_call c = prefill_call(out, query, p, b, s, hn, scale, causal);
+  c.row_pitch = s;
   c.uniform_context = (int)p.bs;
   if (bits.has_value()) {
     const int64_t planes = mask_seqs * mask_heads, qtiles = (s + 127) / 128, tiles = (p.bs + 63) / 64;

@@ -187,15 +187,16 @@ int prefill_checked(const ic_prefill_call &c, const uint8_t *mask, int64_t mask_
       return IC_ERR_BAD_SHAPE;
   } else {
     if (!c.block_tables || !c.cu_seqlens_q) return IC_ERR_NULL_POINTER;
-    if (c.block_table_stride <= 0 || c.row_pitch < 0 || (c.row_pitch > 0 && c.row_pitch < c.max_chunk_len))
-      return IC_ERR_BAD_SHAPE;
+    if (c.block_table_stride <= 0 || c.row_pitch != 0) return IC_ERR_BAD_SHAPE;
   }
   if (c.mask_bits != nullptr) {
     if (c.mask_lists == nullptr) return IC_ERR_NULL_POINTER;
     if (c.context_lens != nullptr || c.causal || mask != nullptr || c.mask_plane_seq < 0 || c.mask_plane_head < 0)
       return IC_ERR_BAD_SHAPE;
   }
-  if (c.row_pitch > 0 && c.row_pitch * c.n_seqs > 0x7fffffff) return IC_ERR_UNSUPPORTED;
+  if (c.rows != nullptr && (c.context_lens == nullptr || c.n_rows <= 0 || c.q_rows <= 0)) return IC_ERR_BAD_SHAPE;
+  if (c.n_rows > 0x7fffffff || c.q_rows > 0x7fffffff || (c.row_pitch > 0 && c.row_pitch * c.n_seqs > 0x7fffffff))
+    return IC_ERR_UNSUPPORTED;
   if (c.out_stride_token < (int64_t)c.hn * c.hd || c.q_stride_token < (int64_t)c.hn * c.hd) return IC_ERR_BAD_SHAPE;
   if (!aligned16(c.q) || !aligned16(c.out) || !aligned16(c.k_pool) || !aligned16(c.v_pool) ||
       !stride16(c.q_stride_token, es) || !stride16(c.out_stride_token, es))
@@ -230,6 +231,9 @@ int prefill_checked(const ic_prefill_call &c, const uint8_t *mask, int64_t mask_
   a.mask_stride_head = mask_stride_head;
   a.mask_stride_row = mask_stride_row;
   a.mask_keys = mask_keys;
+  a.rows = c.rows;
+  a.n_rows = (int)c.n_rows;
+  a.q_rows = (int)c.q_rows;
   a.row_pitch = c.row_pitch;
   a.uniform_context = c.uniform_context;
   a.positions = c.positions;
@@ -470,6 +474,17 @@ int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, i
   if (!mask || !bits || !lists || !flags) return IC_ERR_NULL_POINTER;
   return ic::launch_mask_pack(mask, stride_seq, stride_head, stride_row, n_seqs, heads, rows, keys, bits, lists, flags,
                               static_cast<hipStream_t>(stream));
+}
+
+int ic_zero_unlisted_rows(void *out, int64_t out_stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
+                          const int32_t *bounds, int n_seqs, int row_pitch, void *stream) {
+  if (n_seqs < 0 || row_pitch < 0 || row_bytes <= 0 || n_rows < 0 || out_stride_bytes < row_bytes)
+    return IC_ERR_BAD_SHAPE;
+  if (n_seqs == 0 || row_pitch == 0) return IC_OK;
+  if (!out || !rows || !bounds) return IC_ERR_NULL_POINTER;
+  if (!aligned16(out) || out_stride_bytes % 16 != 0 || row_bytes % 16 != 0) return IC_ERR_ALIGNMENT;
+  return ic::launch_zero_unlisted_rows(static_cast<char *>(out), out_stride_bytes, row_bytes, rows, n_rows, bounds,
+                                       n_seqs, row_pitch, static_cast<hipStream_t>(stream));
 }
 
 int ic_paged_prefill_ex(const ic_prefill_call *call, void *stream) {

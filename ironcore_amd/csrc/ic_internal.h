@@ -105,11 +105,14 @@ struct PrefillArgs {
   int64_t mask_stride_head = 0;
   int64_t mask_stride_row = 0;
   int64_t mask_keys = 0;  // keys a mask row covers; keys from there on are hidden
-  // Rows of sequence i start at i * row_pitch in q and out instead of cu_seqlens_q[i] (0 = packed rows);
-  // output rows from a chunk's end to max_chunk_len are zeroed.
-  int64_t row_pitch = 0;
+  // Row i of the packed chunks (cu_seqlens_q) is row rows[i] of q and out (nullptr: row i): chunks that lie in
+  // padded tensors.  The other rows of out are not written.
+  const int64_t *rows = nullptr;
+  int n_rows = 0;  // entries of rows
+  int q_rows = 0;  // rows of q and out
   // Equal sequences: context_lens, cu_seqlens_q and block_tables may be null; then every context has
-  // uniform_context keys, every chunk max_chunk_len rows, and sequence i is pool block i.
+  // uniform_context keys, every chunk max_chunk_len rows, row_pitch rows apart, and sequence i is pool block i.
+  int64_t row_pitch = 0;
   int uniform_context = 0;
   // Rotary embedding of the query rows as they are loaded (nullptr = none): row r of q uses table row
   // positions[r].
@@ -129,6 +132,8 @@ struct PrefillArgs {
 // dtype/shape) or IC_ERR_LAUNCH.
 int launch_kv_append(const AppendArgs &a, hipStream_t stream);
 int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream);
+int launch_zero_unlisted_rows(char *out, int64_t stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
+                              const int32_t *bounds, int n_seqs, int row_pitch, hipStream_t stream);
 int launch_paged_decode(const DecodeArgs &a, hipStream_t stream);
 int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream);
 int launch_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,

@@ -64,4 +64,33 @@ int launch_kv_append(const AppendArgs &a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
 
+namespace {
+
+// Zeroes the rows of a padded output that no chunk holds, ahead of the attention launch that writes the others.
+// Bound by the bytes written.  Row r of sequence i is known to be listed when entry bounds[i] + r names it (chunks
+// at the start of their rows, what PagedKVCache lays out); a row listed elsewhere is zeroed and written again,
+// which is why this is a launch of its own: inside the attention kernel it would race with that write.
+__global__ __launch_bounds__(kAppendThreads) void zero_unlisted_rows_kernel(
+    char *__restrict__ out, int64_t stride_bytes, int chunks, const int64_t *__restrict__ rows, int64_t n_rows,
+    const int32_t *__restrict__ bounds, int row_pitch, int64_t total) {
+  for (int64_t row = blockIdx.x; row < total; row += gridDim.x) {
+    const int seq = (int)(row / row_pitch);
+    const int64_t at = bounds[seq] + (row - (int64_t)seq * row_pitch);
+    if (at >= 0 && at < bounds[seq + 1] && at < n_rows && rows[at] == row) continue;
+    for (int c = threadIdx.x; c < chunks; c += kAppendThreads)
+      store16(out + row * stride_bytes + (int64_t)c * 16, Vec16{{0u, 0u, 0u, 0u}});
+  }
+}
+
+}  // namespace
+
+int launch_zero_unlisted_rows(char *out, int64_t stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
+                              const int32_t *bounds, int n_seqs, int row_pitch, hipStream_t stream) {
+  const int64_t total = (int64_t)n_seqs * row_pitch;
+  const int64_t most = (int64_t)device_cu_count() * 8;
+  hipLaunchKernelGGL(zero_unlisted_rows_kernel, dim3((unsigned)(total < most ? total : most)), dim3(kAppendThreads), 0,
+                     stream, out, stride_bytes, row_bytes / 16, rows, n_rows, bounds, row_pitch, total);
+  return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
+}
+
 }  // namespace ic

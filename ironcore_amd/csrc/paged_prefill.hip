@@ -116,13 +116,11 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   const bool causal = !MASK && p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
-  if (p.row_pitch > 0 && C < p.max_chunk)
-    zero_padding<HD, 2, kPrefillThreads>(p, q_lo, C, kvh * p.group, p.group, r, per_unit);
   if (q0 >= C) return;
   if (L == 0) {  // query rows without any key (not under the causal rule): zero rows
     const int rows = C - q0 < kBM ? C - q0 : kBM;
     for (int idx = threadIdx.x; idx < rows * (HD / 8); idx += kPrefillThreads)
-      store16(p.out + ((q_lo + q0 + idx / (HD / 8)) * p.out_stride_token + (int64_t)h * HD + (idx % (HD / 8)) * 8) * 2,
+      store16(p.out + (query_row(p, q_lo, q0 + idx / (HD / 8)) * p.out_stride_token + (int64_t)h * HD + (idx % (HD / 8)) * 8) * 2,
               Vec16{{0u, 0u, 0u, 0u}});
     return;
   }
@@ -138,12 +136,13 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   const int my_q = q0 + wave * 32 + n;
   const int qrow = my_q < C ? my_q : C - 1;
   const int limit = causal ? P + qrow : L - 1;  // last key this query row may see
+  const int64_t at_row = query_row(p, q_lo, qrow);
   Vec16 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
-    qf[ks] = load16(p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+    qf[ks] = load16(p.q + (at_row * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
   if (p.positions != nullptr) {
-    const int64_t trig = rope_row(p, q_lo + qrow) + hh * 4;
+    const int64_t trig = rope_row(p, at_row) + hh * 4;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[ks] = rotate_chunk<typename M::E>(qf[ks], p.cos_table + trig + ks * 8, p.sin_table + trig + ks * 8);
@@ -515,7 +514,7 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   if (my_q < C) {
-    T *orow = reinterpret_cast<T *>(p.out) + (q_lo + my_q) * p.out_stride_token + (int64_t)h * HD;
+    T *orow = reinterpret_cast<T *>(p.out) + query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD;
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob) {
 #pragma unroll
@@ -609,6 +608,9 @@ int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream) {
   kp.mask_stride_head = a.mask_stride_head;
   kp.mask_stride_row = a.mask_stride_row;
   kp.mask_keys = a.mask_keys > 0x7fffffff ? 0x7fffffff : (int)a.mask_keys;
+  kp.rows = a.rows;
+  kp.n_rows = a.n_rows;
+  kp.q_rows = a.q_rows;
   kp.row_pitch = a.row_pitch;
   kp.max_chunk = a.max_chunk_len;
   kp.uniform_context = a.uniform_context;

@@ -65,21 +65,18 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   const int q0 = (p.n_qtiles - 1 - blockIdx.x % p.n_qtiles) * kF32BM;  // last query tiles (the longest) first
   const int kvh = h / p.group;
   const bool equal = p.context_lens == nullptr;  // equal sequences: nothing to look up
-  int q_lo = equal ? 0 : p.cu_seqlens_q[seq];
+  const int q_lo = equal ? (int)(seq * p.row_pitch) : p.cu_seqlens_q[seq];
   int L = equal ? p.uniform_context : p.context_lens[seq];
   int C = equal ? p.max_chunk : p.cu_seqlens_q[seq + 1] - q_lo;
-  if (p.row_pitch > 0) q_lo = (int)(seq * p.row_pitch);
   const bool causal = MASK == 0 && p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
-  if (p.row_pitch > 0 && C < p.max_chunk)
-    zero_padding<HD, 4, kF32Threads>(p, q_lo, C, h, 1, blockIdx.x % p.n_qtiles, p.n_qtiles);
   if (q0 >= C) return;
   const int tid = threadIdx.x;
   if (L == 0) {  // query rows without any key (not under the causal rule): zero rows
     const int rows = C - q0 < kF32BM ? C - q0 : kF32BM;
     for (int idx = tid; idx < rows * F4R; idx += kF32Threads)
-      store16(p.out + ((q_lo + q0 + idx / F4R) * p.out_stride_token + (int64_t)h * HD + (idx % F4R) * 4) * 4,
+      store16(p.out + (query_row(p, q_lo, q0 + idx / F4R) * p.out_stride_token + (int64_t)h * HD + (idx % F4R) * 4) * 4,
               Vec16{{0u, 0u, 0u, 0u}});
     return;
   }
@@ -93,13 +90,14 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   const int my_q = q0 + wave * 32 + n;
   const int qrow = my_q < C ? my_q : C - 1;
   const int limit = causal ? P + qrow : L - 1;  // last key this query row may see
+  const int64_t at_row = query_row(p, q_lo, qrow);
   float4 qf[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
     qf[j] = *reinterpret_cast<const float4 *>(
-        p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + 8 * j + 4 * hh) * 4);
+        p.q + (at_row * p.q_stride_token + (int64_t)h * HD + 8 * j + 4 * hh) * 4);
   if (p.positions != nullptr) {
-    const int64_t trig = rope_row(p, q_lo + qrow) + 2 * hh;
+    const int64_t trig = rope_row(p, at_row) + 2 * hh;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
       qf[j] = __builtin_bit_cast(float4, rotate_chunk<F32>(__builtin_bit_cast(Vec16, qf[j]), p.cos_table + trig + 4 * j,
@@ -279,7 +277,7 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   if (my_q < C) {
-    float *orow = reinterpret_cast<float *>(p.out) + (q_lo + my_q) * p.out_stride_token + (int64_t)h * HD;
+    float *orow = reinterpret_cast<float *>(p.out) + query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD;
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob) {
 #pragma unroll

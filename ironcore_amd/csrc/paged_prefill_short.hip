@@ -82,8 +82,6 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const bool causal = p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
-  if (p.row_pitch > 0 && C < p.max_chunk)
-    zero_padding<HD, 2, TG * kShortWaves * kWave>(p, q_lo, C, kvh * p.group, p.group, within / kXcds, per_unit);
   // wave blocks per head (a packed mask's lists belong to 128 rows of one head: four blocks, unused ones too)
   const int n_blocks = PACKED ? ((C + 127) >> 7) * kShortWaves : (C + 31) >> 5;
   const int total = n_blocks * p.group;
@@ -111,7 +109,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
     if (mine && tg == 0 && my_q < C)
 #pragma unroll
       for (int c = 0; c < HD / 16; ++c)
-        store16(p.out + ((q_lo + my_q) * p.out_stride_token + (int64_t)h * HD + (hh * (HD / 16) + c) * 8) * 2,
+        store16(p.out + (query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD + (hh * (HD / 16) + c) * 8) * 2,
                 Vec16{{0u, 0u, 0u, 0u}});
     return;
   }
@@ -119,12 +117,13 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 
   const int qrow = my_q < C ? my_q : C - 1;
   const int limit = causal ? P + qrow : L - 1;  // last key this query row may see
+  const int64_t at_row = query_row(p, q_lo, qrow);
   Vec16 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
-    qf[ks] = load16(p.q + ((q_lo + qrow) * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+    qf[ks] = load16(p.q + (at_row * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
   if (p.positions != nullptr) {
-    const int64_t trig = rope_row(p, q_lo + qrow) + hh * 4;
+    const int64_t trig = rope_row(p, at_row) + hh * 4;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[ks] = rotate_chunk<typename M::E>(qf[ks], p.cos_table + trig + ks * 8, p.sin_table + trig + ks * 8);
@@ -409,7 +408,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   if (mine && my_q < C) {
-    T *orow = reinterpret_cast<T *>(p.out) + (q_lo + my_q) * p.out_stride_token + (int64_t)h * HD;
+    T *orow = reinterpret_cast<T *>(p.out) + query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD;
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob) {
 #pragma unroll

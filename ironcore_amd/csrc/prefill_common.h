@@ -44,9 +44,12 @@ struct PrefillKP {
   int64_t mask_stride_head;
   int64_t mask_stride_row;
   int mask_keys;  // keys a mask row covers: keys from there on are hidden and never read
-  int64_t row_pitch;    // rows from one sequence's chunk to the next in q and out (0 = packed, cu_seqlens_q)
-  int max_chunk;        // longest chunk; with row_pitch, output rows from a chunk's end to here are zeroed
-  int uniform_context;  // context_lens == nullptr: keys of every context (every chunk has max_chunk rows)
+  const int64_t *rows;  // row of q and out that row i of the packed chunks is (nullptr: i itself)
+  int n_rows;           // entries of `rows`
+  int q_rows;           // rows of q and out, which bound them
+  int64_t row_pitch;    // equal sequences: rows from one chunk to the next in q and out
+  int max_chunk;        // ... and rows of every chunk
+  int uniform_context;  // context_lens == nullptr (equal sequences): keys of every context
   const int32_t *positions;  // rotary embedding of the query rows (nullptr: none)
   const float *cos_table;
   const float *sin_table;
@@ -165,19 +168,17 @@ __device__ __forceinline__ void pick_sequence(const PrefillKP &p, int rank, int 
     L = p.context_lens[seq];
     C = p.cu_seqlens_q[seq + 1] - q_lo;
   }
-  if (p.row_pitch > 0) q_lo = (int)(seq * p.row_pitch);
 }
 
-// Output rows C .. max_chunk-1 of a sequence, `heads` heads of HD elements from head0 on: zeros.  Share
-// `share` of `shares` takes every shares-th row.
-template <int HD, int ES, int THREADS>
-__device__ __forceinline__ void zero_padding(const PrefillKP &p, int64_t row0, int C, int head0, int heads, int share,
-                                             int shares) {
-  const int chunks = heads * (HD * ES / 16);
-  for (int r = C + share; r < p.max_chunk; r += shares) {
-    char *row = p.out + ((row0 + r) * p.out_stride_token + (int64_t)head0 * HD) * ES;
-    for (int c = threadIdx.x; c < chunks; c += THREADS) store16(row + c * 16, Vec16{{0u, 0u, 0u, 0u}});
+// Row of q and out that is row r of the chunk whose rows start at q_lo.
+__device__ __forceinline__ int64_t query_row(const PrefillKP &p, int q_lo, int r) {
+  int64_t row = q_lo + r;
+  if (p.rows != nullptr) {
+    row = p.rows[row < p.n_rows ? row : p.n_rows - 1];
+    row = row < 0 ? 0 : row;  // a corrupt entry must not become an address outside the tensors
+    row = row < p.q_rows ? row : p.q_rows - 1;
   }
+  return row;
 }
 
 // The tiles a query tile visits under a packed mask: entry i (clamped to the last one) holds the tile and the

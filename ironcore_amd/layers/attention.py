@@ -344,13 +344,14 @@ class Attention(BaseModule):
                                           None if rope is None else rope.sin_emb, *here)
             if out is not None:
                 return out
-        elif here is not None and (rows is None or meta.max_chunk_len == sq):
+        elif here is not None:
             rope = rotary_pos_emb
             bounds = meta.cu_seqlens_q
             if bounds is None:
                 bounds = torch.arange(0, (b + 1) * sq, sq, dtype=torch.int32, device=query.device)
             out = _lib.host().prefill_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
-                                           meta.slot_mapping, bounds, 1.0 / self.scale_factor, meta.positions,
+                                           meta.slot_mapping, bounds, rows, sq if rows is None else meta.max_chunk_len,
+                                           1.0 / self.scale_factor, meta.positions,
                                            None if rope is None else rope.cos_emb,
                                            None if rope is None else rope.sin_emb, *here)
             if out is not None:

@@ -127,6 +127,42 @@ def test_prefill_step(gpu, monkeypatch, dtype, precision, rope, hn, gn, hd, pref
 
 
 @pytest.mark.parametrize("dtype,precision", [(torch.bfloat16, "bf16"), (torch.float32, "fp32")])
+@pytest.mark.parametrize("placement", ["left", "packed", "reversed"])
+@pytest.mark.parametrize("hn,gn,hd,prefix,chunks", [(6, 2, 64, (0, 90), (1, 70)), (8, 8, 128, (1300, 1400), (250, 256))])
+def test_chunk_rows_anywhere(gpu, monkeypatch, dtype, precision, placement, hn, gn, hd, prefix, chunks):
+    """chunk_rows names the rows of the padded tensors that exist, wherever they are: at the ends of
+    their sequences' rows (padding on the left), all of them first, or each chunk last row first."""
+    n = 20 if prefix[0] > 1000 else 4
+    wl = workloads.make_prefill_workload(n, hn, gn, hd, *prefix, *chunks, dtype=dtype, seed=hn + hd)
+    meta, query, key, value = _ragged(gpu, wl, dtype, 16, 5)
+    width = query.shape[1]
+    lens = (wl.cu_seqlens_q[1:] - wl.cu_seqlens_q[:-1]).tolist()
+    old = meta.chunk_rows.tolist()
+    if placement == "left":
+        new = [i * width + width - c + t for i, c in enumerate(lens) for t in range(c)]
+    elif placement == "packed":
+        new = list(range(len(old)))
+    else:
+        new = [i * width + c - 1 - t for i, c in enumerate(lens) for t in range(c)]
+    slots, positions = torch.full_like(meta.slot_mapping, -1), torch.zeros_like(meta.positions)
+    slots[new], positions[new] = meta.slot_mapping[old], meta.positions[old]
+    meta.chunk_rows, meta.slot_mapping, meta.positions = torch.tensor(new, device=gpu), slots, positions
+    emb = RotaryPositionalEmbedding(hd, max_seq_len=int(wl.context_lens.max())).to(gpu)
+    attn = _layer(hn, gn, hd, precision)
+    pools = [(wl.k_pool.to(gpu), wl.v_pool.to(gpu)) for _ in range(2)]
+    left = list(pools)
+
+    def call():
+        return attn(query, key, value, kv_cache=left.pop(), attn_metadata=meta, rotary_pos_emb=emb)
+    native, plain = _both(monkeypatch, call)
+    padding = torch.ones(n * width, dtype=torch.bool, device=gpu)
+    padding[new] = False
+    assert torch.isfinite(native.float()).all() and torch.equal(native, plain)
+    assert not native.view(n * width, -1)[padding].any()
+    assert torch.equal(pools[0][0], pools[1][0]) and torch.equal(pools[0][1], pools[1][1])
+
+
+@pytest.mark.parametrize("dtype,precision", [(torch.bfloat16, "bf16"), (torch.float32, "fp32")])
 @pytest.mark.parametrize("b,s,hn,gn,hd,masked", [(3, 70, 6, 2, 64, True), (1, 1, 4, 4, 128, False), (2, 129, 4, 1, 128, True),
                                                   (70, 5, 2, 2, 32, True), (1, 2304, 2, 2, 128, False)])
 def test_dense_call(gpu, monkeypatch, dtype, precision, b, s, hn, gn, hd, masked):
