@@ -74,6 +74,7 @@ class PackedMask:
     bits: torch.Tensor    # int64 [planes, 4 * query tiles, key tiles, 32]
     lists: torch.Tensor   # int32 [planes, query tiles, key tiles + 1]
     shape: tuple          # of the byte mask: (1 or b, 1 or hn, sq, sk)
+    stream: int = 0       # raw stream the tensors were allocated on
 
     def bytes(self) -> torch.Tensor:
         """The byte mask again (uint8), for a call the packed kernels do not take."""
@@ -191,7 +192,7 @@ class Attention(BaseModule):
                 elif flags[1] and sq <= sk:
                     kind, data = "causal", None
                 else:
-                    kind, data = "general", PackedMask(packed[0], packed[1], tuple(m.shape))
+                    kind, data = "general", PackedMask(packed[0], packed[1], tuple(m.shape), here[1])
                 return self._remember_mask(attention_mask, version, (b, sq, sk, hn), kind, data)
         visible = m != 0
         i = torch.arange(sq, device=m.device).unsqueeze(1)
@@ -294,6 +295,10 @@ class Attention(BaseModule):
         here = _lib.here(query)
         packed = mask if isinstance(mask, PackedMask) else None
         if here is not None and (mask is None or packed is not None):
+            if packed is not None and packed.stream != here[1]:
+                # kept with the mask, so it may be given up while this stream still reads it
+                for t in (packed.bits, packed.lists):
+                    t.record_stream(torch.cuda.current_stream(query.device))
             bits, lists, planes = (packed.bits, packed.lists, packed.shape) if packed is not None else (None, None, (1, 1))
             out = _lib.host().dense(query, key, value, causal, bits, lists, planes[0], planes[1],
                                     1.0 / self.scale_factor, *here)
