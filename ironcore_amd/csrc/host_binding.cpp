@@ -317,11 +317,13 @@ OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, boo
 
 }  // namespace
 
+// (wrapped, so that torch's exceptions keep their Python types: an allocation that does not fit raises
+// torch.OutOfMemoryError)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("kv_append", &kv_append);
-  m.def("paged_decode", &paged_decode);
-  m.def("decode_step", &decode_step);
-  m.def("prefill_step", &prefill_step);
-  m.def("dense", &dense);
-  m.def("pack_mask", &pack_mask);
+  m.def("kv_append", torch::wrap_pybind_function(kv_append));
+  m.def("paged_decode", torch::wrap_pybind_function(paged_decode));
+  m.def("decode_step", torch::wrap_pybind_function(decode_step));
+  m.def("prefill_step", torch::wrap_pybind_function(prefill_step));
+  m.def("dense", torch::wrap_pybind_function(dense));
+  m.def("pack_mask", torch::wrap_pybind_function(pack_mask));
 }

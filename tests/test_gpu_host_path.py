@@ -175,3 +175,12 @@ def test_dense_call(gpu, monkeypatch, dtype, precision, b, s, hn, gn, hd, masked
     attn = _layer(hn, gn, hd, precision)
     native, plain = _both(monkeypatch, lambda: attn(query, key, value, mask))
     assert torch.equal(native, plain)
+
+
+def test_out_of_memory_keeps_its_type(gpu):
+    """What the allocator raises inside the native call is torch's own exception, as it was from torch.empty."""
+    b, pool = 1 << 22, torch.zeros(1, 1, 16, 128, dtype=torch.bfloat16, device=gpu)
+    query = torch.zeros(1, 512, 128, dtype=torch.bfloat16, device=gpu).expand(b, 512, 128)     # 512 GiB of output
+    tables = torch.zeros(1, 1, dtype=torch.int32, device=gpu).expand(b, 1)
+    with pytest.raises(torch.OutOfMemoryError):
+        paged_ops.paged_decode(query, pool, pool, tables, torch.ones(b, dtype=torch.int32, device=gpu), 16)
