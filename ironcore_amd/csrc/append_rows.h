@@ -1,0 +1,41 @@
+// How the append kernels (kv_append.hip, rope_kv_append.hip) lay token rows over
+// workgroups of kAppendThreads lanes, one 16-byte chunk of a row to a lane.
+#pragma once
+
+#include "ic_internal.h"
+
+namespace ic {
+
+constexpr int kAppendThreads = 256;
+constexpr int kAppendThreadsShift = 8;
+
+// Lanes a row takes in a workgroup, as a shift: a row that fills less than a workgroup shares it.  A few KV
+// heads are a wave's worth of chunks (4 heads of 128 in 16 bits: 64), and with a workgroup to a row the launch
+// is bound by how fast workgroups start and three quarters of their lanes do nothing.
+inline int append_row_shift(int chunks) {
+  int shift = 0;
+  while (shift < kAppendThreadsShift && (1 << shift) < chunks) ++shift;
+  return shift;
+}
+
+// Token (from the slice's first) and chunk of this lane.  A row that fills the workgroup is the same for all
+// its lanes (WIDE: its slot and the division by the block size stay scalar).
+template <bool WIDE>
+__device__ __forceinline__ int64_t append_token(int row_shift) {
+  if (WIDE) return blockIdx.y;
+  return ((int64_t)blockIdx.y << (kAppendThreadsShift - row_shift)) + (threadIdx.x >> row_shift);
+}
+template <bool WIDE>
+__device__ __forceinline__ int append_chunk(int row_shift) {
+  return blockIdx.x * kAppendThreads + (WIDE ? threadIdx.x : threadIdx.x & ((1 << row_shift) - 1));
+}
+
+// Block of a slot in [0, num_slots): where a lane's slots differ, a 64-bit division on the vector unit is some
+// hundred instructions.
+template <bool WIDE>
+__device__ __forceinline__ int64_t slot_block(int64_t slot, int block_size, int64_t num_slots) {
+  if (WIDE || (num_slots >> 32) != 0) return slot / block_size;
+  return (uint32_t)slot / (uint32_t)block_size;
+}
+
+}  // namespace ic

@@ -6,10 +6,12 @@
 //
 // HBM-bound byte copy.  One lane moves one 16-byte chunk with a single
 // dwordx4 load and store; a workgroup covers a contiguous run of chunks of one
-// token row, so both the read of the new row and the write of each
-// (head, token) segment are fully coalesced.  K and V go in the same launch
-// (blockIdx.z).  Algorithmic traffic: 2 * n_tokens * gn * hd * elem bytes read
-// and the same written, plus 8 bytes of slot index per token.
+// token row, or, where a row has fewer chunks than a workgroup lanes, several
+// rows (a row takes a power of two of lanes), so both the read of the new row
+// and the write of each (head, token) segment are fully coalesced.  K and V go
+// in the same launch (blockIdx.z).  Algorithmic traffic: 2 * n_tokens * gn * hd *
+// elem bytes read and the same written, plus 8 bytes of slot index per token.
+#include "append_rows.h"
 #include "ic_device.h"
 #include "ic_internal.h"
 #include "../../include/ironcore_paged.h"
@@ -18,19 +20,18 @@ namespace ic {
 
 namespace {
 
-constexpr int kAppendThreads = 256;
-
+template <bool WIDE>
 __global__ __launch_bounds__(kAppendThreads) void kv_append_kernel(
     const char *__restrict__ k_new, const char *__restrict__ v_new, int64_t new_stride_bytes,
     char *__restrict__ k_pool, char *__restrict__ v_pool, int64_t stride_block_bytes,
     int64_t stride_head_bytes, int64_t stride_token_bytes, const int64_t *__restrict__ slot_mapping,
-    int chunks_per_head, int chunks_per_row, int block_size, int64_t num_slots) {
-  const int64_t t = blockIdx.y;
+    int chunks_per_head, int chunks_per_row, int row_shift, int64_t n_tokens, int block_size, int64_t num_slots) {
+  const int64_t t = append_token<WIDE>(row_shift);
+  const int c = append_chunk<WIDE>(row_shift);
+  if (t >= n_tokens || c >= chunks_per_row) return;
   const int64_t slot = slot_mapping[t];
   if (slot < 0 || slot >= num_slots) return;
-  const int c = blockIdx.x * kAppendThreads + threadIdx.x;
-  if (c >= chunks_per_row) return;
-  const int64_t blk = slot / block_size;
+  const int64_t blk = slot_block<WIDE>(slot, block_size, num_slots);
   const int64_t off = slot - blk * block_size;
   const int head = c / chunks_per_head;
   const int within = c - head * chunks_per_head;
@@ -47,18 +48,20 @@ int launch_kv_append(const AppendArgs &a, hipStream_t stream) {
   const int es = elem_size(a.dtype);
   const int chunks_per_head = a.hd * es / 16;
   const int chunks_per_row = chunks_per_head * a.gn;
-  dim3 grid((chunks_per_row + kAppendThreads - 1) / kAppendThreads, (unsigned)a.n_tokens, 2);
+  const int row_shift = append_row_shift(chunks_per_row);
+  const int rows = kAppendThreads >> row_shift;  // token rows of a workgroup
+  dim3 grid((chunks_per_row + kAppendThreads - 1) / kAppendThreads, 1, 2);
   // gridDim.y is limited to 65535: walk longer appends in slices.
-  const int64_t kMaxY = 65535;
-  for (int64_t t0 = 0; t0 < a.n_tokens; t0 += kMaxY) {
-    const int64_t n = (a.n_tokens - t0 < kMaxY) ? a.n_tokens - t0 : kMaxY;
-    grid.y = (unsigned)n;
-    hipLaunchKernelGGL(kv_append_kernel, grid, dim3(kAppendThreads), 0, stream,
+  const int64_t slice = (int64_t)65535 * rows;
+  for (int64_t t0 = 0; t0 < a.n_tokens; t0 += slice) {
+    const int64_t n = (a.n_tokens - t0 < slice) ? a.n_tokens - t0 : slice;
+    grid.y = (unsigned)((n + rows - 1) / rows);
+    hipLaunchKernelGGL(rows == 1 ? kv_append_kernel<true> : kv_append_kernel<false>, grid, dim3(kAppendThreads), 0, stream,
                        (const char *)a.k_new + t0 * a.new_stride_token * es,
                        (const char *)a.v_new + t0 * a.new_stride_token * es,
                        a.new_stride_token * es, (char *)a.k_pool, (char *)a.v_pool,
                        a.pool.stride_block * es, a.pool.stride_head * es, a.pool.stride_token * es,
-                       a.slot_mapping + t0, chunks_per_head, chunks_per_row, a.pool.block_size,
+                       a.slot_mapping + t0, chunks_per_head, chunks_per_row, row_shift, n, a.pool.block_size,
                        a.pool.num_blocks * a.pool.block_size);
   }
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;

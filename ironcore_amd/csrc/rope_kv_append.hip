@@ -20,10 +20,11 @@
 // caller's decision (its true position in the sequence for a cached decoder).
 //
 // HBM-bound: one lane handles one 16-byte chunk (4 pairs in 16-bit types, 2
-// in fp32) and the matching 16 or 8 bytes of each table row; blockIdx.z picks
-// K, V or Q.  Algorithmic traffic: K and V rows read once and written once,
-// Q rows read and written in place, 12 bytes of slot and position per token;
-// the table rows in use stay in cache.
+// in fp32) and the matching 16 or 8 bytes of each table row; rows of few
+// chunks share a workgroup; blockIdx.z picks K, V or Q.  Algorithmic traffic:
+// K and V rows read once and written once, Q rows read and written in place,
+// 12 bytes of slot and position per token; the table rows in use stay in cache.
+#include "append_rows.h"
 #include "ic_internal.h"
 #include "rope_device.h"
 #include "../../include/ironcore_paged.h"
@@ -31,8 +32,6 @@
 namespace ic {
 
 namespace {
-
-constexpr int kRopeThreads = 256;
 
 struct RopeKP {
   const char *q;          // or nullptr
@@ -56,16 +55,20 @@ struct RopeKP {
   int chunks_per_head;
   int q_chunks;   // per token
   int kv_chunks;  // per token
+  int q_row_shift;   // lanes of a row in a workgroup
+  int kv_row_shift;
   int block_size;
   int half_hd;
 };
 
-template <class E>
-__global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(const RopeKP p, int64_t t0) {
+template <class E, bool WIDE>
+__global__ __launch_bounds__(kAppendThreads) void rope_kv_append_kernel(const RopeKP p, int64_t t0, int64_t n_tokens) {
   constexpr int PAIRS = E::EPL / 2;  // pairs in one 16-byte chunk
-  const int64_t t = t0 + blockIdx.y;
   const int part = blockIdx.z;  // 0: K, 1: V, 2: Q
-  const int c = blockIdx.x * kRopeThreads + threadIdx.x;
+  const int row_shift = part == 2 ? p.q_row_shift : p.kv_row_shift;
+  const int64_t t = t0 + append_token<WIDE>(row_shift);
+  const int c = append_chunk<WIDE>(row_shift);
+  if (t >= n_tokens) return;
   int64_t pos = p.positions[t];
   pos = pos < 0 ? 0 : pos;
   pos = pos >= p.table_rows ? p.table_rows - 1 : pos;
@@ -80,7 +83,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(const Rope
   if (p.k_new == nullptr || c >= p.kv_chunks) return;
   const int64_t slot = p.slot_mapping[t];
   if (slot < 0 || slot >= p.num_slots) return;
-  const int64_t blk = slot / p.block_size;
+  const int64_t blk = slot_block<WIDE>(slot, p.block_size, p.num_slots);
   const int64_t off = slot - blk * p.block_size;
   const int head = c / p.chunks_per_head;
   const int within = c - head * p.chunks_per_head;
@@ -98,11 +101,15 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(const Rope
 template <class E>
 int launch_typed(const RopeKP &kp, int64_t n_tokens, hipStream_t stream) {
   const int widest = kp.q_chunks > kp.kv_chunks ? kp.q_chunks : kp.kv_chunks;
-  dim3 grid((widest + kRopeThreads - 1) / kRopeThreads, 1, 3);
-  const int64_t kMaxY = 65535;  // gridDim.y limit: walk longer batches in slices
-  for (int64_t t0 = 0; t0 < n_tokens; t0 += kMaxY) {
-    grid.y = (unsigned)((n_tokens - t0 < kMaxY) ? n_tokens - t0 : kMaxY);
-    hipLaunchKernelGGL(rope_kv_append_kernel<E>, grid, dim3(kRopeThreads), 0, stream, kp, t0);
+  const int shift = kp.q_row_shift > kp.kv_row_shift ? kp.q_row_shift : kp.kv_row_shift;
+  const int rows = kAppendThreads >> shift;  // token rows of a workgroup, at least
+  dim3 grid((widest + kAppendThreads - 1) / kAppendThreads, 1, kp.q_chunks > 0 ? 3 : 2);
+  const bool wide = kp.kv_row_shift == kAppendThreadsShift && (kp.q_chunks == 0 || kp.q_row_shift == kAppendThreadsShift);
+  const int64_t slice = (int64_t)65535 * rows;  // gridDim.y limit: walk longer batches in slices
+  for (int64_t t0 = 0; t0 < n_tokens; t0 += slice) {
+    const int64_t n = n_tokens - t0 < slice ? n_tokens - t0 : slice;
+    grid.y = (unsigned)((n + rows - 1) / rows);
+    hipLaunchKernelGGL((wide ? rope_kv_append_kernel<E, true> : rope_kv_append_kernel<E, false>), grid, dim3(kAppendThreads), 0, stream, kp, t0, t0 + n);
   }
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
@@ -135,6 +142,8 @@ int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream) {
   kp.chunks_per_head = ap.hd * es / 16;
   kp.q_chunks = a.q ? kp.chunks_per_head * a.hn : 0;
   kp.kv_chunks = ap.k_new ? kp.chunks_per_head * ap.gn : 0;
+  kp.q_row_shift = append_row_shift(kp.q_chunks);
+  kp.kv_row_shift = append_row_shift(kp.kv_chunks);
   kp.block_size = ap.pool.block_size;
   kp.half_hd = ap.hd / 2;
   switch (ap.dtype) {
