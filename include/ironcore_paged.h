@@ -470,6 +470,24 @@ int ic_paged_decode_masked(void *out, int64_t out_stride_seq,
                            void *workspace, size_t workspace_bytes,
                            int dtype, void *stream);
 
+/*
+ * y = x W (+ bias) for at most IC_LINEAR_ROWS_MAX rows: the projections of a
+ * decode step (the reference's linears, W stored [in, out]:
+ * ironcore/parallel/tensor_parallel/layers.py:41,194-204).  fp32 sums.
+ *
+ *   out [m, n], x [m, k], w [k, n], bias [n] or NULL: one element type, rows
+ *       16-byte aligned; strides in elements.
+ *   n a multiple of 16 bytes of elements, k of 64 bytes.
+ *   splits  workgroups that share a column's k range; 0 lets the library choose.
+ *   workspace  ic_linear_rows_workspace_bytes(m, n, k, splits, dtype) bytes.
+ */
+#define IC_LINEAR_ROWS_MAX 32
+size_t ic_linear_rows_workspace_bytes(int m, int n, int k, int splits, int dtype);
+int ic_linear_rows(void *out, int64_t out_stride, const void *x, int64_t x_stride,
+                   const void *w, int64_t w_stride, const void *bias,
+                   int m, int n, int k, int splits,
+                   void *workspace, size_t workspace_bytes, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -90,6 +90,12 @@ SIGNATURES = {
         c_int, c_int, c_int, c_int,             # hn, gn, hd, block_size
         c_int64, c_float, c_int,                # num_blocks, scale, causal
         c_int, c_void_p]),                      # dtype, stream
+    "ic_linear_rows_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "ic_linear_rows": (c_int, [
+        c_void_p, c_int64, c_void_p, c_int64,   # out, out_stride, x, x_stride
+        c_void_p, c_int64, c_void_p,            # w, w_stride, bias
+        c_int, c_int, c_int, c_int,             # m, n, k, splits
+        c_void_p, c_size_t, c_int, c_void_p]),  # workspace, workspace_bytes, dtype, stream
     "ic_mask_pack": (c_int, [
         c_void_p, c_int64, c_int64, c_int64,    # mask, strides: seq, head, row
         c_int, c_int, c_int, c_int,             # n_seqs, heads, rows, keys

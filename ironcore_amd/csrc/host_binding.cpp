@@ -12,6 +12,12 @@
 // and serves a capturing stream from the graph's own pool.
 #include <torch/extension.h>
 
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+
+#include <climits>
+
 #include "../../include/ironcore_paged.h"
 
 namespace {
@@ -315,6 +321,47 @@ OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, boo
   return out;
 }
 
+// ---- the model's linears --------------------------------------------------------------------
+
+// Nothing but values: no subclass, no functorch or forward-mode wrapper, no view that a kernel would misread.
+bool plain(const Tensor &t) {
+  return !at::isTensorSubclassLike(t) && !t.is_conj() && !t.is_neg() && !t._fw_grad(0).defined();
+}
+
+// y = x W (+ bias) for the few rows of a decode step; x [..., k] contiguous, W [k, n].  What a dispatched product
+// would do beside it (autograd, autocast, tracing, dispatch modes) is left to that.
+OptTensor linear_rows(const Tensor &x, const Tensor &w, const OptTensor &bias, int64_t device, int64_t stream) {
+  if (x.dim() < 2 || w.dim() != 2 || !on(x, device) || !on(w, device) || x.scalar_type() != w.scalar_type() ||
+      x.size(-1) != w.size(0) || x.numel() == 0 || !x.is_contiguous() || w.stride(1) != 1 || !plain(x) || !plain(w) ||
+      c10::impl::dispatch_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA))
+    return c10::nullopt;
+  const int dtype = dtype_code(x.scalar_type());
+  const int64_t k = w.size(0), n = w.size(1), m = x.numel() / k;
+  if (dtype < 0 || m > IC_LINEAR_ROWS_MAX || n > INT_MAX || k > INT_MAX) return c10::nullopt;
+  if (bias.has_value() && (!index_vector(*bias, x.scalar_type(), n, device) || bias->dim() != 1 || !plain(*bias)))
+    return c10::nullopt;
+  if (at::GradMode::is_enabled() &&
+      (x.requires_grad() || w.requires_grad() || (bias.has_value() && bias->requires_grad())))
+    return c10::nullopt;
+  const int es = (int)x.element_size();
+  if (n % (16 / es) != 0 || k % (64 / es) != 0 || (w.stride(0) * es) % 16 != 0 || w.stride(0) < n) return c10::nullopt;
+  const size_t need = ic_linear_rows_workspace_bytes((int)m, (int)n, (int)k, 0, dtype);
+  // Without a bias to fuse and with nothing to gain from split sums the library's product is as fast or faster for
+  // short columns and for more than 16 rows (bf16, this kernel / the library: 16 rows, 1 024 x 1 024 6.8 / 6.0 us,
+  // 1 024 x 5 504 9.4 / 8.9; 32 rows, 4 096 x 22 016 42.3 / 40.4).
+  if (!bias.has_value() && need == 0 && (m > 16 || k * es <= 2048)) return c10::nullopt;
+  auto sizes = x.sizes().vec();
+  sizes.back() = n;
+  const Tensor out = at::empty(sizes, x.options());
+  Tensor ws;
+  if (need > 0) ws = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
+  if (ic_linear_rows(out.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), w.stride(0),
+                     bias.has_value() ? bias->data_ptr() : nullptr, (int)m, (int)n, (int)k, 0,
+                     need > 0 ? ws.data_ptr() : nullptr, need, dtype, (void *)stream) != IC_OK)
+    return c10::nullopt;
+  return out;
+}
+
 }  // namespace
 
 // (wrapped, so that torch's exceptions keep their Python types: an allocation that does not fit raises
@@ -325,5 +372,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_step", torch::wrap_pybind_function(decode_step));
   m.def("prefill_step", torch::wrap_pybind_function(prefill_step));
   m.def("dense", torch::wrap_pybind_function(dense));
+  m.def("linear_rows", torch::wrap_pybind_function(linear_rows));
   m.def("pack_mask", torch::wrap_pybind_function(pack_mask));
 }

@@ -466,6 +466,35 @@ int ic_paged_decode_static(void *out, int64_t out_stride_seq, const void *q, int
                         kStaticMaxWaves, dtype, stream);
 }
 
+size_t ic_linear_rows_workspace_bytes(int m, int n, int k, int splits, int dtype) {
+  if (m < 1 || m > IC_LINEAR_ROWS_MAX || n < 1 || k < 1 || !dtype_ok(dtype)) return 0;
+  const int got = ic::linear_rows_splits(n, k, dtype, splits);
+  return got > 1 ? (size_t)got * m * n * sizeof(float) : 0;
+}
+
+int ic_linear_rows(void *out, int64_t out_stride, const void *x, int64_t x_stride, const void *w, int64_t w_stride,
+                   const void *bias, int m, int n, int k, int splits, void *workspace, size_t workspace_bytes,
+                   int dtype, void *stream) {
+  if (m < 0 || n < 0 || k <= 0 || splits < 0) return IC_ERR_BAD_SHAPE;
+  if (!dtype_ok(dtype)) return IC_ERR_UNSUPPORTED;
+  if (m == 0 || n == 0) return IC_OK;
+  const int es = ic::elem_size(dtype), block = 16 / es;
+  if (m > IC_LINEAR_ROWS_MAX || n % block != 0 || k % (4 * block) != 0) return IC_ERR_UNSUPPORTED;
+  if (out_stride < n || x_stride < k || w_stride < n) return IC_ERR_BAD_SHAPE;
+  if (!out || !x || !w) return IC_ERR_NULL_POINTER;
+  if (!aligned16(out) || !aligned16(x) || !aligned16(w) || !stride16(out_stride, es) || !stride16(x_stride, es) ||
+      !stride16(w_stride, es))
+    return IC_ERR_ALIGNMENT;
+  const size_t need = ic_linear_rows_workspace_bytes(m, n, k, splits, dtype);
+  if (need > 0 && (!workspace || !aligned16(workspace))) return IC_ERR_WORKSPACE;
+  if (workspace_bytes < need) return IC_ERR_WORKSPACE;
+  ic::LinearArgs a;
+  a.x = x, a.w = w, a.bias = bias, a.out = out;
+  a.x_stride = x_stride, a.w_stride = w_stride, a.out_stride = out_stride;
+  a.m = m, a.n = n, a.k = k, a.splits = splits, a.dtype = dtype, a.workspace = workspace;
+  return ic::launch_linear_rows(a, static_cast<hipStream_t>(stream));
+}
+
 int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,
                  int heads, int rows, int keys, uint64_t *bits, int32_t *lists, int32_t *flags, void *stream) {
   if (n_seqs < 0 || heads < 0 || rows < 0 || keys < 0 || stride_seq < 0 || stride_head < 0 || stride_row < 0)

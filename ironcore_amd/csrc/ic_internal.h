@@ -45,6 +45,17 @@ struct RopeAppendArgs {
   int64_t table_rows;
 };
 
+// y = x W (+ bias), a few rows (linear_rows.hip).
+struct LinearArgs {
+  const void *x, *w, *bias;  // [m, k], [k, n], [n] or nullptr
+  void *out;                 // [m, n]
+  int64_t x_stride, w_stride, out_stride;  // elements
+  int m, n, k;
+  int splits;  // of k; 0: the rule's
+  int dtype;
+  void *workspace;
+};
+
 struct DecodeArgs {
   void *out;
   int64_t out_stride_seq;
@@ -134,6 +145,8 @@ int launch_kv_append(const AppendArgs &a, hipStream_t stream);
 int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream);
 int launch_zero_unlisted_rows(char *out, int64_t stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
                               const int32_t *bounds, int n_seqs, int row_pitch, hipStream_t stream);
+int launch_linear_rows(const LinearArgs &a, hipStream_t stream);
+int linear_rows_splits(int n, int k, int dtype, int want);
 int launch_paged_decode(const DecodeArgs &a, hipStream_t stream);
 int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream);
 int launch_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,

@@ -8,9 +8,10 @@ transformer.py:77-162) and generates by re-running that forward on the whole
 growing sequence every step (examples/generate_text.py:12-46).  The classes
 below keep that arithmetic and those parameter names, add the two optional
 arguments that carry the KV cache down to ``Attention.forward``, and replace
-the full recompute by prefill + cached decode.  The GEMMs, norms and the
-activation are plain torch calls on the GPU (plumbing around the hot path);
-attention and the KV append are the HIP kernels.
+the full recompute by prefill + cached decode.  Attention, the KV append and the
+linears of a decode step (up to 32 rows) are the HIP kernels; the other GEMMs,
+the norms and the activation are plain torch calls on the GPU (plumbing around
+the hot path).
 
 Built: pre/post-LN with LayerNorm or RMSNorm, learned absolute positions or
 rotary embeddings, GELU/ReLU/SiLU and gated (GLU/SwiGLU/GeGLU/SiGLU) MLPs, tied or
@@ -28,10 +29,27 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _lib
 from .kv_cache import PagedKVCache
 from .layers.attention import Attention, PagedAttentionMetadata
 from .layers.module import BaseModule, get_model_dtype
 from .layers.rotary import RotaryPositionalEmbedding
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``x @ weight (+ bias)``, the weight ``[in, out]``.  The few rows of a decode
+    step go through the package's kernel (csrc/linear_rows.hip); more rows, and
+    calls that torch has to see (autograd, autocast, tracing, subclasses), through
+    torch's product."""
+    if not (torch.overrides.has_torch_function_variadic(x, weight) or torch.compiler.is_compiling()
+            or torch.jit.is_tracing()):
+        here = _lib.here(x)
+        if here is not None:
+            y = _lib.host().linear_rows(x, weight, bias, *here)
+            if y is not None:
+                return y
+    y = torch.matmul(x, weight)
+    return y + bias if bias is not None else y
 
 
 class Linear(BaseModule):
@@ -45,8 +63,7 @@ class Linear(BaseModule):
         self.bias = nn.Parameter(torch.empty(output_size)) if bias else None
 
     def forward(self, x):
-        y = torch.matmul(x, self.weight)
-        return y + self.bias if self.bias is not None else y
+        return linear(x, self.weight, self.bias)
 
 
 class LayerNorm(BaseModule):
@@ -297,7 +314,7 @@ class LanguageModel(BaseModule):
         x = self.model(x, attention_mask, self.rotary_pos_emb, kv_cache=kv_cache, attn_metadata=meta)
         x = self.output_layernorm(x)
         if self.config.model.untie_embed:
-            return torch.matmul(x, self.output_layer.weight)
+            return linear(x, self.output_layer.weight)
         return torch.matmul(x, self.embedding.word_embeddings.weight.transpose(0, 1))
 
 

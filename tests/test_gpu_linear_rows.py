@@ -1,0 +1,77 @@
+"""The few-row linear (csrc/linear_rows.hip) at the edges of its tiles: one k
+step and many, columns that end inside a tile, splits that do not divide, one
+row, a full 16, one more, 32; against float64, and what it leaves to torch."""
+import pytest
+import torch
+
+from ironcore_amd import _lib, generation
+
+pytestmark = pytest.mark.gpu
+
+# rounding to the element type; fp32: sums of up to 2 816 products in another order
+TOL = {torch.bfloat16: 4e-3, torch.float16: 5e-4, torch.float32: 2e-6}
+
+
+def _operands(gpu, dtype, m, k, n, seed):
+    g = torch.Generator().manual_seed(seed)
+    x, w, bias = torch.randn(m, k, generator=g), torch.randn(k, n, generator=g) * 0.05, torch.randn(n, generator=g)
+    return tuple(t.to(dtype).to(gpu) for t in (x, w, bias))
+
+
+def _distance(got, want):
+    return ((got.double().cpu() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,k,n", [(1, 32, 8), (1, 64, 136), (4, 768, 768), (16, 2816, 264), (17, 256, 1000),
+                                   (32, 4096, 128), (3, 96, 72)])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_against_float64(gpu, dtype, m, k, n, with_bias):
+    x, w, bias = _operands(gpu, dtype, m, k, n, m + n)
+    bias = bias if with_bias else torch.zeros_like(bias)
+    got = _lib.host().linear_rows(x, w, bias, *_lib.here(x))
+    want = x.double().cpu() @ w.double().cpu()
+    if with_bias:
+        want = want + bias.double().cpu()
+    assert got.shape == (m, n) and got.dtype == dtype
+    assert _distance(got, want) <= TOL[dtype]
+    wide = torch.zeros(k, n + 8, dtype=dtype, device=gpu)
+    wide[:, :n] = w                                     # rows further apart than long: the same sums
+    assert torch.equal(_lib.host().linear_rows(x, wide[:, :n], bias, *_lib.here(x)), got)
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3, 5])
+def test_any_split(gpu, splits):
+    x, w, bias = _operands(gpu, torch.float32, 7, 1056, 200, splits)    # 66 steps: splits of unequal length
+    lib, dev = _lib.load(), x.device
+    need = lib.ic_linear_rows_workspace_bytes(7, 200, 1056, splits, 2)
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+    out = torch.empty(7, 200, device=dev)
+    args = (out.data_ptr(), 200, x.data_ptr(), 1056, w.data_ptr(), 200, bias.data_ptr(), 7, 200, 1056, splits)
+    assert lib.ic_linear_rows(*args, ws.data_ptr(), need, 2, _lib.current_stream_ptr(dev)) == 0
+    want = x.double().cpu() @ w.double().cpu() + bias.double().cpu()
+    assert _distance(out, want) <= TOL[torch.float32]
+    if need:
+        assert lib.ic_linear_rows(*args, ws.data_ptr(), need - 1, 2, _lib.current_stream_ptr(dev)) == -4
+
+
+def test_what_is_left_to_torch(gpu):
+    """Gradients, autocast, vmap and shapes that the kernel does not take go through torch's product."""
+    x, w, bias = _operands(gpu, torch.float32, 4, 64, 32, 1)
+    want = torch.matmul(x, w) + bias
+    host, here = _lib.host(), _lib.here(x)
+    wg = w.clone().requires_grad_()
+    assert host.linear_rows(x, wg, bias, *here) is None
+    generation.linear(x, wg, bias).sum().backward()
+    assert torch.allclose(wg.grad, x.sum(0).unsqueeze(1).expand(64, 32), atol=1e-4)
+    with torch.no_grad():
+        assert host.linear_rows(x, wg, bias, *here) is not None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert torch.matmul(x, w).dtype == torch.bfloat16 and host.linear_rows(x, w, None, *here) is None
+        assert torch.allclose(torch.vmap(lambda v: generation.linear(v, w, bias))(x), want, atol=1e-4)
+        assert host.linear_rows(x, w, None, *here) is None      # short columns, no bias: torch's is as fast
+        for bad in (x[:, ::2], x.double(), torch.zeros(33, 64, device=gpu), torch.zeros(0, 64, device=gpu)):
+            assert host.linear_rows(bad, w, bias, *here) is None
+        assert host.linear_rows(x, w[:, :30], bias[:30], *here) is None and host.linear_rows(x, w.t(), None, *here) is None
+        odd = torch.empty(4 * 64 + 1, device=gpu)[1:].view(4, 64).copy_(x)      # not 16-byte aligned
+        assert torch.allclose(generation.linear(odd, w, bias), want, atol=1e-4)
