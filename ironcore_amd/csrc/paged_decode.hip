@@ -304,6 +304,175 @@ __global__ __launch_bounds__(NW *kWave) void paged_decode_kernel(const DecodeKP 
   }
 }
 
+// Small batches of short contexts (a few sequences of a small model, a few hundred tokens): with shares of a tile
+// the split above turns them into partials that a second launch merges, 8 + 5 us of which the tiles themselves take
+// two (4 sequences of up to 160 tokens, 12 heads of 64, fp32: 13.0 us, here 3.8).  Here a workgroup owns a whole pair: its eight waves take the pair's tiles in turn (a wave's table entries come
+// in one load, one per lane: at most 64 tiles), keep the running softmax of the kernel above and merge through LDS; one launch, no
+// workspace.  All types; the arithmetic is the vector-ALU kernel's (fp32 probabilities and sums).
+// Bound by the chain of round trips: context length and table, tile, merge.
+constexpr int kPairWaves = 8;
+
+template <class E, int HD, int GT>
+__global__ __launch_bounds__(kPairWaves *kWave) void paged_decode_pair_kernel(const DecodeKP p) {
+  using T = typename E::type;
+  constexpr int EPL = E::EPL;
+  constexpr int ES = sizeof(T);
+  constexpr int LPR = HD / EPL;     // lanes sharing one token row
+  constexpr int RPL = kWave / LPR;  // token rows per load instruction
+  constexpr int BS = 16;
+  constexpr int NLD = BS / RPL;     // load instructions per tile
+  __shared__ __attribute__((aligned(16))) float s_acc[kPairWaves][GT][HD];
+  __shared__ float s_m[kPairWaves][GT], s_l[kPairWaves][GT];
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int col = lane % LPR;
+  const int rowg = lane / LPR;
+  const int seq = blockIdx.y;
+  const int kvh = blockIdx.x;
+  const int heads = p.group;  // (at most GT: groups are not cut here)
+  const int head0 = kvh * heads;
+
+  int ctx = p.context_lens[seq];
+  ctx = ctx < p.max_ctx ? ctx : p.max_ctx;
+  ctx = ctx < 0 ? 0 : ctx;
+  const int tiles = (ctx + BS - 1) / BS;
+  const int mine = __builtin_amdgcn_readfirstlane(tiles > wave ? (tiles - wave + kPairWaves - 1) / kPairWaves : 0);
+  // lane r: byte offset of this wave's tile of round r
+  int64_t tile_off = 0;
+  if (lane < mine) {
+    const int tile = wave + lane * kPairWaves;
+    const int blk = tile / p.tiles_per_block;
+    int64_t phys = p.block_tables[seq * p.bt_stride + blk];
+    // A corrupt table entry must not become an out-of-pool address.
+    phys = phys < 0 ? 0 : phys;
+    phys = phys >= p.num_blocks ? p.num_blocks - 1 : phys;
+    tile_off = (phys * p.stride_block + kvh * p.stride_head +
+                (int64_t)(tile - blk * p.tiles_per_block) * BS * p.stride_token) * ES;
+  }
+  Vec16 qreg[GT];
+#pragma unroll
+  for (int g = 0; g < GT; ++g) {
+    const int h = head0 + (g < heads ? g : heads - 1);
+    qreg[g] = load16(p.q + (seq * p.q_stride_seq + (int64_t)h * HD + col * EPL) * ES);
+  }
+  uint32_t lane_off[NLD];
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) lane_off[i] = (uint32_t)(((i * RPL + rowg) * p.stride_token + col * EPL) * ES);
+
+  float m[GT], l[GT], acc[GT][EPL];
+#pragma unroll
+  for (int g = 0; g < GT; ++g) {
+    m[g] = kNegInf;
+    l[g] = 0.f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[g][e] = 0.f;
+  }
+  auto issue = [&](int r, Vec16 *kk, Vec16 *vv) {
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)tile_off, r);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)tile_off >> 32), r);
+    const int64_t at = (int64_t)(((uint64_t)hi << 32) | lo);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) kk[i] = load16(p.k_pool + at + lane_off[i]);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) vv[i] = load16(p.v_pool + at + lane_off[i]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto consume = [&](int r, Vec16 *kk, Vec16 *vv) {
+    float s[GT][NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i)
+#pragma unroll
+      for (int g = 0; g < GT; ++g) s[g][i] = group_sum<LPR>(E::dot(kk[i], qreg[g], 0.f)) * p.scale_log2e;
+    const int tok0 = (wave + r * kPairWaves) * BS;
+    if (tok0 + BS > ctx) {  // the sequence's last tile may be partly filled
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        if (tok0 + i * RPL + rowg >= ctx) {
+#pragma unroll
+          for (int g = 0; g < GT; ++g) s[g][i] = kNegInf;
+          vv[i] = Vec16{{0u, 0u, 0u, 0u}};
+        }
+      }
+    }
+    float vf[NLD][EPL];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) E::widen(vv[i], vf[i]);
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+      float mx = m[g];
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) mx = fmaxf(mx, s[g][i]);
+      const float ms = (mx == kNegInf) ? 0.f : mx;
+      const float alpha = __builtin_amdgcn_exp2f(m[g] - ms);
+      float pr[NLD];
+      float ps = 0.f;
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        pr[i] = __builtin_amdgcn_exp2f(s[g][i] - ms);
+        ps += pr[i];
+      }
+      l[g] = l[g] * alpha + ps;
+      m[g] = mx;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        float a = acc[g][e] * alpha;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) a = __builtin_fmaf(pr[i], vf[i][e], a);
+        acc[g][e] = a;
+      }
+    }
+  };
+  Vec16 ka[NLD], va[NLD], kb[NLD], vb[NLD];
+  if (mine > 0) issue(0, ka, va);
+  for (int r = 0; r < mine; r += 2) {
+    issue(r + 1 < mine ? r + 1 : r, kb, vb);
+    consume(r, ka, va);
+    if (r + 1 >= mine) break;
+    issue(r + 2 < mine ? r + 2 : r + 1, ka, va);
+    consume(r + 1, kb, vb);
+  }
+
+  // ---- merge: the row groups of a wave by exchange, the waves through LDS ----------------------
+#pragma unroll
+  for (int g = 0; g < GT; ++g) {
+    float mx = m[g];
+#pragma unroll
+    for (int off = LPR; off < kWave; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+    const float w = (m[g] == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m[g] - mx);
+    float ls = l[g] * w;
+#pragma unroll
+    for (int off = LPR; off < kWave; off <<= 1) ls += __shfl_xor(ls, off, kWave);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      float a = acc[g][e] * w;
+#pragma unroll
+      for (int off = LPR; off < kWave; off <<= 1) a += __shfl_xor(a, off, kWave);
+      if (rowg == 0) s_acc[wave][g][col * EPL + e] = a;
+    }
+    if (lane == 0) {
+      s_m[wave][g] = mx;
+      s_l[wave][g] = ls;
+    }
+  }
+  __syncthreads();
+  T *orow = reinterpret_cast<T *>(p.out) + seq * p.out_stride_seq + (int64_t)head0 * HD;
+  for (int o = threadIdx.x; o < heads * HD; o += kPairWaves * kWave) {
+    const int g = o / HD, d = o % HD;
+    float mx = kNegInf;
+#pragma unroll
+    for (int v = 0; v < kPairWaves; ++v) mx = fmaxf(mx, s_m[v][g]);
+    float sum = 0.f, a = 0.f;
+#pragma unroll
+    for (int v = 0; v < kPairWaves; ++v) {
+      const float w = s_m[v][g] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(s_m[v][g] - mx);
+      sum = __builtin_fmaf(s_l[v][g], w, sum);
+      a = __builtin_fmaf(s_acc[v][g][d], w, a);
+    }
+    orow[o] = E::narrow(tiles == 0 ? 0.f : a / sum);  // no visible token: zero rows
+  }
+}
+
 constexpr int kReduceThreads = 256;
 
 // Where the split-K partials of one (sequence, pair) lie.  A pair's tiles in a
@@ -552,8 +721,43 @@ void launch_valu_main(DecodeKP &kp, hipStream_t stream) {
   hipLaunchKernelGGL((paged_decode_kernel<E, HD, GT, BS, NW>), dim3(wgs), dim3(NW * kWave), 0, stream, kp);
 }
 
+// Whether a call is the pair kernel's.  us of the split (main kernel and reduce) / of the pair kernel, contexts up to
+// 48, 160, 300, 600, 1 200 tokens:
+//   fp32, 12 / 12 heads of 64, 4 sequences     9.8 / 3.1   13.0 / 3.8   15.6 / 4.3   19.3 / 5.5   27.9 / 8.1
+//   fp32, 32 / 32 of 128, 4                   11.6 / 3.7   14.1 / 5.0   18.9 / 7.7   26.8 / 13.8  35.6 / 22.4
+//   bf16, 32 / 32 of 128, 4                   11.0 / 3.6   13.0 / 4.5   14.8 / 5.1   20.2 / 8.0   24.6 / 13.9
+//   bf16, 16 / 16 of 64, 40                   14.4 / 4.7   18.3 / 5.6   22.3 / 9.4
+//   bf16, 32 / 8 of 128, 4                    10.2 / 6.4   13.0 / 8.4   15.2 / 10.1  19.7 / 14.3  18.2 / 21.3
+//   bf16, 32 / 8 of 128, 40                   12.2 / 11.8  16.0 / 15.2  19.9 / 20.9
+//   bf16, 28 / 4 of 128, 4                    10.1 / 10.4  13.2 / 14.1  15.2 / 17.1
+// One head per pair wins throughout; the lines keep a batch with a single long row among short ones, which the split
+// balances (8-10 us at least) and a workgroup walks alone, from losing.  Grouped heads cost this kernel vector work
+// for each head, hence short contexts only, and none from five heads on.
+bool decode_takes_pairs(const DecodeKP &kp, int row_bytes) {
+  if (kp.cohort_size != 1 || kp.key_mask != nullptr || kp.min_chunk > 1 || kp.max_ctx <= 0 || kp.group > 4) return false;
+  const int64_t rounds = ((int64_t)kp.max_ctx + 16 * kPairWaves - 1) / (16 * kPairWaves);
+  const int64_t pairs = (int64_t)kp.n_seqs * kp.pairs_per_seq;
+  if (kp.group > 1) return rounds <= 2 && pairs <= device_cu_count();
+  return rounds <= 10 && rounds * row_bytes <= 2560 && pairs <= 2 * device_cu_count();
+}
+
+template <class E, int HD>
+void launch_pairs(const DecodeKP &kp, hipStream_t stream) {
+  const dim3 grid(kp.pairs_per_seq, kp.n_seqs), block(kPairWaves * kWave);
+  if (kp.group == 1)
+    hipLaunchKernelGGL((paged_decode_pair_kernel<E, HD, 1>), grid, block, 0, stream, kp);
+  else if (kp.group == 2)
+    hipLaunchKernelGGL((paged_decode_pair_kernel<E, HD, 2>), grid, block, 0, stream, kp);
+  else
+    hipLaunchKernelGGL((paged_decode_pair_kernel<E, HD, 4>), grid, block, 0, stream, kp);
+}
+
 template <class E, int HD>
 int launch_group(DecodeKP &kp, int dtype, hipStream_t stream) {
+  if (decode_takes_pairs(kp, HD * (int)sizeof(typename E::type))) {
+    launch_pairs<E, HD>(kp, stream);
+    return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
+  }
   if constexpr (sizeof(typename E::type) == 2) {
     // 16-bit element types: the matrix-core kernel, whatever the group size.
     if (!launch_decode_mfma_main(kp, dtype, HD, stream)) return IC_ERR_UNSUPPORTED;
