@@ -12,6 +12,8 @@ constexpr int kAppendThreadsShift = 8;
 // Lanes a row takes in a workgroup, as a shift: a row that fills less than a workgroup shares it.  A few KV
 // heads are a wave's worth of chunks (4 heads of 128 in 16 bits: 64), and with a workgroup to a row the launch
 // is bound by how fast workgroups start and three quarters of their lanes do nothing.
+// 9 chunks padded to 701 tokens, 4 KV heads of 128, rotary, query rotated elsewhere: 4 us (the layer call
+// 56.2 -> 51.9); 8 192 tokens of 32 heads, whose rows fill their workgroups, as before.
 inline int append_row_shift(int chunks) {
   int shift = 0;
   while (shift < kAppendThreadsShift && (1 << shift) < chunks) ++shift;
