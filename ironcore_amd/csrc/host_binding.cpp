@@ -290,34 +290,62 @@ c10::optional<std::tuple<Tensor, Tensor, Tensor>> pack_mask(const Tensor &mask, 
   return std::make_tuple(bits, lists, flags);
 }
 
-// The dense call: query [b, sq, hn, hd] on key / value [b, sk, gn, hd], which the kernel walks as a pool of
-// one block per sequence, at whatever strides they have.
-// `bits`, `lists`: a packed mask of mask_seqs x mask_heads planes (1 or b, 1 or hn).
-OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, bool causal, const OptTensor &bits,
-                const OptTensor &lists, int64_t mask_seqs, int64_t mask_heads, double scale, int64_t device,
-                int64_t stream) {
-  if (query.dim() != 4 || key.dim() != 4 || key.size(1) == 0 || query.size(1) == 0) return c10::nullopt;
+// [b, s, heads, hd] row by row, the strides of size-1 dimensions included (is_contiguous() lets those be anything).
+Tensor row_major(const Tensor &t) {
+  const auto s = t.sizes(), st = t.strides();
+  if (st[3] == 1 && st[2] == s[3] && st[1] == s[2] * s[3] && st[0] == s[1] * s[2] * s[3]) return t;
+  return t.clone(at::MemoryFormat::Contiguous);
+}
+
+struct DenseMask {
+  bool causal;
+  const OptTensor &bits, &lists;  // packed: seqs x heads planes (1 or b, 1 or hn)
+  int64_t seqs, heads;
+};
+
+// The dense call on tensors as they lie: the kernel walks key and value as a pool of one block per sequence, at
+// whatever strides they share.
+OptTensor dense_as_laid(const Tensor &query, const Tensor &key, const Tensor &value, const DenseMask &m, double scale,
+                        int64_t device, void *stream) {
   const Pool p(key.permute({0, 2, 1, 3}), value.permute({0, 2, 1, 3}), device);
   const int64_t b = query.size(0), s = query.size(1), hn = query.size(2);
   if (!p.ok || !p.attends() || p.nb != b || hn % p.gn != 0 || !rows4(query, b, s, hn, p.hd) || !on(query, device) ||
       query.scalar_type() != key.scalar_type() || (b == 1 && p.sb < p.bs * p.st))
     return c10::nullopt;
   const Tensor out = at::empty({b, s, hn * p.hd}, query.options());
-  ic_prefill_call c = prefill_call(out, query, p, b, s, hn, scale, causal);
+  ic_prefill_call c = prefill_call(out, query, p, b, s, hn, scale, m.causal);
   c.row_pitch = s;
   c.uniform_context = (int)p.bs;
-  if (bits.has_value()) {
-    const int64_t planes = mask_seqs * mask_heads, qtiles = (s + 127) / 128, tiles = (p.bs + 63) / 64;
-    if (causal || !lists.has_value() || (mask_seqs != 1 && mask_seqs != b) || (mask_heads != 1 && mask_heads != hn) ||
-        !index_vector(*bits, at::kLong, planes * qtiles * 4 * tiles * 32, device) ||
-        !index_vector(*lists, at::kInt, planes * qtiles * (tiles + 1), device))
+  if (m.bits.has_value()) {
+    const int64_t planes = m.seqs * m.heads, qtiles = (s + 127) / 128, tiles = (p.bs + 63) / 64;
+    if (m.causal || !m.lists.has_value() || (m.seqs != 1 && m.seqs != b) || (m.heads != 1 && m.heads != hn) ||
+        !index_vector(*m.bits, at::kLong, planes * qtiles * 4 * tiles * 32, device) ||
+        !index_vector(*m.lists, at::kInt, planes * qtiles * (tiles + 1), device))
       return c10::nullopt;
-    c.mask_bits = reinterpret_cast<const uint64_t *>(bits->data_ptr<int64_t>());
-    c.mask_lists = lists->data_ptr<int32_t>();
-    c.mask_plane_head = mask_heads > 1 ? 1 : 0;
-    c.mask_plane_seq = mask_seqs > 1 ? (int)mask_heads : 0;
+    c.mask_bits = reinterpret_cast<const uint64_t *>(m.bits->data_ptr<int64_t>());
+    c.mask_lists = m.lists->data_ptr<int32_t>();
+    c.mask_plane_head = m.heads > 1 ? 1 : 0;
+    c.mask_plane_seq = m.seqs > 1 ? (int)m.heads : 0;
   }
-  if (ic_paged_prefill_ex(&c, (void *)stream) != IC_OK) return c10::nullopt;
+  if (ic_paged_prefill_ex(&c, stream) != IC_OK) return c10::nullopt;
+  return out;
+}
+
+// The dense call: query [b, sq, hn, hd] on key / value [b, sk, gn, hd].  Tensors that do not lie as the kernel walks
+// them are copied: a query whose rows are not one stride apart, keys and values with strides of their own (a rotary
+// model rotates the keys into a tensor of their own and leaves the values a slice of the projection).
+OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, bool causal, const OptTensor &bits,
+                const OptTensor &lists, int64_t mask_seqs, int64_t mask_heads, double scale, int64_t device,
+                int64_t stream) {
+  if (query.dim() != 4 || key.dim() != 4 || value.dim() != 4 || key.size(1) == 0 || query.size(1) == 0)
+    return c10::nullopt;
+  const DenseMask m{causal, bits, lists, mask_seqs, mask_heads};
+  const Tensor q = rows4(query, query.size(0), query.size(1), query.size(2), query.size(3)) ? query : row_major(query);
+  OptTensor out = dense_as_laid(q, key, value, m, scale, device, (void *)stream);
+  if (!out.has_value()) {
+    const Tensor k = row_major(key), v = row_major(value);
+    if (!k.is_same(key) || !v.is_same(value)) out = dense_as_laid(q, k, v, m, scale, device, (void *)stream);
+  }
   return out;
 }
 

@@ -79,9 +79,10 @@ class PackedMask:
     def bytes(self) -> torch.Tensor:
         """The byte mask again (uint8), for a call the packed kernels do not take."""
         n, heads, rows, keys = self.shape
-        words = self.bits.permute(0, 1, 3, 2).reshape(n * heads, -1, self.bits.shape[2], 1)
-        bit = (words >> torch.arange(64, device=words.device)) & 1
-        return bit.reshape(n, heads, bit.shape[1], -1)[:, :, :rows, :keys].to(torch.uint8).contiguous()
+        parts = self.bits.view(torch.uint8).view(*self.bits.shape, 8).transpose(2, 3)      # ..., row, tile, byte of 8 keys
+        bit = parts.reshape(n * heads, -1, parts.shape[3] * 8, 1) >> torch.arange(8, dtype=torch.uint8, device=parts.device)
+        bit &= 1
+        return bit.view(n, heads, bit.shape[1], -1)[:, :, :rows, :keys].contiguous()
 
 
 @dataclass
