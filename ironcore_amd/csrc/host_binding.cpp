@@ -35,6 +35,17 @@ int dtype_code(at::ScalarType t) {
   }
 }
 
+// Whether a library call was made: false for arguments that it does not take, which the Python wrapper then handles
+// or refuses by name.  A launch that failed is raised from here, as _lib.PagedLibraryError: the library has read (and
+// so cleared) HIP's last error, and a second try by the wrapper would hide it.
+bool made(const char *func, int rc) {
+  if (rc == IC_ERR_LAUNCH) {
+    py::gil_scoped_acquire gil;
+    py::module_::import("ironcore_amd._lib").attr("check")(func, rc);
+  }
+  return rc == IC_OK;
+}
+
 bool on(const Tensor &t, int64_t device) { return t.is_cuda() && t.get_device() == device; }
 
 struct Pool {
@@ -75,8 +86,9 @@ int64_t row_stride4(const Tensor &t) { return t.size(1) > 1 ? t.stride(1) : t.st
 
 bool append_rows(const void *k, const void *v, int64_t stride, const Pool &p, const Tensor &slots, int64_t n,
                  void *stream) {
-  return ic_kv_append(k, v, stride, const_cast<void *>(p.k), const_cast<void *>(p.v), p.sb, p.sh, p.st,
-                      slots.data_ptr<int64_t>(), n, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream) == IC_OK;
+  return made("ic_kv_append",
+              ic_kv_append(k, v, stride, const_cast<void *>(p.k), const_cast<void *>(p.v), p.sb, p.sh, p.st,
+                           slots.data_ptr<int64_t>(), n, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream));
 }
 
 struct Decode {
@@ -99,12 +111,13 @@ bool decode(const Tensor &out, const void *q, int64_t q_stride, const Pool &p, i
   const size_t need = ic_paged_decode_shared_workspace_bytes((int)b, (int)hn, (int)p.gn, (int)p.hd, (int)d.cohort);
   if (need == 0) return false;
   const Tensor ws = at::empty({(int64_t)need}, out.options().dtype(at::kByte));
-  return ic_paged_decode_shared(out.data_ptr(), out.stride(0), q, q_stride, p.k, p.v, p.sb, p.sh, p.st,
-                                d.tables.data_ptr<int32_t>(), d.tables.stride(0), d.lens.data_ptr<int32_t>(), (int)b,
-                                (int)hn, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, (int)d.max_ctx, (float)d.scale,
-                                (int)d.min_chunk, (int)d.cohort,
-                                d.cohort > 1 ? d.shared->data_ptr<int32_t>() : nullptr, ws.data_ptr(), need, p.dtype,
-                                stream) == IC_OK;
+  return made("ic_paged_decode_shared",
+              ic_paged_decode_shared(out.data_ptr(), out.stride(0), q, q_stride, p.k, p.v, p.sb, p.sh, p.st,
+                                     d.tables.data_ptr<int32_t>(), d.tables.stride(0), d.lens.data_ptr<int32_t>(),
+                                     (int)b, (int)hn, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, (int)d.max_ctx,
+                                     (float)d.scale, (int)d.min_chunk, (int)d.cohort,
+                                     d.cohort > 1 ? d.shared->data_ptr<int32_t>() : nullptr, ws.data_ptr(), need,
+                                     p.dtype, stream));
 }
 
 // ---- tensor-level calls (paged_ops) ----------------------------------------------------------
@@ -177,10 +190,11 @@ struct NewRows {
 // Append with the keys rotated on their way; q_out == nullptr: the query is left alone.
 bool rope_append(const Tensor &key, const Tensor &value, const Pool &p, const Tensor &slots, const Rope &r, int64_t n,
                  void *q_out, const void *q, int64_t q_stride, int64_t hn, void *stream) {
-  return ic_rope_kv_append_to(q_out, hn * p.hd, q_out ? q : nullptr, q_stride, (int)hn, key.data_ptr(),
-                              value.data_ptr(), row_stride4(key), const_cast<void *>(p.k), const_cast<void *>(p.v),
-                              p.sb, p.sh, p.st, slots.data_ptr<int64_t>(), r.positions, r.cos, r.sin, r.rows, n,
-                              (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream) == IC_OK;
+  return made("ic_rope_kv_append_to",
+              ic_rope_kv_append_to(q_out, hn * p.hd, q_out ? q : nullptr, q_stride, (int)hn, key.data_ptr(),
+                                   value.data_ptr(), row_stride4(key), const_cast<void *>(p.k),
+                                   const_cast<void *>(p.v), p.sb, p.sh, p.st, slots.data_ptr<int64_t>(), r.positions,
+                                   r.cos, r.sin, r.rows, n, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream));
 }
 
 // One cached decode step of a layer (sq == 1): append, then attend.  With rotary tables the query is
@@ -258,8 +272,9 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
     c.rows = rows->data_ptr<int64_t>();
     c.n_rows = rows->numel(), c.q_rows = in.b * in.s;
     const int row_bytes = (int)(in.hn * p.hd * query.element_size());
-    if (ic_zero_unlisted_rows(c.out, row_bytes, row_bytes, c.rows, c.n_rows, bounds.data_ptr<int32_t>(), (int)in.b,
-                              (int)in.s, (void *)stream) != IC_OK)
+    if (!made("ic_zero_unlisted_rows",
+              ic_zero_unlisted_rows(c.out, row_bytes, row_bytes, c.rows, c.n_rows, bounds.data_ptr<int32_t>(),
+                                    (int)in.b, (int)in.s, (void *)stream)))
       return c10::nullopt;
   }
   c.block_tables = tables.data_ptr<int32_t>();
@@ -268,7 +283,7 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
   c.cu_seqlens_q = bounds.data_ptr<int32_t>();
   c.positions = rope.positions;
   c.cos_table = rope.cos, c.sin_table = rope.sin, c.table_rows = rope.rows;
-  if (ic_paged_prefill_ex(&c, (void *)stream) != IC_OK) return c10::nullopt;
+  if (!made("ic_paged_prefill_ex", ic_paged_prefill_ex(&c, (void *)stream))) return c10::nullopt;
   return out;
 }
 
@@ -283,9 +298,10 @@ c10::optional<std::tuple<Tensor, Tensor, Tensor>> pack_mask(const Tensor &mask, 
   const Tensor bits = at::empty({n * heads, qtiles * 4, tiles, 32}, mask.options().dtype(at::kLong));
   const Tensor lists = at::empty({n * heads, qtiles, tiles + 1}, mask.options().dtype(at::kInt));
   const Tensor flags = at::ones({2}, mask.options().dtype(at::kInt));
-  if (ic_mask_pack(mask.data_ptr<uint8_t>(), mask.stride(0), mask.stride(1), mask.stride(2), (int)n, (int)heads,
-                   (int)rows, (int)keys, reinterpret_cast<uint64_t *>(bits.data_ptr<int64_t>()),
-                   lists.data_ptr<int32_t>(), flags.data_ptr<int32_t>(), (void *)stream) != IC_OK)
+  if (!made("ic_mask_pack",
+            ic_mask_pack(mask.data_ptr<uint8_t>(), mask.stride(0), mask.stride(1), mask.stride(2), (int)n, (int)heads,
+                         (int)rows, (int)keys, reinterpret_cast<uint64_t *>(bits.data_ptr<int64_t>()),
+                         lists.data_ptr<int32_t>(), flags.data_ptr<int32_t>(), (void *)stream)))
     return c10::nullopt;
   return std::make_tuple(bits, lists, flags);
 }
@@ -327,7 +343,7 @@ OptTensor dense_as_laid(const Tensor &query, const Tensor &key, const Tensor &va
     c.mask_plane_head = m.heads > 1 ? 1 : 0;
     c.mask_plane_seq = m.seqs > 1 ? (int)m.heads : 0;
   }
-  if (ic_paged_prefill_ex(&c, stream) != IC_OK) return c10::nullopt;
+  if (!made("ic_paged_prefill_ex", ic_paged_prefill_ex(&c, stream))) return c10::nullopt;
   return out;
 }
 
@@ -383,9 +399,10 @@ OptTensor linear_rows(const Tensor &x, const Tensor &w, const OptTensor &bias, i
   const Tensor out = at::empty(sizes, x.options());
   Tensor ws;
   if (need > 0) ws = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
-  if (ic_linear_rows(out.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), w.stride(0),
-                     bias.has_value() ? bias->data_ptr() : nullptr, (int)m, (int)n, (int)k, 0,
-                     need > 0 ? ws.data_ptr() : nullptr, need, dtype, (void *)stream) != IC_OK)
+  if (!made("ic_linear_rows",
+            ic_linear_rows(out.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), w.stride(0),
+                           bias.has_value() ? bias->data_ptr() : nullptr, (int)m, (int)n, (int)k, 0,
+                           need > 0 ? ws.data_ptr() : nullptr, need, dtype, (void *)stream)))
     return c10::nullopt;
   return out;
 }

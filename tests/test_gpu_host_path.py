@@ -184,3 +184,37 @@ def test_out_of_memory_keeps_its_type(gpu):
     tables = torch.zeros(1, 1, dtype=torch.int32, device=gpu).expand(b, 1)
     with pytest.raises(torch.OutOfMemoryError):
         paged_ops.paged_decode(query, pool, pool, tables, torch.ones(b, dtype=torch.int32, device=gpu), 16)
+
+
+def _failed_hip_call():
+    """Leaves a last error in the runtime that the library was linked to, by a call that the host refuses."""
+    import ctypes
+    with open("/proc/self/maps") as maps:
+        path = next(line.split()[-1] for line in maps if "libamdhip64" in line)
+    assert ctypes.CDLL(path).hipSetDevice(1 << 20) != 0
+
+
+def test_a_failed_launch_is_reported(gpu, monkeypatch):
+    """A launch error raises, as it does from the Python path, and is not tried away; the next call runs."""
+    wl = workloads.make_decode_workload(3, 4, 2, 64, 20, 40, seed=1).to(gpu)
+    k = torch.randn(3, 2, 64, device=gpu).bfloat16()
+    q, slots = torch.randn(3, 4, 64, device=gpu).bfloat16(), torch.tensor([0, 17, 33], device=gpu)
+    meta = PagedAttentionMetadata(block_tables=wl.block_tables, context_lens=wl.context_lens, slot_mapping=slots,
+                                  max_context_len=wl.max_context_len)
+    attn = _layer(4, 2, 64, "bf16")
+    x, w = torch.randn(4, 64, device=gpu), torch.randn(64, 32, device=gpu)
+    calls = [lambda: paged_ops.kv_append(k, k, wl.k_pool, wl.v_pool, slots),
+             lambda: paged_ops.paged_decode(wl.query, wl.k_pool, wl.v_pool, wl.block_tables, wl.context_lens,
+                                            wl.max_context_len),
+             lambda: attn(q[:, None], k[:, None], k[:, None], kv_cache=(wl.k_pool, wl.v_pool), attn_metadata=meta),
+             lambda: attn(q[None], k[None], k[None]),
+             lambda: _lib.host().linear_rows(x, w, w[0], *_lib.here(x))]
+    for n, call in enumerate(calls):
+        call()                                              # memory for its output is at hand
+        torch.cuda.synchronize()
+        _failed_hip_call()
+        with pytest.raises(_lib.PagedLibraryError) as err:
+            call()
+        assert err.value.code == -5, n
+        call()
+        torch.cuda.synchronize()
