@@ -4,10 +4,13 @@
 // bound by this path (three launches of a few microseconds each behind 33 us of
 // Python on one core); the functions here leave 2-3 us of it.
 //
-// Each function handles the ordinary case completely, or does nothing and
-// returns None: the Python wrapper (paged_ops.py, layers/attention.py) then takes
-// its own path, which makes tensors contiguous, switches the device or names
-// what is wrong with the arguments.  Nothing is kept between calls: outputs and
+// Each function handles the ordinary case completely, or returns None: the Python
+// wrapper (paged_ops.py, layers/attention.py) then takes its own path, which makes
+// tensors contiguous, switches the device or names what is wrong with the arguments.
+// What a layer call's attention does not take is looked for before its append is
+// launched; where only the library's own limits refuse it (2^31 rows, a 4 GiB block),
+// the append has been made, and the wrapper makes it again, the same rows into the
+// same slots.  Nothing is kept between calls: outputs and
 // workspaces come from torch's allocator, which orders their reuse on the stream
 // and serves a capturing stream from the graph's own pool.
 #include <torch/extension.h>
@@ -84,6 +87,11 @@ bool rows4(const Tensor &t, int64_t b, int64_t s, int64_t heads, int64_t hd) {
 }
 int64_t row_stride4(const Tensor &t) { return t.size(1) > 1 ? t.stride(1) : t.stride(0); }
 
+// Rows that a kernel reads in 16-byte pieces, `row` elements each.
+bool rows16(const void *p, int64_t stride, int64_t row, int64_t element_size) {
+  return reinterpret_cast<uintptr_t>(p) % 16 == 0 && (stride * element_size) % 16 == 0 && stride >= row;
+}
+
 bool append_rows(const void *k, const void *v, int64_t stride, const Pool &p, const Tensor &slots, int64_t n,
                  void *stream) {
   return made("ic_kv_append",
@@ -100,7 +108,9 @@ struct Decode {
 
 bool decode_fits(const Pool &p, int64_t b, int64_t hn, const Decode &d, int64_t device) {
   if (!p.attends() || hn % p.gn != 0 || b == 0 || !table(d.tables, b, device) ||
-      !index_vector(d.lens, at::kInt, b, device) || d.max_ctx > d.tables.size(1) * p.bs || d.cohort < 1)
+      !index_vector(d.lens, at::kInt, b, device) || d.max_ctx > d.tables.size(1) * p.bs || d.cohort < 1 ||
+      p.bs % 16 != 0 ||
+      ic_paged_decode_shared_workspace_bytes((int)b, (int)hn, (int)p.gn, (int)p.hd, (int)d.cohort) == 0)
     return false;
   return d.cohort == 1 ||
          (d.shared.has_value() && index_vector(*d.shared, at::kInt, (b + d.cohort - 1) / d.cohort, device));
@@ -109,7 +119,6 @@ bool decode_fits(const Pool &p, int64_t b, int64_t hn, const Decode &d, int64_t 
 bool decode(const Tensor &out, const void *q, int64_t q_stride, const Pool &p, int64_t b, int64_t hn, const Decode &d,
             void *stream) {
   const size_t need = ic_paged_decode_shared_workspace_bytes((int)b, (int)hn, (int)p.gn, (int)p.hd, (int)d.cohort);
-  if (need == 0) return false;
   const Tensor ws = at::empty({(int64_t)need}, out.options().dtype(at::kByte));
   return made("ic_paged_decode_shared",
               ic_paged_decode_shared(out.data_ptr(), out.stride(0), q, q_stride, p.k, p.v, p.sb, p.sh, p.st,
@@ -213,6 +222,7 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
   if (!rope.ok || !decode_fits(p, in.b, in.hn, d, device)) return c10::nullopt;
   const void *q = query.data_ptr();
   int64_t q_stride = row_stride4(query);
+  if (!rows16(q, q_stride, in.hn * p.hd, query.element_size())) return c10::nullopt;
   Tensor rotated;
   if (rope.used) {
     rotated = at::empty({in.b, in.hn * p.hd}, query.options());
@@ -250,14 +260,17 @@ ic_prefill_call prefill_call(const Tensor &out, const Tensor &query, const Pool 
 // kernel.
 OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
                        const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
-                       const Tensor &bounds, const OptTensor &rows, int64_t longest, double scale, const OptTensor &positions, const OptTensor &cos,
-                       const OptTensor &sin, int64_t device, int64_t stream) {
+                       const Tensor &bounds, const OptTensor &rows, int64_t longest, double scale,
+                       const OptTensor &positions, const OptTensor &cos, const OptTensor &sin, int64_t device,
+                       int64_t stream) {
   const Pool p(k_pool, v_pool, device);
   if (!p.ok || !p.attends()) return c10::nullopt;
   const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
   if (!in.ok || in.hn % p.gn != 0 || !index_vector(slots, at::kLong, in.b * in.s, device) ||
       !table(tables, in.b, device) || !index_vector(lens, at::kInt, in.b, device) ||
       !index_vector(bounds, at::kInt, in.b + 1, device) || longest > in.s ||
+      !rows16(query.data_ptr(), row_stride4(query), in.hn * p.hd, query.element_size()) ||
+      (p.dtype != IC_DTYPE_F32 && p.bs % 16 != 0 && tables.stride(0) != 1) ||  // 16 bits: whole groups of 16 rows
       (rows.has_value() && (rows->numel() == 0 || !index_vector(*rows, at::kLong, rows->numel(), device))))
     return c10::nullopt;
   const Rope rope(positions, cos, sin, in.b * in.s, p.hd, device);

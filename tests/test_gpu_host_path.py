@@ -218,3 +218,23 @@ def test_a_failed_launch_is_reported(gpu, monkeypatch):
         assert err.value.code == -5, n
         call()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("why", ["block size", "query start"])
+def test_nothing_is_appended_for_a_call_that_is_not_taken(gpu, why):
+    """The binding looks for what the attention does not take before it launches the append."""
+    hn, gn, hd, bs = 4, 2, 64, 24 if why == "block size" else 16
+    pools = torch.zeros(2, 6, gn, bs, hd, dtype=torch.bfloat16, device=gpu)
+    k = torch.ones(3, 1, gn, hd, dtype=torch.bfloat16, device=gpu)
+    start = 1 if why == "query start" else 0
+    q = torch.ones(3 * hn * hd + 1, dtype=torch.bfloat16, device=gpu)[start:start + 3 * hn * hd].view(3, 1, hn, hd)
+    tables = torch.arange(6, dtype=torch.int32, device=gpu).view(3, 2)
+    lens, slots = torch.full((3,), 5, dtype=torch.int32, device=gpu), torch.arange(3, device=gpu) * 2 * bs
+    host, here = _lib.host(), _lib.here(q)
+    assert host.decode_step(q, k, k, *pools, tables, lens, slots, 5, 0.125, 1, None, None, None, None, *here) is None
+    assert host.prefill_step(q, k, k, *pools, tables, lens, slots, torch.arange(4, dtype=torch.int32, device=gpu), None, 1,
+                             0.125, None, None, None, *here) is None
+    assert not pools.any()
+    meta = PagedAttentionMetadata(block_tables=tables, context_lens=lens, slot_mapping=slots, max_context_len=5)
+    with pytest.raises(_lib.PagedLibraryError):     # and the layer refuses it by name, as before
+        _layer(hn, gn, hd, "bf16")(q, k, k, kv_cache=tuple(pools), attn_metadata=meta)
