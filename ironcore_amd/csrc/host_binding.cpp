@@ -423,13 +423,14 @@ OptTensor linear_rows(const Tensor &x, const Tensor &w, const OptTensor &bias, i
 }  // namespace
 
 // (wrapped, so that torch's exceptions keep their Python types: an allocation that does not fit raises
-// torch.OutOfMemoryError)
+// torch.OutOfMemoryError.  The GIL is given up for the call: a launch may wait on a full queue and an allocation on the
+// GPU, and other threads go on meanwhile.)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("kv_append", torch::wrap_pybind_function(kv_append));
-  m.def("paged_decode", torch::wrap_pybind_function(paged_decode));
-  m.def("decode_step", torch::wrap_pybind_function(decode_step));
-  m.def("prefill_step", torch::wrap_pybind_function(prefill_step));
-  m.def("dense", torch::wrap_pybind_function(dense));
-  m.def("linear_rows", torch::wrap_pybind_function(linear_rows));
-  m.def("pack_mask", torch::wrap_pybind_function(pack_mask));
+  m.def("kv_append", torch::wrap_pybind_function_no_gil(kv_append));
+  m.def("paged_decode", torch::wrap_pybind_function_no_gil(paged_decode));
+  m.def("decode_step", torch::wrap_pybind_function_no_gil(decode_step));
+  m.def("prefill_step", torch::wrap_pybind_function_no_gil(prefill_step));
+  m.def("dense", torch::wrap_pybind_function_no_gil(dense));
+  m.def("linear_rows", torch::wrap_pybind_function_no_gil(linear_rows));
+  m.def("pack_mask", torch::wrap_pybind_function_no_gil(pack_mask));
 }
