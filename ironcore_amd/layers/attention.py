@@ -340,26 +340,22 @@ class Attention(BaseModule):
         k_pool, v_pool = kv_cache
         rows = getattr(meta, "chunk_rows", None)
         here = _lib.here(query)
+        rope = None if rotary_pos_emb is None else (meta.positions, rotary_pos_emb.cos_emb, rotary_pos_emb.sin_emb)
         if here is not None and sq == 1 and rows is None:
-            rope = rotary_pos_emb
-            cohort = meta.cohort_size if query.dtype != torch.float32 else 1
+            cohort = int(meta.cohort_size) if query.dtype != torch.float32 else 1
             out = _lib.host().decode_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
-                                          meta.slot_mapping, meta.max_context_len, 1.0 / self.scale_factor, cohort,
-                                          meta.cohort_shared_blocks if cohort > 1 else None, meta.positions,
-                                          None if rope is None else rope.cos_emb,
-                                          None if rope is None else rope.sin_emb, *here)
+                                          meta.slot_mapping, int(meta.max_context_len), 1.0 / self.scale_factor, cohort,
+                                          meta.cohort_shared_blocks if cohort > 1 else None,
+                                          *(rope or (None, None, None)), *here)
             if out is not None:
                 return out
-        elif here is not None:
-            rope = rotary_pos_emb
+        elif here is not None and (rows is None or meta.cu_seqlens_q is not None):   # (rows come with their bounds)
             bounds = meta.cu_seqlens_q
             if bounds is None:
                 bounds = torch.arange(0, (b + 1) * sq, sq, dtype=torch.int32, device=query.device)
             out = _lib.host().prefill_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
-                                           meta.slot_mapping, bounds, rows, sq if rows is None else meta.max_chunk_len,
-                                           1.0 / self.scale_factor, meta.positions,
-                                           None if rope is None else rope.cos_emb,
-                                           None if rope is None else rope.sin_emb, *here)
+                                           meta.slot_mapping, bounds, rows, sq if rows is None else int(meta.max_chunk_len),
+                                           1.0 / self.scale_factor, *(rope or (None, None, None)), *here)
             if out is not None:
                 return out
         if rotary_pos_emb is None:

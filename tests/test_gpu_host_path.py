@@ -238,3 +238,33 @@ def test_nothing_is_appended_for_a_call_that_is_not_taken(gpu, why):
     meta = PagedAttentionMetadata(block_tables=tables, context_lens=lens, slot_mapping=slots, max_context_len=5)
     with pytest.raises(_lib.PagedLibraryError):     # and the layer refuses it by name, as before
         _layer(hn, gn, hd, "bf16")(q, k, k, kv_cache=tuple(pools), attn_metadata=meta)
+
+
+def test_metadata_as_the_python_path_takes_it(gpu, monkeypatch):
+    """Bounds that are floats, metadata of another class with only the fields a call needs; and chunk rows
+    without their bounds, which neither path takes."""
+    from types import SimpleNamespace
+    hn, gn, hd, b = 4, 2, 64, 4
+    attn = _layer(hn, gn, hd, "bf16")
+    wl = workloads.make_grpo_workload(2, 2, hn, gn, hd, 64, 1, 90, seed=2).to(gpu)
+    last = wl.context_lens.long() - 1
+    slots = wl.block_tables.long().gather(1, (last // 16).unsqueeze(1)).squeeze(1) * 16 + last % 16
+    shared = torch.full((2,), 4, dtype=torch.int32, device=gpu)
+    meta = SimpleNamespace(block_tables=wl.block_tables, context_lens=wl.context_lens, slot_mapping=slots,
+                           max_context_len=float(wl.max_context_len), cohort_size=2.0, cohort_shared_blocks=shared)
+    k = torch.randn(b, 1, gn, hd, device=gpu).bfloat16()
+    q = torch.randn(b, 1, hn, hd, device=gpu).bfloat16()
+    native, plain = _both(monkeypatch, lambda: attn(q, k, k, kv_cache=(wl.k_pool, wl.v_pool), attn_metadata=meta))
+    assert torch.equal(native, plain)
+
+    wl = workloads.make_prefill_workload(3, hn, gn, hd, 0, 20, 1, 30, seed=4)
+    meta, q, k, v = _ragged(gpu, wl, torch.bfloat16, 16, 1)
+    pools = wl.k_pool.to(gpu), wl.v_pool.to(gpu)
+    fields = {name: getattr(meta, name) for name in ("block_tables", "context_lens", "slot_mapping", "max_context_len",
+                                                     "cu_seqlens_q", "chunk_rows")}
+    meta = SimpleNamespace(**fields, max_chunk_len=float(meta.max_chunk_len))
+    native, plain = _both(monkeypatch, lambda: attn(q, k, v, kv_cache=pools, attn_metadata=meta))
+    assert torch.equal(native, plain)
+    meta.cu_seqlens_q = None
+    with pytest.raises(AttributeError):
+        attn(q, k, v, kv_cache=pools, attn_metadata=meta)
