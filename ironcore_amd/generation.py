@@ -41,8 +41,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     step go through the package's kernel (csrc/linear_rows.hip); more rows, and
     calls that torch has to see (autograd, autocast, tracing, subclasses), through
     torch's product."""
-    if not (torch.overrides.has_torch_function_variadic(x, weight) or torch.compiler.is_compiling()
-            or torch.jit.is_tracing()):
+    given = (x, weight) if bias is None else (x, weight, bias)
+    # (a fake tensor says that it is on a GPU where there is none)
+    if type(x) in (torch.Tensor, nn.Parameter) and not (
+            torch.overrides.has_torch_function_variadic(*given) or torch.compiler.is_compiling() or torch.jit.is_tracing()):
         here = _lib.here(x)
         if here is not None:
             y = _lib.host().linear_rows(x, weight, bias, *here)

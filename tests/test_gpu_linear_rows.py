@@ -75,3 +75,11 @@ def test_what_is_left_to_torch(gpu):
         assert host.linear_rows(x, w[:, :30], bias[:30], *here) is None and host.linear_rows(x, w.t(), None, *here) is None
         odd = torch.empty(4 * 64 + 1, device=gpu)[1:].view(4, 64).copy_(x)      # not 16-byte aligned
         assert torch.allclose(generation.linear(odd, w, bias), want, atol=1e-4)
+
+
+def test_a_bias_that_torch_has_to_see(gpu):
+    class Seen(torch.Tensor):
+        pass
+    x, w, bias = _operands(gpu, torch.float32, 4, 64, 32, 1)
+    y = generation.linear(x, w, bias.as_subclass(Seen))
+    assert type(y) is Seen and torch.equal(y.as_subclass(torch.Tensor), torch.matmul(x, w) + bias)

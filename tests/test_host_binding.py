@@ -7,7 +7,7 @@ import time
 import pytest
 import torch
 
-from ironcore_amd import _lib
+from ironcore_amd import _lib, generation
 
 
 def _calls():
@@ -51,3 +51,13 @@ def test_other_threads_run_during_a_call(name):
         sys.setswitchinterval(switch)
     thread.join()
     assert during
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_on_fake_tensors(bias):
+    """Shapes worked out without a GPU, as torch's product does: nothing asks for the device."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x, w = torch.empty(4, 64, device="cuda"), torch.empty(64, 32, device="cuda")
+        y = generation.linear(x, w, torch.empty(32, device="cuda") if bias else None)
+        assert y.shape == (4, 32) and y.is_cuda
