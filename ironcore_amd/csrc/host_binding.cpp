@@ -385,6 +385,29 @@ bool plain(const Tensor &t) {
   return !at::isTensorSubclassLike(t) && !t.is_conj() && !t.is_neg() && !t._fw_grad(0).defined();
 }
 
+// Whether torch's product, and its addition of the bias, is as fast or faster for m rows, the weights read from memory.
+// (splits: what the kernel would take; a tile is a workgroup's 64 columns in fp32, 128 in 16 bits.)  Library / kernel, us:
+//  * more columns than the CUs hold tiles of at once, so that a second, short wave of workgroups runs alone: 1 024 x
+//    50 304 fp32 39 / 47, 4 096 x 50 304 bf16 68 / 74; x 32 000 28 / 26 and 53 / 47;
+//  * fp32, more than 16 rows, one split (each workgroup reads all of x twice over): 4 096 x 11 008 46 / 58, with the
+//    bias 48 / 57; short columns have a bias's launch to gain: 512 x 2 048 11 / 8;
+//  * two splits of 113 to 128 tiles: 4 096 x 8 192 fp32 26 / 29, 4 096 x 16 384 bf16 26 / 28, while 8 192 x 8 192 is
+//    57 / 53, 1 536 x 8 192 fp32 16 / 14 and 1 088 x 16 384 bf16 13 / 11;
+//  * short columns, whose split pays for its second launch only by a bias: fp32, 8 rows 640 x 4 096 7.0 / 7.6, 768 x
+//    3 072 8.0 / 7.5, 17 rows 1 024 x 4 096 9.1 / 10.3, 3 072 x 3 072 18 / 17; bf16, 16 rows 1 536 x 1 536 7 / 8, x
+//    6 144 12 / 10, 2 048 x 2 048 9 / 8, 17 rows 1 792 x 2 048 8 / 9; without a split, 1 024 x 1 024 6.0 / 6.8.
+bool library_as_fast(int64_t m, int64_t n, int64_t k, bool fp32, int64_t splits, bool bias) {
+  const int64_t tiles = (n + (fp32 ? 63 : 127)) / (fp32 ? 64 : 128);
+  const bool many = m > 16;
+  if (tiles > (fp32 ? 512 : 256) && (fp32 || !bias)) return true;
+  const bool two_splits = splits == 2 && tiles > 112 && k < 8192 && k >= (fp32 ? 2048 : 1280);
+  if (bias) return fp32 && many && (splits == 1 ? k > 768 || n > 16384 : two_splits);
+  if (splits == 1) return many || k * (fp32 ? 4 : 2) <= 2048;
+  if (two_splits) return true;
+  if (many) return fp32 ? splits < 8 && k < 3072 : k < 2048;
+  return fp32 ? k < (m > 8 ? 1024 : 768) : k < 2048 && n < 5120;
+}
+
 // y = x W (+ bias) for the few rows of a decode step; x [..., k] contiguous, W [k, n].  What a dispatched product
 // would do beside it (autograd, autocast, tracing, dispatch modes) is left to that.
 OptTensor linear_rows(const Tensor &x, const Tensor &w, const OptTensor &bias, int64_t device, int64_t stream) {
@@ -403,10 +426,8 @@ OptTensor linear_rows(const Tensor &x, const Tensor &w, const OptTensor &bias, i
   const int es = (int)x.element_size();
   if (n % (16 / es) != 0 || k % (64 / es) != 0 || (w.stride(0) * es) % 16 != 0 || w.stride(0) < n) return c10::nullopt;
   const size_t need = ic_linear_rows_workspace_bytes((int)m, (int)n, (int)k, 0, dtype);
-  // Without a bias to fuse and with nothing to gain from split sums the library's product is as fast or faster for
-  // short columns and for more than 16 rows (bf16, this kernel / the library: 16 rows, 1 024 x 1 024 6.8 / 6.0 us,
-  // 1 024 x 5 504 9.4 / 8.9; 32 rows, 4 096 x 22 016 42.3 / 40.4).
-  if (!bias.has_value() && need == 0 && (m > 16 || k * es <= 2048)) return c10::nullopt;
+  const int64_t splits = need > 0 ? (int64_t)need / (4 * m * n) : 1;
+  if (library_as_fast(m, n, k, dtype == IC_DTYPE_F32, splits, bias.has_value())) return c10::nullopt;
   auto sizes = x.sizes().vec();
   sizes.back() = n;
   const Tensor out = at::empty(sizes, x.options());

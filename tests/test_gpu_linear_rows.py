@@ -83,3 +83,28 @@ def test_a_bias_that_torch_has_to_see(gpu):
     x, w, bias = _operands(gpu, torch.float32, 4, 64, 32, 1)
     y = generation.linear(x, w, bias.as_subclass(Seen))
     assert type(y) is Seen and torch.equal(y.as_subclass(torch.Tensor), torch.matmul(x, w) + bias)
+
+
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+@pytest.mark.parametrize("dtype,with_bias,m,k,n,taken", [
+    (F32, False, 8, 768, 1024, True), (F32, False, 8, 704, 1024, False), (F32, False, 9, 768, 1024, False),
+    (F32, False, 9, 1024, 1024, True), (F32, False, 17, 1024, 2048, True), (F32, False, 17, 1024, 4096, False),
+    (F32, False, 17, 3072, 4096, True), (F32, False, 4, 2048, 8192, False), (F32, False, 4, 1536, 8192, True),
+    (F32, False, 4, 4096, 7168, True), (F32, False, 4, 8192, 8192, True), (F32, False, 16, 1024, 11008, True),
+    (F32, False, 17, 1024, 11008, False), (F32, False, 4, 640, 32768, True), (F32, False, 4, 640, 32772, False),
+    (F32, True, 32, 512, 2048, True), (F32, True, 16, 1024, 11008, True), (F32, True, 17, 1024, 11008, False),
+    (F32, True, 17, 768, 16384, True), (F32, True, 17, 768, 16388, False), (F32, True, 4, 640, 32772, False),
+    (F32, True, 4, 2048, 8192, True), (F32, True, 17, 2048, 8192, False), (F32, True, 32, 2048, 4096, True),
+    (BF16, False, 16, 2048, 1024, True), (BF16, False, 16, 1792, 1024, False), (BF16, False, 16, 1536, 5120, True),
+    (BF16, False, 17, 1536, 5120, False), (BF16, False, 17, 2048, 2048, True), (BF16, False, 4, 4096, 16384, False),
+    (BF16, False, 4, 4096, 14336, True), (BF16, False, 4, 8192, 16384, True), (BF16, False, 4, 1088, 16384, True),
+    (BF16, False, 4, 2048, 32768, True), (BF16, False, 4, 2048, 32776, False), (BF16, True, 32, 256, 256, True),
+    (BF16, True, 4, 2048, 32776, True)])
+def test_what_the_library_does_as_fast(gpu, dtype, with_bias, m, k, n, taken):
+    """The lines of the rule by size, from both sides (a GPU of 256 CUs)."""
+    x, w = torch.zeros(m, k, dtype=dtype, device=gpu), torch.zeros(k, n, dtype=dtype, device=gpu)
+    bias = torch.zeros(n, dtype=dtype, device=gpu) if with_bias else None
+    y = _lib.host().linear_rows(x, w, bias, *_lib.here(x))
+    assert (y is not None) == taken and (not taken or not y.any())
