@@ -536,18 +536,17 @@ int launch_hd(PrefillKP kp, const PrefillArgs &a, hipStream_t stream) {
   const int64_t wgs = slices * kXcds * kp.group * kp.n_qtiles;
   if (wgs > 0x7fffffff) return IC_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs);
-  switch (a.hd) {
-    case 32:
+  if (a.hd == 128) {
+    hipLaunchKernelGGL((paged_prefill_kernel<M, 128, SINGLE, MASK>), grid, dim3(kPrefillThreads), 0, stream, kp);
+  } else if constexpr (MASK) {  // (without a byte mask head dims 32 and 64 are the short kernel's, whatever the size)
+    if (a.hd == 32)
       hipLaunchKernelGGL((paged_prefill_kernel<M, 32, SINGLE, MASK>), grid, dim3(kPrefillThreads), 0, stream, kp);
-      break;
-    case 64:
+    else if (a.hd == 64)
       hipLaunchKernelGGL((paged_prefill_kernel<M, 64, SINGLE, MASK>), grid, dim3(kPrefillThreads), 0, stream, kp);
-      break;
-    case 128:
-      hipLaunchKernelGGL((paged_prefill_kernel<M, 128, SINGLE, MASK>), grid, dim3(kPrefillThreads), 0, stream, kp);
-      break;
-    default:
+    else
       return IC_ERR_UNSUPPORTED;
+  } else {
+    return IC_ERR_UNSUPPORTED;
   }
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
