@@ -18,6 +18,17 @@ def _operands(gpu, dtype, m, k, n, seed):
     return tuple(t.to(dtype).to(gpu) for t in (x, w, bias))
 
 
+def _product(x, w, bias, splits=0):
+    """The library's entry point itself: none of the binding's rules about what is worth it."""
+    lib, dev, (m, k), n = _lib.load(), x.device, x.shape, w.shape[1]
+    need = lib.ic_linear_rows_workspace_bytes(m, n, k, splits, _lib.IC_DTYPE[x.dtype])
+    ws, out = torch.empty(max(need, 1), dtype=torch.uint8, device=dev), torch.empty(m, n, dtype=x.dtype, device=dev)
+    assert lib.ic_linear_rows(out.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), w.stride(0),
+                              bias.data_ptr() if bias is not None else None, m, n, k, splits, ws.data_ptr(), need,
+                              _lib.IC_DTYPE[x.dtype], _lib.current_stream_ptr(dev)) == 0
+    return out
+
+
 def _distance(got, want):
     return ((got.double().cpu() - want).norm() / want.norm()).item()
 
@@ -28,8 +39,9 @@ def _distance(got, want):
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_against_float64(gpu, dtype, m, k, n, with_bias):
     x, w, bias = _operands(gpu, dtype, m, k, n, m + n)
-    bias = bias if with_bias else torch.zeros_like(bias)
-    got = _lib.host().linear_rows(x, w, bias, *_lib.here(x))
+    def call(w):
+        return _lib.host().linear_rows(x, w, bias, *_lib.here(x)) if with_bias else _product(x, w, None)
+    got = call(w)
     want = x.double().cpu() @ w.double().cpu()
     if with_bias:
         want = want + bias.double().cpu()
@@ -37,7 +49,23 @@ def test_against_float64(gpu, dtype, m, k, n, with_bias):
     assert _distance(got, want) <= TOL[dtype]
     wide = torch.zeros(k, n + 8, dtype=dtype, device=gpu)
     wide[:, :n] = w                                     # rows further apart than long: the same sums
-    assert torch.equal(_lib.host().linear_rows(x, wide[:, :n], bias, *_lib.here(x)), got)
+    assert torch.equal(call(wide[:, :n]), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("splits", [1, 2, 4])
+@pytest.mark.parametrize("m", [1, 16, 17, 32])
+def test_without_a_bias(gpu, dtype, splits, m):
+    """Stored by the products' kernel (one split) and by the sums' (several), one and two blocks of 16 rows."""
+    x, w, _ = _operands(gpu, dtype, m, 2080, 200, m + splits)
+    want = x.double().cpu() @ w.double().cpu()
+    assert _distance(_product(x, w, None, splits), want) <= TOL[dtype]
+
+
+def test_without_a_bias_through_the_binding(gpu):
+    x, w, _ = _operands(gpu, torch.bfloat16, 16, 2048, 256, 3)
+    got = _lib.host().linear_rows(x, w, None, *_lib.here(x))
+    assert torch.equal(got, _product(x, w, None)) and torch.equal(generation.linear(x, w), got)
 
 
 @pytest.mark.parametrize("splits", [1, 2, 3, 5])
