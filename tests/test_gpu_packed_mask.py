@@ -95,3 +95,30 @@ def test_layer(gpu, dtype, precision, b, sq, sk, hn, gn, hd, kind):
                                   mask=m.to(torch.uint8).to(gpu)).view(b, sq, -1)
     bar = {torch.bfloat16: 8e-3, torch.float16: 1e-3, torch.float32: 1e-5}[dtype]   # two roundings of the same sums
     assert ((out - old).abs() <= bar * old.abs().clamp(min=1)).all()
+
+
+def test_a_mask_given_up_while_another_stream_reads_it(gpu):
+    """A mask packed on one stream and used on a second one, then dropped: its packed form is not handed out
+    again on the first stream before the second has read it."""
+    from ironcore_amd.layers import attention
+    n, h, hd = 200, 4, 64
+    attn = Attention(ic_config.MainConfig(
+        model=ic_config.ModelConfig(d_model=h * hd, num_attention_heads=h, num_attention_groups=h, head_dim=hd,
+                                    dropout_attn=0.0, precision="bf16"),
+        trainer=ic_config.TrainerConfig(use_flash_attn=False))).eval()
+    q = torch.randn(1, n, h, hd, device=gpu).bfloat16()
+    mask = _mask(1, 1, n, n, "random", 1).to(gpu)
+    want = attn(q, q, q, mask)
+    torch.cuda.synchronize()
+    packed = attention._MASK_CLASSES[id(mask)][3]
+    pieces = [(t.data_ptr(), t.shape, t.dtype) for t in (packed.bits, packed.lists)]
+    del packed
+    second = torch.cuda.Stream()
+    with torch.cuda.stream(second):
+        torch.cuda._sleep(50_000_000)
+        got = attn(q, q, q, mask)
+    del mask                                            # the packed form goes with it
+    again = [torch.zeros(shape, dtype=dtype, device=gpu) for _, shape, dtype in pieces]
+    assert not {t.data_ptr() for t in again} & {at for at, _, _ in pieces}
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
