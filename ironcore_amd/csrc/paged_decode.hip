@@ -306,9 +306,10 @@ __global__ __launch_bounds__(NW *kWave) void paged_decode_kernel(const DecodeKP 
 
 // Small batches of short contexts (a few sequences of a small model, a few hundred tokens): with shares of a tile
 // the split above turns them into partials that a second launch merges, 8 + 5 us of which the tiles themselves take
-// two (4 sequences of up to 160 tokens, 12 heads of 64, fp32: 13.0 us, here 3.8).  Here a workgroup owns a whole pair: its eight waves take the pair's tiles in turn (a wave's table entries come
-// in one load, one per lane: at most 64 tiles), keep the running softmax of the kernel above and merge through LDS; one launch, no
-// workspace.  All types; the arithmetic is the vector-ALU kernel's (fp32 probabilities and sums).
+// two (4 sequences of up to 160 tokens, 12 heads of 64, fp32: 13.0 us, here 3.8).  Here a workgroup owns a whole pair:
+// its eight waves take the pair's tiles in turn (a wave's table entries come in one load, one per lane: at most 64
+// tiles), keep the running softmax of the kernel above and merge through LDS; one launch, no workspace.  All types;
+// the arithmetic is the vector-ALU kernel's (fp32 probabilities and sums).
 // Bound by the chain of round trips: context length and table, tile, merge.
 constexpr int kPairWaves = 8;
 
@@ -730,9 +731,11 @@ void launch_valu_main(DecodeKP &kp, hipStream_t stream) {
 //   bf16, 32 / 8 of 128, 4                    10.2 / 6.4   13.0 / 8.4   15.2 / 10.1  19.7 / 14.3  18.2 / 21.3
 //   bf16, 32 / 8 of 128, 40                   12.2 / 11.8  16.0 / 15.2  19.9 / 20.9
 //   bf16, 28 / 4 of 128, 4                    10.1 / 10.4  13.2 / 14.1  15.2 / 17.1
-// One head per pair wins throughout; the lines keep a batch with a single long row among short ones, which the split
-// balances (8-10 us at least) and a workgroup walks alone, from losing.  Grouped heads cost this kernel vector work
-// for each head, hence short contexts only, and none from five heads on.
+// One head per pair wins throughout, the 640 pairs of 40 sequences included; the rounds are limited so that a batch
+// with a single long row among short ones, which the split balances (8-10 us at least) and a workgroup walks alone,
+// does not lose.  The limit on the pairs (512 on 256 CUs) does not follow from these figures: beyond it only the even
+// batch of 640 pairs has been measured, and no row says where the split becomes faster.  Grouped heads cost this
+// kernel vector work for each head, hence short contexts only, and none from five heads on.
 bool decode_takes_pairs(const DecodeKP &kp, int row_bytes) {
   if (kp.cohort_size != 1 || kp.key_mask != nullptr || kp.min_chunk > 1 || kp.max_ctx <= 0 || kp.group > 4) return false;
   const int64_t rounds = ((int64_t)kp.max_ctx + 16 * kPairWaves - 1) / (16 * kPairWaves);

@@ -49,10 +49,11 @@ except ImportError:
     flash_attn_varlen_func = None
 
 
-# attention_mask tensor -> what _classify_mask found for it: id -> (weak reference, (version, shapes), kind, bytes).
+# attention_mask tensor -> what _classify_mask found for it: id -> (weak reference, (version, shapes), kind, data).
 # An entry goes when its mask tensor dies (the weak reference's callback) and when more than
-# _MASK_CLASSES_MAX masks are alive at once (oldest first): the byte copy of a general mask is as
-# large as the mask, and a model that builds a new document mask per batch must not pile them up.
+# _MASK_CLASSES_MAX masks are alive at once (oldest first): the packed form of a general mask is an
+# eighth of its bytes (rows rounded up to 128), and a model that builds a new document mask per batch
+# must not pile them up.
 _MASK_CLASSES: dict = {}
 _MASK_CLASSES_MAX = 4
 
