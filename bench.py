@@ -226,7 +226,7 @@ def event_pass(torch, step, first, n):
 def after_idle(torch, step, idle_s, warmup, steps):
     """What the first launches after an idle GPU cost.  The wall-timed steps
     follow the parity gate, during which the CPU oracle runs for seconds and
-    the GPU does nothing; with the driver's counts (5 + 20 steps) they are the
+    the GPU does nothing; with 5 + 20 steps they are the
     first few milliseconds of work after that gap.  This pass repeats the
     situation (GPU idle for `idle_s`, then `n` steps, every call bracketed by
     events) so that the line can say how much of a step's wall time beyond its
