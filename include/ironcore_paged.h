@@ -488,6 +488,68 @@ int ic_linear_rows(void *out, int64_t out_stride, const void *x, int64_t x_strid
                    int m, int n, int k, int splits,
                    void *workspace, size_t workspace_bytes, int dtype, void *stream);
 
+/*
+ * A linear of a decode step with what stands around it in a transformer layer
+ * (ironcore/models/transformer.py:77-135), for at most IC_LINEAR_ROWS_MAX rows, in
+ * one of three forms:
+ *
+ *   out = act(x W + bias)
+ *   [q | k | v] = x W + bias, stored as an append   (slot_mapping not NULL)
+ *   out = x W + bias + residual, norm_out = norm(out)   (residual or norm given)
+ *
+ * One element type throughout, fp32 sums, rounded to the element type only on
+ * the way to out and norm_out (the norm takes out as rounded).  Rows of x, residual,
+ * out, norm_out, w, w2, norm_weight and norm_bias 16-byte aligned, strides in elements;
+ * k a multiple of 64 bytes of elements, n, n2 and half of a gated n of 16 bytes.
+ *
+ *   w2     a second matrix [k, n2] whose columns follow the first one's, or NULL
+ *          (third form: NULL).
+ *   act    IC_ACT_*, first form; the gated ones take the columns [feature | gate] and
+ *          give n / 2: GLU feature * sigmoid(gate), SWIGLU silu(feature) * gate.
+ *   slot_mapping  second form: the columns are hn heads of queries, gn of keys and gn
+ *          of values (w and w2 together); queries go to out, keys and values into
+ *          the pools as ic_kv_append stores them.  With cos_table and sin_table
+ *          queries and keys are rotated on the way as by ic_rope_kv_append, row i at
+ *          positions[i].
+ *   norm   third form: IC_NORM_* over the n values of a row, weight [n], bias [n] or
+ *          NULL; out may be NULL then.  With w NULL the product and the bias are left out.
+ *          n up to IC_STEP_LINEAR_ROW_MAX.
+ *   tile_bytes  64, 128 or 256: bytes of a row of W that a workgroup takes; splits:
+ *          workgroups that share a column's k range; 0 lets the library choose.
+ *   workspace  ic_step_linear_workspace_bytes(call) bytes, 16-byte aligned.
+ */
+enum { IC_NORM_NONE = 0, IC_NORM_LAYER = 1, IC_NORM_RMS = 2 };
+enum { IC_ACT_NONE = 0, IC_ACT_RELU = 1, IC_ACT_GELU = 2, IC_ACT_SILU = 3, IC_ACT_GLU = 4, IC_ACT_SWIGLU = 5 };
+#define IC_STEP_LINEAR_ROW_MAX 16384
+typedef struct ic_step_linear_call {
+  void *out, *norm_out;
+  int64_t out_stride, norm_out_stride;
+  const void *x;
+  int64_t x_stride;
+  const void *w, *bias;
+  int64_t w_stride;
+  const void *w2, *bias2;
+  int64_t w2_stride;
+  const void *residual;
+  int64_t residual_stride;
+  const void *norm_weight, *norm_bias;
+  int m, k, n, n2;
+  int norm, act;
+  float eps;
+  int dtype, tile_bytes, splits;
+  void *k_pool, *v_pool;
+  int64_t pool_stride_block, pool_stride_head, pool_stride_token, num_blocks;
+  int hn, gn, hd, block_size;
+  const int64_t *slot_mapping;
+  const int32_t *positions;
+  const float *cos_table, *sin_table;
+  int64_t table_rows;
+  void *workspace;
+  size_t workspace_bytes;
+} ic_step_linear_call;
+size_t ic_step_linear_workspace_bytes(const ic_step_linear_call *call);
+int ic_step_linear(const ic_step_linear_call *call, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -19,6 +19,7 @@
 #include <ATen/autocast_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 
+#include <algorithm>
 #include <climits>
 
 #include "../../include/ironcore_paged.h"
@@ -441,6 +442,145 @@ OptTensor linear_rows(const Tensor &x, const Tensor &w, const OptTensor &bias, i
   return out;
 }
 
+// ---- a transformer layer's decode step -------------------------------------------------------
+
+// A parameter or activation of a step: plain values of one type on the device, rows of 16-byte pieces.
+bool step_tensor(const Tensor &t, at::ScalarType type, int64_t device) {
+  return on(t, device) && t.scalar_type() == type && plain(t) && !(at::GradMode::is_enabled() && t.requires_grad());
+}
+bool step_vector(const OptTensor &t, int64_t n, at::ScalarType type, int64_t device) {
+  return !t.has_value() || (step_tensor(*t, type, device) && t->dim() == 1 && t->numel() == n && t->is_contiguous() &&
+                            reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0);
+}
+bool step_matrix(const OptTensor &t, int64_t k, int64_t n, at::ScalarType type, int64_t device) {
+  return t.has_value() && step_tensor(*t, type, device) && t->dim() == 2 && t->size(0) == k && t->size(1) == n &&
+         t->stride(1) == 1 && n * t->element_size() % 16 == 0 && k * t->element_size() % 64 == 0 &&
+         rows16(t->data_ptr(), t->stride(0), n, t->element_size());
+}
+const void *data(const OptTensor &t) { return t.has_value() ? t->data_ptr() : nullptr; }
+
+// Whether a step may go past the dispatcher at all.
+bool step_outside_torch() { return c10::impl::dispatch_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA); }
+
+// The norm of up to 32 rows [b, 1, n].
+OptTensor norm_rows(const Tensor &x, const Tensor &weight, const OptTensor &bias, int64_t norm, double eps,
+                    int64_t device, int64_t stream) {
+  const at::ScalarType type = x.scalar_type();
+  const int dtype = dtype_code(type);
+  const int64_t n = x.size(-1), m = n > 0 ? x.numel() / n : 0;
+  if (dtype < 0 || m < 1 || m > IC_LINEAR_ROWS_MAX || n > IC_STEP_LINEAR_ROW_MAX || !step_tensor(x, type, device) ||
+      !x.is_contiguous() || !rows16(x.data_ptr(), n, n, x.element_size()) || !step_vector(weight, n, type, device) ||
+      !step_vector(bias, n, type, device) || step_outside_torch())
+    return c10::nullopt;
+  const Tensor out = at::empty(x.sizes(), x.options());
+  ic_step_linear_call c = {};
+  c.norm_out = out.data_ptr(), c.norm_out_stride = n;
+  c.residual = x.data_ptr(), c.residual_stride = n;
+  c.norm_weight = weight.data_ptr(), c.norm_bias = data(bias);
+  c.m = (int)m, c.n = (int)n, c.norm = (int)norm, c.eps = (float)eps, c.dtype = dtype;
+  if (!made("ic_step_linear", ic_step_linear(&c, (void *)stream))) return c10::nullopt;
+  return out;
+}
+
+// One layer of a decode step: hidden [b, 1, d] and its input norm in, the layer's output and the norm that follows it
+// (the next layer's, or the model's last) out.  `w`: q, kv, attention output, post-attention norm, up, down, next norm, a
+// weight and a bias each.  Seven launches and more: projections with the append, attention (one or two), output projection
+// with residual and norm (two), up-projection with the activation, down-projection with residual and norm (two).
+c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
+    const Tensor &hidden, const Tensor &normed, const std::vector<OptTensor> &w, int64_t hn, int64_t gn, int64_t hd,
+    int64_t act, int64_t norm, double eps, int64_t next_norm, double next_eps, bool post_ln, const Tensor &k_pool, const Tensor &v_pool,
+    const Tensor &tables, const Tensor &lens, const Tensor &slots, int64_t max_ctx, double scale, int64_t cohort,
+    const OptTensor &shared, const OptTensor &positions, const OptTensor &cos, const OptTensor &sin, int64_t device,
+    int64_t stream) {
+  const Pool p(k_pool, v_pool, device);
+  const at::ScalarType type = hidden.scalar_type();
+  if (w.size() != 14 || !p.ok || p.gn != gn || p.hd != hd || hidden.dim() != 3 || hidden.size(1) != 1 || k_pool.scalar_type() != type ||
+      normed.sizes() != hidden.sizes() || !step_tensor(hidden, type, device) || !step_tensor(normed, type, device) ||
+      !hidden.is_contiguous() || !normed.is_contiguous() || step_outside_torch())
+    return c10::nullopt;
+  const int64_t b = hidden.size(0), d = hidden.size(2), q_cols = hn * p.hd, kv_cols = p.gn * p.hd;
+  if (b < 1 || b > IC_LINEAR_ROWS_MAX || d > IC_STEP_LINEAR_ROW_MAX || !w[8].has_value() || w[8]->dim() != 2)
+    return c10::nullopt;
+  const int64_t up_cols = w[8]->size(1), f = act >= IC_ACT_GLU ? up_cols / 2 : up_cols;
+  const int es = (int)hidden.element_size();
+  if (!rows16(hidden.data_ptr(), d, d, es) || !rows16(normed.data_ptr(), d, d, es) ||
+      !step_matrix(w[0], d, q_cols, type, device) || !step_vector(w[1], q_cols, type, device) ||
+      !step_matrix(w[2], d, 2 * kv_cols, type, device) || !step_vector(w[3], 2 * kv_cols, type, device) ||
+      !step_matrix(w[4], q_cols, d, type, device) || !step_vector(w[5], d, type, device) || !w[6].has_value() ||
+      !step_vector(w[6], d, type, device) || !step_vector(w[7], d, type, device) ||
+      !step_matrix(w[8], d, up_cols, type, device) || !step_vector(w[9], up_cols, type, device) ||
+      up_cols > (1 << 30) || (act >= IC_ACT_GLU && (up_cols * es) % 32 != 0) || !step_matrix(w[10], f, d, type, device) ||
+      !step_vector(w[11], d, type, device) || !w[12].has_value() || !step_vector(w[12], d, type, device) ||
+      !step_vector(w[13], d, type, device) || !index_vector(slots, at::kLong, b, device))
+    return c10::nullopt;
+  const Decode dec{tables, lens, max_ctx, 0, cohort, shared, scale};
+  const Rope rope(positions, cos, sin, b, p.hd, device);
+  if (!rope.ok || !decode_fits(p, b, hn, dec, device) ||
+      !rows16(p.k, p.sb, 1, es) || !rows16(p.v, p.sb, 1, es) || (p.sh * es) % 16 != 0 || (p.st * es) % 16 != 0)
+    return c10::nullopt;
+
+  ic_step_linear_call qkv = {}, proj = {}, up = {}, down = {};
+  qkv.m = proj.m = up.m = down.m = (int)b;
+  qkv.dtype = proj.dtype = up.dtype = down.dtype = p.dtype;
+  qkv.x = normed.data_ptr(), qkv.x_stride = d, qkv.k = (int)d;
+  qkv.w = data(w[0]), qkv.bias = data(w[1]), qkv.w_stride = w[0]->stride(0), qkv.n = (int)q_cols;
+  qkv.w2 = data(w[2]), qkv.bias2 = data(w[3]), qkv.w2_stride = w[2]->stride(0), qkv.n2 = (int)(2 * kv_cols);
+  qkv.out_stride = q_cols;
+  qkv.k_pool = const_cast<void *>(p.k), qkv.v_pool = const_cast<void *>(p.v);
+  qkv.pool_stride_block = p.sb, qkv.pool_stride_head = p.sh, qkv.pool_stride_token = p.st, qkv.num_blocks = p.nb;
+  qkv.hn = (int)hn, qkv.gn = (int)p.gn, qkv.hd = (int)p.hd, qkv.block_size = (int)p.bs;
+  qkv.slot_mapping = slots.data_ptr<int64_t>();
+  qkv.positions = rope.positions, qkv.cos_table = rope.cos, qkv.sin_table = rope.sin, qkv.table_rows = rope.rows;
+  proj.x_stride = q_cols, proj.k = (int)q_cols;
+  proj.w = data(w[4]), proj.bias = data(w[5]), proj.w_stride = w[4]->stride(0), proj.n = (int)d;
+  proj.residual = post_ln ? normed.data_ptr() : hidden.data_ptr(), proj.residual_stride = d;
+  proj.norm = (int)norm, proj.eps = (float)eps, proj.norm_weight = data(w[6]), proj.norm_bias = data(w[7]);
+  proj.out_stride = proj.norm_out_stride = d;
+  up.x_stride = d, up.k = (int)d;
+  up.w = data(w[8]), up.bias = data(w[9]), up.w_stride = w[8]->stride(0), up.n = (int)up_cols;
+  up.act = (int)act, up.out_stride = f;
+  down.x_stride = f, down.k = (int)f;
+  down.w = data(w[10]), down.bias = data(w[11]), down.w_stride = w[10]->stride(0), down.n = (int)d;
+  down.norm = (int)next_norm, down.eps = (float)next_eps, down.norm_weight = data(w[12]), down.norm_bias = data(w[13]);
+  down.residual_stride = down.out_stride = down.norm_out_stride = d;
+
+  // one allocation for what the layer's launches hand to each other
+  const Tensor out = at::empty({b, 1, d}, hidden.options()), out_normed = at::empty({b, 1, d}, hidden.options());
+  down.residual = out.data_ptr();  // (any address: what the workspace depends on)
+  size_t work = 0;
+  for (const ic_step_linear_call *c : {&qkv, &proj, &up, &down}) work = std::max(work, ic_step_linear_workspace_bytes(c));
+  const size_t decode_work =
+      ic_paged_decode_shared_workspace_bytes((int)b, (int)hn, (int)p.gn, (int)p.hd, (int)cohort);
+  size_t total = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = total;
+    total += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t at_q = take(b * q_cols * es), at_att = take(b * q_cols * es), at_mid = take(b * d * es),
+               at_mid_normed = take(b * d * es), at_act = take(b * f * es), at_work = take(std::max(work, decode_work));
+  const Tensor scratch = at::empty({(int64_t)total}, hidden.options().dtype(at::kByte));
+  char *base = static_cast<char *>(scratch.data_ptr());
+  qkv.out = base + at_q;
+  proj.x = base + at_att, proj.out = base + at_mid, proj.norm_out = base + at_mid_normed;
+  up.x = base + at_mid_normed, up.out = base + at_act;
+  down.x = base + at_act, down.residual = post_ln ? proj.norm_out : proj.out;
+  down.out = out.data_ptr(), down.norm_out = out_normed.data_ptr();
+  for (ic_step_linear_call *c : {&qkv, &proj, &up, &down}) c->workspace = base + at_work, c->workspace_bytes = work;
+
+  auto linear = [&](const ic_step_linear_call &c) { return made("ic_step_linear", ic_step_linear(&c, (void *)stream)); };
+  if (!linear(qkv) ||
+      !made("ic_paged_decode_shared",
+            ic_paged_decode_shared(base + at_att, q_cols, qkv.out, q_cols, p.k, p.v, p.sb, p.sh, p.st,
+                                   tables.data_ptr<int32_t>(), tables.stride(0), lens.data_ptr<int32_t>(), (int)b,
+                                   (int)hn, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, (int)max_ctx, (float)scale, 0,
+                                   (int)cohort, cohort > 1 ? shared->data_ptr<int32_t>() : nullptr, base + at_work,
+                                   decode_work, p.dtype, (void *)stream)) ||
+      !linear(proj) || !linear(up) || !linear(down))
+    return c10::nullopt;
+  return std::make_tuple(out, out_normed);
+}
+
 }  // namespace
 
 // (wrapped, so that torch's exceptions keep their Python types: an allocation that does not fit raises
@@ -453,5 +593,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("prefill_step", torch::wrap_pybind_function_no_gil(prefill_step));
   m.def("dense", torch::wrap_pybind_function_no_gil(dense));
   m.def("linear_rows", torch::wrap_pybind_function_no_gil(linear_rows));
+  m.def("norm_rows", torch::wrap_pybind_function_no_gil(norm_rows));
+  m.def("decoder_layer", torch::wrap_pybind_function_no_gil(decoder_layer));
   m.def("pack_mask", torch::wrap_pybind_function_no_gil(pack_mask));
 }

@@ -495,6 +495,67 @@ int ic_linear_rows(void *out, int64_t out_stride, const void *x, int64_t x_strid
   return ic::launch_linear_rows(a, static_cast<hipStream_t>(stream));
 }
 
+// Sizes and modes of a step linear, without its pointers (what the workspace depends on).
+static int step_linear_sizes(const ic_step_linear_call &a) {
+  if (a.m < 0 || a.n < 0 || a.n2 < 0 || a.k < 0 || a.splits < 0) return IC_ERR_BAD_SHAPE;
+  if (!dtype_ok(a.dtype) || a.norm < IC_NORM_NONE || a.norm > IC_NORM_RMS || a.act < IC_ACT_NONE ||
+      a.act > IC_ACT_SWIGLU || (a.tile_bytes != 0 && a.tile_bytes != 64 && a.tile_bytes != 128 && a.tile_bytes != 256))
+    return IC_ERR_UNSUPPORTED;
+  const int block = 16 / ic::elem_size(a.dtype);
+  const bool gated = a.act >= IC_ACT_GLU, append = a.slot_mapping != nullptr;
+  const bool rows = a.residual != nullptr || a.norm != IC_NORM_NONE;
+  if (a.m > IC_LINEAR_ROWS_MAX || (int64_t)a.n + a.n2 > (1 << 30) || a.n % (gated ? 2 * block : block) != 0 ||
+      a.n2 % block != 0 || a.k % (4 * block) != 0 || (a.n == 0 && a.n2 > 0) ||
+      (append && (rows || a.act != IC_ACT_NONE)) || ((gated || rows) && a.n2 != 0) ||
+      (rows && (a.act != IC_ACT_NONE || a.n > IC_STEP_LINEAR_ROW_MAX)))
+    return IC_ERR_UNSUPPORTED;
+  if (a.w == nullptr ? !rows : a.k == 0) return a.w == nullptr ? IC_ERR_NULL_POINTER : IC_ERR_BAD_SHAPE;
+  return IC_OK;
+}
+
+size_t ic_step_linear_workspace_bytes(const ic_step_linear_call *call) {
+  if (call == nullptr || call->m == 0 || call->n == 0 || step_linear_sizes(*call) != IC_OK) return 0;
+  const ic::StepPlan plan = ic::step_linear_plan(*call);
+  return plan.partial ? (size_t)plan.splits * call->m * ((size_t)call->n + call->n2) * sizeof(float) : 0;
+}
+
+int ic_step_linear(const ic_step_linear_call *call, void *stream) {
+  if (call == nullptr) return IC_ERR_NULL_POINTER;
+  const ic_step_linear_call &a = *call;
+  if (const int rc = step_linear_sizes(a); rc != IC_OK) return rc;
+  if (a.m == 0 || a.n == 0) return IC_OK;
+  const int es = ic::elem_size(a.dtype);
+  const bool append = a.slot_mapping != nullptr;
+  const int64_t columns = a.act >= IC_ACT_GLU ? a.n / 2 : append ? (int64_t)a.hn * a.hd : (int64_t)a.n + a.n2;
+  if ((a.out && a.out_stride < columns) || (a.w && (a.x_stride < a.k || a.w_stride < a.n)) ||
+      (a.n2 > 0 && a.w2_stride < a.n2) || (a.residual && a.residual_stride < columns) ||
+      (a.norm != IC_NORM_NONE && a.norm_out_stride < columns))
+    return IC_ERR_BAD_SHAPE;
+  if ((a.w && !a.x) || (a.n2 > 0 && !a.w2) || (!a.out && a.norm == IC_NORM_NONE) ||
+      (a.norm != IC_NORM_NONE && (!a.norm_weight || !a.norm_out)))
+    return IC_ERR_NULL_POINTER;
+  auto whole = [&](const void *ptr, int64_t stride) { return ptr == nullptr || (aligned16(ptr) && stride16(stride, es)); };
+  if (!whole(a.out, a.out_stride) || !whole(a.norm_out, a.norm_out_stride) || !whole(a.x, a.x_stride) ||
+      !whole(a.w, a.w_stride) || !whole(a.w2, a.w2_stride) || !whole(a.residual, a.residual_stride) ||
+      !whole(a.norm_weight, 0) || !whole(a.norm_bias, 0))
+    return IC_ERR_ALIGNMENT;
+  if (append) {
+    if (a.hn <= 0 || a.gn <= 0 || a.hd <= 0 || a.hd % 2 != 0 || a.block_size <= 0 || a.num_blocks <= 0 ||
+        ((int64_t)a.hn + 2 * a.gn) * a.hd != (int64_t)a.n + a.n2 || a.pool_stride_block <= 0 ||
+        a.pool_stride_head <= 0 || a.pool_stride_token <= 0)
+      return IC_ERR_BAD_SHAPE;
+    if (!a.k_pool || !a.v_pool || (a.cos_table != nullptr) != (a.sin_table != nullptr) ||
+        (a.cos_table && (!a.positions || a.table_rows <= 0)))
+      return IC_ERR_NULL_POINTER;
+    if (!aligned16(a.k_pool) || !aligned16(a.v_pool) || !stride16(a.pool_stride_block, es) ||
+        !stride16(a.pool_stride_head, es) || !stride16(a.pool_stride_token, es))
+      return IC_ERR_ALIGNMENT;
+  }
+  const size_t need = ic_step_linear_workspace_bytes(call);
+  if (need > 0 && (!a.workspace || !aligned16(a.workspace) || a.workspace_bytes < need)) return IC_ERR_WORKSPACE;
+  return ic::launch_step_linear(a, static_cast<hipStream_t>(stream));
+}
+
 int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,
                  int heads, int rows, int keys, uint64_t *bits, int32_t *lists, int32_t *flags, void *stream) {
   if (n_seqs < 0 || heads < 0 || rows < 0 || keys < 0 || stride_seq < 0 || stride_head < 0 || stride_row < 0)

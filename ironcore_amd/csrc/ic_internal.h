@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "../../include/ironcore_paged.h"
+
 namespace ic {
 
 struct PoolLayout {
@@ -147,6 +149,14 @@ int launch_zero_unlisted_rows(char *out, int64_t stride_bytes, int row_bytes, co
                               const int32_t *bounds, int n_seqs, int row_pitch, hipStream_t stream);
 int launch_linear_rows(const LinearArgs &a, hipStream_t stream);
 int linear_rows_splits(int n, int k, int dtype, int want);
+int launch_step_linear(const ic_step_linear_call &a, hipStream_t stream);
+// How a step linear is laid out: bytes of a row of W to a workgroup, workgroups that share a column's k range,
+// whether sums go through the workspace, whether a workgroup then takes a whole row.
+struct StepPlan {
+  int tile_bytes, splits, per_split, tiles, tiles0;
+  bool partial, rows;
+};
+StepPlan step_linear_plan(const ic_step_linear_call &a);
 int launch_paged_decode(const DecodeArgs &a, hipStream_t stream);
 int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream);
 int launch_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,

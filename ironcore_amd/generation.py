@@ -9,8 +9,8 @@ growing sequence every step (examples/generate_text.py:12-46).  The classes
 below keep that arithmetic and those parameter names, add the two optional
 arguments that carry the KV cache down to ``Attention.forward``, and replace
 the full recompute by prefill + cached decode.  Attention, the KV append and the
-linears of a decode step (up to 32 rows) are the HIP kernels; the other GEMMs,
-the norms and the activation are plain torch calls on the GPU (plumbing around
+layers of a decode step (up to 32 rows) are HIP kernels; the other GEMMs,
+norms and activations are plain torch calls on the GPU (plumbing around
 the hot path).
 
 Built: pre/post-LN with LayerNorm or RMSNorm, learned absolute positions or
@@ -228,6 +228,90 @@ class TransformerModel(BaseModule):
         return hidden_states
 
 
+# ---- a decode step past the modules --------------------------------------------------------------
+# The layers of a decode step (one new token a sequence) can run as a handful of native launches each, norms,
+# biases, activations, residuals and the cache append on the launches of the products (csrc/step_linear.hip).  The
+# modules are then not called, so that path is taken only where nobody could tell: every module of the known
+# type, without hooks, its forward its own.
+
+def _own(*classes):
+    return {cls: cls.forward for cls in classes}
+
+
+_OWN_FORWARD = _own(Linear, LayerNorm, RmsNorm, nn.LayerNorm, nn.RMSNorm, nn.ReLU, nn.GELU, nn.SiLU, GLUActivation, MLP,
+                    Attention, TransformerLayer, TransformerModel)
+_OWN_FORWARD_ITEMS = tuple(_OWN_FORWARD.items())
+_OWN_PAGED = Attention._paged
+
+
+def _untouched(module, *kinds) -> bool:
+    """Whether calling the module would do what its class says and nothing else."""
+    return (type(module) in kinds and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks and "forward" not in module.__dict__)
+
+
+def _step_norm(norm, d):
+    """(kind, eps, weight, bias) for the native step, or None."""
+    if not _untouched(norm, LayerNorm, RmsNorm):
+        return None
+    inner = norm.layernorm
+    kind = 1 if _untouched(inner, nn.LayerNorm) else 2 if _untouched(inner, nn.RMSNorm) else 0
+    if not kind or inner.weight is None or inner.eps is None or tuple(inner.normalized_shape) != (d,):
+        return None
+    return kind, inner.eps, inner.weight, inner.bias if kind == 1 else None
+
+
+def _step_activation(act):
+    if _untouched(act, nn.ReLU):
+        return 1
+    if _untouched(act, nn.GELU):
+        return 2 if act.approximate == "none" else None
+    if _untouched(act, nn.SiLU):
+        return 3
+    if _untouched(act, GLUActivation):
+        return {"glu": 4, "swiglu": 5}.get(act.variant)
+    return None
+
+
+def _step_layer(layer, d):
+    """What the native step needs of a layer: (weights and biases, heads, groups, head dimension, activation, norm
+    kind and eps, post-LN, scale, input norm), or None."""
+    if not _untouched(layer, TransformerLayer):
+        return None
+    attention, mlp = layer.self_attention, layer.mlp
+    linears = (layer.linear_q, layer.linear_kv, layer.attn_output, mlp.up_proj, mlp.down_proj) if _untouched(mlp, MLP) else ()
+    norm, first = _step_norm(layer.post_attn_layernorm, d), _step_norm(layer.input_layernorm, d)
+    act = _step_activation(mlp.activation) if linears else None
+    hn, gn, hd = layer.num_local_attention_heads, layer.num_local_attention_groups, layer.head_dimension
+    if (act is None or norm is None or first is None or not _untouched(attention, Attention)
+            or "_paged" in attention.__dict__ or not all(_untouched(x, Linear) for x in linears)
+            or (attention.num_local_attention_heads, attention.num_local_attention_groups, attention.head_dimension) != (hn, gn, hd)
+            or (attention.training and attention.config.model.dropout_attn > 0.0)):
+        return None
+    q, kv, out, up, down = linears
+    return ([q.weight, q.bias, kv.weight, kv.bias, out.weight, out.bias, norm[2], norm[3], up.weight, up.bias,
+             down.weight, down.bias], hn, gn, hd, act, norm[0], norm[1], bool(layer.config.model.post_ln),
+            1.0 / attention.scale_factor, first)
+
+
+def _step_plan(model, d):
+    """The layers of ``model`` (a LanguageModel) for the native step and its last norm, or None where a module has
+    to be called."""
+    stack = model.model
+    if not (_untouched(stack, TransformerModel) and _untouched_by_anyone()
+            and all(cls.forward is forward for cls, forward in _OWN_FORWARD_ITEMS) and Attention._paged is _OWN_PAGED):
+        return None
+    layers = [_step_layer(layer, d) for layer in stack.layers]
+    last = _step_norm(model.output_layernorm, d)
+    return None if last is None or None in layers or not layers else (layers, last)
+
+
+def _untouched_by_anyone() -> bool:
+    module = torch.nn.modules.module
+    return not (module._global_forward_hooks or module._global_forward_pre_hooks or module._global_backward_hooks
+                or module._global_backward_pre_hooks)
+
+
 class LanguageModelEmbedding(BaseModule):
     """ironcore/layers/embedding.py:9-50 (word + learned absolute position)."""
 
@@ -313,11 +397,50 @@ class LanguageModel(BaseModule):
             attention_mask = None
             position_ids = (torch.tensor(past, device=dev).unsqueeze(1) + torch.arange(s, device=dev).unsqueeze(0))
         x = self.embedding(input_ids, position_ids)
-        x = self.model(x, attention_mask, self.rotary_pos_emb, kv_cache=kv_cache, attn_metadata=meta)
-        x = self.output_layernorm(x)
+        normed = self._native_step(x, kv_cache, meta) if s == 1 and meta is not None else None
+        if normed is not None:
+            x = normed
+        else:
+            x = self.model(x, attention_mask, self.rotary_pos_emb, kv_cache=kv_cache, attn_metadata=meta)
+            x = self.output_layernorm(x)
         if self.config.model.untie_embed:
             return linear(x, self.output_layer.weight)
         return torch.matmul(x, self.embedding.word_embeddings.weight.transpose(0, 1))
+
+
+    def _native_step(self, x, kv_cache, meta):
+        """The layers and the last norm of a decode step by native calls, one a layer, or None: ``x`` [b, 1, d] are
+        the embedded tokens.  Where a layer's call is not taken (sizes, types, strides), the layer runs as a module."""
+        here = _lib.here(x) if type(x) is torch.Tensor else None
+        if (here is None or getattr(meta, "chunk_rows", None) is not None or x.dim() != 3
+                or torch.overrides.has_torch_function_unary(x) or torch.compiler.is_compiling() or torch.jit.is_tracing()):
+            return None
+        plan = _step_plan(self, x.shape[-1])
+        if plan is None:
+            return None
+        layers, last = plan
+        host, rope = _lib.host(), self.rotary_pos_emb
+        kind, eps, weight, bias = layers[0][9]
+        normed = host.norm_rows(x, weight, bias, kind, eps, *here)
+        if normed is None:
+            return None
+        cohort = int(meta.cohort_size) if x.dtype != torch.float32 else 1
+        shared = meta.cohort_shared_blocks if cohort > 1 else None
+        angles = (None, None, None) if rope is None else (meta.positions, rope.cos_emb, rope.sin_emb)
+        longest = int(meta.max_context_len)
+        for index, (weights, hn, gn, hd, act, kind, eps, post_ln, scale, _) in enumerate(layers):
+            following = last if index + 1 == len(layers) else layers[index + 1][9]
+            pools = kv_cache.layer(index)
+            got = host.decoder_layer(x, normed, weights + [following[2], following[3]], hn, gn, hd, act, kind, eps,
+                                     following[0], following[1], post_ln, *pools, meta.block_tables, meta.context_lens,
+                                     meta.slot_mapping, longest, scale, cohort, shared, *angles, *here)
+            if got is None:
+                x = self.model.layers[index](x, None, rope, kv_cache=pools, attn_metadata=meta)
+                normed = (self.output_layernorm if index + 1 == len(layers)
+                          else self.model.layers[index + 1].input_layernorm)(x)
+            else:
+                x, normed = got
+        return normed
 
 
 def sample_next(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 0,
