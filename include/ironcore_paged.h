@@ -550,6 +550,56 @@ typedef struct ic_step_linear_call {
 size_t ic_step_linear_workspace_bytes(const ic_step_linear_call *call);
 int ic_step_linear(const ic_step_linear_call *call, void *stream);
 
+/*
+ * The next token of each row of logits, greedily (examples/generate_text.py:27-28 at
+ * temperature 0): the first of the largest values, NaN counting as the largest.
+ *
+ *   logits [rows, n] of dtype, rows 16-byte aligned, n a multiple of 16 bytes and >= 2.
+ *   tokens, margins  [rows, columns] or NULL: the token and best - second best (of
+ *          equal values the second is as large as the best) go to column *column
+ *          (NULL: 0); a column outside [0, columns) is not stored.
+ *   next   [rows] or NULL: the token once more.
+ *   finished  [rows] or NULL: a row with a nonzero byte gets eos, and a row whose
+ *          token is eos gets a nonzero byte.
+ *   workspace  ic_greedy_workspace_bytes(rows, n) bytes, 16-byte aligned.
+ */
+typedef struct ic_greedy_call {
+  const void *logits;
+  int64_t stride;
+  int rows, n, dtype;
+  int64_t *tokens;
+  int64_t token_stride;
+  float *margins;
+  int64_t margin_stride;
+  const int64_t *column;
+  int64_t columns;
+  int64_t *next;
+  uint8_t *finished;
+  int64_t eos;
+  void *workspace;
+  size_t workspace_bytes;
+} ic_greedy_call;
+size_t ic_greedy_workspace_bytes(int rows, int n);
+int ic_greedy(const ic_greedy_call *call, void *stream);
+
+/*
+ * The bookkeeping of a decode step on the device: row i's new token has position
+ * p = context_lens[i] (written to positions and token_positions), its pool slot is
+ * block_tables[i][p / block_size] * block_size + p % block_size (-1 beyond
+ * table_width), and context_lens[i] becomes p + 1.  *column (if given) grows by 1.
+ */
+typedef struct ic_advance_call {
+  int32_t *context_lens;
+  const int32_t *block_tables;
+  int64_t block_table_stride;
+  int rows, table_width, block_size;
+  int32_t *positions;
+  int64_t *token_positions;
+  int64_t *slot_mapping;
+  int64_t *column;
+} ic_advance_call;
+int ic_advance(const ic_advance_call *call, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

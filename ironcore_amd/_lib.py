@@ -98,6 +98,9 @@ SIGNATURES = {
         c_void_p, c_size_t, c_int, c_void_p]),  # workspace, workspace_bytes, dtype, stream
     "ic_step_linear_workspace_bytes": (c_size_t, [c_void_p]),   # call descriptor
     "ic_step_linear": (c_int, [c_void_p, c_void_p]),    # call descriptor, stream
+    "ic_greedy_workspace_bytes": (c_size_t, [c_int, c_int]),   # rows, n
+    "ic_greedy": (c_int, [c_void_p, c_void_p]),         # call descriptor, stream
+    "ic_advance": (c_int, [c_void_p, c_void_p]),        # call descriptor, stream
     "ic_mask_pack": (c_int, [
         c_void_p, c_int64, c_int64, c_int64,    # mask, strides: seq, head, row
         c_int, c_int, c_int, c_int,             # n_seqs, heads, rows, keys

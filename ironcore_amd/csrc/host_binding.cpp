@@ -581,6 +581,61 @@ c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
   return std::make_tuple(out, out_normed);
 }
 
+// ---- greedy decoding --------------------------------------------------------------------------
+
+// The next token of each row of logits [b, n] and, wanted, how far it is ahead: stored into column `*column` of `tokens`
+// [b, columns] and `margins`, and into `next` [b, 1].  `finished` comes with an eos token.
+bool greedy(const Tensor &logits, const OptTensor &column, const OptTensor &tokens, const OptTensor &margins,
+            const OptTensor &next, const OptTensor &finished, int64_t eos, int64_t device, int64_t stream) {
+  const int dtype = dtype_code(logits.scalar_type());
+  if (dtype < 0 || logits.dim() != 2 || logits.size(0) == 0 || logits.size(1) < 2 || logits.size(0) > INT_MAX / 64 ||
+      logits.size(1) > INT_MAX / 2 || logits.stride(1) != 1 || !on(logits, device) || !plain(logits) ||
+      c10::impl::dispatch_mode_enabled())
+    return false;
+  const int64_t b = logits.size(0), n = logits.size(1), es = logits.element_size();
+  const int64_t stride = b > 1 ? logits.stride(0) : n;
+  auto table = [&](const OptTensor &t, at::ScalarType type) {
+    return !t.has_value() || (on(*t, device) && t->scalar_type() == type && t->dim() == 2 && t->size(0) == b &&
+                              t->size(1) > 0 && t->is_contiguous());
+  };
+  if (!rows16(logits.data_ptr(), stride, n, es) || (n * es) % 16 != 0 || !table(tokens, at::kLong) ||
+      !table(margins, at::kFloat) || (tokens.has_value() && margins.has_value() && tokens->size(1) != margins->size(1)) ||
+      (column.has_value() && !index_vector(*column, at::kLong, 1, device)) ||
+      (next.has_value() && !index_vector(*next, at::kLong, b, device)) ||
+      (finished.has_value() && !index_vector(*finished, at::kBool, b, device)))
+    return false;
+  ic_greedy_call c = {};
+  c.logits = logits.data_ptr(), c.stride = stride;
+  c.rows = (int)b, c.n = (int)n, c.dtype = dtype;
+  if (tokens.has_value()) c.tokens = tokens->data_ptr<int64_t>(), c.token_stride = c.columns = tokens->size(1);
+  if (margins.has_value()) c.margins = margins->data_ptr<float>(), c.margin_stride = c.columns = margins->size(1);
+  if (column.has_value()) c.column = column->data_ptr<int64_t>();
+  if (next.has_value()) c.next = next->data_ptr<int64_t>();
+  if (finished.has_value()) c.finished = reinterpret_cast<uint8_t *>(finished->data_ptr<bool>()), c.eos = eos;
+  c.workspace_bytes = ic_greedy_workspace_bytes(c.rows, c.n);
+  const Tensor ws = at::empty({(int64_t)c.workspace_bytes}, logits.options().dtype(at::kByte));
+  c.workspace = ws.data_ptr();
+  return made("ic_greedy", ic_greedy(&c, (void *)stream));
+}
+
+// Position, slot and context length of the next token of each row (see ic_advance).
+bool advance(const Tensor &lens, const Tensor &tables, int64_t block_size, const Tensor &positions,
+             const Tensor &token_positions, const Tensor &slots, const Tensor &column, int64_t device, int64_t stream) {
+  const int64_t b = lens.numel();
+  if (b == 0 || b > INT_MAX / 512 || !index_vector(lens, at::kInt, b, device) || !table(tables, b, device) ||
+      tables.size(1) > INT_MAX || block_size > INT_MAX || !index_vector(positions, at::kInt, b, device) ||
+      !index_vector(token_positions, at::kLong, b, device) || !index_vector(slots, at::kLong, b, device) ||
+      !index_vector(column, at::kLong, 1, device))
+    return false;
+  ic_advance_call c = {};
+  c.context_lens = lens.data_ptr<int32_t>();
+  c.block_tables = tables.data_ptr<int32_t>(), c.block_table_stride = tables.stride(0);
+  c.rows = (int)b, c.table_width = (int)tables.size(1), c.block_size = (int)block_size;
+  c.positions = positions.data_ptr<int32_t>(), c.token_positions = token_positions.data_ptr<int64_t>();
+  c.slot_mapping = slots.data_ptr<int64_t>(), c.column = column.data_ptr<int64_t>();
+  return made("ic_advance", ic_advance(&c, (void *)stream));
+}
+
 }  // namespace
 
 // (wrapped, so that torch's exceptions keep their Python types: an allocation that does not fit raises
@@ -595,5 +650,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_rows", torch::wrap_pybind_function_no_gil(linear_rows));
   m.def("norm_rows", torch::wrap_pybind_function_no_gil(norm_rows));
   m.def("decoder_layer", torch::wrap_pybind_function_no_gil(decoder_layer));
+  m.def("greedy", torch::wrap_pybind_function_no_gil(greedy));
+  m.def("advance", torch::wrap_pybind_function_no_gil(advance));
   m.def("pack_mask", torch::wrap_pybind_function_no_gil(pack_mask));
 }

@@ -556,6 +556,34 @@ int ic_step_linear(const ic_step_linear_call *call, void *stream) {
   return ic::launch_step_linear(a, static_cast<hipStream_t>(stream));
 }
 
+size_t ic_greedy_workspace_bytes(int rows, int n) { return rows > 0 && n > 0 ? ic::greedy_workspace_bytes(rows, n) : 0; }
+
+int ic_greedy(const ic_greedy_call *call, void *stream) {
+  if (call == nullptr) return IC_ERR_NULL_POINTER;
+  const ic_greedy_call &a = *call;
+  if (a.rows < 0 || a.n < 2 || a.stride < a.n || ((a.tokens || a.margins) && a.columns < 1) ||
+      (a.tokens && a.token_stride < a.columns) || (a.margins && a.margin_stride < a.columns))
+    return IC_ERR_BAD_SHAPE;
+  if (!dtype_ok(a.dtype)) return IC_ERR_UNSUPPORTED;
+  if (a.rows == 0) return IC_OK;
+  const int es = ic::elem_size(a.dtype);
+  if (!a.logits) return IC_ERR_NULL_POINTER;
+  if (!aligned16(a.logits) || !stride16(a.stride, es) || !stride16(a.n, es)) return IC_ERR_ALIGNMENT;
+  if (!a.workspace || !aligned16(a.workspace) || a.workspace_bytes < ic_greedy_workspace_bytes(a.rows, a.n))
+    return IC_ERR_WORKSPACE;
+  return ic::launch_greedy(a, static_cast<hipStream_t>(stream));
+}
+
+int ic_advance(const ic_advance_call *call, void *stream) {
+  if (call == nullptr) return IC_ERR_NULL_POINTER;
+  const ic_advance_call &a = *call;
+  if (a.rows < 0 || a.table_width < 0 || a.block_size < 1 || a.block_table_stride < a.table_width) return IC_ERR_BAD_SHAPE;
+  if (a.rows == 0) return IC_OK;
+  if (!a.context_lens || !a.block_tables || !a.positions || !a.token_positions || !a.slot_mapping)
+    return IC_ERR_NULL_POINTER;
+  return ic::launch_advance(a, static_cast<hipStream_t>(stream));
+}
+
 int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,
                  int heads, int rows, int keys, uint64_t *bits, int32_t *lists, int32_t *flags, void *stream) {
   if (n_seqs < 0 || heads < 0 || rows < 0 || keys < 0 || stride_seq < 0 || stride_head < 0 || stride_row < 0)

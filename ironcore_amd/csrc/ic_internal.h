@@ -157,6 +157,9 @@ struct StepPlan {
   bool partial, rows;
 };
 StepPlan step_linear_plan(const ic_step_linear_call &a);
+size_t greedy_workspace_bytes(int rows, int n);
+int launch_greedy(const ic_greedy_call &a, hipStream_t stream);
+int launch_advance(const ic_advance_call &a, hipStream_t stream);
 int launch_paged_decode(const DecodeArgs &a, hipStream_t stream);
 int launch_paged_prefill(const PrefillArgs &a, hipStream_t stream);
 int launch_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, int64_t stride_row, int n_seqs,

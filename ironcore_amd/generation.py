@@ -459,6 +459,19 @@ def sample_next(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 0,
     return torch.multinomial(probs, num_samples=1, generator=generator)
 
 
+def _greedy(logits: torch.Tensor, with_margin: bool):
+    """``sample_next`` at temperature 0 and how far the token is ahead of the second best, natively, or
+    ``(None, None)``."""
+    here = _lib.here(logits) if type(logits) is torch.Tensor and logits.dim() == 2 else None
+    if here is None or torch.overrides.has_torch_function_unary(logits):
+        return None, None
+    nxt = torch.empty(logits.shape[0], 1, dtype=torch.int64, device=logits.device)
+    margin = torch.empty(logits.shape[0], 1, dtype=torch.float32, device=logits.device) if with_margin else None
+    if not _lib.host().greedy(logits, None, None, margin, nxt, None, 0, *here):
+        return None, None
+    return nxt, margin.squeeze(1) if with_margin else None
+
+
 @torch.no_grad()
 def generate(model: LanguageModel, input_ids: torch.Tensor, max_new_tokens: int, *,
              block_size: int = 16, temperature: float = 0.0, top_k: int = 0,
@@ -508,10 +521,14 @@ def generate(model: LanguageModel, input_ids: torch.Tensor, max_new_tokens: int,
             logits = _prefill_logits(model, input_ids, prompt_lens, kv_cache, seq_ids)
         else:
             logits = model(step_input, kv_cache=kv_cache, seq_ids=seq_ids)[:, -1, :]
+        nxt, margin = _greedy(logits, return_margins) if temperature == 0.0 else (None, None)
         if return_margins:
-            top2 = torch.topk(logits.float(), 2, dim=-1)[0]
-            margins.append(top2[:, 0] - top2[:, 1])
-        nxt = sample_next(logits, temperature, top_k, generator)
+            if margin is None:
+                top2 = torch.topk(logits.float(), 2, dim=-1)[0]
+                margin = top2[:, 0] - top2[:, 1]
+            margins.append(margin)
+        if nxt is None:
+            nxt = sample_next(logits, temperature, top_k, generator)
         if eos_token_id is not None:
             nxt = torch.where(finished.unsqueeze(1), torch.full_like(nxt, eos_token_id), nxt)
             finished |= nxt.squeeze(1) == eos_token_id
@@ -581,6 +598,10 @@ def _generate_graphed(model, input_ids, max_new_tokens, block_size, eos_token_id
     finished = torch.zeros(b, dtype=torch.bool, device=dev)
 
     def select(logits):
+        here = _lib.here(logits)
+        if here is not None and _lib.host().greedy(logits, col.view(1), new_tokens, margins, step_input,
+                                                   None if eos_token_id is None else finished, eos_token_id or 0, *here):
+            return
         if margins is not None:
             top2 = torch.topk(logits.float(), 2, dim=-1)[0]
             margins.scatter_(1, col.expand(b, 1), (top2[:, 0] - top2[:, 1]).unsqueeze(1))
@@ -589,19 +610,25 @@ def _generate_graphed(model, input_ids, max_new_tokens, block_size, eos_token_id
             nxt = torch.where(finished.unsqueeze(1), torch.full_like(nxt, eos_token_id), nxt)
             finished.logical_or_(nxt.squeeze(1) == eos_token_id)
         new_tokens.scatter_(1, col.expand(b, 1), nxt)
-        col.add_(1)
         step_input.copy_(nxt)
 
     def decode_step():
-        pos = ctx.clone()                                    # the new token's position = tokens cached so far
-        ctx.add_(1)
-        block = tables.gather(1, (pos // bs).long().unsqueeze(1)).squeeze(1)
+        # the new token's position = tokens cached so far; its slot from the table, its column the next one
+        pos, token_pos = torch.empty_like(ctx), torch.empty(b, 1, dtype=torch.int64, device=dev)
+        slots = torch.empty(b, dtype=torch.int64, device=dev)
+        here = _lib.here(ctx)
+        if here is None or not _lib.host().advance(ctx, tables, bs, pos, token_pos, slots, col.view(1), *here):
+            pos.copy_(ctx)
+            token_pos.copy_(ctx.unsqueeze(1))
+            ctx.add_(1)
+            col.add_(1)
+            block = tables.gather(1, (pos // bs).long().unsqueeze(1)).squeeze(1)
+            slots.copy_(block.long() * bs + (pos % bs).long())
         meta = PagedAttentionMetadata(
-            block_tables=tables, context_lens=ctx, slot_mapping=block.long() * bs + (pos % bs).long(),
+            block_tables=tables, context_lens=ctx, slot_mapping=slots,
             max_context_len=cached_at_end, cu_seqlens_q=None, cohort_size=1, cohort_shared_blocks=None,
             positions=pos)
-        step_logits = model(step_input, kv_cache=kv_cache, attn_metadata=meta,
-                            position_ids=pos.long().unsqueeze(1))[:, -1, :]
+        step_logits = model(step_input, kv_cache=kv_cache, attn_metadata=meta, position_ids=token_pos)[:, -1, :]
         select(step_logits)
 
     select(logits)
