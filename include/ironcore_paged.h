@@ -551,6 +551,35 @@ size_t ic_step_linear_workspace_bytes(const ic_step_linear_call *call);
 int ic_step_linear(const ic_step_linear_call *call, void *stream);
 
 /*
+ * A decode step's append and attention in one launch: ic_kv_append (with cos_table and
+ * sin_table ic_rope_kv_append_to, the query rows rotated on their way and not stored) of the
+ * n_seqs new rows, then ic_paged_decode, which sees all of them, whichever sequence's
+ * slot they are in.  For small batches of short contexts (at most 64 sequences);
+ * IC_ERR_UNSUPPORTED for the others, with nothing launched.  No workspace.
+ */
+typedef struct ic_decode_append_call {
+  void *out;
+  int64_t out_stride_seq;
+  const void *q;
+  int64_t q_stride_seq;
+  const void *k_new, *v_new;
+  int64_t new_stride_token;
+  void *k_pool, *v_pool;
+  int64_t pool_stride_block, pool_stride_head, pool_stride_token, num_blocks;
+  const int32_t *block_tables;
+  int64_t block_table_stride;
+  const int32_t *context_lens;
+  const int64_t *slot_mapping;
+  const int32_t *positions;
+  const float *cos_table, *sin_table;
+  int64_t table_rows;
+  int n_seqs, hn, gn, hd, block_size, max_context_len;
+  float scale;
+  int dtype;
+} ic_decode_append_call;
+int ic_paged_decode_append(const ic_decode_append_call *call, void *stream);
+
+/*
  * The next token of each row of logits, greedily (examples/generate_text.py:27-28 at
  * temperature 0): the first of the largest values, NaN counting as the largest.
  *

@@ -81,10 +81,11 @@ bool table(const Tensor &t, int64_t rows, int64_t device) {
 bool rows3(const Tensor &t, int64_t heads, int64_t hd) {
   return t.dim() == 3 && t.size(1) == heads && t.size(2) == hd && t.stride(2) == 1 && t.stride(1) == hd;
 }
-// [b, s, heads, hd] that is [b*s, heads, hd] rows at one stride.
+// [b, s, heads, hd] that is [b*s, heads, hd] rows at one stride (that of a dimension of size 1 says nothing: half of a
+// projection's row, as a decode step hands it over, keeps the half's length there).
 bool rows4(const Tensor &t, int64_t b, int64_t s, int64_t heads, int64_t hd) {
   return t.dim() == 4 && t.size(0) == b && t.size(1) == s && t.size(2) == heads && t.size(3) == hd &&
-         t.stride(3) == 1 && t.stride(2) == hd && (b == 1 || t.stride(0) == s * t.stride(1));
+         t.stride(3) == 1 && t.stride(2) == hd && (b == 1 || s == 1 || t.stride(0) == s * t.stride(1));
 }
 int64_t row_stride4(const Tensor &t) { return t.size(1) > 1 ? t.stride(1) : t.stride(0); }
 
@@ -224,6 +225,22 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
   const void *q = query.data_ptr();
   int64_t q_stride = row_stride4(query);
   if (!rows16(q, q_stride, in.hn * p.hd, query.element_size())) return c10::nullopt;
+  if (cohort == 1 && rows16(key.data_ptr(), row_stride4(key), p.gn * p.hd, key.element_size()) &&
+      rows16(value.data_ptr(), row_stride4(value), p.gn * p.hd, key.element_size())) {
+    const Tensor out = at::empty({in.b, 1, in.hn * p.hd}, query.options());
+    ic_decode_append_call c = {};
+    c.out = out.data_ptr(), c.out_stride_seq = in.hn * p.hd;
+    c.q = q, c.q_stride_seq = q_stride;
+    c.k_new = key.data_ptr(), c.v_new = value.data_ptr(), c.new_stride_token = row_stride4(key);
+    c.k_pool = const_cast<void *>(p.k), c.v_pool = const_cast<void *>(p.v);
+    c.pool_stride_block = p.sb, c.pool_stride_head = p.sh, c.pool_stride_token = p.st, c.num_blocks = p.nb;
+    c.block_tables = tables.data_ptr<int32_t>(), c.block_table_stride = tables.stride(0);
+    c.context_lens = lens.data_ptr<int32_t>(), c.slot_mapping = slots.data_ptr<int64_t>();
+    c.positions = rope.positions, c.cos_table = rope.cos, c.sin_table = rope.sin, c.table_rows = rope.rows;
+    c.n_seqs = (int)in.b, c.hn = (int)in.hn, c.gn = (int)p.gn, c.hd = (int)p.hd, c.block_size = (int)p.bs;
+    c.max_context_len = (int)max_ctx, c.scale = (float)scale, c.dtype = p.dtype;
+    if (made("ic_paged_decode_append", ic_paged_decode_append(&c, (void *)stream))) return out;
+  }
   Tensor rotated;
   if (rope.used) {
     rotated = at::empty({in.b, in.hn * p.hd}, query.options());

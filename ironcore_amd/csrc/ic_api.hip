@@ -72,7 +72,7 @@ int decode_checked(void *out, int64_t out_stride_seq, const void *q, int64_t q_s
                    int min_chunk_tokens, int cohort_size, const int32_t *cohort_shared_blocks,
                    void *workspace, size_t workspace_bytes, int max_waves, int dtype, void *stream,
                    const uint8_t *key_mask = nullptr, int64_t key_mask_stride_seq = 0,
-                   int64_t key_mask_stride_head = 0) {
+                   int64_t key_mask_stride_head = 0, const ic::AppendRows *rows = nullptr) {
   if (n_seqs < 0 || hn <= 0 || gn <= 0 || hn % gn != 0 || max_context_len < 0 || cohort_size < 1)
     return IC_ERR_BAD_SHAPE;
   if (key_mask != nullptr) {
@@ -101,7 +101,15 @@ int decode_checked(void *out, int64_t out_stride_seq, const void *q, int64_t q_s
   // the matrix-core kernel stores 8- or 16-byte pieces of output rows
   if (es == 2 && (!aligned16(out) || !stride16(out_stride_seq, es))) return IC_ERR_ALIGNMENT;
   const ic::DecodeWorkspace ws = ic::decode_workspace(n_seqs, hn, gn, hd, cohort_size, max_waves);
-  if (!workspace || workspace_bytes < ws.total() || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+  if (rows != nullptr) {
+    if (!rows->k_new || !rows->v_new || !rows->slots || (rows->cos_table != nullptr) != (rows->sin_table != nullptr) ||
+        (rows->cos_table && !rows->positions))
+      return IC_ERR_NULL_POINTER;
+    if (rows->new_stride_token < (int64_t)gn * hd || (rows->cos_table && rows->table_rows <= 0)) return IC_ERR_BAD_SHAPE;
+    if (!aligned16(rows->k_new) || !aligned16(rows->v_new) || !stride16(rows->new_stride_token, es) ||
+        !aligned16(rows->cos_table) || !aligned16(rows->sin_table))
+      return IC_ERR_ALIGNMENT;
+  } else if (!workspace || workspace_bytes < ws.total() || (reinterpret_cast<uintptr_t>(workspace) & 255u))
     return IC_ERR_WORKSPACE;
 
   ic::DecodeArgs a;
@@ -134,6 +142,7 @@ int decode_checked(void *out, int64_t out_stride_seq, const void *q, int64_t q_s
   a.key_mask_stride_seq = key_mask_stride_seq;
   a.key_mask_stride_head = key_mask_stride_head;
   a.dtype = dtype;
+  a.rows = rows;
   return ic::launch_paged_decode(a, static_cast<hipStream_t>(stream));
 }
 
@@ -554,6 +563,17 @@ int ic_step_linear(const ic_step_linear_call *call, void *stream) {
   const size_t need = ic_step_linear_workspace_bytes(call);
   if (need > 0 && (!a.workspace || !aligned16(a.workspace) || a.workspace_bytes < need)) return IC_ERR_WORKSPACE;
   return ic::launch_step_linear(a, static_cast<hipStream_t>(stream));
+}
+
+int ic_paged_decode_append(const ic_decode_append_call *call, void *stream) {
+  if (call == nullptr) return IC_ERR_NULL_POINTER;
+  const ic_decode_append_call &c = *call;
+  const ic::AppendRows rows = {c.k_new,     c.v_new,     c.new_stride_token, c.slot_mapping,
+                               c.positions, c.cos_table, c.sin_table,        c.table_rows};
+  return decode_checked(c.out, c.out_stride_seq, c.q, c.q_stride_seq, c.k_pool, c.v_pool, c.pool_stride_block,
+                        c.pool_stride_head, c.pool_stride_token, c.block_tables, c.block_table_stride, c.context_lens,
+                        c.n_seqs, c.hn, c.gn, c.hd, c.block_size, c.num_blocks, c.max_context_len, c.scale, 0, 1,
+                        nullptr, nullptr, 0, ic::kMaxDecodeWaves, c.dtype, stream, nullptr, 0, 0, &rows);
 }
 
 size_t ic_greedy_workspace_bytes(int rows, int n) { return rows > 0 && n > 0 ? ic::greedy_workspace_bytes(rows, n) : 0; }

@@ -58,6 +58,16 @@ struct LinearArgs {
   void *workspace;
 };
 
+// A decode step's new rows, where the append is part of the launch.
+struct AppendRows {
+  const void *k_new, *v_new;  // [n_seqs, gn, hd]
+  int64_t new_stride_token;   // elements
+  const int64_t *slots;       // [n_seqs]
+  const int32_t *positions;   // [n_seqs] rows of the rotary tables
+  const float *cos_table, *sin_table;  // or nullptr
+  int64_t table_rows;
+};
+
 struct DecodeArgs {
   void *out;
   int64_t out_stride_seq;
@@ -89,6 +99,7 @@ struct DecodeArgs {
   const uint8_t *key_mask = nullptr;
   int64_t key_mask_stride_seq = 0;
   int64_t key_mask_stride_head = 0;
+  const AppendRows *rows = nullptr;  // append these first, in the same launch
 };
 
 struct PrefillArgs {
