@@ -11,6 +11,11 @@
 //    (ceil(C / 32) per head), and a workgroup takes four neighbouring ones, so
 //    short chunks of several heads share a workgroup and its K/V tiles: 13 rows
 //    x 7 heads are two workgroups, not seven with 5 % of their rows in use.
+//    Blocks are numbered row block by row block, the heads of a row block side by
+//    side: the waves of a workgroup reach about equally far (a packed mask's
+//    lists belong to a head's rows: there head by head).
+//  * Chunks of unequal length: workgroups are numbered over all sequences, the longest sweep
+//    first (by_sweep below), KV heads round the XCDs.
 //  * Every wave stages a 16-row group of K AND of V of each tile, into two
 //    buffers (a third gained nothing); one barrier per tile.  64 KiB of LDS at head dim 128, 32 KiB at 64:
 //    two, resp. four, workgroups share a CU, and what the two-sided schedule of
@@ -28,6 +33,10 @@
 //    are mixed.  2 x 1 024 tokens in packed documents, 16 heads of 64: 149 us with
 //    the byte mask of the long kernel (32 byte loads per lane and tile, every tile
 //    walked), 11.9 us here, launch to launch.
+//
+//  * Query rows and outputs move as whole rows of a head and change places in LDS: as the MFMA lays them out a
+//    load touched 32 cache lines for 1 KiB, rotary tables likewise (query rows ready after 3.8 instead of 5.3 us of
+//    a workgroup's 17; 80 sequences of 129 tokens, 12 heads of 64: 20.8 -> 18.8 us).
 //
 // Bound by the latency of a tile (load, two products and a softmax in one wave's
 // instruction stream, about 1 us at head dim 128) at the sizes it is for; 80
@@ -47,10 +56,71 @@ constexpr int kBN = 64;         // tokens per K/V tile
 
 constexpr int kShortBuffers = 2;  // LDS buffers per pool and tile group
 
+// Chunks of unequal length, at most one sequence per lane: workgroup `index` of a KV head, numbered over the sequences by
+// the tiles it has to walk, most first.  Workgroup w of a sequence walks more tiles than its workgroup w - 1, so the number
+// that walk more than t tiles is a formula, and a binary search over t finds the index's t, then its sequence.
+// False: past the last one.  v0: its first wave block.
+//
+// 9 prompts of 3-701 tokens, 28 / 4 heads of 128, rotary: numbered sequence by sequence (units of a KV head on an
+// XCD) the XCDs had 82 to 102 workgroups, and the longest of a middle sequence began when half the launch was over
+// (the layer call 51.7 -> 49.2 us; with whole rows of queries and outputs, below, 40.4).
+__device__ __forceinline__ bool pick_by_sweep(const PrefillKP &p, int index, int &seq, int &q_lo, int &L, int &C, int &v0) {
+  const int n_seqs = p.n_units / p.gn, ln = threadIdx.x & (kWave - 1), group = p.group;
+  const bool in = ln < n_seqs;
+  const int lo = in ? p.cu_seqlens_q[ln] : 0, chunk = in ? p.cu_seqlens_q[ln + 1] - lo : 0;
+  int len = in ? p.context_lens[ln] : 0;
+  len = len < 0 ? 0 : len;
+  const int rows = p.causal && chunk > len ? len : chunk;
+  const int blocks = rows > 0 ? (rows + 31) >> 5 : 0;
+  const int wgs = (blocks * group + kShortWaves - 1) / kShortWaves;
+  const int prefix = len - rows;
+  // workgroups of this lane's sequence that walk more than t tiles (t == 0: all of them)
+  auto longer = [&](int t) {
+    if (t == 0) return wgs;
+    const int keys = t * kBN;
+    if (keys >= len) return 0;
+    if (!p.causal) return wgs;
+    const int block = keys > prefix ? (keys - prefix) >> 5 : 0;  // the first that sees past `keys`
+    const int first = (block * group) / kShortWaves;             // the workgroup that holds it (and rows of no later block)
+    return wgs > first ? wgs - first : 0;
+  };
+  // (counts are exact in fp32; up to 16 sequences stay inside a row of lanes, whose exchanges are vector instructions)
+  auto total = [&](int t) {
+    const float n = (float)longer(t);
+    return __builtin_amdgcn_readfirstlane((int)(n_seqs <= 16 ? group_sum<16>(n) : group_sum<kWave>(n)));
+  };
+  if (index >= total(0)) return false;
+  int above = 1;  // total(t) > index >= total(above)
+  while (total(above) > index) above *= 2;
+  int t = above >> 1;
+  while (above - t > 1) {
+    const int mid = (t + above) >> 1;
+    if (total(mid) > index)
+      t = mid;
+    else
+      above = mid;
+  }
+  const int beyond = longer(t + 1), here = longer(t) - beyond;
+  int rest = index - total(t + 1);
+  seq = 0;
+  for (int j = 0; j < n_seqs; ++j) {
+    const int n = __builtin_amdgcn_readlane(here, j);
+    if (rest < n) {
+      seq = j;
+      break;
+    }
+    rest -= n;
+  }
+  q_lo = __builtin_amdgcn_readlane(lo, seq);
+  L = __builtin_amdgcn_readlane(len, seq);
+  C = __builtin_amdgcn_readlane(chunk, seq);
+  v0 = (__builtin_amdgcn_readlane(wgs - beyond, seq) - 1 - rest) * kShortWaves;
+  return true;
+}
+
 template <class M, int HD, bool SINGLE, int TG, bool PACKED>
 __global__ __launch_bounds__(TG *kShortWaves *kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 2 : 4)))
 void paged_prefill_short_kernel(const PrefillKP p) {
-  using T = typename M::T;
   constexpr int KS = HD / 16;      // k-steps of the QK contraction
   constexpr int OB = HD / 32;      // 32-wide blocks of the output head dim
   constexpr int TB = kBN / 32;     // 32-token blocks per tile
@@ -70,15 +140,26 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 
   // XCD-aware placement as in the long kernel: the workgroups of one (sequence, KV head) unit get ids
   // that differ by a multiple of 8.
+  int seq, q_lo, L, C, kvh, v0 = 0, slice = 0, r = 0;
   const int per_unit = p.n_qtiles;  // workgroups per unit
-  const int slice = blockIdx.x / (kXcds * per_unit);
-  const int within = blockIdx.x - slice * (kXcds * per_unit);
-  const int unit = slice * kXcds + (within % kXcds);
-  if (unit >= p.n_units) return;
-  const int rank = unit / p.gn;
-  const int kvh = unit - rank * p.gn;
-  int seq, q_lo, L, C;
-  pick_sequence(p, rank, seq, q_lo, L, C);
+  if (!PACKED && p.by_sweep) {
+    kvh = blockIdx.x % p.gn;
+    if (!pick_by_sweep(p, blockIdx.x / p.gn, seq, q_lo, L, C, v0)) return;
+  } else {
+    slice = blockIdx.x / (kXcds * per_unit);
+    const int within = blockIdx.x - slice * (kXcds * per_unit);
+    const int unit = slice * kXcds + (within % kXcds);
+    if (unit >= p.n_units) return;
+    const int rank = unit / p.gn;
+    kvh = unit - rank * p.gn;
+    r = within / kXcds;
+    pick_sequence(p, rank, seq, q_lo, L, C);
+  }
+  // (one value for the workgroup on either way here: the tiles' addresses are scalars)
+  seq = __builtin_amdgcn_readfirstlane(seq);
+  kvh = __builtin_amdgcn_readfirstlane(kvh);
+  L = __builtin_amdgcn_readfirstlane(L);
+  C = __builtin_amdgcn_readfirstlane(C);
   const bool causal = p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
@@ -87,8 +168,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const int total = n_blocks * p.group;
   // The last blocks (the longest sweeps) first; in the slices that share the CUs with the first ones when
   // the whole grid is resident, last: a CU then holds a long and a short sweep, not two of the same length.
-  const int r = within / kXcds;
-  const int v0 = (slice < p.flip_slice ? per_unit - 1 - r : r) * kShortWaves;
+  if (PACKED || !p.by_sweep) v0 = (slice < p.flip_slice ? per_unit - 1 - r : r) * kShortWaves;
   if (v0 >= total) return;
 
   const int tid = threadIdx.x;
@@ -100,8 +180,8 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const int n = lane & 31;  // query column of this lane within the wave's 32-row block
   const int hh = lane >> 5;  // which half of each k-step this lane feeds
   const int v = v0 + wave < total ? v0 + wave : total - 1;
-  const int head = v / n_blocks;
-  const int row0 = (v - head * n_blocks) * 32;
+  const int head = PACKED ? v / n_blocks : v % p.group;
+  const int row0 = (PACKED ? v - head * n_blocks : v / p.group) * 32;
   const bool mine = v0 + wave < total && row0 < C;
   const int h = kvh * p.group + head;
   const int my_q = row0 + n;
@@ -117,17 +197,34 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 
   const int qrow = my_q < C ? my_q : C - 1;
   const int limit = causal ? P + qrow : L - 1;  // last key this query row may see
-  const int64_t at_row = query_row(p, q_lo, qrow);
+  // Query rows come in whole rows of the head, CPR lanes to a row (a lane's MFMA operands are 16-byte pieces of 32 rows,
+  // and loads of those cost a cache line look-up each), are rotated there, and change places through the part
+  // of this wave's second tile buffers.
+  const int cc = lane % CPR;    // 16-byte chunk of a row this lane moves, here and in the staging below
+  const int rsub = lane / CPR;  // row within the rows one load covers
+  const int k_lane = n * ROWB + ((hh ^ tile_swizzle_k<CPR>(n)) << 4);  // operand reads of rows stored as K tiles are
+  const int my_row = (int)query_row(p, q_lo, qrow);
+  int table_row_of_mine = 0;
+  if (p.positions != nullptr) table_row_of_mine = rope_position(p, my_row);
+  char *const s_q = (wave < 2 ? tiles_k : tiles_v) + (NB - 1) * TILEB + (wave & 1) * (TILEB / 2);
   Vec16 qf[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-    qf[ks] = load16(p.q + (at_row * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+  for (int i = 0; i < KS; ++i)
+    qf[i] = load16(p.q + ((int64_t)__shfl(my_row, i * WR + rsub, kWave) * p.q_stride_token + (int64_t)h * HD + cc * 8) * 2);
   if (p.positions != nullptr) {
-    const int64_t trig = rope_row(p, at_row) + hh * 4;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qf[ks] = rotate_chunk<typename M::E>(qf[ks], p.cos_table + trig + ks * 8, p.sin_table + trig + ks * 8);
+    for (int i = 0; i < KS; ++i) {
+      const int64_t trig = (int64_t)__shfl(table_row_of_mine, i * WR + rsub, kWave) * p.half_hd + cc * 4;
+      qf[i] = rotate_chunk<typename M::E>(qf[i], p.cos_table + trig, p.sin_table + trig);
+    }
   }
+#pragma unroll
+  for (int i = 0; i < KS; ++i) {
+    const int r = i * WR + rsub;
+    store16(s_q + r * ROWB + ((cc ^ tile_swizzle_k<CPR>(r)) << 4), qf[i]);
+  }
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) qf[ks] = load16(s_q + (k_lane ^ (ks * 32)));
 
   f32x16_t o[OB];
   float m = kNegInf, l = 0.f;
@@ -136,10 +233,9 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[ob][i] = 0.f;
 
-  // tiles this wave's rows reach, and the most that any wave of the workgroup does: a workgroup whose
-  // blocks span two heads holds a head's last block
+  // tiles this wave's rows reach, and the most that any wave of the workgroup does: its last block's
   const int v_last = v0 + kShortWaves < total ? v0 + kShortWaves - 1 : total - 1;
-  const int last_row = v0 / n_blocks == v_last / n_blocks ? (v_last % n_blocks) * 32 + 32 : C;
+  const int last_row = (v_last / p.group) * 32 + 32;  // (a packed mask has its lists instead)
   int kv_end = causal ? P + last_row : L;
   kv_end = kv_end < L ? kv_end : L;
   MaskList list;
@@ -151,8 +247,6 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 
   // ---- tile staging: memory -> LDS (see the long kernel: one table entry and one base address per
   // 16-row group, fixed lane offsets, unconditional loads) -----------------------------------------
-  const int cc = lane % CPR;    // LDS slot (16-byte chunk of the row) this lane fills
-  const int rsub = lane / CPR;  // row within the rows one load covers
   const int64_t head_bytes = (int64_t)kvh * p.stride_head * 2;
   const uint32_t block_bytes = (uint32_t)(p.stride_block * 2);
   const uint32_t token_bytes = (uint32_t)(p.stride_token * 2);
@@ -231,7 +325,6 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   };
 
   // per-lane LDS offsets of the operand reads (the swizzles seen from the reading side)
-  const int k_lane = n * ROWB + ((hh ^ tile_swizzle_k<CPR>(n)) << 4);
   const int vq = (lane & 15) >> 2;
   const int v_lane = (4 * hh + vq) * ROWB + ((tile_swizzle_v<CPR>(vq) >> 2) << 6) + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
   const int mask_from = __builtin_amdgcn_readfirstlane(causal ? (P + row0 + 1) / kBN : L / kBN);
@@ -407,19 +500,28 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   both_halves(l, l_a, l_b);
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  if (mine && my_q < C) {
-    T *orow = reinterpret_cast<T *>(p.out) + query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD;
+  // Out in whole rows of the head again, through LDS: the tiles are done with (with two tile groups the first group's
+  // wave takes the slab it has just read).
+  if constexpr (TG == 1) __syncthreads();
+  char *const s_o = TG == 1 ? s_tiles + wave * 32 * ROWB : s_tiles + wave * (OB * 16 + 2) * kWave * 4;
 #pragma unroll
-    for (int ob = 0; ob < OB; ++ob) {
+  for (int ob = 0; ob < OB; ++ob) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int d = ob * 32 + 4 * hh + 8 * j;
-        uint2 w;
-        w.x = M::pack2(o[ob][4 * j] * inv, o[ob][4 * j + 1] * inv);
-        w.y = M::pack2(o[ob][4 * j + 2] * inv, o[ob][4 * j + 3] * inv);
-        *reinterpret_cast<uint2 *>(orow + d) = w;
-      }
+    for (int j = 0; j < 4; ++j) {
+      uint2 w;
+      w.x = M::pack2(o[ob][4 * j] * inv, o[ob][4 * j + 1] * inv);
+      w.y = M::pack2(o[ob][4 * j + 2] * inv, o[ob][4 * j + 3] * inv);
+      *reinterpret_cast<uint2 *>(s_o + n * ROWB + (((ob * 4 + j) ^ tile_swizzle_k<CPR>(n)) << 4) + hh * 8) = w;
     }
+  }
+#pragma unroll
+  for (int i = 0; i < KS; ++i) {
+    const int r = i * WR + rsub;
+    // (a packed mask comes with equal sequences, whose rows need no register until here)
+    const int64_t row = PACKED ? q_lo + row0 + r : __shfl(my_row, r, kWave);
+    const int64_t to = row * p.out_stride_token + (int64_t)h * HD + cc * 8;
+    const Vec16 v = load16(s_o + r * ROWB + ((cc ^ tile_swizzle_k<CPR>(r)) << 4));
+    if (mine && row0 + r < C) store16(p.out + to * 2, v);
   }
 }
 
@@ -498,7 +600,14 @@ bool prefill_takes_short(const PrefillArgs &a) {
 int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t stream) {
   const int64_t per_unit = short_workgroups_per_unit(a);
   const int64_t slices = (kp.n_units + kXcds - 1) / kXcds;
-  const int64_t wgs = slices * kXcds * per_unit;
+  int64_t wgs = slices * kXcds * per_unit;
+  // Chunks that lie in padded rows are of unequal length: at most so many workgroups, a sequence's last one and row
+  // block not full.
+  kp.by_sweep = a.rows != nullptr && a.mask_bits == nullptr && a.n_seqs <= kWave;
+  if (kp.by_sweep) {
+    const int64_t blocks = a.n_rows / 32 + a.n_seqs;
+    wgs = a.gn * ((blocks * kp.group + kShortWaves - 1) / kShortWaves + a.n_seqs);
+  }
   if (wgs > 0x7fffffff) return IC_ERR_UNSUPPORTED;
   kp.n_qtiles = (int)per_unit;
   const int cus = device_cu_count();

@@ -34,6 +34,7 @@ struct PrefillKP {
   int gn;           // KV heads
   int n_units;      // n_seqs * gn
   int n_qtiles;     // query tiles per chunk (grid sizing); short kernel: workgroups per unit
+  int by_sweep;     // short kernel: workgroups are numbered over all sequences, longest sweep first
   int flip_slice;   // short kernel: first slice of units whose workgroups take their blocks shortest sweep first
   int causal;
   float scale_log2e;
@@ -200,11 +201,13 @@ struct MaskList {
 };
 
 // The rotary tables' row of query row `row` (clamped into them).
-__device__ __forceinline__ int64_t rope_row(const PrefillKP &p, int64_t row) {
+__device__ __forceinline__ int rope_position(const PrefillKP &p, int64_t row) {
   int pos = p.positions[row];
   pos = pos < 0 ? 0 : pos;
-  pos = pos >= p.table_rows ? p.table_rows - 1 : pos;
-  return (int64_t)pos * p.half_hd;
+  return pos >= p.table_rows ? p.table_rows - 1 : pos;
+}
+__device__ __forceinline__ int64_t rope_row(const PrefillKP &p, int64_t row) {
+  return (int64_t)rope_position(p, row) * p.half_hd;
 }
 
 constexpr float kLazySlack = 8.0f;  // log2 units
