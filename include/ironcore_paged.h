@@ -551,6 +551,32 @@ size_t ic_step_linear_workspace_bytes(const ic_step_linear_call *call);
 int ic_step_linear(const ic_step_linear_call *call, void *stream);
 
 /*
+ * The append of a step's chunks in one launch: ic_kv_append, or with cos_table and
+ * sin_table ic_rope_kv_append_to without queries, and with rows not NULL
+ * ic_zero_unlisted_rows (zero_out, zero_stride_bytes, zero_row_bytes, rows, n_rows, bounds,
+ * n_seqs, row_pitch) beside it.
+ */
+typedef struct ic_append_call {
+  const void *k_new, *v_new;
+  int64_t new_stride_token;
+  void *k_pool, *v_pool;
+  int64_t pool_stride_block, pool_stride_head, pool_stride_token, num_blocks;
+  const int64_t *slot_mapping;
+  int64_t n_tokens;
+  int gn, hd, block_size, dtype;
+  const int32_t *positions;
+  const float *cos_table, *sin_table;
+  int64_t table_rows;
+  void *zero_out;
+  int64_t zero_stride_bytes;
+  const int64_t *rows;
+  int64_t n_rows;
+  const int32_t *bounds;
+  int zero_row_bytes, n_seqs, row_pitch;
+} ic_append_call;
+int ic_append_chunks(const ic_append_call *call, void *stream);
+
+/*
  * A decode step's append and attention in one launch: ic_kv_append (with cos_table and
  * sin_table ic_rope_kv_append_to, the query rows rotated on their way and not stored) of the
  * n_seqs new rows, then ic_paged_decode, which sees all of them, whichever sequence's

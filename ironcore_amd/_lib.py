@@ -98,6 +98,7 @@ SIGNATURES = {
         c_void_p, c_size_t, c_int, c_void_p]),  # workspace, workspace_bytes, dtype, stream
     "ic_step_linear_workspace_bytes": (c_size_t, [c_void_p]),   # call descriptor
     "ic_step_linear": (c_int, [c_void_p, c_void_p]),    # call descriptor, stream
+    "ic_append_chunks": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_paged_decode_append": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_greedy_workspace_bytes": (c_size_t, [c_int, c_int]),   # rows, n
     "ic_greedy": (c_int, [c_void_p, c_void_p]),         # call descriptor, stream

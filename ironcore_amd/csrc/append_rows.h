@@ -2,6 +2,7 @@
 // workgroups of kAppendThreads lanes, one 16-byte chunk of a row to a lane.
 #pragma once
 
+#include "ic_device.h"
 #include "ic_internal.h"
 
 namespace ic {
@@ -38,6 +39,28 @@ template <bool WIDE>
 __device__ __forceinline__ int64_t slot_block(int64_t slot, int block_size, int64_t num_slots) {
   if (WIDE || (num_slots >> 32) != 0) return slot / block_size;
   return (uint32_t)slot / (uint32_t)block_size;
+}
+
+// Zeroes the rows of a padded output that no chunk holds, ahead of the attention launch that writes the others.
+// Bound by the bytes written.  Row r of sequence i is known to be listed when entry bounds[i] + r names it (chunks
+// at the start of their rows, what PagedKVCache lays out); a row listed elsewhere is zeroed and written again,
+// which is why this comes before the attention kernel: inside it it would race with that write.  It is a part of the
+// append's launch (9 prompts padded to 701 rows of 28 heads of 128: one launch of 7 us instead of 7 + 6).
+__device__ __forceinline__ void zero_unlisted_rows(const ZeroRows &z, int64_t group, int64_t groups) {
+  for (int64_t row = group; row < z.total; row += groups) {
+    const int seq = (int)(row / z.row_pitch);
+    const int64_t at = z.bounds[seq] + (row - (int64_t)seq * z.row_pitch);
+    if (at >= 0 && at < z.bounds[seq + 1] && at < z.n_rows && z.rows[at] == row) continue;
+    for (int c = threadIdx.x; c < z.chunks; c += kAppendThreads)
+      store16(z.out + row * z.stride_bytes + (int64_t)c * 16, Vec16{{0u, 0u, 0u, 0u}});
+  }
+}
+
+// The last z slice of an append's grid is that, if there is anything to zero.
+__device__ __forceinline__ bool zero_part(const ZeroRows &z) {
+  if (z.total == 0 || blockIdx.z + 1 != gridDim.z) return false;
+  zero_unlisted_rows(z, (int64_t)blockIdx.y * gridDim.x + blockIdx.x, (int64_t)gridDim.y * gridDim.x);
+  return true;
 }
 
 }  // namespace ic

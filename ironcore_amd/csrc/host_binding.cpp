@@ -293,21 +293,23 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
     return c10::nullopt;
   const Rope rope(positions, cos, sin, in.b * in.s, p.hd, device);
   if (!rope.ok) return c10::nullopt;
-  if (rope.used ? !rope_append(key, value, p, slots, rope, in.b * in.s, nullptr, nullptr, 0, in.hn, (void *)stream)
-                : !append_rows(key.data_ptr(), value.data_ptr(), row_stride4(key), p, slots, in.b * in.s,
-                               (void *)stream))
-    return c10::nullopt;
   const Tensor out = at::empty({in.b, in.s, in.hn * p.hd}, query.options());
   ic_prefill_call c = prefill_call(out, query, p, in.b, longest, in.hn, scale, true);
-  if (rows.has_value()) {
-    c.rows = rows->data_ptr<int64_t>();
-    c.n_rows = rows->numel(), c.q_rows = in.b * in.s;
-    const int row_bytes = (int)(in.hn * p.hd * query.element_size());
-    if (!made("ic_zero_unlisted_rows",
-              ic_zero_unlisted_rows(c.out, row_bytes, row_bytes, c.rows, c.n_rows, bounds.data_ptr<int32_t>(),
-                                    (int)in.b, (int)in.s, (void *)stream)))
-      return c10::nullopt;
+  ic_append_call ap = {};
+  ap.k_new = key.data_ptr(), ap.v_new = value.data_ptr(), ap.new_stride_token = row_stride4(key);
+  ap.k_pool = const_cast<void *>(p.k), ap.v_pool = const_cast<void *>(p.v);
+  ap.pool_stride_block = p.sb, ap.pool_stride_head = p.sh, ap.pool_stride_token = p.st, ap.num_blocks = p.nb;
+  ap.slot_mapping = slots.data_ptr<int64_t>(), ap.n_tokens = in.b * in.s;
+  ap.gn = (int)p.gn, ap.hd = (int)p.hd, ap.block_size = (int)p.bs, ap.dtype = p.dtype;
+  ap.positions = rope.positions, ap.cos_table = rope.cos, ap.sin_table = rope.sin, ap.table_rows = rope.rows;
+  if (rows.has_value()) {  // the rows that no chunk holds become zeros beside the append
+    c.rows = ap.rows = rows->data_ptr<int64_t>();
+    c.n_rows = ap.n_rows = rows->numel(), c.q_rows = in.b * in.s;
+    ap.zero_out = out.data_ptr();
+    ap.zero_row_bytes = (int)(in.hn * p.hd * query.element_size()), ap.zero_stride_bytes = ap.zero_row_bytes;
+    ap.bounds = bounds.data_ptr<int32_t>(), ap.n_seqs = (int)in.b, ap.row_pitch = (int)in.s;
   }
+  if (!made("ic_append_chunks", ic_append_chunks(&ap, (void *)stream))) return c10::nullopt;
   c.block_tables = tables.data_ptr<int32_t>();
   c.block_table_stride = tables.stride(0);
   c.context_lens = lens.data_ptr<int32_t>();

@@ -18,6 +18,18 @@ struct PoolLayout {
   int block_size;
 };
 
+// Rows of a padded output to zero beside an append (total == 0: none).
+struct ZeroRows {
+  char *out = nullptr;
+  int64_t stride_bytes = 0;
+  const int64_t *rows = nullptr;    // the rows that exist, chunk by chunk
+  int64_t n_rows = 0;
+  const int32_t *bounds = nullptr;  // of the chunks in `rows`
+  int64_t total = 0;                // rows of out, row_pitch to a sequence
+  int chunks = 0;                   // 16-byte pieces of a row
+  int row_pitch = 1;
+};
+
 struct AppendArgs {
   const void *k_new;
   const void *v_new;
@@ -30,6 +42,7 @@ struct AppendArgs {
   int gn;
   int hd;
   int dtype;
+  ZeroRows zero;
 };
 
 // KV append with rotary embedding: the plain append's arguments (k_new / v_new
@@ -156,8 +169,7 @@ struct PrefillArgs {
 // dtype/shape) or IC_ERR_LAUNCH.
 int launch_kv_append(const AppendArgs &a, hipStream_t stream);
 int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream);
-int launch_zero_unlisted_rows(char *out, int64_t stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
-                              const int32_t *bounds, int n_seqs, int row_pitch, hipStream_t stream);
+int launch_zero_unlisted_rows(const ZeroRows &z, hipStream_t stream);
 int launch_linear_rows(const LinearArgs &a, hipStream_t stream);
 int linear_rows_splits(int n, int k, int dtype, int want);
 int launch_step_linear(const ic_step_linear_call &a, hipStream_t stream);

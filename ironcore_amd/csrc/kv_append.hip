@@ -25,7 +25,9 @@ __global__ __launch_bounds__(kAppendThreads) void kv_append_kernel(
     const char *__restrict__ k_new, const char *__restrict__ v_new, int64_t new_stride_bytes,
     char *__restrict__ k_pool, char *__restrict__ v_pool, int64_t stride_block_bytes,
     int64_t stride_head_bytes, int64_t stride_token_bytes, const int64_t *__restrict__ slot_mapping,
-    int chunks_per_head, int chunks_per_row, int row_shift, int64_t n_tokens, int block_size, int64_t num_slots) {
+    int chunks_per_head, int chunks_per_row, int row_shift, int64_t n_tokens, int block_size, int64_t num_slots,
+    const ZeroRows zero) {
+  if (zero_part(zero)) return;
   const int64_t t = append_token<WIDE>(row_shift);
   const int c = append_chunk<WIDE>(row_shift);
   if (t >= n_tokens || c >= chunks_per_row) return;
@@ -51,48 +53,37 @@ int launch_kv_append(const AppendArgs &a, hipStream_t stream) {
   const int row_shift = append_row_shift(chunks_per_row);
   const int rows = kAppendThreads >> row_shift;  // token rows of a workgroup
   dim3 grid((chunks_per_row + kAppendThreads - 1) / kAppendThreads, 1, 2);
+  ZeroRows zero = a.zero;
   // gridDim.y is limited to 65535: walk longer appends in slices.
   const int64_t slice = (int64_t)65535 * rows;
   for (int64_t t0 = 0; t0 < a.n_tokens; t0 += slice) {
     const int64_t n = (a.n_tokens - t0 < slice) ? a.n_tokens - t0 : slice;
     grid.y = (unsigned)((n + rows - 1) / rows);
+    grid.z = zero.total > 0 ? 3 : 2;
     hipLaunchKernelGGL(rows == 1 ? kv_append_kernel<true> : kv_append_kernel<false>, grid, dim3(kAppendThreads), 0, stream,
                        (const char *)a.k_new + t0 * a.new_stride_token * es,
                        (const char *)a.v_new + t0 * a.new_stride_token * es,
                        a.new_stride_token * es, (char *)a.k_pool, (char *)a.v_pool,
                        a.pool.stride_block * es, a.pool.stride_head * es, a.pool.stride_token * es,
                        a.slot_mapping + t0, chunks_per_head, chunks_per_row, row_shift, n, a.pool.block_size,
-                       a.pool.num_blocks * a.pool.block_size);
+                       a.pool.num_blocks * a.pool.block_size, zero);
+    zero.total = 0;  // the first slice's
   }
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
 
 namespace {
 
-// Zeroes the rows of a padded output that no chunk holds, ahead of the attention launch that writes the others.
-// Bound by the bytes written.  Row r of sequence i is known to be listed when entry bounds[i] + r names it (chunks
-// at the start of their rows, what PagedKVCache lays out); a row listed elsewhere is zeroed and written again,
-// which is why this is a launch of its own: inside the attention kernel it would race with that write.
-__global__ __launch_bounds__(kAppendThreads) void zero_unlisted_rows_kernel(
-    char *__restrict__ out, int64_t stride_bytes, int chunks, const int64_t *__restrict__ rows, int64_t n_rows,
-    const int32_t *__restrict__ bounds, int row_pitch, int64_t total) {
-  for (int64_t row = blockIdx.x; row < total; row += gridDim.x) {
-    const int seq = (int)(row / row_pitch);
-    const int64_t at = bounds[seq] + (row - (int64_t)seq * row_pitch);
-    if (at >= 0 && at < bounds[seq + 1] && at < n_rows && rows[at] == row) continue;
-    for (int c = threadIdx.x; c < chunks; c += kAppendThreads)
-      store16(out + row * stride_bytes + (int64_t)c * 16, Vec16{{0u, 0u, 0u, 0u}});
-  }
+__global__ __launch_bounds__(kAppendThreads) void zero_unlisted_rows_kernel(const ZeroRows z) {
+  zero_unlisted_rows(z, blockIdx.x, gridDim.x);
 }
 
 }  // namespace
 
-int launch_zero_unlisted_rows(char *out, int64_t stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
-                              const int32_t *bounds, int n_seqs, int row_pitch, hipStream_t stream) {
-  const int64_t total = (int64_t)n_seqs * row_pitch;
+int launch_zero_unlisted_rows(const ZeroRows &z, hipStream_t stream) {
   const int64_t most = (int64_t)device_cu_count() * 8;
-  hipLaunchKernelGGL(zero_unlisted_rows_kernel, dim3((unsigned)(total < most ? total : most)), dim3(kAppendThreads), 0,
-                     stream, out, stride_bytes, row_bytes / 16, rows, n_rows, bounds, row_pitch, total);
+  hipLaunchKernelGGL(zero_unlisted_rows_kernel, dim3((unsigned)(z.total < most ? z.total : most)), dim3(kAppendThreads), 0,
+                     stream, z);
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
 

@@ -62,7 +62,9 @@ struct RopeKP {
 };
 
 template <class E, bool WIDE>
-__global__ __launch_bounds__(kAppendThreads) void rope_kv_append_kernel(const RopeKP p, int64_t t0, int64_t n_tokens) {
+__global__ __launch_bounds__(kAppendThreads) void rope_kv_append_kernel(const RopeKP p, int64_t t0, int64_t n_tokens,
+                                                                             const ZeroRows zero) {
+  if (zero_part(zero)) return;
   constexpr int PAIRS = E::EPL / 2;  // pairs in one 16-byte chunk
   const int part = blockIdx.z;  // 0: K, 1: V, 2: Q
   const int row_shift = part == 2 ? p.q_row_shift : p.kv_row_shift;
@@ -99,17 +101,20 @@ __global__ __launch_bounds__(kAppendThreads) void rope_kv_append_kernel(const Ro
 }
 
 template <class E>
-int launch_typed(const RopeKP &kp, int64_t n_tokens, hipStream_t stream) {
+int launch_typed(const RopeKP &kp, int64_t n_tokens, ZeroRows zero, hipStream_t stream) {
   const int widest = kp.q_chunks > kp.kv_chunks ? kp.q_chunks : kp.kv_chunks;
   const int shift = kp.q_row_shift > kp.kv_row_shift ? kp.q_row_shift : kp.kv_row_shift;
   const int rows = kAppendThreads >> shift;  // token rows of a workgroup, at least
   dim3 grid((widest + kAppendThreads - 1) / kAppendThreads, 1, kp.q_chunks > 0 ? 3 : 2);
   const bool wide = kp.kv_row_shift == kAppendThreadsShift && (kp.q_chunks == 0 || kp.q_row_shift == kAppendThreadsShift);
   const int64_t slice = (int64_t)65535 * rows;  // gridDim.y limit: walk longer batches in slices
+  const unsigned parts = grid.z;
   for (int64_t t0 = 0; t0 < n_tokens; t0 += slice) {
     const int64_t n = n_tokens - t0 < slice ? n_tokens - t0 : slice;
     grid.y = (unsigned)((n + rows - 1) / rows);
-    hipLaunchKernelGGL((wide ? rope_kv_append_kernel<E, true> : rope_kv_append_kernel<E, false>), grid, dim3(kAppendThreads), 0, stream, kp, t0, t0 + n);
+    grid.z = parts + (zero.total > 0 ? 1 : 0);
+    hipLaunchKernelGGL((wide ? rope_kv_append_kernel<E, true> : rope_kv_append_kernel<E, false>), grid, dim3(kAppendThreads), 0, stream, kp, t0, t0 + n, zero);
+    zero.total = 0;  // the first slice's
   }
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
@@ -147,9 +152,9 @@ int launch_rope_kv_append(const RopeAppendArgs &a, hipStream_t stream) {
   kp.block_size = ap.pool.block_size;
   kp.half_hd = ap.hd / 2;
   switch (ap.dtype) {
-    case IC_DTYPE_BF16: return launch_typed<Bf16>(kp, ap.n_tokens, stream);
-    case IC_DTYPE_F16: return launch_typed<F16>(kp, ap.n_tokens, stream);
-    case IC_DTYPE_F32: return launch_typed<F32>(kp, ap.n_tokens, stream);
+    case IC_DTYPE_BF16: return launch_typed<Bf16>(kp, ap.n_tokens, ap.zero, stream);
+    case IC_DTYPE_F16: return launch_typed<F16>(kp, ap.n_tokens, ap.zero, stream);
+    case IC_DTYPE_F32: return launch_typed<F32>(kp, ap.n_tokens, ap.zero, stream);
     default: return IC_ERR_UNSUPPORTED;
   }
 }

@@ -1,0 +1,121 @@
+"""Chunks of unequal length (rows named one by one): workgroups numbered over all sequences by the length of their
+sweep, against the same chunks numbered sequence by sequence; the append's launch with the zeroing beside it."""
+import ctypes
+from ctypes import c_float, c_int, c_int64, c_void_p
+
+import pytest
+import torch
+
+from ironcore_amd import _lib, paged_ops, workloads
+from ironcore_amd.layers import RotaryPositionalEmbedding
+
+pytestmark = pytest.mark.gpu
+
+
+class Prefill(ctypes.Structure):
+    _fields_ = [(n, t) for names, t in (
+        ("out", c_void_p), ("out_stride_token", c_int64), ("q", c_void_p), ("q_stride_token", c_int64), ("k_pool v_pool", c_void_p),
+        ("pool_stride_block pool_stride_head pool_stride_token", c_int64), ("block_tables", c_void_p),
+        ("block_table_stride", c_int64), ("context_lens cu_seqlens_q", c_void_p),
+        ("n_seqs max_chunk_len hn gn hd block_size", c_int), ("num_blocks", c_int64), ("scale", c_float),
+        ("causal dtype uniform_context", c_int), ("row_pitch", c_int64), ("rows", c_void_p), ("n_rows q_rows", c_int64),
+        ("positions cos_table sin_table", c_void_p), ("table_rows", c_int64), ("mask_bits mask_lists", c_void_p),
+        ("mask_plane_seq mask_plane_head", c_int)) for n in names.split()]
+
+
+class Append(ctypes.Structure):
+    _fields_ = [(n, t) for names, t in (
+        ("k_new v_new", c_void_p), ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
+        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("slot_mapping", c_void_p),
+        ("n_tokens", c_int64), ("gn hd block_size dtype", c_int), ("positions cos_table sin_table", c_void_p),
+        ("table_rows", c_int64), ("zero_out", c_void_p), ("zero_stride_bytes", c_int64), ("rows", c_void_p),
+        ("n_rows", c_int64), ("bounds", c_void_p), ("zero_row_bytes n_seqs row_pitch", c_int)) for n in names.split()]
+
+
+def _attend(d, hn, gn, hd, causal, rows, positions, emb, out, q):
+    call = Prefill(out=out.data_ptr(), out_stride_token=hn * hd, q=q.data_ptr(), q_stride_token=hn * hd,
+                   k_pool=d.k_pool.data_ptr(), v_pool=d.v_pool.data_ptr(), pool_stride_block=d.k_pool.stride(0),
+                   pool_stride_head=d.k_pool.stride(1), pool_stride_token=d.k_pool.stride(2), block_tables=d.block_tables.data_ptr(),
+                   block_table_stride=d.block_tables.stride(0), context_lens=d.context_lens.data_ptr(),
+                   cu_seqlens_q=d.cu_seqlens_q.data_ptr(), n_seqs=len(d.context_lens), max_chunk_len=d.max_chunk_len, hn=hn, gn=gn,
+                   hd=hd, block_size=d.k_pool.shape[2], num_blocks=d.k_pool.shape[0], scale=hd ** -0.5, causal=causal,
+                   dtype=_lib.IC_DTYPE[q.dtype])
+    if rows is not None:
+        call.rows, call.n_rows, call.q_rows = rows.data_ptr(), rows.numel(), q.shape[0]
+    if emb is not None:
+        call.positions, call.cos_table, call.sin_table = positions.data_ptr(), emb.cos_emb.data_ptr(), emb.sin_emb.data_ptr()
+        call.table_rows = emb.cos_emb.shape[0]
+    assert _lib.load().ic_paged_prefill_ex(ctypes.byref(call), _lib.current_stream_ptr(q.device)) == 0
+    return out
+
+
+@pytest.mark.parametrize("n_seqs,hn,gn,hd,block,prefix,chunks,dtype", [
+    (1, 7, 1, 128, 16, (0, 0), (97, 97), torch.bfloat16),      # one sequence, a group that fills no workgroup
+    (16, 8, 8, 128, 16, (0, 200), (0, 300), torch.bfloat16),   # as many as a row of lanes holds; empty chunks
+    (17, 4, 2, 64, 48, (0, 700), (1, 65), torch.float16),
+    (64, 6, 2, 32, 16, (0, 40), (0, 140), torch.bfloat16),     # a sequence to every lane
+    (65, 6, 2, 64, 16, (0, 40), (1, 70), torch.bfloat16),      # one more: numbered sequence by sequence
+    (3, 28, 4, 128, 16, (1500, 1600), (1, 130), torch.bfloat16),
+    (9, 12, 12, 128, 16, (0, 0), (3, 700), torch.bfloat16)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("rope", [False, True])
+def test_by_sweep(gpu, n_seqs, hn, gn, hd, block, prefix, chunks, dtype, causal, rope):
+    wl = workloads.make_prefill_workload(n_seqs, hn, gn, hd, *prefix, *chunks, block_size=block, dtype=dtype, seed=n_seqs)
+    d = wl.to(gpu)
+    paged_ops.kv_append(d.k_new, d.v_new, d.k_pool, d.v_pool, d.slot_mapping)
+    if not causal and n_seqs > 1:
+        d.context_lens[n_seqs // 2] = 0        # rows without a key: zeros
+    total = d.query.shape[0]
+    emb = RotaryPositionalEmbedding(hd, max_seq_len=300).to(gpu) if rope else None
+    g = torch.Generator().manual_seed(n_seqs)
+    positions = torch.randint(-2, 320, (total,), generator=g, dtype=torch.int32).to(gpu)
+    want = torch.empty(total, hn * hd, dtype=dtype, device=gpu)
+    _attend(d, hn, gn, hd, causal, None, positions, emb, want, d.query)
+    spread = torch.randperm(2 * total + 3, generator=g)[:total].to(gpu)                   # any rows of a larger tensor
+    q = torch.full((2 * total + 3, hn, hd), float("nan"), dtype=dtype, device=gpu)
+    q[spread] = d.query
+    at = torch.full((2 * total + 3,), -1, dtype=torch.int32, device=gpu)
+    at[spread] = positions
+    out = torch.full((2 * total + 3, hn * hd), 7.0, dtype=dtype, device=gpu)
+    _attend(d, hn, gn, hd, causal, spread, at, emb, out, q)
+    # the same sums, in two tile groups or one: a rounding of the result apart
+    assert torch.allclose(out[spread].float(), want.float(), rtol=2 ** -7, atol=2 ** -9)
+    untouched = torch.ones(2 * total + 3, dtype=torch.bool, device=gpu)
+    untouched[spread] = False
+    assert (out[untouched] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_seqs,width,gn,hd", [(1, 5, 1, 32), (3, 40, 2, 64), (2, 70, 33, 128)])
+@pytest.mark.parametrize("rope", [False, True])
+def test_append_and_zeroing(gpu, dtype, n_seqs, width, gn, hd, rope):
+    g = torch.Generator(device=gpu).manual_seed(width)
+    n = n_seqs * width
+    k, v = (torch.randn(n, gn, hd, generator=g, device=gpu).to(dtype) for _ in range(2))
+    lens = [width - 3 * i for i in range(n_seqs)]
+    rows = torch.tensor([i * width + t for i, c in enumerate(lens) for t in range(c)], device=gpu)
+    bounds = torch.tensor([0] + lens, dtype=torch.int32, device=gpu).cumsum(0, dtype=torch.int32)
+    slots = torch.full((n,), -1, dtype=torch.int64, device=gpu)
+    slots[rows] = torch.randperm(160, device=gpu, generator=g)[:len(rows)]
+    positions = torch.randint(0, 90, (n,), generator=g, device=gpu, dtype=torch.int32)
+    emb = RotaryPositionalEmbedding(hd, max_seq_len=90).to(gpu)
+    pools = [torch.zeros(10, gn, 16, hd, dtype=dtype, device=gpu) for _ in range(4)]
+    if rope:
+        paged_ops.rope_kv_append(torch.zeros(n, 1, hd, dtype=dtype, device=gpu), k, v, pools[0], pools[1], slots, positions,
+                                 emb.cos_emb, emb.sin_emb)
+    else:
+        paged_ops.kv_append(k, v, pools[0], pools[1], slots)
+    out = torch.full((n, 3 * hd), 7.0, dtype=dtype, device=gpu)
+    call = Append(k_new=k.data_ptr(), v_new=v.data_ptr(), new_stride_token=gn * hd, k_pool=pools[2].data_ptr(),
+                  v_pool=pools[3].data_ptr(), pool_stride_block=gn * 16 * hd, pool_stride_head=16 * hd, pool_stride_token=hd,
+                  num_blocks=10, slot_mapping=slots.data_ptr(), n_tokens=n, gn=gn, hd=hd, block_size=16,
+                  dtype=_lib.IC_DTYPE[dtype], positions=positions.data_ptr(), table_rows=90, zero_out=out.data_ptr(),
+                  zero_stride_bytes=3 * hd * k.element_size(), rows=rows.data_ptr(), n_rows=len(rows), bounds=bounds.data_ptr(),
+                  zero_row_bytes=3 * hd * k.element_size(), n_seqs=n_seqs, row_pitch=width)
+    if rope:
+        call.cos_table, call.sin_table = emb.cos_emb.data_ptr(), emb.sin_emb.data_ptr()
+    assert _lib.load().ic_append_chunks(ctypes.byref(call), _lib.current_stream_ptr(gpu)) == 0
+    assert torch.equal(pools[0], pools[2]) and torch.equal(pools[1], pools[3])
+    listed = torch.zeros(n, dtype=torch.bool, device=gpu)
+    listed[rows] = True
+    assert (out[listed] == 7).all() and not out[~listed].any()
