@@ -305,7 +305,7 @@ __global__ __launch_bounds__(NW *kWave) void paged_decode_kernel(const DecodeKP 
   }
 }
 
-// Small batches of short contexts (a few sequences of a small model, a few hundred tokens): with shares of a tile
+// Short contexts (up to about a thousand tokens, see decode_takes_pairs for the lines): with shares of a tile
 // the split above turns them into partials that a second launch merges, 8 + 5 us of which the tiles themselves take
 // two (4 sequences of up to 160 tokens, 12 heads of 64, fp32: 13.0 us, here 3.8).  Here a workgroup owns a whole pair:
 // its eight waves take the pair's tiles in turn (a wave's table entries come in one load, one per lane: at most 64
@@ -799,17 +799,34 @@ void launch_valu_main(DecodeKP &kp, hipStream_t stream) {
 //   bf16, 32 / 8 of 128, 4                    10.2 / 6.4   13.0 / 8.4   15.2 / 10.1  19.7 / 14.3  18.2 / 21.3
 //   bf16, 32 / 8 of 128, 40                   12.2 / 11.8  16.0 / 15.2  19.9 / 20.9
 //   bf16, 28 / 4 of 128, 4                    10.1 / 10.4  13.2 / 14.1  15.2 / 17.1
-// One head per pair wins throughout, the 640 pairs of 40 sequences included; the rounds are limited so that a batch
-// with a single long row among short ones, which the split balances (8-10 us at least) and a workgroup walks alone,
-// does not lose.  The limit on the pairs (512 on 256 CUs) does not follow from these figures: beyond it only the even
-// batch of 640 pairs has been measured, and no row says where the split becomes faster.  Grouped heads cost this
-// kernel vector work for each head, hence short contexts only, and none from five heads on.
-bool decode_takes_pairs(const DecodeKP &kp, int row_bytes) {
+// Larger batches, contexts of 20-64, 20-200, 17-512, 50-1 000 and 30-2 000 tokens, split / this kernel:
+//   bf16, 16 / 16 of 64, 64      19.7 / 7.4   22.1 / 10.1  30.7 / 19.3   42.0 / 31.6    67.8 / 58.1
+//   bf16, 16 / 16 of 64, 233     23.9 / 19.4  39.9 / 28.4  67.6 / 51.6   111.5 / 95.2   200.0 / 180.6
+//   bf16, 32 / 32 of 128, 64     20.6 / 18.7  34.1 / 29.0  64.0 / 56.6   110.8 / 105.2  211.6 / 197.8
+//   bf16, 32 / 32 of 128, 233    49.0 / 54.7  98.9 / 88.0  201.1 / 181.9 363.7 / 349.5  678.9 / 669.3
+//   fp32, 32 / 32 of 128, 64     31.2 / 33.5  56.8 / 55.9  112.9 / 102.9 201.7 / 193.1  393.7 / 379.8
+//   fp32, 32 / 32 of 128, 233    83.3 / 109   179 / 182    380 / 350     708 / 681
+//   bf16, 8 / 4 of 64, 233       20.0 / 11.4  22.6 / 13.6  30.2 / 20.0   41.3 / 32.5    56.5 / 56.6
+//   bf16, 16 / 8 of 128, 4       13.3 / 6.5   14.7 / 7.6   16.1 / 9.3    17.1 / 13.4    16.4 / 20.3
+//   bf16, 16 / 8 of 128, 256     21.3 / 22.9  35.7 / 33.7  68.0 / 58.9   114.3 / 106.8  204.7 / 199.2
+//   bf16, 16 / 4 of 64, 4        12.0 / 8.1   13.7 / 9.9   14.6 / 11.6   19.6 / 15.2    16.3 / 22.4
+//   bf16, 16 / 4 of 64, 256      20.7 / 18.8  23.3 / 22.8  32.2 / 30.3   44.1 / 42.2    64.5 / 66.8
+// and batches with one long row among rows of 20 tokens, which the split balances and a workgroup walks alone (1 000, 2 000):
+//   bf16, 16 / 16 of 64, 4 and 233       20.6 / 7.4, 21.0 / 10.4 and 26.7 / 18.0, 27.7 / 20.7
+//   bf16, 32 / 32 of 128, 4 and 64       16.9 / 10.9, 18.8 / 16.0 and 24.9 / 19.3, 29.3 / 30.4
+//   fp32, 32 / 32 of 128, 4              20.1 / 15.8, 25.2 / 42.3
+// So the rows a workgroup walks are limited by their bytes (a round is 128 tokens), and the pairs by theirs: tens of
+// thousands of short rows start more workgroups than the split does.  Grouped heads cost this kernel vector work for
+// each head, hence lower limits, and none from five heads on.
+bool decode_takes_pairs(const DecodeKP &kp, int hd, int row_bytes) {
   if (kp.cohort_size != 1 || kp.key_mask != nullptr || kp.min_chunk > 1 || kp.max_ctx <= 0 || kp.group > 4) return false;
   const int64_t rounds = ((int64_t)kp.max_ctx + 16 * kPairWaves - 1) / (16 * kPairWaves);
   const int64_t pairs = (int64_t)kp.n_seqs * kp.pairs_per_seq;
-  if (kp.group > 1) return rounds <= 2 && pairs <= device_cu_count();
-  return rounds <= 10 && rounds * row_bytes <= 2560 && pairs <= 2 * device_cu_count();
+  if (rounds > 16 || kp.n_seqs > 65535) return false;
+  if (kp.group == 1) return rounds * row_bytes <= 4096 && pairs * row_bytes < (rounds == 1 ? 1 << 20 : 2 << 20);
+  if (kp.group == 2) return rounds * row_bytes <= 2048 && pairs * row_bytes < 1 << 19;
+  if (hd <= 64) return rounds <= 8 && pairs <= 2 * device_cu_count();
+  return rounds <= 2 && pairs <= device_cu_count();
 }
 
 template <class E, int HD, bool APPEND>
@@ -826,9 +843,12 @@ int launch_pairs(const DecodeKP &kp, const PairAppend &rows, hipStream_t stream)
 
 template <class E, int HD>
 int launch_group(DecodeKP &kp, int dtype, const AppendRows *rows, hipStream_t stream) {
-  const bool pairs = decode_takes_pairs(kp, HD * (int)sizeof(typename E::type));
+  const bool pairs = decode_takes_pairs(kp, HD, HD * (int)sizeof(typename E::type));
   if (rows != nullptr) {  // with the append: only in one launch
-    if (!pairs || kp.n_seqs > kPairAppendRows || kp.num_blocks * kp.tiles_per_block >= (int64_t)1 << 31)
+    // (larger grids are bound by what their workgroups do: 233 sequences of 17-512 tokens, 16 heads of 64, rotary 87 us
+    // so, 54 with a launch for the append)
+    if (!pairs || kp.n_seqs > kPairAppendRows || (int64_t)kp.n_seqs * kp.pairs_per_seq > 2 * device_cu_count() ||
+        kp.num_blocks * kp.tiles_per_block >= (int64_t)1 << 31)
       return IC_ERR_UNSUPPORTED;
     PairAppend n;
     n.k_new = (const char *)rows->k_new, n.v_new = (const char *)rows->v_new;

@@ -106,10 +106,13 @@ def test_rows_that_see_each_other(gpu, dtype, rope, hn, gn, hd):
     _compare(gpu, dtype, lens, tables, slots, hn, gn, hd, block, n_blocks, rope, 3)
 
 
-def test_batches_of_64_rows_and_more(gpu):
-    for b, one in ((64, True), (65, False)):
-        wl = workloads.make_decode_workload(b, 4, 4, 64, 20, 40, dtype=torch.bfloat16, seed=b)
-        last = wl.context_lens.long() - 1
-        slots = wl.block_tables.long().gather(1, (last // 16).unsqueeze(1)).squeeze(1) * 16 + last % 16
-        _compare(gpu, torch.bfloat16, wl.context_lens.tolist(), wl.block_tables, slots, 4, 4, 64, 16, wl.k_pool.shape[0],
-                 True, b, one_launch=one)
+@pytest.mark.parametrize("b,one", [(64, True), (65, False), (300, False)])
+def test_a_row_to_every_lane_and_more(gpu, b, one):
+    wl = workloads.make_decode_workload(b, 2, 2, 64, 20, 40, dtype=torch.bfloat16, seed=b)
+    last = wl.context_lens.long() - 1
+    slots = wl.block_tables.long().gather(1, (last // 16).unsqueeze(1)).squeeze(1) * 16 + last % 16
+    tables = wl.block_tables.clone()
+    tables[3], slots[3] = tables[b - 1], slots[b - 1] - 1          # row 3 is the last row's sequence, a token earlier
+    wl.context_lens[3] = wl.context_lens[b - 1]
+    _compare(gpu, torch.bfloat16, wl.context_lens.tolist(), tables, slots, 2, 2, 64, 16, wl.k_pool.shape[0],
+             True, b, one_launch=one)
