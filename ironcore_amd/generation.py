@@ -377,6 +377,10 @@ class LanguageModel(BaseModule):
                 new_token_counts: Optional[Sequence[int]] = None):
         if labels is not None:
             raise NotImplementedError("loss computation is a training feature")
+        return self._logits(self._hidden(input_ids, kv_cache, seq_ids, attn_metadata, position_ids, new_token_counts))
+
+    def _hidden(self, input_ids, kv_cache, seq_ids, attn_metadata, position_ids, new_token_counts):
+        """What the output layer takes: [b, s, d], normed."""
         b, s = input_ids.shape
         dev = input_ids.device
         if attn_metadata is not None:
@@ -391,22 +395,29 @@ class LanguageModel(BaseModule):
         else:
             if seq_ids is None or len(seq_ids) != b:
                 raise ValueError("one cache sequence id per batch row")
-            past = [kv_cache.length(sid) for sid in seq_ids]
             # new_token_counts: row i of input_ids holds that many new tokens, the rest is padding
-            meta = kv_cache.prepare(seq_ids, s if new_token_counts is None else list(new_token_counts))
+            counts = s if new_token_counts is None else list(new_token_counts)
             attention_mask = None
-            position_ids = (torch.tensor(past, device=dev).unsqueeze(1) + torch.arange(s, device=dev).unsqueeze(0))
+            if type(kv_cache) is PagedKVCache and kv_cache.device == dev:
+                # (used on this stream only, so the host need not wait for what is still running on it)
+                meta, position_ids = kv_cache._prepare(seq_ids, counts)
+            else:
+                past = [kv_cache.length(sid) for sid in seq_ids]
+                meta = kv_cache.prepare(seq_ids, counts)
+                position_ids = (torch.tensor(past, device=dev).unsqueeze(1) + torch.arange(s, device=dev).unsqueeze(0))
+            if position_ids.shape[1] != s:   # no row is as long as input_ids
+                position_ids = position_ids[:, :1] + torch.arange(s, device=dev).unsqueeze(0)
         x = self.embedding(input_ids, position_ids)
         normed = self._native_step(x, kv_cache, meta) if s == 1 and meta is not None else None
         if normed is not None:
-            x = normed
-        else:
-            x = self.model(x, attention_mask, self.rotary_pos_emb, kv_cache=kv_cache, attn_metadata=meta)
-            x = self.output_layernorm(x)
+            return normed
+        x = self.model(x, attention_mask, self.rotary_pos_emb, kv_cache=kv_cache, attn_metadata=meta)
+        return self.output_layernorm(x)
+
+    def _logits(self, x):
         if self.config.model.untie_embed:
             return linear(x, self.output_layer.weight)
         return torch.matmul(x, self.embedding.word_embeddings.weight.transpose(0, 1))
-
 
     def _native_step(self, x, kv_cache, meta):
         """The layers and the last norm of a decode step by native calls, one a layer, or None: ``x`` [b, 1, d] are
@@ -441,6 +452,9 @@ class LanguageModel(BaseModule):
             else:
                 x, normed = got
         return normed
+
+
+_MODEL_FORWARD = LanguageModel.forward
 
 
 def sample_next(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 0,
@@ -546,12 +560,17 @@ def generate(model: LanguageModel, input_ids: torch.Tensor, max_new_tokens: int,
 
 
 def _prefill_logits(model, input_ids, prompt_lens, kv_cache, seq_ids):
-    """Logits ``[b, vocab]`` at each prompt's last token after one prefill step."""
-    if prompt_lens is None:
-        return model(input_ids, kv_cache=kv_cache, seq_ids=seq_ids)[:, -1, :]
+    """Logits ``[b, vocab]`` at each prompt's last token after one prefill step: only those, unless somebody watches
+    the model's call."""
+    b, s = input_ids.shape
+    last = None if prompt_lens is None else torch.tensor(prompt_lens, device=input_ids.device) - 1
+    rows = torch.arange(b, device=input_ids.device) if last is not None else None
+    if (_untouched(model, LanguageModel) and LanguageModel.forward is _MODEL_FORWARD and _untouched_by_anyone()
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()):
+        x = model._hidden(input_ids, kv_cache, seq_ids, None, None, prompt_lens)
+        return model._logits((x[:, -1] if last is None else x[rows, last]).contiguous())
     logits = model(input_ids, kv_cache=kv_cache, seq_ids=seq_ids, new_token_counts=prompt_lens)
-    last = torch.tensor(prompt_lens, device=input_ids.device) - 1
-    return logits[torch.arange(len(prompt_lens), device=input_ids.device), last]
+    return logits[:, -1, :] if last is None else logits[rows, last]
 
 
 def _with_prompts(tokens, s, prompt_lens):

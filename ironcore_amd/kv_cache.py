@@ -23,6 +23,7 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Iterable, Sequence
 
+import numpy as np
 import torch
 
 from .layers.attention import PagedAttentionMetadata
@@ -167,6 +168,33 @@ class PagedKVCache:
         seq.length += 1
         return blk * bs + off
 
+    def _slots_for_append(self, seq: _Sequence, n_tokens: int) -> list:
+        """Slots of the next ``n_tokens`` tokens: :meth:`_slot_for_append`, a block at a time."""
+        slots = []
+        while n_tokens > 0:
+            first = self._slot_for_append(seq)
+            more = min(n_tokens, self.block_size - first % self.block_size) - 1
+            slots.extend(range(first, first + more + 1))
+            seq.length += more
+            n_tokens -= more + 1
+        return slots
+
+    def _upload(self, arrays: dict, wait: bool) -> dict:
+        """The numpy arrays as tensors on the cache's device, in one copy from pinned memory.  Without ``wait`` the
+        copy is only ordered on the current stream."""
+        if self.device.type != "cuda":
+            return {name: torch.from_numpy(a).to(self.device) for name, a in arrays.items()}
+        starts, total = [], 0
+        for a in arrays.values():
+            starts.append(total)
+            total += -(-a.nbytes // 16) * 16
+        host = torch.empty(max(total, 16), dtype=torch.uint8, pin_memory=True)
+        for start, a in zip(starts, arrays.values()):
+            host.numpy()[start:start + a.nbytes] = a.reshape(-1).view(np.uint8)
+        there = host.to(self.device, non_blocking=not wait)
+        return {name: there[start:start + a.nbytes].view(getattr(torch, str(a.dtype))).view(a.shape)
+                for start, (name, a) in zip(starts, arrays.items())}
+
     # ---- decoding without per-step host work ---------------------------------------------
     def reserve(self, sid: int, total_length: int) -> None:
         """Give the sequence every block it needs to grow to ``total_length``
@@ -218,6 +246,15 @@ class PagedKVCache:
         ``cohort_size`` > 1 groups consecutive ``seq_ids`` into cohorts and
         records how many leading blocks each cohort's members alias (forks of
         one prompt listed next to each other), so decode streams them once."""
+        return self._prepare(seq_ids, new_tokens, cohort_size, wait=True)[0]
+
+    def _prepare(self, seq_ids, new_tokens, cohort_size=1, wait=False):
+        """:meth:`prepare` and the index int64 ``[n, longest]`` that each row of the step has in its sequence
+        (padding counted on).  Without ``wait`` the tensors are for work on the current stream."""
+        if self.device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            # (a graph would replay this step's values)
+            raise RuntimeError("the bookkeeping of a step cannot be captured: reserve() the blocks and hand the model "
+                               "attn_metadata that the device keeps up to date")
         n = len(seq_ids)
         counts = [new_tokens] * n if isinstance(new_tokens, int) else list(new_tokens)
         if len(counts) != n:
@@ -230,38 +267,34 @@ class PagedKVCache:
         need = sum(self._blocks_needed(self._seqs[sid], c) for sid, c in zip(seq_ids, counts))
         if need > self.allocator.num_free:
             raise OutOfBlocks(f"{need} KV blocks needed for this step, {self.allocator.num_free} free")
-        slots, positions = [], []
-        for sid, c in zip(seq_ids, counts):
+        slots = np.full((n, width), -1, dtype=np.int64)
+        past = np.zeros((n, 1), dtype=np.int64)
+        for i, (sid, c) in enumerate(zip(seq_ids, counts)):
             seq = self._seqs[sid]
-            start = seq.length
-            row = [self._slot_for_append(seq) for _ in range(c)]
-            slots.extend(row + [-1] * (width - c))
-            positions.extend(list(range(start, start + c)) + [0] * (width - c))
+            past[i] = seq.length
+            if c > 0:
+                slots[i, :c] = self._slots_for_append(seq, c)
+        index = past + np.arange(width)
+        there = np.arange(width) < np.asarray(counts, dtype=np.int64).reshape(n, 1)
         lens = [self._seqs[s].length for s in seq_ids]
         max_blocks = max((len(self._seqs[s].blocks) for s in seq_ids), default=1) or 1
-        table = [self._seqs[s].blocks + [0] * (max_blocks - len(self._seqs[s].blocks)) for s in seq_ids]
-        dev = self.device
-        cu = chunk_rows = None
+        table = np.zeros((n, max_blocks), dtype=np.int32)
+        for row, sid in zip(table, seq_ids):
+            row[:len(self._seqs[sid].blocks)] = self._seqs[sid].blocks
+        arrays = {"slots": slots.reshape(-1), "index": index, "table": table, "lens": np.asarray(lens, dtype=np.int32),
+                  "positions": np.where(there, index, 0).astype(np.int32).reshape(-1)}
         if ragged:
             # rows are padded to `width` ([b, width, ...] tensors); the kernels get the true bounds
             # and the layer packs the rows that exist
-            bounds = [0]
-            for c in counts:
-                bounds.append(bounds[-1] + c)
-            cu = torch.tensor(bounds, dtype=torch.int32, device=dev)
-            chunk_rows = torch.tensor([i * width + t for i, c in enumerate(counts) for t in range(c)],
-                                      dtype=torch.int64, device=dev)
-        shared = None
+            arrays["cu"] = np.cumsum([0] + counts).astype(np.int32)
+            arrays["rows"] = np.flatnonzero(there).astype(np.int64)
         if cohort_size > 1 and n > 0:
             from .paged_ops import shared_prefix_blocks
-            shared = torch.from_numpy(shared_prefix_blocks(table, lens, self.block_size, cohort_size)).to(dev)
+            arrays["shared"] = np.ascontiguousarray(
+                shared_prefix_blocks(table.tolist(), lens, self.block_size, cohort_size))
+        t = self._upload(arrays, wait)
         return PagedAttentionMetadata(
-            block_tables=torch.tensor(table, dtype=torch.int32, device=dev).view(n, max_blocks),
-            context_lens=torch.tensor(lens, dtype=torch.int32, device=dev),
-            slot_mapping=torch.tensor(slots, dtype=torch.int64, device=dev),
-            max_context_len=max(lens, default=0),
-            cu_seqlens_q=cu,
-            cohort_size=cohort_size if shared is not None else 1,
-            cohort_shared_blocks=shared,
-            positions=torch.tensor(positions, dtype=torch.int32, device=dev),
-            chunk_rows=chunk_rows, max_chunk_len=width)
+            block_tables=t["table"], context_lens=t["lens"], slot_mapping=t["slots"],
+            max_context_len=max(lens, default=0), cu_seqlens_q=t.get("cu"),
+            cohort_size=cohort_size if "shared" in t else 1, cohort_shared_blocks=t.get("shared"),
+            positions=t["positions"], chunk_rows=t.get("rows"), max_chunk_len=width), t["index"]
