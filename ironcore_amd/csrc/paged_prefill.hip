@@ -68,7 +68,6 @@ constexpr int kStageBuffers = 4;          // LDS buffers per pool: a tile is fet
 // query row walks all L keys and a chunk may be longer than its context.
 template <class M, int HD, bool SINGLE, bool MASK>
 __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const PrefillKP p) {
-  using T = typename M::T;
   constexpr int KS = HD / 16;          // k-steps of the QK contraction
   constexpr int OB = HD / 32;          // 32-wide blocks of the output head dim
   constexpr int TB = kBN / 32;         // 32-token blocks per tile
@@ -513,19 +512,26 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   both_halves(l, l_a, l_b);
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  if (my_q < C) {
-    T *orow = reinterpret_cast<T *>(p.out) + query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD;
+  // Out in whole rows of the head, CPR lanes to a row, through LDS (as the MFMA lays them out a store touches 32
+  // cache lines for 512 bytes): the tiles are done with.  16 x 512 rows behind up to 4 096, 32 heads: 372 -> 365 us.
+  __syncthreads();
+  char *const s_o = &s_k[0][0] + wave * 32 * ROWB;  // (256 rows: as many as the K buffers hold)
 #pragma unroll
-    for (int ob = 0; ob < OB; ++ob) {
+  for (int ob = 0; ob < OB; ++ob) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int d = ob * 32 + 4 * hh + 8 * j;
-        uint2 w;
-        w.x = M::pack2(o[ob][4 * j] * inv, o[ob][4 * j + 1] * inv);
-        w.y = M::pack2(o[ob][4 * j + 2] * inv, o[ob][4 * j + 3] * inv);
-        *reinterpret_cast<uint2 *>(orow + d) = w;
-      }
+    for (int j = 0; j < 4; ++j) {
+      uint2 w;
+      w.x = M::pack2(o[ob][4 * j] * inv, o[ob][4 * j + 1] * inv);
+      w.y = M::pack2(o[ob][4 * j + 2] * inv, o[ob][4 * j + 3] * inv);
+      *reinterpret_cast<uint2 *>(s_o + n * ROWB + (((ob * 4 + j) ^ swz_k(n)) << 4) + hh * 8) = w;
     }
+  }
+  constexpr int OWR = kWave / CPR;
+#pragma unroll
+  for (int i = 0; i < 32 / OWR; ++i) {
+    const int r = i * OWR + lane / CPR, chunk = lane % CPR, row = q0 + wave * 32 + r;
+    const Vec16 v = load16(s_o + r * ROWB + ((chunk ^ swz_k(r)) << 4));
+    if (row < C) store16(p.out + (query_row(p, q_lo, row) * p.out_stride_token + (int64_t)h * HD + chunk * 8) * 2, v);
   }
 }
 
