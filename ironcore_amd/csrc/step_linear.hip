@@ -133,16 +133,45 @@ struct alignas(2 * sizeof(T)) Pair {
   T a, b;
 };
 
+// What the end of a product needs beside its sums, fetched before them: the bias of two neighbouring columns (and of
+// their gates), and where a row's new keys and values go.
+struct Extras {
+  float a = 0.f, b = 0.f, gate_a = 0.f, gate_b = 0.f;
+};
+struct Place {
+  int64_t slot = -1, angle = 0;  // pool slot; first element of the row's rotary tables
+};
+
+template <class E>
+__device__ __forceinline__ Extras fetch_extras(const StepKP &p, int col) {
+  Extras x;
+  const int mat = col >= p.n[0] ? 1 : 0;
+  const typename E::type *bias = reinterpret_cast<const typename E::type *>(p.bias[mat]);
+  if (bias == nullptr) return x;
+  bias += col - (mat ? p.n[0] : 0);
+  x.a = static_cast<float>(bias[0]), x.b = static_cast<float>(bias[1]);
+  if (p.gated) x.gate_a = static_cast<float>(bias[p.n[0] / 2]), x.gate_b = static_cast<float>(bias[p.n[0] / 2 + 1]);
+  return x;
+}
+
+__device__ __forceinline__ Place fetch_place(const StepKP &p, int row) {
+  Place at;
+  if (p.slots == nullptr) return at;
+  at.slot = p.slots[row];
+  if (p.cos_table == nullptr) return at;
+  const int64_t pos = p.positions[row];
+  at.angle = (pos < 0 ? 0 : pos >= p.table_rows ? p.table_rows - 1 : pos) * (p.hd / 2);
+  return at;
+}
+
 // Two neighbouring columns of the projections [q | k | v] of row `row`, rotated and stored where they belong.
 template <class E>
-__device__ __forceinline__ void store_qkv(const StepKP &p, int row, int col, float a, float b) {
+__device__ __forceinline__ void store_qkv(const StepKP &p, int row, int col, float a, float b, const Place &place) {
   using T = typename E::type;
   const int q_cols = p.hn * p.hd, kv_cols = p.gn * p.hd;
   const bool value = col >= q_cols + kv_cols;
   if (p.cos_table != nullptr && !value) {
-    int64_t pos = p.positions[row];
-    pos = pos < 0 ? 0 : pos >= p.table_rows ? p.table_rows - 1 : pos;
-    const int64_t at = pos * (p.hd / 2) + (col % p.hd) / 2;
+    const int64_t at = place.angle + (col % p.hd) / 2;
     rotate_pair(a, b, p.cos_table[at], p.sin_table[at], a, b);
   }
   const Pair<T> v{E::narrow(a), E::narrow(b)};
@@ -150,7 +179,7 @@ __device__ __forceinline__ void store_qkv(const StepKP &p, int row, int col, flo
     *reinterpret_cast<Pair<T> *>(reinterpret_cast<T *>(p.out) + row * p.out_stride + col) = v;
     return;
   }
-  const int64_t slot = p.slots[row];
+  const int64_t slot = place.slot;
   if (slot < 0 || slot >= p.num_slots) return;
   const int64_t blk = (p.num_slots >> 32) != 0 ? slot / p.block_size : (uint32_t)slot / (uint32_t)p.block_size;
   const int at = col - q_cols - (value ? kv_cols : 0);
@@ -161,19 +190,12 @@ __device__ __forceinline__ void store_qkv(const StepKP &p, int row, int col, flo
 // Two neighbouring columns of a row, their sums complete but for the bias: bias, activation (with the gate that
 // belongs to a feature), rotation, and the store.  `col` counts over both matrices, or over the features.
 template <class E>
-__device__ __forceinline__ void finish_pair(const StepKP &p, int row, int col, float a, float b, float ga, float gb) {
+__device__ __forceinline__ void finish_pair(const StepKP &p, int row, int col, float a, float b, float ga, float gb,
+                                            const Extras &x, const Place &place) {
   using T = typename E::type;
-  const int mat = col >= p.n[0] ? 1 : 0;
-  const T *bias = reinterpret_cast<const T *>(p.bias[mat]);
-  if (bias != nullptr) {
-    bias += col - (mat ? p.n[0] : 0);
-    a += static_cast<float>(bias[0]), b += static_cast<float>(bias[1]);
-  }
+  a += x.a, b += x.b;
   if (p.gated) {
-    if (bias != nullptr) {
-      bias += p.n[0] / 2;
-      ga += static_cast<float>(bias[0]), gb += static_cast<float>(bias[1]);
-    }
+    ga += x.gate_a, gb += x.gate_b;
     if (p.act == IC_ACT_SWIGLU) {
       a = a * sigmoid(a) * ga, b = b * sigmoid(b) * gb;
     } else {
@@ -183,7 +205,7 @@ __device__ __forceinline__ void finish_pair(const StepKP &p, int row, int col, f
     a = activate(p.act, a), b = activate(p.act, b);
   }
   if (p.slots != nullptr)
-    store_qkv<E>(p, row, col, a, b);
+    store_qkv<E>(p, row, col, a, b, place);
   else
     *reinterpret_cast<Pair<T> *>(reinterpret_cast<T *>(p.out) + row * p.out_stride + col) =
         Pair<T>{E::narrow(a), E::narrow(b)};
@@ -237,6 +259,16 @@ __global__ __launch_bounds__(kStepThreads) void step_linear_kernel(const StepKP 
 #pragma unroll
     for (int t = 0; t < MT; ++t) xv[d][t] = load16(x[t] + (int64_t)step * 64);
   };
+  // The sums' end: a thread takes the same two columns of every row it has (widths are powers of two).
+  const int cols = gated ? TN / 2 : TN, end = gated ? half : n;
+  const int before = mat ? p.n[0] : 0;
+  const int at = 2 * (threadIdx.x % (cols / 2)), first_row = threadIdx.x / (cols / 2), row_step = kStepThreads / (cols / 2);
+  Extras extras;
+  Place place;
+  if constexpr (!SPLIT) {  // (on their way with the first steps)
+    if (n0 + at < end) extras = fetch_extras<E>(p, before + n0 + at);
+    if (first_row < p.m) place = fetch_place(p, first_row);
+  }
   f32x4_t acc[NB][MT];
 #pragma unroll
   for (int j = 0; j < NB; ++j)
@@ -271,8 +303,6 @@ __global__ __launch_bounds__(kStepThreads) void step_linear_kernel(const StepKP 
       if (d < mine) add(d);
   }
   // ---- the waves' sums, 16 rows of x at a time, two columns a thread --------------------------
-  const int cols = gated ? TN / 2 : TN, end = gated ? half : n;
-  const int before = mat ? p.n[0] : 0;
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     if (t > 0) __syncthreads();
@@ -282,8 +312,8 @@ __global__ __launch_bounds__(kStepThreads) void step_linear_kernel(const StepKP 
 #pragma unroll
       for (int j = 0; j < NB; ++j) to[r * NB + j] = acc[j][t][r];
     __syncthreads();
-    for (int e = threadIdx.x; e < 16 * (cols / 2); e += kStepThreads) {
-      const int r = e / (cols / 2), at = 2 * (e % (cols / 2)), row = t * 16 + r;
+    for (int r = first_row; r < 16; r += row_step) {
+      const int row = t * 16 + r;
       if (row >= p.m || n0 + at >= end) continue;
       auto total = [&](int column, float &a, float &b) {
         a = b = 0.f;
@@ -300,7 +330,7 @@ __global__ __launch_bounds__(kStepThreads) void step_linear_kernel(const StepKP 
                                     at) = make_float2(a, b);
       } else {
         if (gated) total(TN / 2 + at, ga, gb);
-        finish_pair<E>(p, row, before + n0 + at, a, b, ga, gb);
+        finish_pair<E>(p, row, before + n0 + at, a, b, ga, gb, extras, row == first_row ? place : fetch_place(p, row));
       }
     }
   }
@@ -334,11 +364,13 @@ __global__ __launch_bounds__(kFinishThreads) void step_finish_kernel(const StepK
   if (col >= cols) return;
   const float *at = p.partials + (int64_t)row * total + col;
   const int64_t pitch = (int64_t)p.m * total;
+  const Extras low = fetch_extras<E>(p, col), high = fetch_extras<E>(p, col + 2);
+  const Place place = fetch_place(p, row);
   const float4 v = sum_partials(at, pitch, p.splits);
   float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
   if (p.gated) g = sum_partials(at + cols, pitch, p.splits);
-  finish_pair<E>(p, row, col, v.x, v.y, g.x, g.y);
-  finish_pair<E>(p, row, col + 2, v.z, v.w, g.z, g.w);
+  finish_pair<E>(p, row, col, v.x, v.y, g.x, g.y, low, place);
+  finish_pair<E>(p, row, col + 2, v.z, v.w, g.z, g.w, high, place);
 }
 
 constexpr int kRowThreads = 1024;
