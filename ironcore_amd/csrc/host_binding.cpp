@@ -198,11 +198,11 @@ struct NewRows {
   }
 };
 
-// Append with the keys rotated on their way; q_out == nullptr: the query is left alone.
+// Append with the keys rotated on their way, the query into a tensor of its own.
 bool rope_append(const Tensor &key, const Tensor &value, const Pool &p, const Tensor &slots, const Rope &r, int64_t n,
                  void *q_out, const void *q, int64_t q_stride, int64_t hn, void *stream) {
   return made("ic_rope_kv_append_to",
-              ic_rope_kv_append_to(q_out, hn * p.hd, q_out ? q : nullptr, q_stride, (int)hn, key.data_ptr(),
+              ic_rope_kv_append_to(q_out, hn * p.hd, q, q_stride, (int)hn, key.data_ptr(),
                                    value.data_ptr(), row_stride4(key), const_cast<void *>(p.k),
                                    const_cast<void *>(p.v), p.sb, p.sh, p.st, slots.data_ptr<int64_t>(), r.positions,
                                    r.cos, r.sin, r.rows, n, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream));
@@ -225,9 +225,9 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
   const void *q = query.data_ptr();
   int64_t q_stride = row_stride4(query);
   if (!rows16(q, q_stride, in.hn * p.hd, query.element_size())) return c10::nullopt;
+  const Tensor out = at::empty({in.b, 1, in.hn * p.hd}, query.options());
   if (cohort == 1 && rows16(key.data_ptr(), row_stride4(key), p.gn * p.hd, key.element_size()) &&
       rows16(value.data_ptr(), row_stride4(value), p.gn * p.hd, key.element_size())) {
-    const Tensor out = at::empty({in.b, 1, in.hn * p.hd}, query.options());
     ic_decode_append_call c = {};
     c.out = out.data_ptr(), c.out_stride_seq = in.hn * p.hd;
     c.q = q, c.q_stride_seq = q_stride;
@@ -251,7 +251,6 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
   } else if (!append_rows(key.data_ptr(), value.data_ptr(), row_stride4(key), p, slots, in.b, (void *)stream)) {
     return c10::nullopt;
   }
-  const Tensor out = at::empty({in.b, 1, in.hn * p.hd}, query.options());
   if (!decode(out, q, q_stride, p, in.b, in.hn, d, (void *)stream)) return c10::nullopt;
   return out;
 }
