@@ -81,11 +81,16 @@ bool table(const Tensor &t, int64_t rows, int64_t device) {
 bool rows3(const Tensor &t, int64_t heads, int64_t hd) {
   return t.dim() == 3 && t.size(1) == heads && t.size(2) == hd && t.stride(2) == 1 && t.stride(1) == hd;
 }
-// [b, s, heads, hd] that is [b*s, heads, hd] rows at one stride (that of a dimension of size 1 says nothing: half of a
-// projection's row, as a decode step hands it over, keeps the half's length there).
+// [b, s, heads, hd] that is [b*s, heads, hd] rows at one stride.
 bool rows4(const Tensor &t, int64_t b, int64_t s, int64_t heads, int64_t hd) {
   return t.dim() == 4 && t.size(0) == b && t.size(1) == s && t.size(2) == heads && t.size(3) == hd &&
-         t.stride(3) == 1 && t.stride(2) == hd && (b == 1 || s == 1 || t.stride(0) == s * t.stride(1));
+         t.stride(3) == 1 && t.stride(2) == hd && (b == 1 || t.stride(0) == s * t.stride(1));
+}
+// The same where one row a sequence may come at any stride.  With s == 1 the stride of that dimension says nothing (half of a
+// projection's row, as a decode step hands it over, keeps the half's length there).
+bool step_rows4(const Tensor &t, int64_t b, int64_t s, int64_t heads, int64_t hd) {
+  return rows4(t, b, s, heads, hd) || (s == 1 && t.dim() == 4 && t.size(0) == b && t.size(1) == 1 && t.size(2) == heads &&
+                                       t.size(3) == hd && t.stride(3) == 1 && t.stride(2) == hd);
 }
 int64_t row_stride4(const Tensor &t) { return t.size(1) > 1 ? t.stride(1) : t.stride(0); }
 
@@ -192,7 +197,7 @@ struct NewRows {
           int64_t device) {
     if (query.dim() != 4) return;
     b = query.size(0), s = query.size(1), hn = query.size(2);
-    ok = rows4(query, b, s, hn, p.hd) && rows4(key, b, s, p.gn, p.hd) && rows4(value, b, s, p.gn, p.hd) &&
+    ok = step_rows4(query, b, s, hn, p.hd) && step_rows4(key, b, s, p.gn, p.hd) && step_rows4(value, b, s, p.gn, p.hd) &&
          row_stride4(key) == row_stride4(value) && query.scalar_type() == type && key.scalar_type() == type &&
          value.scalar_type() == type && on(query, device) && on(key, device) && on(value, device) && b * s > 0;
   }
@@ -357,7 +362,7 @@ OptTensor dense_as_laid(const Tensor &query, const Tensor &key, const Tensor &va
                         int64_t device, void *stream) {
   const Pool p(key.permute({0, 2, 1, 3}), value.permute({0, 2, 1, 3}), device);
   const int64_t b = query.size(0), s = query.size(1), hn = query.size(2);
-  if (!p.ok || !p.attends() || p.nb != b || hn % p.gn != 0 || !rows4(query, b, s, hn, p.hd) || !on(query, device) ||
+  if (!p.ok || !p.attends() || p.nb != b || hn % p.gn != 0 || !step_rows4(query, b, s, hn, p.hd) || !on(query, device) ||
       query.scalar_type() != key.scalar_type() || (b == 1 && p.sb < p.bs * p.st))
     return c10::nullopt;
   const Tensor out = at::empty({b, s, hn * p.hd}, query.options());
@@ -380,7 +385,8 @@ OptTensor dense_as_laid(const Tensor &query, const Tensor &key, const Tensor &va
 }
 
 // The dense call: query [b, sq, hn, hd] on key / value [b, sk, gn, hd].  Tensors that do not lie as the kernel walks
-// them are copied: a query whose rows are not one stride apart, keys and values with strides of their own (a rotary
+// them are copied: a query whose rows are not one stride apart, or, one row a sequence, at a stride that the kernel does
+// not take (one row for the whole batch, rows at an odd distance), keys and values with strides of their own (a rotary
 // model rotates the keys into a tensor of their own and leaves the values a slice of the projection).
 OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, bool causal, const OptTensor &bits,
                 const OptTensor &lists, int64_t mask_seqs, int64_t mask_heads, double scale, int64_t device,
@@ -388,7 +394,11 @@ OptTensor dense(const Tensor &query, const Tensor &key, const Tensor &value, boo
   if (query.dim() != 4 || key.dim() != 4 || value.dim() != 4 || key.size(1) == 0 || query.size(1) == 0)
     return c10::nullopt;
   const DenseMask m{causal, bits, lists, mask_seqs, mask_heads};
-  const Tensor q = rows4(query, query.size(0), query.size(1), query.size(2), query.size(3)) ? query : row_major(query);
+  const int64_t b = query.size(0), s = query.size(1), hn = query.size(2), hd = query.size(3);
+  const bool laid = rows4(query, b, s, hn, hd) ||
+                    (step_rows4(query, b, s, hn, hd) &&
+                     rows16(query.data_ptr(), row_stride4(query), hn * hd, query.element_size()));
+  const Tensor q = laid ? query : row_major(query);
   OptTensor out = dense_as_laid(q, key, value, m, scale, device, (void *)stream);
   if (!out.has_value()) {
     const Tensor k = row_major(key), v = row_major(value);

@@ -122,3 +122,28 @@ def test_unpacking(gpu):
     got = packed.bytes()
     assert torch.cuda.max_memory_allocated() - before <= 4 * m.numel()
     assert got.dtype == torch.uint8 and torch.equal(got, m.to(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype,precision", DTYPES)
+@pytest.mark.parametrize("hn,gn,hd", [(4, 2, 64), (6, 6, 32), (8, 2, 128)])
+@pytest.mark.parametrize("kind", ["none", "documents"])
+@pytest.mark.parametrize("layout", ["one_for_all", "odd_distance", "odd_start", "last_of_a_row"])
+def test_one_query_row_a_sequence(gpu, dtype, precision, hn, gn, hd, kind, layout):
+    """Rows of a query [b, 1, hn, hd] wherever they lie: one for the whole batch (stride 0), at a distance or a start
+    that is no multiple of 16 bytes, and at one that is."""
+    b, sk = 3, 77
+    g = torch.Generator().manual_seed(hn + hd)
+    k, v = (torch.randn(b, sk, gn, hd, generator=g).to(dtype) for _ in range(2))
+    if layout == "one_for_all":
+        q = torch.randn(1, 1, hn, hd, generator=g).to(dtype).to(gpu).expand(b, 1, hn, hd)
+    elif layout == "odd_distance":
+        q = torch.randn(b, hn * hd + 2, generator=g).to(dtype).to(gpu)[:, :hn * hd].unflatten(1, (1, hn, hd))
+    elif layout == "odd_start":
+        q = torch.randn(b, hn * hd + 8, generator=g).to(dtype).to(gpu)[:, 1:hn * hd + 1].unflatten(1, (1, hn, hd))
+    else:
+        q = torch.randn(b, 5, hn, hd, generator=g).to(dtype).to(gpu)[:, -1:]
+    mask = _mask(kind, b, 1, sk, gpu)
+    got = _layer(hn, gn, hd, precision)(q, k.to(gpu), v.to(gpu), mask)
+    cpu_mask = None if mask is None else mask.cpu()
+    hold(got, dense_attention(q.cpu(), k, v, cpu_mask),
+         dense_attention(q.cpu().double(), k.double(), v.double(), cpu_mask), dtype, 1 if mask is not None else sk, layout)
