@@ -188,7 +188,7 @@ class PagedKVCache:
         for a in arrays.values():
             starts.append(total)
             total += -(-a.nbytes // 16) * 16
-        host = torch.empty(max(total, 16), dtype=torch.uint8, pin_memory=True)
+        host = torch.empty(max(total, 16), dtype=torch.uint8, device="cpu", pin_memory=True)  # (whatever the default device)
         for start, a in zip(starts, arrays.values()):
             host.numpy()[start:start + a.nbytes] = a.reshape(-1).view(np.uint8)
         there = host.to(self.device, non_blocking=not wait)

@@ -94,3 +94,23 @@ def test_capture_of_the_bookkeeping_is_refused(gpu):
         ids.add(0)
     assert before == (cache.length(sid), cache.blocks(sid))
     assert torch.isfinite(model(ids[:, :1], kv_cache=cache, seq_ids=[sid])).all()
+
+
+@torch.no_grad()
+def test_under_a_default_device(gpu):
+    """The staging memory is the host's, whatever device torch's constructors take by default."""
+    model = _model(gpu, torch.float32, False)
+    ids = torch.randint(0, 1000, (2, 9), generator=torch.Generator().manual_seed(1)).to(gpu)
+
+    def run():
+        cache = PagedKVCache(2, 8, 16, 2, 64, torch.float32, gpu)
+        sids = [cache.add_sequence() for _ in range(2)]
+        first = model(ids, kv_cache=cache, seq_ids=sids)
+        meta = cache.prepare(sids, [3, 1])
+        return first, model(ids[:, :1], kv_cache=cache, seq_ids=sids), meta
+    want = run()
+    with torch.device(gpu):
+        got = run()
+    _same(got[2], want[2])
+    for a, b in zip(got[:2], want[:2]):                     # (under a function mode the modules run, not the native step)
+        assert ((a - b).norm() / b.norm()).item() <= 2e-6   # sums of 256 products in other orders
