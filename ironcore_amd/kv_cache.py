@@ -21,6 +21,7 @@ never reads anything back from the GPU.
 from __future__ import annotations
 
 from dataclasses import dataclass, field
+from operator import index
 from typing import Iterable, Sequence
 
 import numpy as np
@@ -256,7 +257,8 @@ class PagedKVCache:
             raise RuntimeError("the bookkeeping of a step cannot be captured: reserve() the blocks and hand the model "
                                "attn_metadata that the device keeps up to date")
         n = len(seq_ids)
-        counts = [new_tokens] * n if isinstance(new_tokens, int) else list(new_tokens)
+        # (whole numbers of any kind: a tensor's elements, numpy's, truth values)
+        counts = [int(index(c)) for c in ([new_tokens] * n if isinstance(new_tokens, int) else new_tokens)]
         if len(counts) != n:
             raise ValueError("one new-token count per sequence")
         width = max(counts) if counts else 0
@@ -274,15 +276,15 @@ class PagedKVCache:
             past[i] = seq.length
             if c > 0:
                 slots[i, :c] = self._slots_for_append(seq, c)
-        index = past + np.arange(width)
+        row_index = past + np.arange(width)
         there = np.arange(width) < np.asarray(counts, dtype=np.int64).reshape(n, 1)
         lens = [self._seqs[s].length for s in seq_ids]
         max_blocks = max((len(self._seqs[s].blocks) for s in seq_ids), default=1) or 1
         table = np.zeros((n, max_blocks), dtype=np.int32)
         for row, sid in zip(table, seq_ids):
             row[:len(self._seqs[sid].blocks)] = self._seqs[sid].blocks
-        arrays = {"slots": slots.reshape(-1), "index": index, "table": table, "lens": np.asarray(lens, dtype=np.int32),
-                  "positions": np.where(there, index, 0).astype(np.int32).reshape(-1)}
+        arrays = {"slots": slots.reshape(-1), "index": row_index, "table": table, "lens": np.asarray(lens, dtype=np.int32),
+                  "positions": np.where(there, row_index, 0).astype(np.int32).reshape(-1)}
         if ragged:
             # rows are padded to `width` ([b, width, ...] tensors); the kernels get the true bounds
             # and the layer packs the rows that exist

@@ -299,3 +299,23 @@ def test_masks_built_under_inference_mode_and_the_mask_cache_stays_small():
     del masks, m, again
     gc.collect()
     assert len(attention_module._MASK_CLASSES) == 0
+
+
+@pytest.mark.parametrize("given", [[3, 5], (3, 5), torch.tensor([3, 5]), torch.tensor([3, 5], dtype=torch.int32),
+                                   [torch.tensor(3), 5]], ids=str)
+def test_prepare_takes_counts_of_any_whole_number_type(given):
+    metas = []
+    for counts in ([3, 5], given):
+        cache = PagedKVCache(1, 8, 16, 1, 32, torch.float32, "cpu")
+        ids = [cache.add_sequence() for _ in range(2)]
+        metas.append(cache.prepare(ids, counts))
+        assert [cache.length(s) for s in ids] == [3, 5] and all(type(cache.length(s)) is int for s in ids)
+    for name in ("block_tables", "context_lens", "slot_mapping", "cu_seqlens_q", "positions", "chunk_rows"):
+        assert torch.equal(getattr(metas[0], name), getattr(metas[1], name)), name
+
+
+def test_prepare_takes_truth_values_as_counts():
+    cache = PagedKVCache(1, 8, 16, 1, 32, torch.float32, "cpu")
+    ids = [cache.add_sequence() for _ in range(2)]
+    assert cache.prepare(ids, [True, False]).context_lens.tolist() == [1, 0]
+    assert cache.prepare(ids, True).context_lens.tolist() == [2, 1]
