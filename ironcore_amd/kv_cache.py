@@ -261,6 +261,8 @@ class PagedKVCache:
         counts = [int(index(c)) for c in ([new_tokens] * n if isinstance(new_tokens, int) else new_tokens)]
         if len(counts) != n:
             raise ValueError("one new-token count per sequence")
+        if any(c < 0 for c in counts):
+            raise ValueError("a sequence cannot have a negative number of new tokens")
         width = max(counts) if counts else 0
         ragged = any(c != width for c in counts)
         if ragged and cohort_size > 1:

@@ -319,3 +319,13 @@ def test_prepare_takes_truth_values_as_counts():
     ids = [cache.add_sequence() for _ in range(2)]
     assert cache.prepare(ids, [True, False]).context_lens.tolist() == [1, 0]
     assert cache.prepare(ids, True).context_lens.tolist() == [2, 1]
+
+
+@pytest.mark.parametrize("counts", [[-1, 2], [2, -1], [-2, -2], -1])
+def test_prepare_refuses_negative_counts(counts):
+    """The bounds of the packed chunks would start below 0, and the kernels read the row list there."""
+    cache = PagedKVCache(1, 8, 16, 1, 32, torch.float32, "cpu")
+    ids = [cache.add_sequence() for _ in range(2)]
+    with pytest.raises(ValueError, match="negative"):
+        cache.prepare(ids, counts)
+    assert [cache.length(s) for s in ids] == [0, 0] and cache.allocator.num_free == 8
