@@ -398,7 +398,8 @@ class LanguageModel(BaseModule):
             # new_token_counts: row i of input_ids holds that many new tokens, the rest is padding
             counts = s if new_token_counts is None else list(new_token_counts)
             attention_mask = None
-            if type(kv_cache) is PagedKVCache and kv_cache.device == dev:
+            if (type(kv_cache) is PagedKVCache and kv_cache.device == dev and "prepare" not in kv_cache.__dict__
+                    and PagedKVCache.prepare is _OWN_PREPARE):
                 # (used on this stream only, so the host need not wait for what is still running on it)
                 meta, position_ids = kv_cache._prepare(seq_ids, counts)
             else:
@@ -455,6 +456,7 @@ class LanguageModel(BaseModule):
 
 
 _MODEL_FORWARD = LanguageModel.forward
+_OWN_PREPARE = PagedKVCache.prepare
 
 
 def sample_next(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 0,

@@ -114,3 +114,23 @@ def test_under_a_default_device(gpu):
     _same(got[2], want[2])
     for a, b in zip(got[:2], want[:2]):                     # (under a function mode the modules run, not the native step)
         assert ((a - b).norm() / b.norm()).item() <= 2e-6   # sums of 256 products in other orders
+
+
+@pytest.mark.parametrize("where", ["instance", "class"])
+@torch.no_grad()
+def test_a_prepare_of_the_users_own_is_called(gpu, monkeypatch, where):
+    model = _model(gpu, torch.float32, False)
+    cache = PagedKVCache(2, 8, 16, 2, 64, torch.float32, gpu)
+    sid, calls, own = cache.add_sequence(), [], PagedKVCache.prepare
+
+    def prepare(self, seq_ids, new_tokens, *rest):
+        calls.append(new_tokens)
+        return own(self, seq_ids, new_tokens, *rest)
+    if where == "class":
+        monkeypatch.setattr(PagedKVCache, "prepare", prepare)
+    else:
+        cache.prepare = lambda *args: prepare(cache, *args)
+    ids = torch.randint(0, 1000, (1, 9)).to(gpu)
+    model(ids, kv_cache=cache, seq_ids=[sid])
+    model(ids[:, :1], kv_cache=cache, seq_ids=[sid])
+    assert calls == [9, 1]
