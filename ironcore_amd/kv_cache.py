@@ -86,9 +86,9 @@ class PagedKVCache:
         self.num_layers = num_layers
         self.num_blocks = num_blocks
         self.block_size = block_size
-        self.device = torch.device(device)
         shape = (num_layers, num_blocks, num_kv_heads, block_size, head_dim)
-        self.k_pools = torch.zeros(shape, dtype=dtype, device=self.device)
+        self.k_pools = torch.zeros(shape, dtype=dtype, device=torch.device(device))
+        self.device = self.k_pools.device    # with its index, whatever the spelling
         self.v_pools = torch.zeros(shape, dtype=dtype, device=self.device)
         self.allocator = BlockAllocator(num_blocks)
         self._seqs: dict[int, _Sequence] = {}

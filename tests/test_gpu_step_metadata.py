@@ -134,3 +134,14 @@ def test_a_prepare_of_the_users_own_is_called(gpu, monkeypatch, where):
     model(ids, kv_cache=cache, seq_ids=[sid])
     model(ids[:, :1], kv_cache=cache, seq_ids=[sid])
     assert calls == [9, 1]
+
+
+@torch.no_grad()
+def test_a_device_without_an_index(gpu, monkeypatch):
+    """A cache on "cuda" is on the current GPU, so a model's step does not wait for the upload of its metadata."""
+    model = _model(gpu, torch.float32, False)
+    cache, waits, upload = PagedKVCache(2, 8, 16, 2, 64, torch.float32, "cuda"), [], PagedKVCache._upload
+    monkeypatch.setattr(PagedKVCache, "_upload", lambda self, arrays, wait: (waits.append(wait), upload(self, arrays, wait))[1])
+    ids = torch.randint(0, 1000, (1, 9)).to(gpu)
+    model(ids, kv_cache=cache, seq_ids=[cache.add_sequence()])
+    assert cache.device == cache.k_pools.device == ids.device and waits == [False]
