@@ -552,9 +552,10 @@ int ic_step_linear(const ic_step_linear_call *call, void *stream);
 
 /*
  * The append of a step's chunks in one launch: ic_kv_append, or with cos_table and
- * sin_table ic_rope_kv_append_to without queries, and with rows not NULL
+ * sin_table ic_rope_kv_append_to without queries, and with zero_out not NULL
  * ic_zero_unlisted_rows (zero_out, zero_stride_bytes, zero_row_bytes, rows, n_rows, bounds,
- * n_seqs, row_pitch) beside it.
+ * n_seqs, row_pitch) beside it, also where there is no token to append (n_tokens 0) or no
+ * row that a chunk holds (n_rows 0: rows may be NULL then).
  */
 typedef struct ic_append_call {
   const void *k_new, *v_new;

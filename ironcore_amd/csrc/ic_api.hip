@@ -620,7 +620,7 @@ static int zero_rows(void *out, int64_t out_stride_bytes, int row_bytes, const i
   if (n_seqs < 0 || row_pitch < 0 || row_bytes <= 0 || n_rows < 0 || out_stride_bytes < row_bytes)
     return IC_ERR_BAD_SHAPE;
   if (n_seqs == 0 || row_pitch == 0) return IC_OK;
-  if (!out || !rows || !bounds) return IC_ERR_NULL_POINTER;
+  if (!out || !bounds) return IC_ERR_NULL_POINTER;
   if (!aligned16(out) || out_stride_bytes % 16 != 0 || row_bytes % 16 != 0) return IC_ERR_ALIGNMENT;
   z.out = static_cast<char *>(out), z.stride_bytes = out_stride_bytes, z.chunks = row_bytes / 16;
   z.rows = rows, z.n_rows = n_rows, z.bounds = bounds;
@@ -631,6 +631,7 @@ static int zero_rows(void *out, int64_t out_stride_bytes, int row_bytes, const i
 int ic_zero_unlisted_rows(void *out, int64_t out_stride_bytes, int row_bytes, const int64_t *rows, int64_t n_rows,
                           const int32_t *bounds, int n_seqs, int row_pitch, void *stream) {
   ic::ZeroRows z;
+  if (n_seqs > 0 && row_pitch > 0 && out && !rows) return IC_ERR_NULL_POINTER;
   if (const int rc = zero_rows(out, out_stride_bytes, row_bytes, rows, n_rows, bounds, n_seqs, row_pitch, z); rc != IC_OK)
     return rc;
   return z.total == 0 ? IC_OK : ic::launch_zero_unlisted_rows(z, static_cast<hipStream_t>(stream));
@@ -645,7 +646,15 @@ int ic_append_chunks(const ic_append_call *call, void *stream) {
   if (const int rc = check_pool(c.pool_stride_block, c.pool_stride_head, c.pool_stride_token, c.gn, c.hd, c.block_size,
                                 c.num_blocks, es))
     return rc;
-  if (c.n_tokens == 0) return IC_OK;
+  ic::RopeAppendArgs a = {};
+  if (c.zero_out != nullptr || c.rows != nullptr) {  // rows to zero, also where no token is appended or no row is listed
+    if (c.rows == nullptr && c.n_rows != 0) return IC_ERR_NULL_POINTER;
+    const int rc = zero_rows(c.zero_out, c.zero_stride_bytes, c.zero_row_bytes, c.rows, c.n_rows, c.bounds, c.n_seqs,
+                             c.row_pitch, a.append.zero);
+    if (rc != IC_OK) return rc;
+  }
+  if (c.n_tokens == 0)
+    return a.append.zero.total == 0 ? IC_OK : ic::launch_zero_unlisted_rows(a.append.zero, static_cast<hipStream_t>(stream));
   if (!c.k_new || !c.v_new || !c.k_pool || !c.v_pool || !c.slot_mapping ||
       (c.cos_table != nullptr) != (c.sin_table != nullptr) || (c.cos_table && !c.positions))
     return IC_ERR_NULL_POINTER;
@@ -653,17 +662,11 @@ int ic_append_chunks(const ic_append_call *call, void *stream) {
   if (!aligned16(c.k_new) || !aligned16(c.v_new) || !aligned16(c.k_pool) || !aligned16(c.v_pool) ||
       !stride16(c.new_stride_token, es) || !aligned16(c.cos_table) || !aligned16(c.sin_table))
     return IC_ERR_ALIGNMENT;
-  ic::RopeAppendArgs a = {};
   a.append.k_new = c.k_new, a.append.v_new = c.v_new, a.append.new_stride_token = c.new_stride_token;
   a.append.k_pool = c.k_pool, a.append.v_pool = c.v_pool;
   a.append.pool = {c.pool_stride_block, c.pool_stride_head, c.pool_stride_token, c.num_blocks, c.block_size};
   a.append.slot_mapping = c.slot_mapping, a.append.n_tokens = c.n_tokens;
   a.append.gn = c.gn, a.append.hd = c.hd, a.append.dtype = c.dtype;
-  if (c.rows != nullptr) {
-    const int rc = zero_rows(c.zero_out, c.zero_stride_bytes, c.zero_row_bytes, c.rows, c.n_rows, c.bounds, c.n_seqs,
-                             c.row_pitch, a.append.zero);
-    if (rc != IC_OK) return rc;
-  }
   if (c.cos_table == nullptr) return ic::launch_kv_append(a.append, static_cast<hipStream_t>(stream));
   a.positions = c.positions, a.cos_table = c.cos_table, a.sin_table = c.sin_table, a.table_rows = c.table_rows;
   return ic::launch_rope_kv_append(a, static_cast<hipStream_t>(stream));

@@ -119,3 +119,43 @@ def test_append_and_zeroing(gpu, dtype, n_seqs, width, gn, hd, rope):
     listed = torch.zeros(n, dtype=torch.bool, device=gpu)
     listed[rows] = True
     assert (out[listed] == 7).all() and not out[~listed].any()
+
+
+def _padded(gpu, n_seqs, width, lens):
+    """(a padded output to zero, the rows that exist, their bounds, which rows those are)"""
+    rows = torch.tensor([i * width + t for i, c in enumerate(lens) for t in range(c)], dtype=torch.int64, device=gpu)
+    bounds = torch.tensor([0] + list(lens), dtype=torch.int32, device=gpu).cumsum(0, dtype=torch.int32)
+    listed = torch.zeros(n_seqs * width, dtype=torch.bool, device=gpu)
+    listed[rows] = True
+    return torch.full((n_seqs * width, 72), 7.0, dtype=torch.bfloat16, device=gpu), rows, bounds, listed
+
+
+@pytest.mark.parametrize("width,lens", [(1, (0, 1, 0)), (5, (5, 0, 2)), (40, (0, 0, 0)), (1200, (1200, 3, 700))])
+def test_zeroing_alone(gpu, width, lens):
+    """The entry point without an append; rows wider than what is zeroed keep the rest."""
+    out, rows, bounds, listed = _padded(gpu, len(lens), width, lens)
+    rows = torch.cat([rows, rows.new_full((1,), -5)])         # (an address for the list without entries)
+    assert _lib.load().ic_zero_unlisted_rows(out.data_ptr(), 144, 128, rows.data_ptr(), len(rows) - 1, bounds.data_ptr(),
+                                             len(lens), width, _lib.current_stream_ptr(gpu)) == 0
+    assert (out[listed] == 7).all() and not out[~listed][:, :64].any() and (out[:, 64:] == 7).all()
+
+
+@pytest.mark.parametrize("tokens", [0, 6])
+@pytest.mark.parametrize("lens", [(2, 1), (0, 0)])
+def test_zeroing_without_tokens_or_listed_rows(gpu, tokens, lens):
+    """The zeroing is done whether or not there is a token to append or a row that a chunk holds."""
+    out, rows, bounds, listed = _padded(gpu, 2, 3, lens)
+    k = torch.randn(6, 2, 32, device=gpu).bfloat16()
+    pool = torch.zeros(1, 2, 16, 32, dtype=torch.bfloat16, device=gpu)
+    slots = torch.arange(6, device=gpu)
+    call = Append(k_new=k.data_ptr(), v_new=k.data_ptr(), new_stride_token=64, k_pool=pool.data_ptr(), v_pool=pool.data_ptr(),
+                  pool_stride_block=1024, pool_stride_head=512, pool_stride_token=32, num_blocks=1,
+                  slot_mapping=slots.data_ptr(), n_tokens=tokens, gn=2, hd=32, block_size=16, dtype=0,
+                  zero_out=out.data_ptr(), zero_stride_bytes=144, rows=rows.data_ptr() if len(rows) else None,
+                  n_rows=len(rows), bounds=bounds.data_ptr(), zero_row_bytes=144, n_seqs=2, row_pitch=3)
+    lib, stream = _lib.load(), _lib.current_stream_ptr(gpu)
+    assert lib.ic_append_chunks(ctypes.byref(call), stream) == 0
+    assert (out[listed] == 7).all() and not out[~listed].any()
+    assert torch.equal(pool[0, :, :tokens], k[:tokens].transpose(0, 1)) and not pool[0, :, tokens:].any()
+    call.rows, call.n_rows = None, 3                           # rows that are counted but not given
+    assert lib.ic_append_chunks(ctypes.byref(call), stream) == -1
