@@ -27,7 +27,7 @@ __global__ __launch_bounds__(kAppendThreads) void kv_append_kernel(
     int64_t stride_head_bytes, int64_t stride_token_bytes, const int64_t *__restrict__ slot_mapping,
     int chunks_per_head, int chunks_per_row, int row_shift, int64_t n_tokens, int block_size, int64_t num_slots,
     const ZeroRows zero) {
-  if (zero_part(zero)) return;
+  if (zero_part(zero, 2)) return;
   const int64_t t = append_token<WIDE>(row_shift);
   const int c = append_chunk<WIDE>(row_shift);
   if (t >= n_tokens || c >= chunks_per_row) return;
@@ -59,7 +59,7 @@ int launch_kv_append(const AppendArgs &a, hipStream_t stream) {
   for (int64_t t0 = 0; t0 < a.n_tokens; t0 += slice) {
     const int64_t n = (a.n_tokens - t0 < slice) ? a.n_tokens - t0 : slice;
     grid.y = (unsigned)((n + rows - 1) / rows);
-    grid.z = zero.total > 0 ? 3 : 2;
+    grid.z = 2 + zero_slices(zero, grid);
     hipLaunchKernelGGL(rows == 1 ? kv_append_kernel<true> : kv_append_kernel<false>, grid, dim3(kAppendThreads), 0, stream,
                        (const char *)a.k_new + t0 * a.new_stride_token * es,
                        (const char *)a.v_new + t0 * a.new_stride_token * es,
@@ -81,9 +81,7 @@ __global__ __launch_bounds__(kAppendThreads) void zero_unlisted_rows_kernel(cons
 }  // namespace
 
 int launch_zero_unlisted_rows(const ZeroRows &z, hipStream_t stream) {
-  const int64_t most = (int64_t)device_cu_count() * 8;
-  hipLaunchKernelGGL(zero_unlisted_rows_kernel, dim3((unsigned)(z.total < most ? z.total : most)), dim3(kAppendThreads), 0,
-                     stream, z);
+  hipLaunchKernelGGL(zero_unlisted_rows_kernel, dim3((unsigned)zero_workgroups(z.total)), dim3(kAppendThreads), 0, stream, z);
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
 

@@ -64,7 +64,7 @@ struct RopeKP {
 template <class E, bool WIDE>
 __global__ __launch_bounds__(kAppendThreads) void rope_kv_append_kernel(const RopeKP p, int64_t t0, int64_t n_tokens,
                                                                              const ZeroRows zero) {
-  if (zero_part(zero)) return;
+  if (zero_part(zero, p.q_chunks > 0 ? 3 : 2)) return;
   constexpr int PAIRS = E::EPL / 2;  // pairs in one 16-byte chunk
   const int part = blockIdx.z;  // 0: K, 1: V, 2: Q
   const int row_shift = part == 2 ? p.q_row_shift : p.kv_row_shift;
@@ -112,7 +112,7 @@ int launch_typed(const RopeKP &kp, int64_t n_tokens, ZeroRows zero, hipStream_t 
   for (int64_t t0 = 0; t0 < n_tokens; t0 += slice) {
     const int64_t n = n_tokens - t0 < slice ? n_tokens - t0 : slice;
     grid.y = (unsigned)((n + rows - 1) / rows);
-    grid.z = parts + (zero.total > 0 ? 1 : 0);
+    grid.z = parts + zero_slices(zero, grid);
     hipLaunchKernelGGL((wide ? rope_kv_append_kernel<E, true> : rope_kv_append_kernel<E, false>), grid, dim3(kAppendThreads), 0, stream, kp, t0, t0 + n, zero);
     zero.total = 0;  // the first slice's
   }

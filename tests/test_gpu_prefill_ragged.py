@@ -1,6 +1,7 @@
 """Chunks of unequal length (rows named one by one): workgroups numbered over all sequences by the length of their
 sweep, against the same chunks numbered sequence by sequence; the append's launch with the zeroing beside it."""
 import ctypes
+import json
 from ctypes import c_float, c_int, c_int64, c_void_p
 
 import pytest
@@ -159,3 +160,26 @@ def test_zeroing_without_tokens_or_listed_rows(gpu, tokens, lens):
     assert torch.equal(pool[0, :, :tokens], k[:tokens].transpose(0, 1)) and not pool[0, :, tokens:].any()
     call.rows, call.n_rows = None, 3                           # rows that are counted but not given
     assert lib.ic_append_chunks(ctypes.byref(call), stream) == -1
+
+
+@pytest.mark.parametrize("gn,hd", [(1, 64), (1, 32), (8, 128)])
+def test_zeroing_has_workgroups_of_its_own(gpu, tmp_path, gn, hd):
+    """Beside an append of any width the padding rows get a workgroup each: not the few that a narrow append has."""
+    from torch.profiler import ProfilerActivity, profile
+    n, rows = 120, 2 * 60
+    out, listed, bounds, _ = _padded(gpu, 2, 60, (60, 3))
+    k = torch.randn(n, gn, hd, device=gpu).bfloat16()
+    pool = torch.zeros(8, gn, 16, hd, dtype=torch.bfloat16, device=gpu)
+    slots = torch.arange(n, device=gpu)
+    call = Append(k_new=k.data_ptr(), v_new=k.data_ptr(), new_stride_token=gn * hd, k_pool=pool.data_ptr(), v_pool=pool.data_ptr(),
+                  pool_stride_block=gn * 16 * hd, pool_stride_head=16 * hd, pool_stride_token=hd, num_blocks=8,
+                  slot_mapping=slots.data_ptr(), n_tokens=n, gn=gn, hd=hd, block_size=16, dtype=0, zero_out=out.data_ptr(),
+                  zero_stride_bytes=144, rows=listed.data_ptr(), n_rows=63, bounds=bounds.data_ptr(), zero_row_bytes=144,
+                  n_seqs=2, row_pitch=60)
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as prof:
+        assert _lib.load().ic_append_chunks(ctypes.byref(call), _lib.current_stream_ptr(gpu)) == 0
+        torch.cuda.synchronize()
+    prof.export_chrome_trace(str(tmp_path / "trace.json"))
+    grids = [e["args"]["grid"] for e in json.loads((tmp_path / "trace.json").read_text())["traceEvents"]
+             if e.get("cat") == "kernel" and "kv_append_kernel" in e["name"]]
+    assert len(grids) == 1 and grids[0][0] * grids[0][1] * (grids[0][2] - 2) >= rows, grids
