@@ -581,7 +581,8 @@ int ic_append_chunks(const ic_append_call *call, void *stream);
  * A decode step's append and attention in one launch: ic_kv_append (with cos_table and
  * sin_table ic_rope_kv_append_to, the query rows rotated on their way and not stored) of the
  * n_seqs new rows, then ic_paged_decode, which sees all of them, whichever sequence's
- * slot they are in.  For small batches of short contexts (at most 64 sequences);
+ * slot they are in.  For small batches of short contexts (at most 64 sequences, a KV
+ * head of one to each CU, fewer where query heads share a KV head or contexts are longer);
  * IC_ERR_UNSUPPORTED for the others, with nothing launched.  No workspace.
  */
 typedef struct ic_decode_append_call {

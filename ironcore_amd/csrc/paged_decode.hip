@@ -790,6 +790,9 @@ void launch_valu_main(DecodeKP &kp, hipStream_t stream) {
   hipLaunchKernelGGL((paged_decode_kernel<E, HD, GT, BS, NW>), dim3(wgs), dim3(NW * kWave), 0, stream, kp);
 }
 
+// Tiles in turn of the pair kernel's waves on the longest row.
+int64_t pair_rounds(const DecodeKP &kp) { return ((int64_t)kp.max_ctx + 16 * kPairWaves - 1) / (16 * kPairWaves); }
+
 // Whether a call is the pair kernel's.  us of the split (main kernel and reduce) / of the pair kernel, contexts up to
 // 48, 160, 300, 600, 1 200 tokens:
 //   fp32, 12 / 12 heads of 64, 4 sequences     9.8 / 3.1   13.0 / 3.8   15.6 / 4.3   19.3 / 5.5   27.9 / 8.1
@@ -820,13 +823,43 @@ void launch_valu_main(DecodeKP &kp, hipStream_t stream) {
 // each head, hence lower limits, and none from five heads on.
 bool decode_takes_pairs(const DecodeKP &kp, int hd, int row_bytes) {
   if (kp.cohort_size != 1 || kp.key_mask != nullptr || kp.min_chunk > 1 || kp.max_ctx <= 0 || kp.group > 4) return false;
-  const int64_t rounds = ((int64_t)kp.max_ctx + 16 * kPairWaves - 1) / (16 * kPairWaves);
+  const int64_t rounds = pair_rounds(kp);
   const int64_t pairs = (int64_t)kp.n_seqs * kp.pairs_per_seq;
   if (rounds > 16 || kp.n_seqs > 65535) return false;
   if (kp.group == 1) return rounds * row_bytes <= 4096 && pairs * row_bytes < (rounds == 1 ? 1 << 20 : 2 << 20);
   if (kp.group == 2) return rounds * row_bytes <= 2048 && pairs * row_bytes < 1 << 19;
   if (hd <= 64) return rounds <= 8 && pairs <= 2 * device_cu_count();
   return rounds <= 2 && pairs <= device_cu_count();
+}
+
+// Whether the append rides on the pair kernel's launch.  It saves a launch of about a microsecond and costs each workgroup
+// the comparison of its tiles with all new slots: worth it while a CU has one workgroup, not with two.  us of one launch / of
+// two (append, attention), by pairs (KV heads times sequences), contexts up to 250, 500, 1 000 and 2 000 tokens:
+//   fp32, 12 / 12 heads of 64             48    5.0 / 6.2    6.0 / 7.2    8.1 / 9.0    15.0 / 16.0
+//                                        192    5.3 / 6.3    7.7 / 8.5   13.9 / 14.6   22.3 / 23.2
+//                                        384   10.7 / 9.5   16.5 / 16.3  26.2 / 25.9   52.4 / 51.2
+//   bf16, 16 / 16 of 64, rotary           64    5.5 / 6.4    6.3 / 7.1    7.8 / 8.5    10.8 / 10.9
+//                                        256    6.1 / 6.5    6.6 / 7.3   13.0 / 12.8   18.6 / 18.5
+//                                        512    8.8 / 7.7   15.5 / 13.8  21.7 / 20.6   34.7 / 33.5
+//   bf16, 8 / 8 of 128, rotary            32    6.3 / 7.1    7.6 / 8.2   10.2 / 10.2   15.1 / 14.1
+//                                        256    7.0 / 7.4   13.2 / 13.3  19.7 / 20.0   32.4 / 32.4
+//                                        512   14.5 / 13.2  21.2 / 19.5  33.9 / 31.5   79.0 / 69.5
+// Grouped heads rotate a query row for each of them, in every wave: fewer pairs, fewer rounds.
+//   bf16, 8 / 4 of 64, rotary             16    7.1 / 7.7    8.3 / 8.9   10.6 / 10.7   15.2 / 14.6
+//                                        128    7.5 / 7.9    8.7 / 9.0   11.8 / 11.0   18.1 / 16.6
+//                                        256    8.0 / 8.1    9.8 / 9.6   15.6 / 14.9   22.0 / 21.5
+//   bf16, 16 / 8 of 128, rotary           32    7.8 / 8.6    9.7 / 10.3  13.6 / 13.8
+//                                        128    8.1 / 8.6   10.0 / 10.4  16.6 / 15.8
+//                                        512   20.5 / 15.0  26.8 / 21.5  38.8 / 34.2
+//   fp16, 8 / 2 of 64, rotary              8   10.3 / 10.5  12.2 / 12.2  16.1 / 15.9
+//                                         64   10.5 / 10.6  12.4 / 12.4  16.3 / 16.0
+//   bf16, 16 / 4 of 64, rotary           256   11.6 / 11.2  14.0 / 13.2  21.8 / 19.1
+bool append_joins_pairs(const DecodeKP &kp, int hd) {
+  const int64_t rounds = pair_rounds(kp), pairs = (int64_t)kp.n_seqs * kp.pairs_per_seq, cus = device_cu_count();
+  if (kp.n_seqs > kPairAppendRows || pairs > cus) return false;
+  if (kp.group == 1) return rounds * hd <= 1024;
+  if (kp.group == 2) return rounds <= 8 && pairs * rounds <= 2 * cus;
+  return rounds <= 4 && pairs * rounds <= cus && 2 * pairs <= cus;
 }
 
 template <class E, int HD, bool APPEND>
@@ -845,10 +878,7 @@ template <class E, int HD>
 int launch_group(DecodeKP &kp, int dtype, const AppendRows *rows, hipStream_t stream) {
   const bool pairs = decode_takes_pairs(kp, HD, HD * (int)sizeof(typename E::type));
   if (rows != nullptr) {  // with the append: only in one launch
-    // (larger grids are bound by what their workgroups do: 233 sequences of 17-512 tokens, 16 heads of 64, rotary 87 us
-    // so, 54 with a launch for the append)
-    if (!pairs || kp.n_seqs > kPairAppendRows || (int64_t)kp.n_seqs * kp.pairs_per_seq > 2 * device_cu_count() ||
-        kp.num_blocks * kp.tiles_per_block >= (int64_t)1 << 31)
+    if (!pairs || !append_joins_pairs(kp, HD) || kp.num_blocks * kp.tiles_per_block >= (int64_t)1 << 31)
       return IC_ERR_UNSUPPORTED;
     PairAppend n;
     n.k_new = (const char *)rows->k_new, n.v_new = (const char *)rows->v_new;

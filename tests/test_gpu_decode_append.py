@@ -116,3 +116,26 @@ def test_a_row_to_every_lane_and_more(gpu, b, one):
     wl.context_lens[3] = wl.context_lens[b - 1]
     _compare(gpu, torch.bfloat16, wl.context_lens.tolist(), tables, slots, 2, 2, 64, 16, wl.k_pool.shape[0],
              True, b, one_launch=one)
+
+
+@pytest.mark.parametrize("dtype,hn,gn,hd,b,longest,one", [
+    (torch.bfloat16, 4, 4, 128, 3, 1024, True), (torch.bfloat16, 4, 4, 128, 3, 1025, False),      # rounds x head dim
+    (torch.float32, 3, 3, 64, 5, 2048, True), (torch.float16, 8, 8, 32, 4, 2047, True),
+    (torch.float32, 3, 3, 64, 5, 2049, False),                                                    # the split's
+    (torch.bfloat16, 4, 2, 64, 2, 1024, True), (torch.bfloat16, 4, 2, 64, 2, 1025, False),
+    (torch.bfloat16, 6, 2, 64, 3, 512, True), (torch.bfloat16, 8, 2, 64, 3, 513, False),
+    (torch.bfloat16, 16, 16, 64, 16, 130, True), (torch.bfloat16, 16, 16, 64, 17, 130, False),    # a pair to a CU (256)
+    (torch.bfloat16, 8, 4, 64, 64, 256, True), (torch.bfloat16, 8, 4, 64, 64, 257, False),        # pairs x rounds
+    (torch.bfloat16, 16, 4, 64, 32, 256, True), (torch.bfloat16, 16, 4, 64, 33, 128, False)])
+@pytest.mark.parametrize("rope", [False, True])
+def test_rounds_and_the_line_to_two_launches(gpu, dtype, hn, gn, hd, b, longest, one, rope):
+    wl = workloads.make_decode_workload(b, hn, gn, hd, longest, longest, dtype=dtype, seed=longest)
+    wl.context_lens -= torch.arange(b, dtype=torch.int32)
+    wl.context_lens[1] = longest // 2
+    last = wl.context_lens.long() - 1
+    slots = wl.block_tables.long().gather(1, (last // 16).unsqueeze(1)).squeeze(1) * 16 + last % 16
+    tables = wl.block_tables.clone()
+    tables[1, :-1] = tables[0, :-1]            # row 1 is in the middle of row 0's context
+    slots[1] = tables[1, last[1] // 16].long() * 16 + last[1] % 16
+    _compare(gpu, dtype, wl.context_lens.tolist(), tables, slots, hn, gn, hd, 16, wl.k_pool.shape[0], rope, b,
+             one_launch=one)
