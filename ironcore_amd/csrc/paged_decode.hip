@@ -305,7 +305,7 @@ __global__ __launch_bounds__(NW *kWave) void paged_decode_kernel(const DecodeKP 
   }
 }
 
-// Short contexts (up to about a thousand tokens, see decode_takes_pairs for the lines): with shares of a tile
+// Short contexts (up to 2 048 tokens at most, see decode_takes_pairs for the lines): with shares of a tile
 // the split above turns them into partials that a second launch merges, 8 + 5 us of which the tiles themselves take
 // two (4 sequences of up to 160 tokens, 12 heads of 64, fp32: 13.0 us, here 3.8).  Here a workgroup owns a whole pair:
 // its eight waves take the pair's tiles in turn (a wave's table entries come in one load, one per lane: at most 64

@@ -48,3 +48,24 @@ def test_table_entries_out_of_the_pool_are_clamped(gpu):
     wl.block_tables[0, 1], wl.block_tables[1, 2] = -7, 10 ** 6
     ref = oracle_paged.paged_decode(wl.query, wl.k_pool, wl.v_pool, want, wl.context_lens)
     assert (_run(wl, gpu) - ref).abs().max().item() <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("dtype,hn,gn,hd", [(torch.bfloat16, 4, 4, 128), (torch.bfloat16, 6, 6, 64), (torch.float32, 3, 3, 64),
+                                            (torch.float16, 4, 2, 64), (torch.bfloat16, 4, 2, 128), (torch.bfloat16, 8, 2, 64)])
+@pytest.mark.parametrize("longest", [1024, 1025, 1280, 1281, 2047, 2048, 2049])
+def test_rounds_up_to_the_limits(gpu, dtype, hn, gn, hd, longest):
+    """Contexts of 8 to 16 rounds, and past what the pair kernel takes (fewer rounds with wide rows or grouped heads)."""
+    lens = (longest, 1, longest - 127, longest // 2, 129)
+    wl = workloads.make_decode_workload(len(lens), hn, gn, hd, longest, longest, dtype=dtype, seed=longest)
+    wl.context_lens = torch.tensor(lens, dtype=torch.int32)
+    ref = oracle_paged.paged_decode(wl.query, wl.k_pool, wl.v_pool, wl.block_tables, wl.context_lens)
+    assert (_run(wl, gpu).float() - ref.float()).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("batch,hn,gn,hd,dtype", [
+    (300, 4, 4, 64, torch.bfloat16), (700, 4, 2, 64, torch.float16), (300, 3, 3, 64, torch.float32),
+    (127, 16, 4, 64, torch.bfloat16), (129, 16, 4, 64, torch.bfloat16)])      # 508 and 516 pairs: the pair kernel's, the split's
+def test_large_batches(gpu, batch, hn, gn, hd, dtype):
+    wl = workloads.make_decode_workload(batch, hn, gn, hd, 1, 300, dtype=dtype, seed=batch)
+    ref = oracle_paged.paged_decode(wl.query, wl.k_pool, wl.v_pool, wl.block_tables, wl.context_lens)
+    assert (_run(wl, gpu).float() - ref.float()).abs().max().item() <= TOL[dtype]

@@ -151,13 +151,15 @@ def test_decode_scaled_llama7b_slice(gpu):
 
 
 @pytest.mark.parametrize("batch", [257, 700, 1100])
-def test_decode_many_short_sequences(gpu, batch):
-    """Batches of more than 256 and of more than 1024 sequences (the prologue
+@pytest.mark.parametrize("min_chunk_tokens", [0, 32])
+def test_decode_many_short_sequences(gpu, batch, min_chunk_tokens):
+    """Batches of more than 256 and of more than 1024 sequences (the split's prologue
     scans the per-sequence tile counts 256 rows at a time, and keeps them in
-    registers only up to 1024 rows), with empty sequences sprinkled in."""
+    registers only up to 1024 rows), with empty sequences sprinkled in.  Without a
+    least share a call like this is the pair kernel's, with one it is the split's."""
     wl = workloads.make_decode_workload(batch, 4, 2, 64, 1, 70, seed=batch)
     wl.context_lens[::97] = 0
-    out = _run(wl, gpu)
+    out = _run(wl, gpu, min_chunk_tokens=min_chunk_tokens)
     ctx = wl.context_lens.clamp(min=1)
     ref = oracle_paged.paged_decode(wl.query, wl.k_pool, wl.v_pool, wl.block_tables, ctx)
     ref[wl.context_lens <= 0] = 0
