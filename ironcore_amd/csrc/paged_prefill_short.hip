@@ -14,8 +14,8 @@
 //    Blocks are numbered row block by row block, the heads of a row block side by
 //    side: the waves of a workgroup reach about equally far (a packed mask's
 //    lists belong to a head's rows: there head by head).
-//  * Chunks of unequal length: workgroups are numbered over all sequences, the longest sweep
-//    first (by_sweep below), KV heads round the XCDs.
+//  * Chunks of unequal length that fill the chip more than once: workgroups are numbered over all
+//    sequences, the longest sweep first (by_sweep below), KV heads round the XCDs.
 //  * Every wave stages a 16-row group of K AND of V of each tile, into two
 //    buffers (a third gained nothing); one barrier per tile.  64 KiB of LDS at head dim 128, 32 KiB at 64:
 //    two, resp. four, workgroups share a CU, and what the two-sided schedule of
@@ -601,10 +601,28 @@ int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t s
   const int64_t per_unit = short_workgroups_per_unit(a);
   const int64_t slices = (kp.n_units + kXcds - 1) / kXcds;
   int64_t wgs = slices * kXcds * per_unit;
-  // Chunks that lie in padded rows are of unequal length: at most so many workgroups, a sequence's last one and row
-  // block not full.
-  kp.by_sweep = a.rows != nullptr && a.mask_bits == nullptr && a.n_seqs <= kWave;
-  if (kp.by_sweep) {
+  // Chunks that lie in padded rows are of unequal length.  Numbered unit by unit, an XCD gets `slices` units and is
+  // uneven against the others where they, or a single one, are more workgroups than its CUs hold at once; where they
+  // are not, everything is resident anyway and the search in each workgroup (1-1.5 us) is lost.  us by sweep / by unit (append
+  // and attention), workgroups of a unit x units of an XCD of the padded chunks, nothing cached and up to 1 024, 8 192 tokens:
+  //   28 / 4 heads of 128, 9 of 3-701 rows     37 x 5     37.6 / 39.7    61.2 / 71.0
+  //                        9 of 100-500        27 x 5     31.2 / 32.4    52.5 / 58.7
+  //                       16 of 10-200         13 x 8     21.2 / 22.7    39.5 / 40.7   166.9 / 175.9
+  //                        9 of 3-60            4 x 5     10.5 / 10.0    24.5 / 22.4   111.5 / 108.3
+  //    8 / 1 of 128,       9 of 3-701          42 x 2     25.5 / 26.1    35.1 / 39.0   120.3 / 146.8
+  //                       32 of 3-60            4 x 4     12.2 / 11.7    29.2 / 25.6
+  //   32 / 32 of 128,     32 of 100-500         4 x 128  168.3 / 193.7
+  //                        2 of 100-500         4 x 8     22.3 / 21.6    33.1 / 31.7
+  //   16 / 4 of 64,        9 of 3-701          21 x 5     25.8 / 24.3    38.6 / 37.3
+  //                       32 of 3-701          22 x 16    47.8 / 51.4    75.4 / 80.2
+  //   16 / 16 of 64,      32 of 100-500         4 x 64    51.6 / 53.9    76.2 / 80.3
+  //                        9 of 100-500         4 x 18    25.3 / 24.3    37.6 / 36.5
+  // (954 sizes measured, 2-60 sequences, 1-32 KV heads: by this line 2.2 % less time than by unit throughout, 2.9 % less
+  // than by sweep throughout, 0.5 % more than the better of the two.)
+  const int64_t xcd_cus = device_cu_count() / kXcds;
+  kp.by_sweep = a.rows != nullptr && a.mask_bits == nullptr && a.n_seqs <= kWave &&
+                (per_unit > xcd_cus || slices * per_unit > xcd_cus * (a.hd == 128 ? 2 : 4));
+  if (kp.by_sweep) {  // (at most so many workgroups, a sequence's last one and row block not full)
     const int64_t blocks = a.n_rows / 32 + a.n_seqs;
     wgs = a.gn * ((blocks * kp.group + kShortWaves - 1) / kShortWaves + a.n_seqs);
   }

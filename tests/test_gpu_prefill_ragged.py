@@ -57,7 +57,13 @@ def _attend(d, hn, gn, hd, causal, rows, positions, emb, out, q):
     (64, 6, 2, 32, 16, (0, 40), (0, 140), torch.bfloat16),     # a sequence to every lane
     (65, 6, 2, 64, 16, (0, 40), (1, 70), torch.bfloat16),      # one more: numbered sequence by sequence
     (3, 28, 4, 128, 16, (1500, 1600), (1, 130), torch.bfloat16),
-    (9, 12, 12, 128, 16, (0, 0), (3, 700), torch.bfloat16)])
+    (9, 12, 12, 128, 16, (0, 0), (3, 700), torch.bfloat16),
+    # more workgroups to an XCD than it holds: 36, 40 and up to 44 of one unit; 16 units of 5 and of 9
+    (1, 36, 1, 128, 16, (0, 0), (97, 97), torch.bfloat16),
+    (3, 64, 4, 128, 16, (1500, 1600), (290, 500), torch.bfloat16),
+    (17, 48, 2, 64, 48, (0, 700), (1, 220), torch.float16),
+    (16, 8, 8, 128, 16, (0, 200), (0, 600), torch.bfloat16),
+    (64, 6, 2, 32, 16, (0, 40), (0, 340), torch.bfloat16)])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("rope", [False, True])
 def test_by_sweep(gpu, n_seqs, hn, gn, hd, block, prefix, chunks, dtype, causal, rope):
