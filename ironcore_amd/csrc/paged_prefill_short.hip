@@ -13,7 +13,7 @@
 //    x 7 heads are two workgroups, not seven with 5 % of their rows in use.
 //    Blocks are numbered row block by row block, the heads of a row block side by
 //    side: the waves of a workgroup reach about equally far (a packed mask's
-//    lists belong to a head's rows: there head by head).
+//    lists belong to a head's rows: there, and with DIRECT, head by head).
 //  * Chunks of unequal length that fill the chip more than once: workgroups are numbered over all
 //    sequences, the longest sweep first (by_sweep below), KV heads round the XCDs.
 //  * Every wave stages a 16-row group of K AND of V of each tile, into two
@@ -34,9 +34,10 @@
 //    the byte mask of the long kernel (32 byte loads per lane and tile, every tile
 //    walked), 11.9 us here, launch to launch.
 //
-//  * Query rows and outputs move as whole rows of a head and change places in LDS: as the MFMA lays them out a
-//    load touched 32 cache lines for 1 KiB, rotary tables likewise (query rows ready after 3.8 instead of 5.3 us of
-//    a workgroup's 17; 80 sequences of 129 tokens, 12 heads of 64: 20.8 -> 18.8 us).
+//  * In full grids and with rotary, query rows and outputs move as whole rows of a head and change places in LDS: as
+//    the MFMA lays them out a load touched 32 cache lines for 1 KiB, rotary tables likewise (query rows ready after 3.8
+//    instead of 5.3 us of a workgroup's 17; 80 sequences of 129 tokens, 12 heads of 64: 20.8 -> 18.8 us).  The others
+//    (DIRECT, prefill_rows_direct) load and store them as they are needed.
 //
 // Bound by the latency of a tile (load, two products and a softmax in one wave's
 // instruction stream, about 1 us at head dim 128) at the sizes it is for; 80
@@ -118,7 +119,9 @@ __device__ __forceinline__ bool pick_by_sweep(const PrefillKP &p, int index, int
   return true;
 }
 
-template <class M, int HD, bool SINGLE, int TG, bool PACKED>
+// DIRECT: query rows and outputs move as the MFMA lays them out, and the row blocks of a head side by side; no rotary
+// (see prefill_rows_direct).
+template <class M, int HD, bool SINGLE, int TG, bool PACKED, bool DIRECT>
 __global__ __launch_bounds__(TG *kShortWaves *kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 2 : 4)))
 void paged_prefill_short_kernel(const PrefillKP p) {
   constexpr int KS = HD / 16;      // k-steps of the QK contraction
@@ -142,7 +145,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   // that differ by a multiple of 8.
   int seq, q_lo, L, C, kvh, v0 = 0, slice = 0, r = 0;
   const int per_unit = p.n_qtiles;  // workgroups per unit
-  if (!PACKED && p.by_sweep) {
+  if (!PACKED && !DIRECT && p.by_sweep) {
     kvh = blockIdx.x % p.gn;
     if (!pick_by_sweep(p, blockIdx.x / p.gn, seq, q_lo, L, C, v0)) return;
   } else {
@@ -168,7 +171,7 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const int total = n_blocks * p.group;
   // The last blocks (the longest sweeps) first; in the slices that share the CUs with the first ones when
   // the whole grid is resident, last: a CU then holds a long and a short sweep, not two of the same length.
-  if (PACKED || !p.by_sweep) v0 = (slice < p.flip_slice ? per_unit - 1 - r : r) * kShortWaves;
+  if (PACKED || DIRECT || !p.by_sweep) v0 = (slice < p.flip_slice ? per_unit - 1 - r : r) * kShortWaves;
   if (v0 >= total) return;
 
   const int tid = threadIdx.x;
@@ -180,8 +183,9 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const int n = lane & 31;  // query column of this lane within the wave's 32-row block
   const int hh = lane >> 5;  // which half of each k-step this lane feeds
   const int v = v0 + wave < total ? v0 + wave : total - 1;
-  const int head = PACKED ? v / n_blocks : v % p.group;
-  const int row0 = (PACKED ? v - head * n_blocks : v / p.group) * 32;
+  constexpr bool kByHead = PACKED || DIRECT;  // wave blocks are numbered head by head
+  const int head = kByHead ? v / n_blocks : v % p.group;
+  const int row0 = (kByHead ? v - head * n_blocks : v / p.group) * 32;
   const bool mine = v0 + wave < total && row0 < C;
   const int h = kvh * p.group + head;
   const int my_q = row0 + n;
@@ -204,27 +208,33 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   const int rsub = lane / CPR;  // row within the rows one load covers
   const int k_lane = n * ROWB + ((hh ^ tile_swizzle_k<CPR>(n)) << 4);  // operand reads of rows stored as K tiles are
   const int my_row = (int)query_row(p, q_lo, qrow);
-  int table_row_of_mine = 0;
-  if (p.positions != nullptr) table_row_of_mine = rope_position(p, my_row);
-  char *const s_q = (wave < 2 ? tiles_k : tiles_v) + (NB - 1) * TILEB + (wave & 1) * (TILEB / 2);
   Vec16 qf[KS];
+  if constexpr (DIRECT) {
 #pragma unroll
-  for (int i = 0; i < KS; ++i)
-    qf[i] = load16(p.q + ((int64_t)__shfl(my_row, i * WR + rsub, kWave) * p.q_stride_token + (int64_t)h * HD + cc * 8) * 2);
-  if (p.positions != nullptr) {
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = load16(p.q + ((int64_t)my_row * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+  } else {
+    int table_row_of_mine = 0;
+    if (p.positions != nullptr) table_row_of_mine = rope_position(p, my_row);
+    char *const s_q = (wave < 2 ? tiles_k : tiles_v) + (NB - 1) * TILEB + (wave & 1) * (TILEB / 2);
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+      qf[i] = load16(p.q + ((int64_t)__shfl(my_row, i * WR + rsub, kWave) * p.q_stride_token + (int64_t)h * HD + cc * 8) * 2);
+    if (p.positions != nullptr) {
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const int64_t trig = (int64_t)__shfl(table_row_of_mine, i * WR + rsub, kWave) * p.half_hd + cc * 4;
+        qf[i] = rotate_chunk<typename M::E>(qf[i], p.cos_table + trig, p.sin_table + trig);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
-      const int64_t trig = (int64_t)__shfl(table_row_of_mine, i * WR + rsub, kWave) * p.half_hd + cc * 4;
-      qf[i] = rotate_chunk<typename M::E>(qf[i], p.cos_table + trig, p.sin_table + trig);
+      const int r = i * WR + rsub;
+      store16(s_q + r * ROWB + ((cc ^ tile_swizzle_k<CPR>(r)) << 4), qf[i]);
     }
-  }
 #pragma unroll
-  for (int i = 0; i < KS; ++i) {
-    const int r = i * WR + rsub;
-    store16(s_q + r * ROWB + ((cc ^ tile_swizzle_k<CPR>(r)) << 4), qf[i]);
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = load16(s_q + (k_lane ^ (ks * 32)));
   }
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) qf[ks] = load16(s_q + (k_lane ^ (ks * 32)));
 
   f32x16_t o[OB];
   float m = kNegInf, l = 0.f;
@@ -235,7 +245,8 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 
   // tiles this wave's rows reach, and the most that any wave of the workgroup does: its last block's
   const int v_last = v0 + kShortWaves < total ? v0 + kShortWaves - 1 : total - 1;
-  const int last_row = (v_last / p.group) * 32 + 32;  // (a packed mask has its lists instead)
+  int last_row = (v_last / p.group) * 32 + 32;  // (a packed mask has its lists instead)
+  if (DIRECT) last_row = v0 / n_blocks == v_last / n_blocks ? (v_last % n_blocks) * 32 + 32 : C;
   int kv_end = causal ? P + last_row : L;
   kv_end = kv_end < L ? kv_end : L;
   MaskList list;
@@ -500,6 +511,23 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   both_halves(l, l_a, l_b);
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if constexpr (DIRECT) {
+    if (mine && my_q < C) {
+      // (a packed mask comes with equal sequences, whose rows need no register until here)
+      char *const orow = p.out + ((PACKED ? q_lo + my_q : my_row) * p.out_stride_token + (int64_t)h * HD + 4 * hh) * 2;
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint2 w;
+          w.x = M::pack2(o[ob][4 * j] * inv, o[ob][4 * j + 1] * inv);
+          w.y = M::pack2(o[ob][4 * j + 2] * inv, o[ob][4 * j + 3] * inv);
+          *reinterpret_cast<uint2 *>(orow + (ob * 32 + 8 * j) * 2) = w;
+        }
+      }
+    }
+    return;
+  }
   // Out in whole rows of the head again, through LDS: the tiles are done with (with two tile groups the first group's
   // wave takes the slab it has just read).
   if constexpr (TG == 1) __syncthreads();
@@ -517,7 +545,6 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 #pragma unroll
   for (int i = 0; i < KS; ++i) {
     const int r = i * WR + rsub;
-    // (a packed mask comes with equal sequences, whose rows need no register until here)
     const int64_t row = PACKED ? q_lo + row0 + r : __shfl(my_row, r, kWave);
     const int64_t to = row * p.out_stride_token + (int64_t)h * HD + cc * 8;
     const Vec16 v = load16(s_o + r * ROWB + ((cc ^ tile_swizzle_k<CPR>(r)) << 4));
@@ -525,18 +552,18 @@ void paged_prefill_short_kernel(const PrefillKP p) {
   }
 }
 
-template <class M, bool SINGLE, int TG, bool PACKED>
+template <class M, bool SINGLE, int TG, bool PACKED, bool DIRECT>
 int launch_short_hd(const PrefillKP &kp, int hd, unsigned wgs, hipStream_t stream) {
   const dim3 grid(wgs), block(TG * kShortWaves * kWave);
   switch (hd) {
     case 32:
-      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 32, SINGLE, TG, PACKED>), grid, block, 0, stream, kp);
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 32, SINGLE, TG, PACKED, DIRECT>), grid, block, 0, stream, kp);
       break;
     case 64:
-      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 64, SINGLE, TG, PACKED>), grid, block, 0, stream, kp);
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 64, SINGLE, TG, PACKED, DIRECT>), grid, block, 0, stream, kp);
       break;
     case 128:
-      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 128, SINGLE, TG, PACKED>), grid, block, 0, stream, kp);
+      hipLaunchKernelGGL((paged_prefill_short_kernel<M, 128, SINGLE, TG, PACKED, DIRECT>), grid, block, 0, stream, kp);
       break;
     default:
       return IC_ERR_UNSUPPORTED;
@@ -544,16 +571,16 @@ int launch_short_hd(const PrefillKP &kp, int hd, unsigned wgs, hipStream_t strea
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
 
-template <class M>
+template <class M, bool DIRECT>
 int launch_short_type(const PrefillKP &kp, const PrefillArgs &a, unsigned wgs, bool split, hipStream_t stream) {
   if (a.mask_bits != nullptr)
-    return split ? launch_short_hd<M, true, 2, true>(kp, a.hd, wgs, stream)
-                 : launch_short_hd<M, true, 1, true>(kp, a.hd, wgs, stream);
+    return split ? launch_short_hd<M, true, 2, true, DIRECT>(kp, a.hd, wgs, stream)
+                 : launch_short_hd<M, true, 1, true, DIRECT>(kp, a.hd, wgs, stream);
   if (a.block_tables == nullptr || a.block_table_stride == 1)
-    return split ? launch_short_hd<M, true, 2, false>(kp, a.hd, wgs, stream)
-                 : launch_short_hd<M, true, 1, false>(kp, a.hd, wgs, stream);
-  return split ? launch_short_hd<M, false, 2, false>(kp, a.hd, wgs, stream)
-               : launch_short_hd<M, false, 1, false>(kp, a.hd, wgs, stream);
+    return split ? launch_short_hd<M, true, 2, false, DIRECT>(kp, a.hd, wgs, stream)
+                 : launch_short_hd<M, true, 1, false, DIRECT>(kp, a.hd, wgs, stream);
+  return split ? launch_short_hd<M, false, 2, false, DIRECT>(kp, a.hd, wgs, stream)
+               : launch_short_hd<M, false, 1, false, DIRECT>(kp, a.hd, wgs, stream);
 }
 
 }  // namespace
@@ -597,6 +624,32 @@ bool prefill_takes_short(const PrefillArgs &a) {
   return !(filled && ctx >= 2 * (int64_t)a.max_chunk_len && ctx >= (a.hn > a.gn ? 2200 : 1250));
 }
 
+// Whether query rows and outputs move as the MFMA lays them out, without the exchange in LDS: that exchange costs a
+// workgroup half a microsecond of latency and saves its CU's cache look-ups, so it loses where the launch is over in a few
+// tiles or leaves the CUs a workgroup or two.  Rotary tables gain from whole rows at every size.  us by whole rows / directly
+// (calls without a cache):
+//   sequences x tokens            1 x 20       18 x 70       3 x 300       4 x 500       60 x 100      30 x 130      2 x 1 024
+//   12 / 12 heads of 64, causal   4.9 / 4.3    6.6 / 5.7     9.3 / 8.2    13.0 / 11.7   11.5 / 10.9   10.1 / 10.1   16.4 / 16.4
+//                  all keys       5.0 / 4.3    6.5 / 6.0     9.5 / 9.0    13.2 / 12.5   11.6 / 12.1   11.7 / 12.9   16.5 / 16.4
+//             packed documents    5.7 / 4.8    7.4 / 6.6     9.9 / 9.0    11.7 / 10.7   12.9 / 12.6   11.0 / 11.0   12.8 / 13.0
+//   16 / 16 of 128, causal        5.9 / 5.4   10.0 / 9.3    11.1 / 10.5   16.7 / 16.1   24.6 / 24.9   21.4 / 22.6   23.2 / 24.0
+//                  all keys       5.8 / 5.1    9.8 / 10.5   11.6 / 12.3   17.5 / 18.1   25.2 / 28.3   23.5 / 27.9   24.3 / 26.2
+//             packed documents    6.3 / 5.6   10.7 / 9.9    11.4 / 11.2   14.7 / 14.5   26.1 / 26.9   22.8 / 24.1   17.4 / 18.9
+//   80 x 129, 12 / 12 of 64, causal (1 920 workgroups): 18.8 / 20.8; packed, 60 x 20, 64 / 8 of 128: 44.1 / 38.1.
+// Grouped heads put one row block of several heads into a workgroup, which reaches equally far, where this numbers head
+// by head: only in grids of a workgroup to a CU (8 / 1 of 64, causal, 8 x 70 6.1 / 5.6, 3 x 300 9.5 / 8.7, 2 x 1 024 23 % faster
+// by whole rows; at head dim 128, 28 / 4, causal, 8 x 70 8.1 / 7.7, 1 x 20 9 % faster by whole rows).
+bool prefill_rows_direct(const PrefillArgs &a, int64_t wgs) {
+  if (a.positions != nullptr) return false;
+  const int64_t cus = device_cu_count(), ctx = context_bound(a);
+  const bool packed = a.mask_bits != nullptr;
+  if (a.hn > a.gn && !packed) return wgs <= cus && (a.hd < 128 ? ctx <= 512 : a.causal && ctx > 64 && ctx <= 128);
+  if (a.hd < 128) return packed || ctx <= 64 || wgs <= (a.causal ? 4 : 1) * cus;
+  if (ctx <= 64) return true;
+  if (packed) return a.max_chunk_len <= 128 && wgs <= 5 * cus;
+  return a.causal ? ctx <= 320 && 2 * wgs <= 5 * cus : ctx <= 128 && wgs <= cus;
+}
+
 int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t stream) {
   const int64_t per_unit = short_workgroups_per_unit(a);
   const int64_t slices = (kp.n_units + kXcds - 1) / kXcds;
@@ -637,8 +690,12 @@ int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t s
   // 22.6 / 69.6 / 137 with one group, 24.4 / 65.4 / 128 with two.
   const int64_t ctx = context_bound(a);
   const bool split = (wgs <= cus && ctx > 512) || (a.hd < 128 && wgs <= 2 * cus && ctx >= 2048);
-  return a.dtype == IC_DTYPE_BF16 ? launch_short_type<MmaBf16>(kp, a, (unsigned)wgs, split, stream)
-                                  : launch_short_type<MmaF16>(kp, a, (unsigned)wgs, split, stream);
+  const bool bf16 = a.dtype == IC_DTYPE_BF16;
+  if (!kp.by_sweep && prefill_rows_direct(a, per_unit * kp.n_units))
+    return bf16 ? launch_short_type<MmaBf16, true>(kp, a, (unsigned)wgs, split, stream)
+                : launch_short_type<MmaF16, true>(kp, a, (unsigned)wgs, split, stream);
+  return bf16 ? launch_short_type<MmaBf16, false>(kp, a, (unsigned)wgs, split, stream)
+              : launch_short_type<MmaF16, false>(kp, a, (unsigned)wgs, split, stream);
 }
 
 }  // namespace prefill

@@ -63,3 +63,16 @@ def test_no_causal_rule_and_empty_chunks(gpu, chunk, prefix):
     _hold(wl, gpu, causal=False)
     wl = workloads.make_prefill_workload(5, 6, 2, 128, prefix, prefix, 0, 3, seed=chunk + 1)
     _hold(wl, gpu)
+
+
+@pytest.mark.parametrize("hn,gn,hd,n_seqs,chunk,prefix,causal", [
+    (4, 4, 128, 2, 64, 0, True), (2, 2, 128, 1, 300, 16, True), (2, 2, 128, 1, 300, 32, True),      # 64, 320 tokens
+    (4, 4, 128, 2, 33, 80, False), (4, 4, 128, 2, 33, 96, False),                                   # 128
+    (12, 12, 64, 85, 70, 0, True), (12, 12, 64, 86, 70, 0, True), (4, 4, 64, 64, 70, 0, False), (4, 4, 64, 65, 70, 0, False),
+    # grouped: 512 tokens, a workgroup to a CU; a workgroup of two heads' and of three heads' blocks
+    (8, 2, 64, 2, 100, 412, True), (8, 2, 64, 2, 100, 413, True), (8, 2, 64, 2, 33, 0, True), (6, 2, 64, 3, 70, 9, False),
+    (8, 1, 32, 1, 20, 0, True), (8, 2, 128, 2, 100, 0, True), (8, 2, 128, 2, 120, 9, True), (16, 2, 64, 40, 70, 0, True)])
+def test_rows_moved_directly_and_whole(gpu, hn, gn, hd, n_seqs, chunk, prefix, causal):
+    """Either side of the lines between the two ways in which query rows and outputs move."""
+    wl = workloads.make_prefill_workload(n_seqs, hn, gn, hd, prefix, prefix, chunk, chunk, seed=n_seqs + chunk)
+    _hold(wl, gpu, causal=causal)
