@@ -19,6 +19,41 @@ HOST_PATH = LIB_PATH.parent / "_host.so"
 IC_OK = 0
 IC_DTYPE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
+# Call descriptors, field by field as in the header (tests hold them to it).
+_FIELDS = {
+    "ic_step_linear_call": (
+        ("out norm_out", c_void_p), ("out_stride norm_out_stride", c_int64), ("x", c_void_p), ("x_stride", c_int64),
+        ("w bias", c_void_p), ("w_stride", c_int64), ("w2 bias2", c_void_p), ("w2_stride", c_int64),
+        ("residual", c_void_p), ("residual_stride", c_int64), ("norm_weight norm_bias", c_void_p), ("m k n n2", c_int),
+        ("norm act", c_int), ("eps", c_float), ("dtype tile_bytes splits", c_int), ("k_pool v_pool", c_void_p),
+        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("hn gn hd block_size", c_int),
+        ("slot_mapping positions cos_table sin_table", c_void_p), ("table_rows", c_int64), ("workspace", c_void_p),
+        ("workspace_bytes", c_size_t)),
+    "ic_append_call": (
+        ("k_new v_new", c_void_p), ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
+        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("slot_mapping", c_void_p),
+        ("n_tokens", c_int64), ("gn hd block_size dtype", c_int), ("positions cos_table sin_table", c_void_p),
+        ("table_rows", c_int64), ("zero_out", c_void_p), ("zero_stride_bytes", c_int64), ("rows", c_void_p),
+        ("n_rows", c_int64), ("bounds", c_void_p), ("zero_row_bytes n_seqs row_pitch", c_int)),
+    "ic_prefill_call": (
+        ("out", c_void_p), ("out_stride_token", c_int64), ("q", c_void_p), ("q_stride_token", c_int64), ("k_pool v_pool", c_void_p),
+        ("pool_stride_block pool_stride_head pool_stride_token", c_int64), ("block_tables", c_void_p),
+        ("block_table_stride", c_int64), ("context_lens cu_seqlens_q", c_void_p),
+        ("n_seqs max_chunk_len hn gn hd block_size", c_int), ("num_blocks", c_int64), ("scale", c_float),
+        ("causal dtype uniform_context", c_int), ("row_pitch", c_int64), ("rows", c_void_p), ("n_rows q_rows", c_int64),
+        ("positions cos_table sin_table", c_void_p), ("table_rows", c_int64), ("mask_bits mask_lists", c_void_p),
+        ("mask_plane_seq mask_plane_head", c_int)),
+    "ic_decode_append_call": (
+        ("out", c_void_p), ("out_stride_seq", c_int64), ("q", c_void_p), ("q_stride_seq", c_int64), ("k_new v_new", c_void_p),
+        ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
+        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("block_tables", c_void_p),
+        ("block_table_stride", c_int64), ("context_lens slot_mapping positions cos_table sin_table", c_void_p),
+        ("table_rows", c_int64), ("n_seqs hn gn hd block_size max_context_len", c_int), ("scale", c_float),
+        ("dtype", c_int)),
+}
+STRUCTS = {name: type(name, (ctypes.Structure,), {"_fields_": [(n, t) for names, t in rows for n in names.split()]})
+           for name, rows in _FIELDS.items()}
+
 # name -> (restype, argtypes); mirrors include/ironcore_paged.h one to one.
 SIGNATURES = {
     "ic_version": (c_int, []),

@@ -24,6 +24,23 @@ def test_header_and_binding_agree():
     assert declared == sorted(_lib.SIGNATURES)
 
 
+C_TYPES = {"float": ctypes.c_float, "size_t": ctypes.c_size_t, "int": ctypes.c_int, "int64_t": ctypes.c_int64}
+
+
+@pytest.mark.parametrize("name", sorted(_lib.STRUCTS))
+def test_descriptors_are_the_header_s(name):
+    text = re.sub(r"/\*.*?\*/", "", HEADER.read_text(), flags=re.S)
+    body = re.search(r"typedef struct %s \{(.*?)\} %s;" % (name, name), text, flags=re.S).group(1)
+    want = []
+    for line in body.split(";")[:-1]:
+        first, *others = line.split(",")
+        base, field = re.match(r"\s*(?:const\s+)?(\w+)\s*(.*)", first, flags=re.S).groups()
+        for f in (field, *others):
+            pointer, field = re.match(r"\s*(\*?)\s*(\w+)\s*$", f).groups()
+            want.append((field, ctypes.c_void_p if pointer else C_TYPES[base]))
+    assert _lib.STRUCTS[name]._fields_ == want
+
+
 def test_library_exports_every_declared_symbol():
     lib = _lib.load()
     for name in _declared_functions():

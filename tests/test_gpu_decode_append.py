@@ -1,7 +1,6 @@
 """A decode step's append inside the attention launch (paged_decode_pair_kernel, APPEND): the same bits, in
 outputs and pools, as the append and the attention one after the other, whoever's context a new row is in."""
 import ctypes
-from ctypes import c_float, c_int, c_int64, c_void_p
 
 import pytest
 import torch
@@ -23,15 +22,7 @@ def _separately(query, key, value, pools, tables, lens, slots, longest, scale, p
                                  emb.sin_emb)
     return paged_ops.paged_decode(q, *pools, tables, lens, longest, scale=scale).view(b, 1, hn * hd)
 
-
-class Call(ctypes.Structure):
-    _fields_ = [(n, t) for names, t in (
-        ("out", c_void_p), ("out_stride_seq", c_int64), ("q", c_void_p), ("q_stride_seq", c_int64), ("k_new v_new", c_void_p),
-        ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
-        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("block_tables", c_void_p),
-        ("block_table_stride", c_int64), ("context_lens slot_mapping positions cos_table sin_table", c_void_p),
-        ("table_rows", c_int64), ("n_seqs hn gn hd block_size max_context_len", c_int), ("scale", c_float),
-        ("dtype", c_int)) for n in names.split()]
+Call = _lib.STRUCTS["ic_decode_append_call"]
 
 
 def _together(query, key, value, pools, tables, lens, slots, longest, scale, positions, emb):

@@ -2,7 +2,6 @@
 sweep, against the same chunks numbered sequence by sequence; the append's launch with the zeroing beside it."""
 import ctypes
 import json
-from ctypes import c_float, c_int, c_int64, c_void_p
 
 import pytest
 import torch
@@ -12,25 +11,8 @@ from ironcore_amd.layers import RotaryPositionalEmbedding
 
 pytestmark = pytest.mark.gpu
 
-
-class Prefill(ctypes.Structure):
-    _fields_ = [(n, t) for names, t in (
-        ("out", c_void_p), ("out_stride_token", c_int64), ("q", c_void_p), ("q_stride_token", c_int64), ("k_pool v_pool", c_void_p),
-        ("pool_stride_block pool_stride_head pool_stride_token", c_int64), ("block_tables", c_void_p),
-        ("block_table_stride", c_int64), ("context_lens cu_seqlens_q", c_void_p),
-        ("n_seqs max_chunk_len hn gn hd block_size", c_int), ("num_blocks", c_int64), ("scale", c_float),
-        ("causal dtype uniform_context", c_int), ("row_pitch", c_int64), ("rows", c_void_p), ("n_rows q_rows", c_int64),
-        ("positions cos_table sin_table", c_void_p), ("table_rows", c_int64), ("mask_bits mask_lists", c_void_p),
-        ("mask_plane_seq mask_plane_head", c_int)) for n in names.split()]
-
-
-class Append(ctypes.Structure):
-    _fields_ = [(n, t) for names, t in (
-        ("k_new v_new", c_void_p), ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
-        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("slot_mapping", c_void_p),
-        ("n_tokens", c_int64), ("gn hd block_size dtype", c_int), ("positions cos_table sin_table", c_void_p),
-        ("table_rows", c_int64), ("zero_out", c_void_p), ("zero_stride_bytes", c_int64), ("rows", c_void_p),
-        ("n_rows", c_int64), ("bounds", c_void_p), ("zero_row_bytes n_seqs row_pitch", c_int)) for n in names.split()]
+Prefill = _lib.STRUCTS["ic_prefill_call"]
+Append = _lib.STRUCTS["ic_append_call"]
 
 
 def _attend(d, hn, gn, hd, causal, rows, positions, emb, out, q):

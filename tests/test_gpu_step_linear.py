@@ -2,7 +2,6 @@
 form against float64 at the edges of tiles, steps and splits; the native step of a model
 against its modules; what is left to the modules."""
 import ctypes
-from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p
 
 import pytest
 import torch
@@ -18,16 +17,7 @@ DTYPES = [torch.bfloat16, torch.float16, torch.float32]
 # one rounding to the element type (2^-9, 2^-12; the norm takes a rounded row: two); fp32: sums of 2 080 products
 TOL = {torch.bfloat16: 5e-3, torch.float16: 6e-4, torch.float32: 1e-6}
 
-
-class Call(ctypes.Structure):
-    _fields_ = [(n, t) for names, t in (
-        ("out norm_out", c_void_p), ("out_stride norm_out_stride", c_int64), ("x", c_void_p), ("x_stride", c_int64),
-        ("w bias", c_void_p), ("w_stride", c_int64), ("w2 bias2", c_void_p), ("w2_stride", c_int64),
-        ("residual", c_void_p), ("residual_stride", c_int64), ("norm_weight norm_bias", c_void_p), ("m k n n2", c_int),
-        ("norm act", c_int), ("eps", c_float), ("dtype tile_bytes splits", c_int), ("k_pool v_pool", c_void_p),
-        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("hn gn hd block_size", c_int),
-        ("slot_mapping positions cos_table sin_table", c_void_p), ("table_rows", c_int64), ("workspace", c_void_p),
-        ("workspace_bytes", c_size_t)) for n in names.split()]
+Call = _lib.STRUCTS["ic_step_linear_call"]
 
 
 def _run(gpu, call, dtype):
