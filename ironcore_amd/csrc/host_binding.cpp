@@ -213,8 +213,9 @@ bool rope_append(const Tensor &key, const Tensor &value, const Pool &p, const Te
                                    r.cos, r.sin, r.rows, n, (int)p.gn, (int)p.hd, (int)p.bs, p.nb, p.dtype, stream));
 }
 
-// One cached decode step of a layer (sq == 1): append, then attend.  With rotary tables the query is
-// rotated into a tensor of its own and the keys on their way into the pool.
+// One cached decode step of a layer (sq == 1): append and attention in one launch where the library takes both together
+// (small batches of short contexts), else one after the other, with rotary tables the query rotated into a tensor of its
+// own and the keys on their way into the pool.
 OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
                       const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
                       int64_t max_ctx, double scale, int64_t cohort, const OptTensor &shared,

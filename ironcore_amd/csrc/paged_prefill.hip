@@ -513,7 +513,8 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(const Pr
   const float lt = l_a + l_b;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   // Out in whole rows of the head, CPR lanes to a row, through LDS (as the MFMA lays them out a store touches 32
-  // cache lines for 512 bytes): the tiles are done with.  16 x 512 rows behind up to 4 096, 32 heads: 372 -> 365 us.
+  // cache lines for 512 bytes): the tiles are done with.  16 x 512 rows behind up to 4 096, 32 heads, with
+  // the append: 373.9 -> 362.2 us in turn on one box (a clock held by power moves the launch as much between runs).
   __syncthreads();
   char *const s_o = &s_k[0][0] + wave * 32 * ROWB;  // (256 rows: as many as the K buffers hold)
 #pragma unroll

@@ -17,7 +17,8 @@
 //    workgroups and a second launch adds the partial sums (fp32) in a fixed order, with everything that follows.
 //    A norm needs whole rows, so its launch has a workgroup to a row, and the product before it is always split.
 //
-// A layer is 7-9 launches instead of 17-19.  GPT-2 small, fp32, batch 4, 128 + 64 tokens by graph replay 66.5 -> 45.3 ms;
+// A layer with plain attention is 7-10 launches instead of 17-19: 2 for each product with a norm, 1 or 2 (split) for the
+// projections and the up-projection, 1 or 2 for attention.  GPT-2 small, fp32, batch 4, 128 + 64 tokens by graph replay 66.5 -> 45.3 ms;
 // a Llama-dims step (four layers, batch 16, bf16) 866 -> 768 us; one of 2 layers, d_model 2 048, 321 -> 140.
 #include "ic_device.h"
 #include "ic_internal.h"
