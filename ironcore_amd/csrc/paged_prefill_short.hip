@@ -636,15 +636,17 @@ bool prefill_takes_short(const PrefillArgs &a) {
 //                  all keys       5.8 / 5.1    9.8 / 10.5   11.6 / 12.3   17.5 / 18.1   25.2 / 28.3   23.5 / 27.9   24.3 / 26.2
 //             packed documents    6.3 / 5.6   10.7 / 9.9    11.4 / 11.2   14.7 / 14.5   26.1 / 26.9   22.8 / 24.1   17.4 / 18.9
 //   80 x 129, 12 / 12 of 64, causal (1 920 workgroups): 18.8 / 20.8; packed, 60 x 20, 64 / 8 of 128: 44.1 / 38.1.
+// (A packed mask at head dim 64 loses where two tile groups share the tiles, 2 x 1 024 tokens of 16 heads 13.0 / 13.3, 1 x 700 of 12
+// 10.0 / 10.3, and gains in the larger grids without, 3 x 1 500 of 12 heads 21.2 / 20.2.)
 // Grouped heads put one row block of several heads into a workgroup, which reaches equally far, where this numbers head
 // by head: only in grids of a workgroup to a CU (8 / 1 of 64, causal, 8 x 70 6.1 / 5.6, 3 x 300 9.5 / 8.7, 2 x 1 024 23 % faster
 // by whole rows; at head dim 128, 28 / 4, causal, 8 x 70 8.1 / 7.7, 1 x 20 9 % faster by whole rows).
-bool prefill_rows_direct(const PrefillArgs &a, int64_t wgs) {
+bool prefill_rows_direct(const PrefillArgs &a, int64_t wgs, bool two_groups) {
   if (a.positions != nullptr) return false;
   const int64_t cus = device_cu_count(), ctx = context_bound(a);
   const bool packed = a.mask_bits != nullptr;
   if (a.hn > a.gn && !packed) return wgs <= cus && (a.hd < 128 ? ctx <= 512 : a.causal && ctx > 64 && ctx <= 128);
-  if (a.hd < 128) return packed || ctx <= 64 || wgs <= (a.causal ? 4 : 1) * cus;
+  if (a.hd < 128) return packed ? !two_groups : ctx <= 64 || wgs <= (a.causal ? 4 : 1) * cus;
   if (ctx <= 64) return true;
   if (packed) return a.max_chunk_len <= 128 && wgs <= 5 * cus;
   return a.causal ? ctx <= 320 && 2 * wgs <= 5 * cus : ctx <= 128 && wgs <= cus;
@@ -691,7 +693,7 @@ int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t s
   const int64_t ctx = context_bound(a);
   const bool split = (wgs <= cus && ctx > 512) || (a.hd < 128 && wgs <= 2 * cus && ctx >= 2048);
   const bool bf16 = a.dtype == IC_DTYPE_BF16;
-  if (!kp.by_sweep && prefill_rows_direct(a, per_unit * kp.n_units))
+  if (!kp.by_sweep && prefill_rows_direct(a, per_unit * kp.n_units, split))
     return bf16 ? launch_short_type<MmaBf16, true>(kp, a, (unsigned)wgs, split, stream)
                 : launch_short_type<MmaF16, true>(kp, a, (unsigned)wgs, split, stream);
   return bf16 ? launch_short_type<MmaBf16, false>(kp, a, (unsigned)wgs, split, stream)
