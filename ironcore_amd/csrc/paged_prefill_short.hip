@@ -34,7 +34,7 @@
 //    the byte mask of the long kernel (32 byte loads per lane and tile, every tile
 //    walked), 11.9 us here, launch to launch.
 //
-//  * In full grids and with rotary, query rows and outputs move as whole rows of a head and change places in LDS: as
+//  * In full grids, and with rotary from a few rows on, query rows and outputs move as whole rows of a head and change places in LDS: as
 //    the MFMA lays them out a load touched 32 cache lines for 1 KiB, rotary tables likewise (query rows ready after 3.8
 //    instead of 5.3 us of a workgroup's 17; 80 sequences of 129 tokens, 12 heads of 64: 20.8 -> 18.8 us).  The others
 //    (DIRECT, prefill_rows_direct) load and store them as they are needed.
@@ -119,8 +119,8 @@ __device__ __forceinline__ bool pick_by_sweep(const PrefillKP &p, int index, int
   return true;
 }
 
-// DIRECT: query rows and outputs move as the MFMA lays them out, and the row blocks of a head side by side; no rotary
-// (see prefill_rows_direct).
+// DIRECT: query rows and outputs move as the MFMA lays them out, and the row blocks of a head side by side (see
+// prefill_rows_direct).
 template <class M, int HD, bool SINGLE, int TG, bool PACKED, bool DIRECT>
 __global__ __launch_bounds__(TG *kShortWaves *kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 2 : 4)))
 void paged_prefill_short_kernel(const PrefillKP p) {
@@ -213,6 +213,12 @@ void paged_prefill_short_kernel(const PrefillKP p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[ks] = load16(p.q + ((int64_t)my_row * p.q_stride_token + (int64_t)h * HD + ks * 16 + hh * 8) * 2);
+    if (!PACKED && p.positions != nullptr) {
+      const int64_t trig = (int64_t)rope_position(p, my_row) * p.half_hd + hh * 4;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        qf[ks] = rotate_chunk<typename M::E>(qf[ks], p.cos_table + trig + ks * 8, p.sin_table + trig + ks * 8);
+    }
   } else {
     int table_row_of_mine = 0;
     if (p.positions != nullptr) table_row_of_mine = rope_position(p, my_row);
@@ -624,10 +630,17 @@ bool prefill_takes_short(const PrefillArgs &a) {
   return !(filled && ctx >= 2 * (int64_t)a.max_chunk_len && ctx >= (a.hn > a.gn ? 2200 : 1250));
 }
 
+namespace {
+// A few query rows to a chunk, which gain nothing from being moved as whole rows (figures below).
+bool few_rows(const PrefillArgs &a) { return a.max_chunk_len <= (a.hd == 128 && a.hn > a.gn ? 4 : 8); }
+
 // Whether query rows and outputs move as the MFMA lays them out, without the exchange in LDS: that exchange costs a
 // workgroup half a microsecond of latency and saves its CU's cache look-ups, so it loses where the launch is over in a few
-// tiles or leaves the CUs a workgroup or two.  Rotary tables gain from whole rows at every size.  us by whole rows / directly
-// (calls without a cache):
+// tiles or leaves the CUs a workgroup or two.  Rotary tables are read by whole rows too, which gains from a few rows on:
+// chunks of 2 / 4 / 8 / 16 / 32 rows (1-42 sequences, nothing to 2 000 cached tokens, append and attention) take 4.5 / 3 / 2 /
+// -1.5 / -9 % more by whole rows at head dim 128, 2 / 1.5 / -1 / -7 / -14 % with grouped heads (42 x 2, 8 / 8 heads of 128:
+// 15.7 / 14.4 us), 4 / 3 / 2 / 0 / -6 % at 64.  As few rows without rotary gain alike (64 x 3, 16 / 4 heads of 128: 13.8 / 13.2).
+// More rows without it, us by whole rows / directly (calls without a cache):
 //   sequences x tokens            1 x 20       18 x 70       3 x 300       4 x 500       60 x 100      30 x 130      2 x 1 024
 //   12 / 12 heads of 64, causal   4.9 / 4.3    6.6 / 5.7     9.3 / 8.2    13.0 / 11.7   11.5 / 10.9   10.1 / 10.1   16.4 / 16.4
 //                  all keys       5.0 / 4.3    6.5 / 6.0     9.5 / 9.0    13.2 / 12.5   11.6 / 12.1   11.7 / 12.9   16.5 / 16.4
@@ -642,15 +655,17 @@ bool prefill_takes_short(const PrefillArgs &a) {
 // by head: only in grids of a workgroup to a CU (8 / 1 of 64, causal, 8 x 70 6.1 / 5.6, 3 x 300 9.5 / 8.7, 2 x 1 024 23 % faster
 // by whole rows; at head dim 128, 28 / 4, causal, 8 x 70 8.1 / 7.7, 1 x 20 9 % faster by whole rows).
 bool prefill_rows_direct(const PrefillArgs &a, int64_t wgs, bool two_groups) {
-  if (a.positions != nullptr) return false;
   const int64_t cus = device_cu_count(), ctx = context_bound(a);
   const bool packed = a.mask_bits != nullptr;
+  if (!packed && few_rows(a)) return true;
+  if (a.positions != nullptr) return false;
   if (a.hn > a.gn && !packed) return wgs <= cus && (a.hd < 128 ? ctx <= 512 : a.causal && ctx > 64 && ctx <= 128);
   if (a.hd < 128) return packed ? !two_groups : ctx <= 64 || wgs <= (a.causal ? 4 : 1) * cus;
   if (ctx <= 64) return true;
   if (packed) return a.max_chunk_len <= 128 && wgs <= 5 * cus;
   return a.causal ? ctx <= 320 && 2 * wgs <= 5 * cus : ctx <= 128 && wgs <= cus;
 }
+}  // namespace
 
 int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t stream) {
   const int64_t per_unit = short_workgroups_per_unit(a);
@@ -675,7 +690,8 @@ int launch_paged_prefill_short(PrefillKP kp, const PrefillArgs &a, hipStream_t s
   // (954 sizes measured, 2-60 sequences, 1-32 KV heads: by this line 2.2 % less time than by unit throughout, 2.9 % less
   // than by sweep throughout, 0.5 % more than the better of the two.)
   const int64_t xcd_cus = device_cu_count() / kXcds;
-  kp.by_sweep = a.rows != nullptr && a.mask_bits == nullptr && a.n_seqs <= kWave &&
+  // (Few rows to a chunk: directly, below, which gains more: 26 chunks of 3-8, 32 / 32 heads of 128: 39.3 / 37.3.)
+  kp.by_sweep = a.rows != nullptr && a.mask_bits == nullptr && a.n_seqs <= kWave && !few_rows(a) &&
                 (per_unit > xcd_cus || slices * per_unit > xcd_cus * (a.hd == 128 ? 2 : 4));
   if (kp.by_sweep) {  // (at most so many workgroups, a sequence's last one and row block not full)
     const int64_t blocks = a.n_rows / 32 + a.n_seqs;

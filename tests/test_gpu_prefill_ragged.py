@@ -74,6 +74,27 @@ def test_by_sweep(gpu, n_seqs, hn, gn, hd, block, prefix, chunks, dtype, causal,
     assert (out[untouched] == 7).all()
 
 
+@pytest.mark.parametrize("hn,gn,hd,dtype", [(4, 4, 128, torch.bfloat16), (14, 2, 128, torch.float16), (6, 2, 64, torch.bfloat16),
+                                            (4, 4, 32, torch.float16)])
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9])
+@pytest.mark.parametrize("named", [False, True])
+def test_few_rows_rotated_on_their_way(gpu, hn, gn, hd, dtype, rows, named):
+    """Either side of the lines from which rotated query rows move as whole rows: the same bits as rows rotated before."""
+    wl = workloads.make_prefill_workload(3, hn, gn, hd, 0, 90, rows if not named else 1, rows, dtype=dtype, seed=rows)
+    wl.max_chunk_len = rows
+    d = wl.to(gpu)
+    paged_ops.kv_append(d.k_new, d.v_new, d.k_pool, d.v_pool, d.slot_mapping)
+    total = d.query.shape[0]
+    emb = RotaryPositionalEmbedding(hd, max_seq_len=100).to(gpu)
+    positions = torch.arange(total, dtype=torch.int32, device=gpu) * 7 - 2                       # clamped into the table
+    list_of_rows = torch.arange(total, device=gpu) if named else None
+    got, want = (torch.empty(total, hn * hd, dtype=dtype, device=gpu) for _ in range(2))
+    _attend(d, hn, gn, hd, True, list_of_rows, positions, emb, got, d.query)
+    before = emb(d.query.view(1, total, hn, hd), positions.clamp(min=0)).view(total, hn, hd)
+    _attend(d, hn, gn, hd, True, list_of_rows, positions, None, want, before)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n_seqs,width,gn,hd", [(1, 5, 1, 32), (3, 40, 2, 64), (2, 70, 33, 128)])
 @pytest.mark.parametrize("rope", [False, True])

@@ -71,6 +71,7 @@ def test_no_causal_rule_and_empty_chunks(gpu, chunk, prefix):
     (12, 12, 64, 85, 70, 0, True), (12, 12, 64, 86, 70, 0, True), (4, 4, 64, 64, 70, 0, False), (4, 4, 64, 65, 70, 0, False),
     # grouped: 512 tokens, a workgroup to a CU; a workgroup of two heads' and of three heads' blocks
     (8, 2, 64, 2, 100, 412, True), (8, 2, 64, 2, 100, 413, True), (8, 2, 64, 2, 33, 0, True), (6, 2, 64, 3, 70, 9, False),
+    (8, 2, 128, 2, 4, 700, True), (8, 2, 128, 2, 5, 700, True), (4, 4, 128, 2, 8, 700, False), (4, 4, 128, 2, 9, 700, False),
     (8, 1, 32, 1, 20, 0, True), (8, 2, 128, 2, 100, 0, True), (8, 2, 128, 2, 120, 9, True), (16, 2, 64, 40, 70, 0, True)])
 def test_rows_moved_directly_and_whole(gpu, hn, gn, hd, n_seqs, chunk, prefix, causal):
     """Either side of the lines between the two ways in which query rows and outputs move."""
