@@ -551,6 +551,61 @@ size_t ic_step_linear_workspace_bytes(const ic_step_linear_call *call);
 int ic_step_linear(const ic_step_linear_call *call, void *stream);
 
 /*
+ * All layers of a decode step in one launch, pre-LN, one new token a row: per layer the
+ * norm, [q | k | v] = x W + bias (rotated with cos_table and sin_table, k and v appended as
+ * by ic_kv_append), ic_paged_decode, output projection and residual, norm, up-projection
+ * with the activation, down-projection and residual; then out (or NULL) = the last
+ * layer's output and norm_out = its norm (norm IC_NORM_NONE: none, NULL).  Rounded to the element type
+ * where ic_step_linear calls round.
+ *
+ * For small models and batches; everything else is IC_ERR_UNSUPPORTED with nothing launched:
+ * m up to IC_STEP_STACK_ROWS, up to IC_STEP_STACK_LAYERS layers of one shape, d up to 1 024,
+ * heads of 64 or 128, at most 4 query heads to a KV head, contexts up to 2 048
+ * tokens.  Matrices [in, out] without gaps, 16-byte aligned; d, f, hn * hd and gn * hd
+ * multiples of 64 bytes of elements.  up_weight has 2 f columns [feature | gate] with a gated act.
+ *
+ *   workspace  ic_step_stack_workspace_bytes(call) bytes, 256-byte aligned (0: unsupported).
+ *   workgroups  0: one to a CU.  draw: nonzero deals the work by a counter, as the launch does
+ *          by itself when other work keeps its workgroups from starting together.
+ */
+#define IC_STEP_STACK_LAYERS 16
+#define IC_STEP_STACK_ROWS 16
+typedef struct ic_step_layer {
+  const void *input_norm_weight, *input_norm_bias;
+  const void *q_weight, *q_bias, *kv_weight, *kv_bias;
+  const void *proj_weight, *proj_bias;
+  const void *post_norm_weight, *post_norm_bias;
+  const void *up_weight, *up_bias, *down_weight, *down_bias;
+  void *k_pool, *v_pool;
+  int input_norm, post_norm;
+  float input_norm_eps, post_norm_eps;
+} ic_step_layer;
+typedef struct ic_step_stack_call {
+  const ic_step_layer *layers;
+  const void *x;
+  void *out, *norm_out;
+  const void *norm_weight, *norm_bias;
+  int num_layers, m, d, f, hn, gn, hd, act;
+  int norm;
+  float eps;
+  int64_t pool_stride_block, pool_stride_head, pool_stride_token, num_blocks;
+  const int32_t *block_tables;
+  int64_t block_table_stride;
+  const int32_t *context_lens;
+  const int64_t *slot_mapping;
+  const int32_t *positions;
+  const float *cos_table, *sin_table;
+  int64_t table_rows;
+  int block_size, max_context_len;
+  float scale;
+  int dtype, workgroups, draw;
+  void *workspace;
+  size_t workspace_bytes;
+} ic_step_stack_call;
+size_t ic_step_stack_workspace_bytes(const ic_step_stack_call *call);
+int ic_step_stack(const ic_step_stack_call *call, void *stream);
+
+/*
  * The append of a step's chunks in one launch: ic_kv_append, or with cos_table and
  * sin_table ic_rope_kv_append_to without queries, and with zero_out not NULL
  * ic_zero_unlisted_rows (zero_out, zero_stride_bytes, zero_row_bytes, rows, n_rows, bounds,

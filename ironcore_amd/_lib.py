@@ -29,6 +29,16 @@ _FIELDS = {
         ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("hn gn hd block_size", c_int),
         ("slot_mapping positions cos_table sin_table", c_void_p), ("table_rows", c_int64), ("workspace", c_void_p),
         ("workspace_bytes", c_size_t)),
+    "ic_step_layer": (
+        ("input_norm_weight input_norm_bias q_weight q_bias kv_weight kv_bias proj_weight proj_bias", c_void_p),
+        ("post_norm_weight post_norm_bias up_weight up_bias down_weight down_bias k_pool v_pool", c_void_p),
+        ("input_norm post_norm", c_int), ("input_norm_eps post_norm_eps", c_float)),
+    "ic_step_stack_call": (
+        ("layers x out norm_out norm_weight norm_bias", c_void_p), ("num_layers m d f hn gn hd act norm", c_int), ("eps", c_float),
+        ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("block_tables", c_void_p),
+        ("block_table_stride", c_int64), ("context_lens slot_mapping positions cos_table sin_table", c_void_p),
+        ("table_rows", c_int64), ("block_size max_context_len", c_int), ("scale", c_float), ("dtype workgroups draw", c_int),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t)),
     "ic_append_call": (
         ("k_new v_new", c_void_p), ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
         ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("slot_mapping", c_void_p),
@@ -133,6 +143,8 @@ SIGNATURES = {
         c_void_p, c_size_t, c_int, c_void_p]),  # workspace, workspace_bytes, dtype, stream
     "ic_step_linear_workspace_bytes": (c_size_t, [c_void_p]),   # call descriptor
     "ic_step_linear": (c_int, [c_void_p, c_void_p]),    # call descriptor, stream
+    "ic_step_stack_workspace_bytes": (c_size_t, [c_void_p]),   # call descriptor
+    "ic_step_stack": (c_int, [c_void_p, c_void_p]),     # call descriptor, stream
     "ic_append_chunks": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_paged_decode_append": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_greedy_workspace_bytes": (c_size_t, [c_int, c_int]),   # rows, n

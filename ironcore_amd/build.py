@@ -23,7 +23,7 @@ HOST_PATH = LIB_DIR / "_host.so"   # native call path (csrc/host_binding.cpp), l
 OBJ_DIR = PKG / "build" / "obj"
 
 SOURCES = ["ic_api.hip", "kv_append.hip", "rope_kv_append.hip", "paged_decode.hip", "paged_decode_mfma.hip", "paged_prefill.hip",
-           "paged_prefill_short.hip", "paged_prefill_f32.hip", "mask_pack.hip", "linear_rows.hip", "step_linear.hip", "choose_token.hip", "mfma_probe.hip"]
+           "paged_prefill_short.hip", "paged_prefill_f32.hip", "mask_pack.hip", "linear_rows.hip", "step_linear.hip", "step_stack.hip", "choose_token.hip", "mfma_probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

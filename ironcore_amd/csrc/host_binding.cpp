@@ -610,6 +610,109 @@ c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
   return std::make_tuple(out, out_normed);
 }
 
+// All layers of a decode step and the norm behind them in one launch (ic_step_stack; more layers than one call holds: in
+// equal parts).  `w`: a layer's weights and biases as decoder_layer takes them, but for the next norm; `norms`: its input
+// norm and its post-attention norm as (kind, eps, weight, bias).  None for what the call does not take, and where the
+// layers' own launches are as fast (stack_pays).
+using Norm = std::tuple<int64_t, double, Tensor, OptTensor>;
+
+// us a layer and token, two rows, 64 to 364 tokens, launches / stack: fp32 d 768, ffn 3 072 36.2 / 26.3, 512 x 2 048 30.5 / 22.3,
+// 256 x 1 024 26.1 / 21.4; bf16 768 x 3 072 32 / 23.5.  Four layers, d 1 024, 16 bits, the step with the output layer: 8 / 8 heads
+// of 128, up to 890 tokens, batch 2 181 / 119, 200 tokens, 10 198 / 138, 1 500 tokens, 16 239 / 213.  A pair's rows are walked by
+// one workgroup and grouped heads cost it vector work, so these have the limit that the attention launch has: 8 / 2
+// heads, 611 tokens, batch 10 205 / 211, 2 048 tokens, 3 210 / 278.  Below 2 MB of weights a layer (256 x 352 24.4 / 20.6) there
+// is little to prefetch, and the layers stay calls of their own, any of which may be a module's.
+bool stack_pays(int64_t group, int64_t max_ctx, int64_t row_bytes, int64_t layer_bytes) {
+  const int64_t rounds = (max_ctx + 127) / 128;
+  if (layer_bytes < 2000000 || group > 4) return false;
+  return group == 1 ? rounds <= 16 && rounds * row_bytes <= 4096 : rounds <= 4;
+}
+
+OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor>> &w,
+                        const std::vector<std::tuple<Norm, Norm>> &norms, const Norm &last, int64_t hn, int64_t gn,
+                        int64_t hd, int64_t act, const std::vector<std::tuple<Tensor, Tensor>> &pools, const Tensor &tables,
+                        const Tensor &lens, const Tensor &slots, int64_t max_ctx, double scale, const OptTensor &positions,
+                        const OptTensor &cos, const OptTensor &sin, int64_t device, int64_t stream) {
+  const at::ScalarType type = x.scalar_type();
+  const size_t layers = w.size();
+  if (layers == 0 || norms.size() != layers || pools.size() != layers || x.dim() != 3 || x.size(1) != 1 ||
+      !step_tensor(x, type, device) || !x.is_contiguous() || dtype_code(type) < 0 || step_outside_torch())
+    return c10::nullopt;
+  const int64_t b = x.size(0), d = x.size(2), q_cols = hn * hd, kv_cols = gn * hd;
+  const int es = (int)x.element_size();
+  if (b < 1 || b > IC_STEP_STACK_ROWS || gn < 1 || !rows16(x.data_ptr(), d, d, es) || w[0].size() != 12 || !w[0][8].has_value() ||
+      w[0][8]->dim() != 2 || !index_vector(slots, at::kLong, b, device))
+    return c10::nullopt;
+  const int64_t up_cols = w[0][8]->size(1), f = act >= IC_ACT_GLU ? up_cols / 2 : up_cols;
+  if (up_cols > (1 << 20) || (act >= IC_ACT_GLU && up_cols % 2 != 0) ||
+      !stack_pays(hn / gn, max_ctx, hd * es, d * (2 * q_cols + 2 * kv_cols + up_cols + f) * es))
+    return c10::nullopt;
+  const Pool first(std::get<0>(pools[0]), std::get<1>(pools[0]), device);
+  const OptTensor none;
+  const Decode dec{tables, lens, max_ctx, 0, 1, none, scale};
+  const Rope rope(positions, cos, sin, b, hd, device);
+  if (!first.ok || !rope.ok || first.gn != gn || first.hd != hd || std::get<0>(pools[0]).scalar_type() != type ||
+      !decode_fits(first, b, hn, dec, device))
+    return c10::nullopt;
+  auto matrix = [&](const OptTensor &t, int64_t k, int64_t n) {
+    return step_matrix(t, k, n, type, device) && t->stride(0) == n;
+  };
+  auto norm_fits = [&](const Norm &n) {
+    return step_vector(std::get<2>(n), d, type, device) && step_vector(std::get<3>(n), d, type, device);
+  };
+  if (!norm_fits(last)) return c10::nullopt;
+  std::vector<ic_step_layer> table(layers);
+  for (size_t i = 0; i < layers; ++i) {
+    const auto &t = w[i];
+    const Norm &in = std::get<0>(norms[i]), &post = std::get<1>(norms[i]);
+    const Pool p(std::get<0>(pools[i]), std::get<1>(pools[i]), device);
+    if (t.size() != 12 || !matrix(t[0], d, q_cols) || !step_vector(t[1], q_cols, type, device) || !matrix(t[2], d, 2 * kv_cols) ||
+        !step_vector(t[3], 2 * kv_cols, type, device) || !matrix(t[4], q_cols, d) || !step_vector(t[5], d, type, device) ||
+        !matrix(t[8], d, up_cols) || !step_vector(t[9], up_cols, type, device) || !matrix(t[10], f, d) ||
+        !step_vector(t[11], d, type, device) || !norm_fits(in) || !norm_fits(post) || !p.ok || p.gn != gn || p.hd != hd ||
+        p.bs != first.bs || p.nb != first.nb || p.sb != first.sb || p.sh != first.sh || p.st != first.st ||
+        p.dtype != first.dtype)
+      return c10::nullopt;
+    ic_step_layer &l = table[i];
+    l.input_norm_weight = std::get<2>(in).data_ptr(), l.input_norm_bias = data(std::get<3>(in));
+    l.q_weight = data(t[0]), l.q_bias = data(t[1]), l.kv_weight = data(t[2]), l.kv_bias = data(t[3]);
+    l.proj_weight = data(t[4]), l.proj_bias = data(t[5]);
+    l.post_norm_weight = std::get<2>(post).data_ptr(), l.post_norm_bias = data(std::get<3>(post));
+    l.up_weight = data(t[8]), l.up_bias = data(t[9]), l.down_weight = data(t[10]), l.down_bias = data(t[11]);
+    l.k_pool = const_cast<void *>(p.k), l.v_pool = const_cast<void *>(p.v);
+    l.input_norm = (int)std::get<0>(in), l.post_norm = (int)std::get<0>(post);
+    l.input_norm_eps = (float)std::get<1>(in), l.post_norm_eps = (float)std::get<1>(post);
+  }
+  ic_step_stack_call c = {};
+  c.m = (int)b, c.d = (int)d, c.f = (int)f, c.hn = (int)hn, c.gn = (int)gn, c.hd = (int)hd, c.act = (int)act;
+  c.pool_stride_block = first.sb, c.pool_stride_head = first.sh, c.pool_stride_token = first.st, c.num_blocks = first.nb;
+  c.block_tables = tables.data_ptr<int32_t>(), c.block_table_stride = tables.stride(0);
+  c.context_lens = lens.data_ptr<int32_t>(), c.slot_mapping = slots.data_ptr<int64_t>();
+  c.positions = rope.positions, c.cos_table = rope.cos, c.sin_table = rope.sin, c.table_rows = rope.rows;
+  c.block_size = (int)first.bs, c.max_context_len = (int)max_ctx, c.scale = (float)scale, c.dtype = first.dtype;
+  const size_t parts = (layers + IC_STEP_STACK_LAYERS - 1) / IC_STEP_STACK_LAYERS;
+  Tensor in = x, out, ws;
+  for (size_t part = 0, from = 0; part < parts; ++part) {
+    const size_t to = layers * (part + 1) / parts;
+    const bool end = part + 1 == parts;
+    c.layers = table.data() + from, c.num_layers = (int)(to - from);
+    out = at::empty({b, 1, d}, x.options());
+    c.x = in.data_ptr();
+    c.out = end ? nullptr : out.data_ptr(), c.norm_out = end ? out.data_ptr() : nullptr;
+    if (end) {
+      c.norm = (int)std::get<0>(last), c.eps = (float)std::get<1>(last);
+      c.norm_weight = std::get<2>(last).data_ptr(), c.norm_bias = data(std::get<3>(last));
+    }
+    c.workspace_bytes = ic_step_stack_workspace_bytes(&c);
+    if (c.workspace_bytes == 0) return c10::nullopt;
+    ws = at::empty({(int64_t)c.workspace_bytes}, x.options().dtype(at::kByte));
+    c.workspace = ws.data_ptr();
+    if (!made("ic_step_stack", ic_step_stack(&c, (void *)stream))) return c10::nullopt;
+    in = out, from = to;
+  }
+  return out;
+}
+
 // ---- greedy decoding --------------------------------------------------------------------------
 
 // The next token of each row of logits [b, n] and, wanted, how far it is ahead: stored into column `*column` of `tokens`
@@ -679,6 +782,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_rows", torch::wrap_pybind_function_no_gil(linear_rows));
   m.def("norm_rows", torch::wrap_pybind_function_no_gil(norm_rows));
   m.def("decoder_layer", torch::wrap_pybind_function_no_gil(decoder_layer));
+  m.def("decoder_stack", torch::wrap_pybind_function_no_gil(decoder_stack));
   m.def("greedy", torch::wrap_pybind_function_no_gil(greedy));
   m.def("advance", torch::wrap_pybind_function_no_gil(advance));
   m.def("pack_mask", torch::wrap_pybind_function_no_gil(pack_mask));

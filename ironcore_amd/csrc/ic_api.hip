@@ -565,6 +565,61 @@ int ic_step_linear(const ic_step_linear_call *call, void *stream) {
   return ic::launch_step_linear(a, static_cast<hipStream_t>(stream));
 }
 
+static int step_stack_sizes(const ic_step_stack_call &a) {
+  if (a.num_layers < 0 || a.m < 0 || a.d <= 0 || a.f <= 0 || a.hn <= 0 || a.gn <= 0 || a.hd <= 0 || a.block_size <= 0 ||
+      a.workgroups < 0 || a.max_context_len < 0)
+    return IC_ERR_BAD_SHAPE;
+  if (!dtype_ok(a.dtype) || a.norm < IC_NORM_NONE || a.norm > IC_NORM_RMS || a.act < IC_ACT_NONE || a.act > IC_ACT_SWIGLU)
+    return IC_ERR_UNSUPPORTED;
+  const int es = ic::elem_size(a.dtype), unit = 64 / es;
+  if (a.num_layers > IC_STEP_STACK_LAYERS || a.m > IC_STEP_STACK_ROWS || a.d > 1024 || a.d % unit != 0 ||
+      a.f % unit != 0 || a.f > (1 << 18) || a.hn > 4096 || a.hn % a.gn != 0 || a.hn / a.gn > 4 || (a.hd != 64 && a.hd != 128) ||
+      a.block_size % 16 != 0 || a.max_context_len > 2048 || a.workgroups > 4096)
+    return IC_ERR_UNSUPPORTED;
+  return IC_OK;
+}
+
+size_t ic_step_stack_workspace_bytes(const ic_step_stack_call *call) {
+  if (call == nullptr || call->m == 0 || call->num_layers == 0 || step_stack_sizes(*call) != IC_OK) return 0;
+  return ic::step_stack_workspace_bytes(*call);
+}
+
+int ic_step_stack(const ic_step_stack_call *call, void *stream) {
+  if (call == nullptr) return IC_ERR_NULL_POINTER;
+  const ic_step_stack_call &a = *call;
+  if (const int rc = step_stack_sizes(a); rc != IC_OK) return rc;
+  if (a.m == 0 || a.num_layers == 0) return IC_OK;
+  const int es = ic::elem_size(a.dtype);
+  if (a.num_blocks <= 0 || a.num_blocks * (a.block_size / 16) >= (int64_t)1 << 31 || a.pool_stride_block <= 0 ||
+      a.pool_stride_head <= 0 || a.pool_stride_token <= 0 ||
+      a.block_table_stride < ((int64_t)a.max_context_len + a.block_size - 1) / a.block_size)
+    return IC_ERR_BAD_SHAPE;
+  if (!a.layers || !a.x || (!a.out && a.norm == IC_NORM_NONE) || (a.norm != IC_NORM_NONE && (!a.norm_weight || !a.norm_out)) ||
+      !a.block_tables || !a.context_lens || !a.slot_mapping || (a.cos_table != nullptr) != (a.sin_table != nullptr) ||
+      (a.cos_table && (!a.positions || a.table_rows <= 0)))
+    return IC_ERR_NULL_POINTER;
+  bool whole = aligned16(a.x) && aligned16(a.out) && aligned16(a.norm_out) && aligned16(a.norm_weight) &&
+               aligned16(a.norm_bias) && stride16(a.pool_stride_block, es) && stride16(a.pool_stride_head, es) &&
+               stride16(a.pool_stride_token, es);
+  for (int i = 0; i < a.num_layers; ++i) {
+    const ic_step_layer &l = a.layers[i];
+    if (!l.input_norm_weight || !l.q_weight || !l.kv_weight || !l.proj_weight || !l.post_norm_weight || !l.up_weight ||
+        !l.down_weight || !l.k_pool || !l.v_pool)
+      return IC_ERR_NULL_POINTER;
+    if (l.input_norm < IC_NORM_LAYER || l.input_norm > IC_NORM_RMS || l.post_norm < IC_NORM_LAYER || l.post_norm > IC_NORM_RMS)
+      return IC_ERR_UNSUPPORTED;
+    for (const void *ptr : {l.input_norm_weight, l.input_norm_bias, l.q_weight, l.q_bias, l.kv_weight, l.kv_bias, l.proj_weight,
+                            l.proj_bias, l.post_norm_weight, l.post_norm_bias, l.up_weight, l.up_bias, l.down_weight,
+                            l.down_bias, (const void *)l.k_pool, (const void *)l.v_pool})
+      whole = whole && aligned16(ptr);
+  }
+  if (!whole) return IC_ERR_ALIGNMENT;
+  if (!a.workspace || reinterpret_cast<uintptr_t>(a.workspace) % 256 != 0 ||
+      a.workspace_bytes < ic::step_stack_workspace_bytes(a))
+    return IC_ERR_WORKSPACE;
+  return ic::launch_step_stack(a, static_cast<hipStream_t>(stream));
+}
+
 int ic_paged_decode_append(const ic_decode_append_call *call, void *stream) {
   if (call == nullptr) return IC_ERR_NULL_POINTER;
   const ic_decode_append_call &c = *call;

@@ -180,6 +180,8 @@ struct StepPlan {
   bool partial, rows;
 };
 StepPlan step_linear_plan(const ic_step_linear_call &a);
+size_t step_stack_workspace_bytes(const ic_step_stack_call &a);
+int launch_step_stack(const ic_step_stack_call &a, hipStream_t stream);
 size_t greedy_workspace_bytes(int rows, int n);
 int launch_greedy(const ic_greedy_call &a, hipStream_t stream);
 int launch_advance(const ic_advance_call &a, hipStream_t stream);

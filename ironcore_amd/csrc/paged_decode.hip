@@ -49,6 +49,7 @@
 // Algorithmic bytes per launch: sum_i ctx_i * 2 * gn * hd * elem (K and V,
 // once per KV head) + q, out, block-table entries and context lengths.
 #include "decode_common.h"
+#include "decode_pair.h"
 #include "rope_device.h"
 #include "../../include/ironcore_paged.h"
 
@@ -308,19 +309,12 @@ __global__ __launch_bounds__(NW *kWave) void paged_decode_kernel(const DecodeKP 
 // Short contexts (up to 2 048 tokens at most, see decode_takes_pairs for the lines): with shares of a tile
 // the split above turns them into partials that a second launch merges, 8 + 5 us of which the tiles themselves take
 // two (4 sequences of up to 160 tokens, 12 heads of 64, fp32: 13.0 us, here 3.8).  Here a workgroup owns a whole pair:
-// its eight waves take the pair's tiles in turn (a wave's table entries come in one load, one per lane: at most 64
-// tiles), keep the running softmax of the kernel above and merge through LDS; one launch, no workspace.  All types;
+// its eight waves take the pair's tiles in turn and merge through LDS (decode_pair.h); one launch, no workspace.  All types;
 // the arithmetic is the vector-ALU kernel's (fp32 probabilities and sums).
 // Bound by the chain of round trips: context length and table, tile, merge.
 //
 // APPEND: the step's append in the same launch (the layer call on 4 sequences of up to 192 tokens, 12 heads of 64,
-// fp32: 11.6 -> 8.0 us).  Each workgroup stores the new rows of its pair and rotates its query rows.  A new row may be
-// visible to any sequence (rows of one sequence at several positions, shared blocks), and another workgroup may store
-// it sooner or later than it is read here, so what a tile holds in a slot of this step is always taken from the new
-// rows: lane j has row j's slot (64 rows at most), and a tile compares its id with all of them at once.
-constexpr int kPairWaves = 8;
-constexpr int kPairAppendRows = kWave;
-
+// fp32: 11.6 -> 8.0 us).  Each workgroup stores the new rows of its pair and rotates its query rows.
 struct PairAppend {
   const char *k_new, *v_new;
   const int64_t *slots;
@@ -330,216 +324,64 @@ struct PairAppend {
 };
 
 template <class E, int HD, int GT, bool APPEND>
-__global__ __launch_bounds__(kPairWaves *kWave) void paged_decode_pair_kernel(const DecodeKP p, const PairAppend n) {
-  using T = typename E::type;
-  constexpr int EPL = E::EPL;
-  constexpr int ES = sizeof(T);
-  constexpr int LPR = HD / EPL;     // lanes sharing one token row
-  constexpr int RPL = kWave / LPR;  // token rows per load instruction
-  constexpr int BS = 16;
-  constexpr int NLD = BS / RPL;     // load instructions per tile
-  __shared__ __attribute__((aligned(16))) float s_acc[kPairWaves][GT][HD];
-  __shared__ float s_m[kPairWaves][GT], s_l[kPairWaves][GT];
-
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int col = lane % LPR;
-  const int rowg = lane / LPR;
-  const int seq = blockIdx.y;
-  const int kvh = blockIdx.x;
-  const int heads = p.group;  // (at most GT: groups are not cut here)
-  const int head0 = kvh * heads;
-
-  int ctx = p.context_lens[seq];
-  ctx = ctx < p.max_ctx ? ctx : p.max_ctx;
-  ctx = ctx < 0 ? 0 : ctx;
-  const int tiles = (ctx + BS - 1) / BS;
-  const int mine = __builtin_amdgcn_readfirstlane(tiles > wave ? (tiles - wave + kPairWaves - 1) / kPairWaves : 0);
+struct PairRows {
+  static constexpr bool kNew = APPEND, kLate = false;
+  static constexpr int EPL = E::EPL, ES = sizeof(typename E::type);
+  const DecodeKP &p;
+  const PairAppend &n;
+  const int seq, kvh, lane, col;
   // the step's new rows: lane j holds row j's slot, the wave this pair's own row (as it is stored)
   int64_t slot = -1;
   Vec16 own_k, own_v;
-  const int new_at = (kvh * HD + col * EPL) * ES;
-  auto table_row = [&](int j) {
+  __device__ __forceinline__ PairRows(const DecodeKP &p, const PairAppend &n, int seq, int kvh)
+      : p(p), n(n), seq(seq), kvh(kvh), lane(threadIdx.x & (kWave - 1)), col(lane % (HD / EPL)) {}
+  __device__ __forceinline__ int64_t table_row(int j) const {
     int64_t pos = n.positions[j];
     pos = pos < 0 ? 0 : pos;
     return (pos >= n.table_rows ? n.table_rows - 1 : pos) * (HD / 2) + col * (EPL / 2);
-  };
-  auto new_key = [&](int j) {
-    const Vec16 k = load16(n.k_new + j * n.new_stride_bytes + new_at);
+  }
+  __device__ __forceinline__ int new_at() const { return (kvh * HD + col * EPL) * ES; }
+  __device__ __forceinline__ Vec16 key(int j) const {
+    const Vec16 k = load16(n.k_new + j * n.new_stride_bytes + new_at());
     if (n.positions == nullptr) return k;
     const int64_t at = table_row(j);
     return rotate_chunk<E>(k, n.cos_table + at, n.sin_table + at);
-  };
-  if constexpr (APPEND) {
-    if (lane < p.n_seqs) slot = n.slots[lane];
-    if (slot >= n.num_slots) slot = -1;
-    own_k = new_key(seq);
-    own_v = load16(n.v_new + seq * n.new_stride_bytes + new_at);
   }
-  // lane r: byte offset of this wave's tile of round r, and the tile's number in the pool
-  int64_t tile_off = 0;
-  int tile_id = -1;
-  if (lane < mine) {
-    const int tile = wave + lane * kPairWaves;
-    const int blk = tile / p.tiles_per_block;
-    int64_t phys = p.block_tables[seq * p.bt_stride + blk];
-    // A corrupt table entry must not become an out-of-pool address.
-    phys = phys < 0 ? 0 : phys;
-    phys = phys >= p.num_blocks ? p.num_blocks - 1 : phys;
-    tile_off = (phys * p.stride_block + kvh * p.stride_head +
-                (int64_t)(tile - blk * p.tiles_per_block) * BS * p.stride_token) * ES;
-    if constexpr (APPEND) tile_id = (int)(phys * p.tiles_per_block) + tile - blk * p.tiles_per_block;
-  }
-  Vec16 qreg[GT];
-#pragma unroll
-  for (int g = 0; g < GT; ++g) {
-    const int h = head0 + (g < heads ? g : heads - 1);
-    qreg[g] = load16(p.q + (seq * p.q_stride_seq + (int64_t)h * HD + col * EPL) * ES);
+  __device__ __forceinline__ Vec16 value(int j) const { return load16(n.v_new + j * n.new_stride_bytes + new_at()); }
+  __device__ __forceinline__ void early() {
     if constexpr (APPEND) {
-      if (n.positions != nullptr) {
-        const int64_t at = table_row(seq);
-        qreg[g] = rotate_chunk<E>(qreg[g], n.cos_table + at, n.sin_table + at);
-      }
+      if (lane < p.n_seqs) slot = n.slots[lane];
+      if (slot >= n.num_slots) slot = -1;
+      own_k = key(seq);
+      own_v = value(seq);
     }
   }
-  uint32_t lane_off[NLD];
+  __device__ __forceinline__ void queries(Vec16 *qreg) const {
 #pragma unroll
-  for (int i = 0; i < NLD; ++i) lane_off[i] = (uint32_t)(((i * RPL + rowg) * p.stride_token + col * EPL) * ES);
-
-  float m[GT], l[GT], acc[GT][EPL];
-#pragma unroll
-  for (int g = 0; g < GT; ++g) {
-    m[g] = kNegInf;
-    l[g] = 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[g][e] = 0.f;
-  }
-  auto issue = [&](int r, Vec16 *kk, Vec16 *vv) {
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)tile_off, r);
-    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)tile_off >> 32), r);
-    const int64_t at = (int64_t)(((uint64_t)hi << 32) | lo);
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) kk[i] = load16(p.k_pool + at + lane_off[i]);
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) vv[i] = load16(p.v_pool + at + lane_off[i]);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto consume = [&](int r, Vec16 *kk, Vec16 *vv) {
-    if constexpr (APPEND) {
-      const int id = __builtin_amdgcn_readlane(tile_id, r);
-      uint64_t rows = __ballot(slot >= 0 && (int)(slot / BS) == id);
-      for (; rows != 0; rows &= rows - 1) {
-        const int j = __builtin_ctzll(rows);
-        const int token = __builtin_amdgcn_readlane((int)(slot % BS), j);
-        Vec16 k = own_k, v = own_v;
-        if (j != seq) k = new_key(j), v = load16(n.v_new + j * n.new_stride_bytes + new_at);
-#pragma unroll
-        for (int i = 0; i < NLD; ++i)
-          if (token == i * RPL + rowg) kk[i] = k, vv[i] = v;
-      }
-    }
-    float s[GT][NLD];
-#pragma unroll
-    for (int i = 0; i < NLD; ++i)
-#pragma unroll
-      for (int g = 0; g < GT; ++g) s[g][i] = group_sum<LPR>(E::dot(kk[i], qreg[g], 0.f)) * p.scale_log2e;
-    const int tok0 = (wave + r * kPairWaves) * BS;
-    if (tok0 + BS > ctx) {  // the sequence's last tile may be partly filled
-#pragma unroll
-      for (int i = 0; i < NLD; ++i) {
-        if (tok0 + i * RPL + rowg >= ctx) {
-#pragma unroll
-          for (int g = 0; g < GT; ++g) s[g][i] = kNegInf;
-          vv[i] = Vec16{{0u, 0u, 0u, 0u}};
+    for (int g = 0; g < GT; ++g) {
+      const int h = kvh * p.group + (g < p.group ? g : p.group - 1);
+      qreg[g] = load16(p.q + (seq * p.q_stride_seq + (int64_t)h * HD + col * EPL) * ES);
+      if constexpr (APPEND) {
+        if (n.positions != nullptr) {
+          const int64_t at = table_row(seq);
+          qreg[g] = rotate_chunk<E>(qreg[g], n.cos_table + at, n.sin_table + at);
         }
       }
     }
-    float vf[NLD][EPL];
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) E::widen(vv[i], vf[i]);
-#pragma unroll
-    for (int g = 0; g < GT; ++g) {
-      float mx = m[g];
-#pragma unroll
-      for (int i = 0; i < NLD; ++i) mx = fmaxf(mx, s[g][i]);
-      const float ms = (mx == kNegInf) ? 0.f : mx;
-      const float alpha = __builtin_amdgcn_exp2f(m[g] - ms);
-      float pr[NLD];
-      float ps = 0.f;
-#pragma unroll
-      for (int i = 0; i < NLD; ++i) {
-        pr[i] = __builtin_amdgcn_exp2f(s[g][i] - ms);
-        ps += pr[i];
-      }
-      l[g] = l[g] * alpha + ps;
-      m[g] = mx;
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        float a = acc[g][e] * alpha;
-#pragma unroll
-        for (int i = 0; i < NLD; ++i) a = __builtin_fmaf(pr[i], vf[i][e], a);
-        acc[g][e] = a;
-      }
-    }
-  };
-  Vec16 ka[NLD], va[NLD], kb[NLD], vb[NLD];
-  if (mine > 0) issue(0, ka, va);
-  if constexpr (APPEND) {
-    // the last wave has the fewest tiles; K from its first row of lanes, V from the second
-    const int64_t to = ((int64_t)__builtin_amdgcn_readlane((uint32_t)((uint64_t)slot >> 32), seq) << 32) |
-                       (uint32_t)__builtin_amdgcn_readlane((uint32_t)slot, seq);
-    if (wave == kPairWaves - 1 && to >= 0 && rowg < 2) {
-      const int64_t blk = (uint64_t)to / (uint32_t)(p.tiles_per_block * BS);
-      const int64_t at = blk * p.stride_block + kvh * p.stride_head + (to - blk * p.tiles_per_block * BS) * p.stride_token;
-      store16(const_cast<char *>(rowg == 0 ? p.k_pool : p.v_pool) + (at + col * EPL) * ES, rowg == 0 ? own_k : own_v);
-    }
   }
-  for (int r = 0; r < mine; r += 2) {
-    issue(r + 1 < mine ? r + 1 : r, kb, vb);
-    consume(r, ka, va);
-    if (r + 1 >= mine) break;
-    issue(r + 2 < mine ? r + 2 : r + 1, ka, va);
-    consume(r + 1, kb, vb);
-  }
+};
 
-  // ---- merge: the row groups of a wave by exchange, the waves through LDS ----------------------
-#pragma unroll
-  for (int g = 0; g < GT; ++g) {
-    float mx = m[g];
-#pragma unroll
-    for (int off = LPR; off < kWave; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-    const float w = (m[g] == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m[g] - mx);
-    float ls = l[g] * w;
-#pragma unroll
-    for (int off = LPR; off < kWave; off <<= 1) ls += __shfl_xor(ls, off, kWave);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      float a = acc[g][e] * w;
-#pragma unroll
-      for (int off = LPR; off < kWave; off <<= 1) a += __shfl_xor(a, off, kWave);
-      if (rowg == 0) s_acc[wave][g][col * EPL + e] = a;
-    }
-    if (lane == 0) {
-      s_m[wave][g] = mx;
-      s_l[wave][g] = ls;
-    }
-  }
+template <class E, int HD, int GT, bool APPEND>
+__global__ __launch_bounds__(kPairWaves *kWave) void paged_decode_pair_kernel(const DecodeKP p, const PairAppend n) {
+  using T = typename E::type;
+  __shared__ PairShared<HD, GT> s;
+  const int seq = blockIdx.y, kvh = blockIdx.x;
+  PairRows<E, HD, GT, APPEND> rows(p, n, seq, kvh);
+  const int tiles = walk_pair<E, HD, GT>(p, p.k_pool, p.v_pool, seq, kvh, threadIdx.x, s, rows);
   __syncthreads();
-  T *orow = reinterpret_cast<T *>(p.out) + seq * p.out_stride_seq + (int64_t)head0 * HD;
-  for (int o = threadIdx.x; o < heads * HD; o += kPairWaves * kWave) {
-    const int g = o / HD, d = o % HD;
-    float mx = kNegInf;
-#pragma unroll
-    for (int v = 0; v < kPairWaves; ++v) mx = fmaxf(mx, s_m[v][g]);
-    float sum = 0.f, a = 0.f;
-#pragma unroll
-    for (int v = 0; v < kPairWaves; ++v) {
-      const float w = s_m[v][g] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(s_m[v][g] - mx);
-      sum = __builtin_fmaf(s_l[v][g], w, sum);
-      a = __builtin_fmaf(s_acc[v][g][d], w, a);
-    }
-    orow[o] = E::narrow(tiles == 0 ? 0.f : a / sum);  // no visible token: zero rows
-  }
+  T *orow = reinterpret_cast<T *>(p.out) + seq * p.out_stride_seq + (int64_t)kvh * p.group * HD;
+  for (int o = threadIdx.x; o < p.group * HD; o += kPairWaves * kWave)
+    orow[o] = E::narrow(tiles == 0 ? 0.f : pair_value(s, o / HD, o % HD));  // no visible token: zero rows
 }
 
 constexpr int kReduceThreads = 256;

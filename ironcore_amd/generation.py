@@ -432,14 +432,23 @@ class LanguageModel(BaseModule):
             return None
         layers, last = plan
         host, rope = _lib.host(), self.rotary_pos_emb
+        cohort = int(meta.cohort_size) if x.dtype != torch.float32 else 1
+        angles = (None, None, None) if rope is None else (meta.positions, rope.cos_emb, rope.sin_emb)
+        longest = int(meta.max_context_len)
+        _, hn, gn, hd, act, _, _, post_ln, scale, _ = layers[0]
+        if not post_ln and cohort == 1 and all(layer[1:5] + layer[7:9] == (hn, gn, hd, act, False, scale) for layer in layers):
+            normed = host.decoder_stack(x, [layer[0][:6] + [None, None] + layer[0][8:] for layer in layers],
+                                        [(layer[9], (layer[5], layer[6], layer[0][6], layer[0][7])) for layer in layers],
+                                        last, hn, gn, hd, act, [kv_cache.layer(i) for i in range(len(layers))],
+                                        meta.block_tables, meta.context_lens, meta.slot_mapping, longest, scale, *angles,
+                                        *here)
+            if normed is not None:
+                return normed
         kind, eps, weight, bias = layers[0][9]
         normed = host.norm_rows(x, weight, bias, kind, eps, *here)
         if normed is None:
             return None
-        cohort = int(meta.cohort_size) if x.dtype != torch.float32 else 1
         shared = meta.cohort_shared_blocks if cohort > 1 else None
-        angles = (None, None, None) if rope is None else (meta.positions, rope.cos_emb, rope.sin_emb)
-        longest = int(meta.max_context_len)
         for index, (weights, hn, gn, hd, act, kind, eps, post_ln, scale, _) in enumerate(layers):
             following = last if index + 1 == len(layers) else layers[index + 1][9]
             pools = kv_cache.layer(index)
