@@ -290,6 +290,229 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   }
 }
 
+// The same for grids that leave the GPU idle.  The kernel above gives a workgroup 128 rows and a wave a serial sweep of its
+// 32 rows over all keys, 3.9 us a tile at head dim 128 (128 matrix instructions of 64 cycles), whether or not there are
+// other rows to share the tiles with: a chunk of 30 rows keeps one wave of a CU busy.  Here a workgroup has 32 rows and its
+// four waves take the tiles in turn, each with its own sums, merged through LDS at the end.  (When: takes_split.)  A wave reads its tiles
+// straight into matrix operands: K 16 bytes a lane of the lane's token, V a word a lane of 32 neighbours; K of the next
+// tile is asked for when the scores are done and arrives under the weighted values, V the other way round, so there is
+// neither staging nor a barrier.  One wave to a SIMD (some 300 registers).  Bound by the matrix instructions of a
+// wave's share, with one round trip at either end.
+template <int HD, bool SINGLE>
+__global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_split_kernel(const PrefillKP p) {
+  constexpr int NJ = HD / 8;
+  constexpr int OB = HD / 32;
+  constexpr int F4R = HD / 4;
+  __shared__ __attribute__((aligned(16))) float s_o[kF32Waves][OB * 16][kWave];
+  __shared__ float s_m[kF32Waves][32], s_l[kF32Waves][32];
+
+  const int seq = blockIdx.y;
+  const int h = blockIdx.x / p.n_qtiles;
+  const int q0 = (p.n_qtiles - 1 - blockIdx.x % p.n_qtiles) * 32;  // the longest first
+  const int kvh = h / p.group;
+  const bool equal = p.context_lens == nullptr;
+  const int q_lo = equal ? (int)(seq * p.row_pitch) : p.cu_seqlens_q[seq];
+  int L = equal ? p.uniform_context : p.context_lens[seq];
+  int C = equal ? p.max_chunk : p.cu_seqlens_q[seq + 1] - q_lo;
+  const bool causal = p.causal;
+  if (L < 0) L = 0;
+  if (causal && C > L) C = L;
+  if (q0 >= C) return;
+  const int tid = threadIdx.x;
+  if (L == 0) {
+    const int rows = C - q0 < 32 ? C - q0 : 32;
+    for (int idx = tid; idx < rows * F4R; idx += kF32Threads)
+      store16(p.out + (query_row(p, q_lo, q0 + idx / F4R) * p.out_stride_token + (int64_t)h * HD + (idx % F4R) * 4) * 4,
+              Vec16{{0u, 0u, 0u, 0u}});
+    return;
+  }
+  const int P = L - C;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int n = lane & 31, hh = lane >> 5;
+  const int my_q = q0 + n;
+  const int qrow = my_q < C ? my_q : C - 1;
+  const int limit = causal ? P + qrow : L - 1;
+  const int64_t at_row = query_row(p, q_lo, qrow);
+
+  int kv_end = causal ? P + q0 + 32 : L;
+  kv_end = kv_end < L ? kv_end : L;
+  const int n_tiles = (kv_end + kF32BN - 1) / kF32BN;
+  const int32_t *table_row = p.block_tables + (int64_t)seq * p.bt_stride;
+  // byte offset of a tile's token n in the pools (rows past the context: the last one, never visible)
+  auto token_row = [&](int t) {
+    int tok = (t < n_tiles ? t : 0) * kF32BN + n;
+    tok = tok < L ? tok : L - 1;
+    int blk = 0, within = tok;
+    if (!SINGLE) {
+      blk = p.block_shift >= 0 ? tok >> p.block_shift : tok / p.block_size;
+      within = tok - blk * p.block_size;
+    }
+    int64_t phys = SINGLE && p.block_tables == nullptr ? seq : table_row[blk];
+    phys = phys < 0 ? 0 : phys;  // a corrupt table entry must not become an out-of-pool address
+    phys = phys >= p.num_blocks ? p.num_blocks - 1 : phys;
+    return (phys * p.stride_block + (int64_t)kvh * p.stride_head + (int64_t)within * p.stride_token) * 4;
+  };
+  float4 kf[NJ];
+  float vf[16][OB];
+  auto fetch_k = [&](int64_t row) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const float4 *>(p.k_pool + row + 32 * j + 16 * hh);
+  };
+  // Matrix instruction i takes token (i % 4) + 8 (i / 4) of a tile in one half of the lanes and the fourth after it in the
+  // other.  Eight tokens lie at one stride where they are all there and in one block; else each lane asks the lane that
+  // has the token's row.
+  const bool strided = (SINGLE || p.block_size % 8 == 0) && p.stride_token < 1 << 24;
+  const uint32_t pitch = (uint32_t)p.stride_token * 4, in_group = (4 * hh) * pitch + n * 4;
+  auto fetch_v = [&](int t, int64_t row) {
+    const uint32_t lo = (uint32_t)row, hi = (uint32_t)((uint64_t)row >> 32);
+    if (strided && (t + 1) * kF32BN <= L) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t first = (int64_t)(((uint64_t)__builtin_amdgcn_readlane(hi, 8 * q) << 32) |
+                                        (uint32_t)__builtin_amdgcn_readlane(lo, 8 * q));
+        const char *base = p.v_pool + first;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int ob = 0; ob < OB; ++ob)
+            vf[4 * q + i][ob] = *reinterpret_cast<const float *>(base + (in_group + i * pitch) + ob * 128);
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int from = (i & 3) + 8 * (i >> 2) + 4 * hh;
+      const char *at = p.v_pool + (int64_t)(((uint64_t)(uint32_t)__shfl(hi, from, kWave) << 32) | (uint32_t)__shfl(lo, from, kWave)) + n * 4;
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob) vf[i][ob] = *reinterpret_cast<const float *>(at + ob * 128);
+    }
+  };
+  int t = wave;
+  int64_t row = token_row(t), row_next = 0;
+  fetch_k(row);
+  fetch_v(t < n_tiles ? t : 0, row);
+  float4 qf[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    qf[j] = *reinterpret_cast<const float4 *>(p.q + (at_row * p.q_stride_token + (int64_t)h * HD + 8 * j + 4 * hh) * 4);
+  if (p.positions != nullptr) {
+    const int64_t trig = rope_row(p, at_row) + 2 * hh;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      qf[j] = __builtin_bit_cast(float4, rotate_chunk<F32>(__builtin_bit_cast(Vec16, qf[j]), p.cos_table + trig + 4 * j,
+                                                           p.sin_table + trig + 4 * j));
+  }
+  f32x16_t o[OB];
+  float m = kNegInf, l = 0.f;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[ob][i] = 0.f;
+  while (t < n_tiles) {
+    const int after = t + kF32Waves;
+    if (after < n_tiles) row_next = token_row(after);
+    // two sums, since an instruction that adds to the last one's result waits for it
+    f32x16_t s, s2;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = s2[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j].x, qf[j].x, s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j].y, qf[j].y, s2, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j].z, qf[j].z, s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j].w, qf[j].w, s2, 0, 0, 0);
+    }
+    if (after < n_tiles) fetch_k(row_next);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] += s2[i];
+    const int tok_base = t * kF32BN + 4 * hh;
+    if (causal ? (t * kF32BN + kF32BN - 1 > P + q0) : (t * kF32BN + kF32BN > L)) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = tok_base + 8 * (i / 4) + (i & 3) > limit ? kNegInf : s[i];
+    }
+    float mx = kNegInf;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    float mx_a, mx_b;
+    both_halves(mx, mx_a, mx_b);
+    mx = fmaxf(mx_a, mx_b) * p.scale_log2e;
+    if (__any(mx > m + kLazySlack)) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = (m == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[ob][i] *= alpha;
+    }
+    const float neg_ms = (m == kNegInf) ? 0.f : -m;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], p.scale_log2e, neg_ms));
+      l += s[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int ob = 0; ob < OB; ++ob) o[ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[i][ob], s[i], o[ob], 0, 0, 0);
+    if (after < n_tiles) fetch_v(after, row_next);
+    __builtin_amdgcn_sched_barrier(0);
+    t = after;
+  }
+  // ---- merge -------------------------------------------------------------------------
+  float l_a, l_b;
+  both_halves(l, l_a, l_b);
+  if (hh == 0) s_m[wave][n] = m, s_l[wave][n] = l_a + l_b;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s_o[wave][ob * 16 + i][lane] = o[ob][i];
+  __syncthreads();
+  float top = kNegInf, lt = 0.f, weight[kF32Waves];
+#pragma unroll
+  for (int w = 0; w < kF32Waves; ++w) top = fmaxf(top, s_m[w][n]);
+#pragma unroll
+  for (int w = 0; w < kF32Waves; ++w) {
+    weight[w] = s_m[w][n] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(s_m[w][n] - top);
+    lt = __builtin_fmaf(s_l[w][n], weight[w], lt);
+  }
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if (my_q >= C) return;
+  float *orow = reinterpret_cast<float *>(p.out) + query_row(p, q_lo, my_q) * p.out_stride_token + (int64_t)h * HD;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob) {  // four dims of each block to a wave
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < kF32Waves; ++w) {
+      const int at = ob * 16 + 4 * wave;
+      sum.x = __builtin_fmaf(s_o[w][at][lane], weight[w], sum.x), sum.y = __builtin_fmaf(s_o[w][at + 1][lane], weight[w], sum.y);
+      sum.z = __builtin_fmaf(s_o[w][at + 2][lane], weight[w], sum.z), sum.w = __builtin_fmaf(s_o[w][at + 3][lane], weight[w], sum.w);
+    }
+    *reinterpret_cast<float4 *>(orow + ob * 32 + 4 * hh + 8 * wave) = make_float4(sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv);
+  }
+}
+
+template <bool SINGLE>
+int launch_split(const PrefillKP &kp, int hd, dim3 grid, hipStream_t stream) {
+  switch (hd) {
+    case 32:
+      hipLaunchKernelGGL((paged_prefill_f32_split_kernel<32, SINGLE>), grid, dim3(kF32Threads), 0, stream, kp);
+      break;
+    case 64:
+      hipLaunchKernelGGL((paged_prefill_f32_split_kernel<64, SINGLE>), grid, dim3(kF32Threads), 0, stream, kp);
+      break;
+    case 128:
+      hipLaunchKernelGGL((paged_prefill_f32_split_kernel<128, SINGLE>), grid, dim3(kF32Threads), 0, stream, kp);
+      break;
+    default:
+      return IC_ERR_UNSUPPORTED;
+  }
+  return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
+}
+
 template <bool SINGLE, int MASK>
 int launch_hd(const PrefillKP &kp, int hd, dim3 grid, hipStream_t stream) {
   switch (hd) {
@@ -308,6 +531,37 @@ int launch_hd(const PrefillKP &kp, int hd, dim3 grid, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? IC_OK : IC_ERR_LAUNCH;
 }
 
+// Whether the rows are cut finer and the keys split.  us of 128 rows to a workgroup / of 32, by blocks of 32 rows (chunks and
+// heads together) and 32-key tiles of the longest sweep:
+//   hd 128, 1 chunk of 100 behind 4 000, 32 heads        128 blocks, 129 tiles   353 / 89
+//           3 of 172-284 behind up to 74, 8              216         12           56 / 24
+//           4 of 4-261 behind up to 275, 16              576         17           80 / 49
+//           21 of 69 behind up to 1 587, 12              756         52          291 / 178
+//           4 of 1 264, 8, dense                       1 280         40          271 / 182
+//           2 of 806 behind up to 56, 32               1 664         27          216 / 188
+//           4 of 600, 32                               2 432         19          238 / 232
+//           1 of 2 000, 8, dense without a mask          504         63          285 / 150
+//           36 of 73, 8, dense                           864          3         32.5 / 37.1
+//           50 of 25, 32, dense                        1 600          1         33.8 / 58.0
+//   hd 64   2 of 75, 32, dense                           192          3         10.9 / 8.8
+//           7 of 437, 8                                  784         14         48.8 / 43.0
+//           8 of 300, 12                                 960         10         55.5 / 43.1
+//           20 of 129, 12, dense                       1 200          5         24.6 / 26.6
+//           8 of 500, 16, dense without a mask         2 048         16         76.7 / 98.8
+//           12 of 117 behind up to 899, 64             3 072         32          165 / 172
+// Long sweeps split until the matrix units are busy either way, later under the causal rule over long chunks, whose
+// workgroups are of unequal length; short ones only while each block has a CU to itself.  (The tables' width stands
+// for the longest context, which the host does not know.)
+bool takes_split(const PrefillArgs &a) {
+  if (a.mask != nullptr || a.mask_bits != nullptr) return false;
+  const bool one_block = a.block_tables == nullptr || a.block_table_stride == 1;
+  if (!one_block && a.pool.block_size < 1) return false;
+  const int64_t blocks = ((int64_t)a.max_chunk_len + 31) / 32 * a.hn * a.n_seqs;
+  const int64_t keys = a.context_lens == nullptr ? a.uniform_context : a.block_table_stride * a.pool.block_size;
+  if (keys < 10 * 32 - 31) return blocks <= device_cu_count();
+  return blocks <= (a.causal && a.max_chunk_len >= 300 ? 1700 : 800);
+}
+
 }  // namespace
 
 int launch_paged_prefill_f32(PrefillKP kp, const PrefillArgs &a, hipStream_t stream) {
@@ -316,6 +570,12 @@ int launch_paged_prefill_f32(PrefillKP kp, const PrefillArgs &a, hipStream_t str
   if (wgs_x > 0x7fffffff || a.n_seqs > 65535) return IC_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs_x, (unsigned)a.n_seqs);
   const bool masked = a.mask != nullptr;
+  if (takes_split(a)) {
+    kp.n_qtiles = (a.max_chunk_len + 31) / 32;
+    const dim3 fine((unsigned)(kp.n_qtiles * a.hn), (unsigned)a.n_seqs);
+    return a.block_tables == nullptr || a.block_table_stride == 1 ? launch_split<true>(kp, a.hd, fine, stream)
+                                                                  : launch_split<false>(kp, a.hd, fine, stream);
+  }
   if (a.mask_bits != nullptr) return launch_hd<true, 2>(kp, a.hd, grid, stream);
   // A one-column block table means one block per sequence, of any length.
   if (a.block_tables == nullptr || a.block_table_stride == 1)
