@@ -283,7 +283,7 @@ ic_prefill_call prefill_call(const Tensor &out, const Tensor &query, const Pool 
 // kernel.
 OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
                        const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
-                       const Tensor &bounds, const OptTensor &rows, int64_t longest, double scale,
+                       const OptTensor &bounds, const OptTensor &rows, int64_t longest, double scale,
                        const OptTensor &positions, const OptTensor &cos, const OptTensor &sin, int64_t device,
                        int64_t stream) {
   const Pool p(k_pool, v_pool, device);
@@ -291,7 +291,8 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
   const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
   if (!in.ok || in.hn % p.gn != 0 || !index_vector(slots, at::kLong, in.b * in.s, device) ||
       !table(tables, in.b, device) || !index_vector(lens, at::kInt, in.b, device) ||
-      !index_vector(bounds, at::kInt, in.b + 1, device) || longest > in.s ||
+      (bounds.has_value() ? !index_vector(*bounds, at::kInt, in.b + 1, device) : rows.has_value() || longest != in.s) ||
+      longest > in.s || in.b * in.s > INT_MAX ||
       !rows16(query.data_ptr(), row_stride4(query), in.hn * p.hd, query.element_size()) ||
       (p.dtype != IC_DTYPE_F32 && p.bs % 16 != 0 && tables.stride(0) != 1) ||  // 16 bits: whole groups of 16 rows
       (rows.has_value() && (rows->numel() == 0 || !index_vector(*rows, at::kLong, rows->numel(), device))))
@@ -312,13 +313,16 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
     c.n_rows = ap.n_rows = rows->numel(), c.q_rows = in.b * in.s;
     ap.zero_out = out.data_ptr();
     ap.zero_row_bytes = (int)(in.hn * p.hd * query.element_size()), ap.zero_stride_bytes = ap.zero_row_bytes;
-    ap.bounds = bounds.data_ptr<int32_t>(), ap.n_seqs = (int)in.b, ap.row_pitch = (int)in.s;
+    ap.bounds = bounds->data_ptr<int32_t>(), ap.n_seqs = (int)in.b, ap.row_pitch = (int)in.s;
   }
   if (!made("ic_append_chunks", ic_append_chunks(&ap, (void *)stream))) return c10::nullopt;
   c.block_tables = tables.data_ptr<int32_t>();
   c.block_table_stride = tables.stride(0);
   c.context_lens = lens.data_ptr<int32_t>();
-  c.cu_seqlens_q = bounds.data_ptr<int32_t>();
+  if (bounds.has_value())
+    c.cu_seqlens_q = bounds->data_ptr<int32_t>();
+  else
+    c.row_pitch = in.s;  // chunks of one length
   c.positions = rope.positions;
   c.cos_table = rope.cos, c.sin_table = rope.sin, c.table_rows = rope.rows;
   if (!made("ic_paged_prefill_ex", ic_paged_prefill_ex(&c, (void *)stream))) return c10::nullopt;

@@ -195,8 +195,10 @@ int prefill_checked(const ic_prefill_call &c, const uint8_t *mask, int64_t mask_
         c.n_seqs > c.num_blocks)
       return IC_ERR_BAD_SHAPE;
   } else {
-    if (!c.block_tables || !c.cu_seqlens_q) return IC_ERR_NULL_POINTER;
-    if (c.block_table_stride <= 0 || c.row_pitch != 0) return IC_ERR_BAD_SHAPE;
+    const bool equal_chunks = c.cu_seqlens_q == nullptr && c.row_pitch > 0;
+    if (!c.block_tables || (!c.cu_seqlens_q && !equal_chunks)) return IC_ERR_NULL_POINTER;
+    if (c.block_table_stride <= 0 || (!equal_chunks && c.row_pitch != 0)) return IC_ERR_BAD_SHAPE;
+    if (equal_chunks && (c.row_pitch < c.max_chunk_len || c.rows != nullptr)) return IC_ERR_BAD_SHAPE;
   }
   if (c.mask_bits != nullptr) {
     if (c.mask_lists == nullptr) return IC_ERR_NULL_POINTER;

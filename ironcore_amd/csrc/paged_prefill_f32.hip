@@ -65,9 +65,9 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_kernel(const Pr
   const int q0 = (p.n_qtiles - 1 - blockIdx.x % p.n_qtiles) * kF32BM;  // last query tiles (the longest) first
   const int kvh = h / p.group;
   const bool equal = p.context_lens == nullptr;  // equal sequences: nothing to look up
-  const int q_lo = equal ? (int)(seq * p.row_pitch) : p.cu_seqlens_q[seq];
+  const int q_lo = chunk_begin(p, seq);
   int L = equal ? p.uniform_context : p.context_lens[seq];
-  int C = equal ? p.max_chunk : p.cu_seqlens_q[seq + 1] - q_lo;
+  int C = chunk_end(p, seq) - q_lo;
   const bool causal = MASK == 0 && p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;  // under the causal rule a chunk cannot be longer than its context
@@ -311,9 +311,9 @@ __global__ __launch_bounds__(kF32Threads) void paged_prefill_f32_split_kernel(co
   const int q0 = (p.n_qtiles - 1 - blockIdx.x % p.n_qtiles) * 32;  // the longest first
   const int kvh = h / p.group;
   const bool equal = p.context_lens == nullptr;
-  const int q_lo = equal ? (int)(seq * p.row_pitch) : p.cu_seqlens_q[seq];
+  const int q_lo = chunk_begin(p, seq);
   int L = equal ? p.uniform_context : p.context_lens[seq];
-  int C = equal ? p.max_chunk : p.cu_seqlens_q[seq + 1] - q_lo;
+  int C = chunk_end(p, seq) - q_lo;
   const bool causal = p.causal;
   if (L < 0) L = 0;
   if (causal && C > L) C = L;

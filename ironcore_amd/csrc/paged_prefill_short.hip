@@ -68,7 +68,7 @@ constexpr int kShortBuffers = 2;  // LDS buffers per pool and tile group
 __device__ __forceinline__ bool pick_by_sweep(const PrefillKP &p, int index, int &seq, int &q_lo, int &L, int &C, int &v0) {
   const int n_seqs = p.n_units / p.gn, ln = threadIdx.x & (kWave - 1), group = p.group;
   const bool in = ln < n_seqs;
-  const int lo = in ? p.cu_seqlens_q[ln] : 0, chunk = in ? p.cu_seqlens_q[ln + 1] - lo : 0;
+  const int lo = in ? chunk_begin(p, ln) : 0, chunk = in ? chunk_end(p, ln) - lo : 0;
   int len = in ? p.context_lens[ln] : 0;
   len = len < 0 ? 0 : len;
   const int rows = p.causal && chunk > len ? len : chunk;

@@ -48,7 +48,7 @@ struct PrefillKP {
   const int64_t *rows;  // row of q and out that row i of the packed chunks is (nullptr: i itself)
   int n_rows;           // entries of `rows`
   int q_rows;           // rows of q and out, which bound them
-  int64_t row_pitch;    // equal sequences: rows from one chunk to the next in q and out
+  int64_t row_pitch;    // no cu_seqlens_q (equal chunks): rows from one chunk to the next in q and out
   int max_chunk;        // ... and rows of every chunk
   int uniform_context;  // context_lens == nullptr (equal sequences): keys of every context
   const int32_t *positions;  // rotary embedding of the query rows (nullptr: none)
@@ -132,6 +132,14 @@ __device__ __forceinline__ int tile_swizzle_v(int r) {
   return CPR == 16 ? ((r & 3) << 2) : CPR == 8 ? (((r >> 1) & 1) << 2) : 0;
 }
 
+// First row of sequence i's chunk, and the one behind its last.
+__device__ __forceinline__ int chunk_begin(const PrefillKP &p, int i) {
+  return p.cu_seqlens_q != nullptr ? p.cu_seqlens_q[i] : (int)(i * p.row_pitch);
+}
+__device__ __forceinline__ int chunk_end(const PrefillKP &p, int i) {
+  return p.cu_seqlens_q != nullptr ? p.cu_seqlens_q[i + 1] : (int)(i * p.row_pitch) + p.max_chunk;
+}
+
 // The sequence that is `rank`th by context length (longest first: workgroups
 // are dispatched in id order and should end together), its first query row,
 // context length and chunk length.  Up to one sequence per lane is ranked on
@@ -151,8 +159,8 @@ __device__ __forceinline__ void pick_sequence(const PrefillKP &p, int rank, int 
     // sequence's come from its lane instead of a second round trip to memory)
     const int ln = threadIdx.x & (kWave - 1);
     const int mine = ln < n_seqs ? p.context_lens[ln] : -0x7fffffff;
-    const int lo_mine = ln < n_seqs ? p.cu_seqlens_q[ln] : 0;
-    const int hi_mine = ln < n_seqs ? p.cu_seqlens_q[ln + 1] : 0;
+    const int lo_mine = ln < n_seqs ? chunk_begin(p, ln) : 0;
+    const int hi_mine = ln < n_seqs ? chunk_end(p, ln) : 0;
     int above = 0;
     for (int j = 0; j < n_seqs; ++j) {
       const int other = __builtin_amdgcn_readlane(mine, j);
@@ -165,9 +173,9 @@ __device__ __forceinline__ void pick_sequence(const PrefillKP &p, int rank, int 
     L = __builtin_amdgcn_readlane(mine, seq);
     C = __builtin_amdgcn_readlane(hi_mine, seq) - q_lo;
   } else {
-    q_lo = p.cu_seqlens_q[seq];
+    q_lo = chunk_begin(p, seq);
     L = p.context_lens[seq];
-    C = p.cu_seqlens_q[seq + 1] - q_lo;
+    C = chunk_end(p, seq) - q_lo;
   }
 }
 

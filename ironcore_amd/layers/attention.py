@@ -351,11 +351,8 @@ class Attention(BaseModule):
             if out is not None:
                 return out
         elif here is not None and (rows is None or meta.cu_seqlens_q is not None):   # (rows come with their bounds)
-            bounds = meta.cu_seqlens_q
-            if bounds is None:
-                bounds = torch.arange(0, (b + 1) * sq, sq, dtype=torch.int32, device=query.device)
             out = _lib.host().prefill_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
-                                           meta.slot_mapping, bounds, rows, sq if rows is None else int(meta.max_chunk_len),
+                                           meta.slot_mapping, meta.cu_seqlens_q, rows, sq if rows is None else int(meta.max_chunk_len),
                                            1.0 / self.scale_factor, *(rope or (None, None, None)), *here)
             if out is not None:
                 return out
