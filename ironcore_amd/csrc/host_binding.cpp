@@ -123,6 +123,21 @@ bool decode_fits(const Pool &p, int64_t b, int64_t hn, const Decode &d, int64_t 
          (d.shared.has_value() && index_vector(*d.shared, at::kInt, (b + d.cohort - 1) / d.cohort, device));
 }
 
+// Whether a cohort's shared blocks are worth reading once.  What its members read again then comes from the cache while all
+// of it fits there (256 MB, beside other data), and without cohorts there is no second phase, the grid fits the rows and small
+// batches take one launch with the append.  us of a layer call with cohorts / without, prompts x samples, prefix + suffix:
+//   16 / 4 heads of 128    22 x 16, 80 + 232       225 MB    40.4 / 29.5        21 x 16, 1 680 + 120     1 239    45.8 / 87.2
+//                          4 x 4, 160 + 41           7       20.4 / 9.9         10 x 16, 816 + 467         420    40.2 / 34.3
+//   32 / 8 of 128          12 x 4, 80 + 55          27       24.3 / 17.7        30 x 8, 240 + 451          679    68.1 / 64.9
+//   12 / 12 of 128         3 x 8, 384 + 289         99       30.4 / 13.3        4 x 4, 2 256 + 55          227    35.1 / 42.6
+//                          14 x 4, 240 + 672       313       41.7 / 31.1        29 x 4, 736 + 43           555    41.4 / 47.0
+//   28 / 4 of 128          29 x 4, 80 + 62          34       26.1 / 19.7        32 x 16, 1 024 + 1 024   2 147    153 / 197
+//   28 / 4 of 64           32 x 16, 160 + 45       107       28.9 / 28.4        3 x 16, 80 + 753            41    26.7 / 27.0
+// Between 200 and 700 MB either may be faster; the line is where none of 64 was slower by more than a percent.
+bool cohorts_pay(const Pool &p, int64_t b, const Decode &d, int64_t element_size) {
+  return d.cohort > 1 && b * d.max_ctx * p.gn * p.hd * 2 * element_size > 192000000;
+}
+
 bool decode(const Tensor &out, const void *q, int64_t q_stride, const Pool &p, int64_t b, int64_t hn, const Decode &d,
             void *stream) {
   const size_t need = ic_paged_decode_shared_workspace_bytes((int)b, (int)hn, (int)p.gn, (int)p.hd, (int)d.cohort);
@@ -225,9 +240,11 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
   if (!p.ok) return c10::nullopt;
   const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
   if (!in.ok || in.s != 1 || !index_vector(slots, at::kLong, in.b, device)) return c10::nullopt;
-  const Decode d{tables, lens, max_ctx, 0, cohort, shared, scale};
+  const Decode asked{tables, lens, max_ctx, 0, cohort, shared, scale};
   const Rope rope(positions, cos, sin, in.b, p.hd, device);
-  if (!rope.ok || !decode_fits(p, in.b, in.hn, d, device)) return c10::nullopt;
+  if (!rope.ok || !decode_fits(p, in.b, in.hn, asked, device)) return c10::nullopt;
+  if (cohort > 1 && !cohorts_pay(p, in.b, asked, query.element_size())) cohort = 1;
+  const Decode d{tables, lens, max_ctx, 0, cohort, shared, scale};
   const void *q = query.data_ptr();
   int64_t q_stride = row_stride4(query);
   if (!rows16(q, q_stride, in.hn * p.hd, query.element_size())) return c10::nullopt;
@@ -551,6 +568,7 @@ c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
   if (!rope.ok || !decode_fits(p, b, hn, dec, device) ||
       !rows16(p.k, p.sb, 1, es) || !rows16(p.v, p.sb, 1, es) || (p.sh * es) % 16 != 0 || (p.st * es) % 16 != 0)
     return c10::nullopt;
+  if (cohort > 1 && !cohorts_pay(p, b, dec, es)) cohort = 1;
 
   ic_step_linear_call qkv = {}, proj = {}, up = {}, down = {};
   qkv.m = proj.m = up.m = down.m = (int)b;

@@ -372,6 +372,8 @@ class Attention(BaseModule):
             return self._ragged_chunks(query, k_pool, v_pool, meta, rows, scale)
         if sq == 1:
             cohort = meta.cohort_size if query.dtype != torch.float32 else 1
+            if not paged_ops.cohorts_pay(k_pool, b, hn, meta.max_context_len, cohort, meta.cohort_shared_blocks):
+                cohort = 1
             out = paged_ops.paged_decode(query.view(b, hn, hd), k_pool, v_pool, meta.block_tables,
                                          meta.context_lens, meta.max_context_len, scale=scale,
                                          cohort_size=cohort,

@@ -335,6 +335,19 @@ def shared_prefix_blocks(block_tables, context_lens, block_size: int, cohort_siz
     return out
 
 
+def cohorts_pay(k_pool: torch.Tensor, b: int, hn: int, max_context_len: int, cohort_size: int, shared) -> bool:
+    """Whether a layer call with cohorts reads their shared blocks once (the native path's rule, with both sides
+    measured: ``cohorts_pay`` in csrc/host_binding.cpp).  Cohorts that a decode call would refuse are left to it."""
+    cohort_size = int(cohort_size)
+    _, gn, _, hd = k_pool.shape
+    if cohort_size <= 1 or b * int(max_context_len) * gn * hd * 2 * k_pool.element_size() > 192000000:
+        return True
+    fits = (shared is not None and shared.dtype == torch.int32 and shared.numel() == -(-b // cohort_size)
+            and shared.is_contiguous() and shared.device == k_pool.device
+            and _lib.load().ic_paged_decode_shared_workspace_bytes(b, hn, gn, hd, cohort_size) > 0)
+    return not fits
+
+
 def paged_prefill(query: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
                   block_tables: torch.Tensor, context_lens: torch.Tensor,
                   cu_seqlens_q: torch.Tensor, max_chunk_len: int, causal: bool = True,
