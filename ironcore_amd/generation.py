@@ -230,7 +230,8 @@ class TransformerModel(BaseModule):
 
 # ---- a decode step past the modules --------------------------------------------------------------
 # The layers of a decode step (one new token a sequence) can run as a handful of native launches each, norms,
-# biases, activations, residuals and the cache append on the launches of the products (csrc/step_linear.hip).  The
+# biases, activations, residuals and the cache append on the launches of the products (csrc/step_linear.hip), those of
+# a small model as one launch together (csrc/step_stack.hip).  The
 # modules are then not called, so that path is taken only where nobody could tell: every module of the known
 # type, without hooks, its forward its own.
 
@@ -421,8 +422,8 @@ class LanguageModel(BaseModule):
         return torch.matmul(x, self.embedding.word_embeddings.weight.transpose(0, 1))
 
     def _native_step(self, x, kv_cache, meta):
-        """The layers and the last norm of a decode step by native calls, one a layer, or None: ``x`` [b, 1, d] are
-        the embedded tokens.  Where a layer's call is not taken (sizes, types, strides), the layer runs as a module."""
+        """The layers and the last norm of a decode step by native calls, one for all of them or one a layer, or None:
+        ``x`` [b, 1, d] are the embedded tokens.  Where a layer's call is not taken (sizes, types, strides), the layer runs as a module."""
         here = _lib.here(x) if type(x) is torch.Tensor else None
         if (here is None or getattr(meta, "chunk_rows", None) is not None or x.dim() != 3
                 or torch.overrides.has_torch_function_unary(x) or torch.compiler.is_compiling() or torch.jit.is_tracing()):
