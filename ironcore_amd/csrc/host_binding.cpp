@@ -635,7 +635,7 @@ c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
 // All layers of a decode step and the norm behind them in one launch (ic_step_stack; more layers than one call holds: in
 // equal parts).  `w`: a layer's weights and biases as decoder_layer takes them, but for the next norm; `norms`: its input
 // norm and its post-attention norm as (kind, eps, weight, bias).  None for what the call does not take, and where the
-// layers' own launches are as fast (stack_pays).
+// layers' own launches are as fast (stack_takes).
 using Norm = std::tuple<int64_t, double, Tensor, OptTensor>;
 
 // us a layer and token, two rows, 64 to 364 tokens, launches / stack: fp32 d 768, ffn 3 072 36.2 / 26.3, 512 x 2 048 30.5 / 22.3,
@@ -650,6 +650,16 @@ bool stack_pays(int64_t group, int64_t max_ctx, int64_t row_bytes, int64_t layer
   return group == 1 ? rounds <= 16 && rounds * row_bytes <= 4096 : rounds <= 4;
 }
 
+// Whether a step of these sizes goes to decoder_stack: asked by itself before the caller gathers the layers' tensors (25 us of
+// the host for four layers, which a step bound by the host would lose for nothing).
+bool stack_takes(int64_t b, int64_t d, int64_t f, int64_t hn, int64_t gn, int64_t hd, int64_t act, int64_t max_ctx,
+                 int64_t element_size) {
+  if (b < 1 || b > IC_STEP_STACK_ROWS || d < 1 || d > 1024 || f < 1 || gn < 1 || hn < gn || hn % gn != 0 || (hd != 64 && hd != 128))
+    return false;
+  const int64_t columns = 2 * hn * hd + 2 * gn * hd + (act >= IC_ACT_GLU ? 3 : 2) * f;
+  return stack_pays(hn / gn, max_ctx, hd * element_size, d * columns * element_size);
+}
+
 OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor>> &w,
                         const std::vector<std::tuple<Norm, Norm>> &norms, const Norm &last, int64_t hn, int64_t gn,
                         int64_t hd, int64_t act, const std::vector<std::tuple<Tensor, Tensor>> &pools, const Tensor &tables,
@@ -662,12 +672,11 @@ OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor
     return c10::nullopt;
   const int64_t b = x.size(0), d = x.size(2), q_cols = hn * hd, kv_cols = gn * hd;
   const int es = (int)x.element_size();
-  if (b < 1 || b > IC_STEP_STACK_ROWS || gn < 1 || !rows16(x.data_ptr(), d, d, es) || w[0].size() != 12 || !w[0][8].has_value() ||
-      w[0][8]->dim() != 2 || !index_vector(slots, at::kLong, b, device))
+  if (!rows16(x.data_ptr(), d, d, es) || w[0].size() != 12 || !w[0][8].has_value() || w[0][8]->dim() != 2 ||
+      !index_vector(slots, at::kLong, b, device))
     return c10::nullopt;
   const int64_t up_cols = w[0][8]->size(1), f = act >= IC_ACT_GLU ? up_cols / 2 : up_cols;
-  if (up_cols > (1 << 20) || (act >= IC_ACT_GLU && up_cols % 2 != 0) ||
-      !stack_pays(hn / gn, max_ctx, hd * es, d * (2 * q_cols + 2 * kv_cols + up_cols + f) * es))
+  if (up_cols > (1 << 20) || (act >= IC_ACT_GLU && up_cols % 2 != 0) || !stack_takes(b, d, f, hn, gn, hd, act, max_ctx, es))
     return c10::nullopt;
   const Pool first(std::get<0>(pools[0]), std::get<1>(pools[0]), device);
   const OptTensor none;
@@ -804,6 +813,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_rows", torch::wrap_pybind_function_no_gil(linear_rows));
   m.def("norm_rows", torch::wrap_pybind_function_no_gil(norm_rows));
   m.def("decoder_layer", torch::wrap_pybind_function_no_gil(decoder_layer));
+  m.attr("STEP_ROWS") = IC_LINEAR_ROWS_MAX;
+  m.def("stack_takes", &stack_takes);
   m.def("decoder_stack", torch::wrap_pybind_function_no_gil(decoder_stack));
   m.def("greedy", torch::wrap_pybind_function_no_gil(greedy));
   m.def("advance", torch::wrap_pybind_function_no_gil(advance));

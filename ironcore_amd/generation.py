@@ -428,16 +428,21 @@ class LanguageModel(BaseModule):
         if (here is None or getattr(meta, "chunk_rows", None) is not None or x.dim() != 3
                 or torch.overrides.has_torch_function_unary(x) or torch.compiler.is_compiling() or torch.jit.is_tracing()):
             return None
+        host = _lib.host()
+        if x.shape[0] > host.STEP_ROWS:   # (more than any of the calls takes: nothing is gathered for them)
+            return None
         plan = _step_plan(self, x.shape[-1])
         if plan is None:
             return None
         layers, last = plan
-        host, rope = _lib.host(), self.rotary_pos_emb
+        rope = self.rotary_pos_emb
         cohort = int(meta.cohort_size) if x.dtype != torch.float32 else 1
         angles = (None, None, None) if rope is None else (meta.positions, rope.cos_emb, rope.sin_emb)
         longest = int(meta.max_context_len)
-        _, hn, gn, hd, act, _, _, post_ln, scale, _ = layers[0]
-        if not post_ln and cohort == 1 and all(layer[1:5] + layer[7:9] == (hn, gn, hd, act, False, scale) for layer in layers):
+        weights, hn, gn, hd, act, _, _, post_ln, scale, _ = layers[0]
+        if (not post_ln and cohort == 1
+                and host.stack_takes(x.shape[0], x.shape[2], weights[10].shape[0], hn, gn, hd, act, longest, x.element_size())
+                and all(layer[1:5] + layer[7:9] == (hn, gn, hd, act, False, scale) for layer in layers)):
             normed = host.decoder_stack(x, [layer[0][:6] + [None, None] + layer[0][8:] for layer in layers],
                                         [(layer[9], (layer[5], layer[6], layer[0][6], layer[0][7])) for layer in layers],
                                         last, hn, gn, hd, act, [kv_cache.layer(i) for i in range(len(layers))],
