@@ -638,26 +638,45 @@ c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
 // layers' own launches are as fast (stack_takes).
 using Norm = std::tuple<int64_t, double, Tensor, OptTensor>;
 
-// us a layer and token, two rows, 64 to 364 tokens, launches / stack: fp32 d 768, ffn 3 072 36.2 / 26.3, 512 x 2 048 30.5 / 22.3,
-// 256 x 1 024 26.1 / 21.4; bf16 768 x 3 072 32 / 23.5.  Four layers, d 1 024, 16 bits, the step with the output layer: 8 / 8 heads
-// of 128, up to 890 tokens, batch 2 181 / 119, 200 tokens, 10 198 / 138, 1 500 tokens, 16 239 / 213.  A pair's rows are walked by
-// one workgroup and grouped heads cost it vector work, so these have the limit that the attention launch has: 8 / 2
-// heads, 611 tokens, batch 10 205 / 211, 2 048 tokens, 3 210 / 278.  Below 2 MB of weights a layer (256 x 352 24.4 / 20.6) there
-// is little to prefetch, and the layers stay calls of their own, any of which may be a module's.
-bool stack_pays(int64_t group, int64_t max_ctx, int64_t row_bytes, int64_t layer_bytes) {
+// us a layer and token of a replayed step, layers' launches / stack (8 layers; heads / KV heads, ffn, context, rows):
+//   fp32 d 768     12 / 12 of 64   3 072     300    1  34 / 25     4  38 / 28     5  38 / 33    16  46 / 40
+//                                           1 700    4  54 / 42    16  69 / 61
+//                                  4 096     300    16  47 / 45    gated, 4  50 / 43    gated, 16  55 / 56
+//                                  8 192     300     4  50 / 47    16  55 / 61
+//                  12 / 3 of 64    3 072     250     4  37 / 31     6  37 / 36    16  40 / 40      500   16  47 / 45
+//                  12 / 6 of 64    3 072     250     4  35 / 32    16  42 / 42      128   16  39 / 40
+//                  6 / 6 of 128    2 304     380     4  39 / 38    16  49 / 51    1 000    4  54 / 63
+//                  6 / 3 of 128    2 304     250     4  36 / 48
+//        d 512     8 / 8 of 64     2 048     300     4  31 / 24    16  35 / 31
+//        d 832     13 / 13 of 64   3 328     300     4  40 / 43    16  47 / 56
+//        d 1 024   8 / 8 of 128    4 096     300     4  48 / 56    16  53 / 69
+//   bf16 d 1 024   8 / 8 of 128    2 752     300    16  45 / 37    2 000   16  67 / 58;   8 192   300   16  59 / 51
+//                  16 / 4 of 64    2 752     500     2  40 / 32    16  45 / 41
+//                  16 / 8 of 64    2 752     128    16  39 / 38      500   16  46 / 42
+//                  8 / 2 of 128    2 752     380     1  42 / 40     4  45 / 43    10  47 / 49      450    2  42 / 43
+//                  8 / 4 of 128    2 752     380     2  37 / 42    16  45 / 53
+//   fp16           8 / 2 of 128    2 752     250     2  39 / 41     4  39 / 42     8  40 / 47
+// In fp32 a row of more than 768 (the product keeps eight steps of weights and not six) and heads of 128 do not fit the registers,
+// nor do the four query rows of grouped heads of 128 (bf16 spills less); above four rows the fp32 product takes 16x16 instructions,
+// mostly for rows that are not there, and long columns weigh more.  A pair's rows are walked by one workgroup, which bounds the
+// contexts of grouped heads.  Below 2 MB of weights a layer (fp32 d 256, ffn 352 24.4 / 20.6) there is little to prefetch, and
+// the layers stay calls of their own, any of which may be a module's.
+bool stack_pays(at::ScalarType type, int64_t b, int64_t d, int64_t f, int64_t group, int64_t hd, int64_t max_ctx, int64_t layer_bytes) {
   const int64_t rounds = (max_ctx + 127) / 128;
-  if (layer_bytes < 2000000 || group > 4) return false;
-  return group == 1 ? rounds <= 16 && rounds * row_bytes <= 4096 : rounds <= 4;
+  if (layer_bytes < 2000000 || f > 8192 || group > 4 || rounds > (group == 1 ? 16 : 4)) return false;
+  if (type == at::kFloat) return d <= 768 && hd == 64 && (b <= 4 || (f <= 4096 && group != 2));
+  return group == 1 || hd == 64 || (type == at::kBFloat16 && group > 2 && b <= 4 && rounds <= 3);
 }
 
 // Whether a step of these sizes goes to decoder_stack: asked by itself before the caller gathers the layers' tensors (25 us of
 // the host for four layers, which a step bound by the host would lose for nothing).
-bool stack_takes(int64_t b, int64_t d, int64_t f, int64_t hn, int64_t gn, int64_t hd, int64_t act, int64_t max_ctx,
-                 int64_t element_size) {
-  if (b < 1 || b > IC_STEP_STACK_ROWS || d < 1 || d > 1024 || f < 1 || gn < 1 || hn < gn || hn % gn != 0 || (hd != 64 && hd != 128))
+bool stack_takes(at::ScalarType type, int64_t b, int64_t d, int64_t f, int64_t hn, int64_t gn, int64_t hd, int64_t act,
+                 int64_t max_ctx) {
+  if (dtype_code(type) < 0 || b < 1 || b > IC_STEP_STACK_ROWS || d < 1 || d > 1024 || f < 1 || gn < 1 || hn < gn || hn % gn != 0 ||
+      (hd != 64 && hd != 128))
     return false;
   const int64_t columns = 2 * hn * hd + 2 * gn * hd + (act >= IC_ACT_GLU ? 3 : 2) * f;
-  return stack_pays(hn / gn, max_ctx, hd * element_size, d * columns * element_size);
+  return stack_pays(type, b, d, f, hn / gn, hd, max_ctx, d * columns * (int64_t)c10::elementSize(type));
 }
 
 OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor>> &w,
@@ -676,7 +695,7 @@ OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor
       !index_vector(slots, at::kLong, b, device))
     return c10::nullopt;
   const int64_t up_cols = w[0][8]->size(1), f = act >= IC_ACT_GLU ? up_cols / 2 : up_cols;
-  if (up_cols > (1 << 20) || (act >= IC_ACT_GLU && up_cols % 2 != 0) || !stack_takes(b, d, f, hn, gn, hd, act, max_ctx, es))
+  if (up_cols > (1 << 20) || (act >= IC_ACT_GLU && up_cols % 2 != 0) || !stack_takes(type, b, d, f, hn, gn, hd, act, max_ctx))
     return c10::nullopt;
   const Pool first(std::get<0>(pools[0]), std::get<1>(pools[0]), device);
   const OptTensor none;

@@ -441,7 +441,7 @@ class LanguageModel(BaseModule):
         longest = int(meta.max_context_len)
         weights, hn, gn, hd, act, _, _, post_ln, scale, _ = layers[0]
         if (not post_ln and cohort == 1
-                and host.stack_takes(x.shape[0], x.shape[2], weights[10].shape[0], hn, gn, hd, act, longest, x.element_size())
+                and host.stack_takes(x.dtype, x.shape[0], x.shape[2], weights[10].shape[0], hn, gn, hd, act, longest)
                 and all(layer[1:5] + layer[7:9] == (hn, gn, hd, act, False, scale) for layer in layers)):
             normed = host.decoder_stack(x, [layer[0][:6] + [None, None] + layer[0][8:] for layer in layers],
                                         [(layer[9], (layer[5], layer[6], layer[0][6], layer[0][7])) for layer in layers],
