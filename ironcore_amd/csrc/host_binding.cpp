@@ -133,9 +133,27 @@ bool decode_fits(const Pool &p, int64_t b, int64_t hn, const Decode &d, int64_t 
 //                          14 x 4, 240 + 672       313       41.7 / 31.1        29 x 4, 736 + 43           555    41.4 / 47.0
 //   28 / 4 of 128          29 x 4, 80 + 62          34       26.1 / 19.7        32 x 16, 1 024 + 1 024   2 147    153 / 197
 //   28 / 4 of 64           32 x 16, 160 + 45       107       28.9 / 28.4        3 x 16, 80 + 753            41    26.7 / 27.0
-// Between 200 and 700 MB either may be faster; the line is where none of 64 was slower by more than a percent.
-bool cohorts_pay(const Pool &p, int64_t b, const Decode &d, int64_t element_size) {
-  return d.cohort > 1 && b * d.max_ctx * p.gn * p.hd * 2 * element_size > 192000000;
+// Between 200 and 700 MB either may be faster; the line is where none of 64 was slower by more than a percent.  (Passes over one
+// layer's pools, which stay in that cache.  With 1.2 GB of pools in turn: 138 MB 36.4 / 28.2, 251 MB 34.3 / 31.4, 7 MB 25.1 / 17.2, and
+// in a model's step, us a layer, 147 MB 127 / 119, 21 MB 69 / 62: the line stays.)
+// At head dim 64 a cohort of more than 64 query rows is the exception: it fills both of the kernel's column tiles and all eight waves,
+// while the plain call, where it is not the pair kernel (decode_takes_pairs), streams grouped heads of 64 at half its rate.
+// Hot and cold, from three quarters of the CUs in pairs on (fewer leave CUs for the plain call's splits):
+//   28 / 4 of 64           10 x 16, 576 + 36    100 MB    25.6 / 28.5   27.4 / 30.1       3 x 16, 912 + 40    47    25.6 / 27.8   27.0 / 28.8
+//                          5 x 10, 576 + 36      31       23.4 / 27.8   24.7 / 28.8       5 x 16, 160 + 400   46    27.4 / 25.4   29.1 / 27.1
+//                          2 x 16, 576 + 36      20       26.0 / 25.1   27.4 / 25.8       2 x 16, 1 504 + 100 53    29.2 / 20.0   30.3 / 21.0
+//                          30 x 8, 400 + 40     108       36.1 / 28.0   38.2 / 30.7       20 x 4, 304 + 60    30    36.0 / 24.5   38.3 / 25.7
+//   64 / 8 of 64           2 x 16, 576 + 36      40       24.4 / 29.8   25.4 / 30.9       2 x 10, 912 + 36    39    28.4 / 26.8   29.4 / 28.0
+//   32 / 8 of 64           3 x 24, 576 + 36      90       23.7 / 27.1   25.2 / 28.5       2 x 32, 576 + 36    80    24.7 / 19.4   26.2 / 19.6
+//   12 / 4 of 64           6 x 24, 576 + 36      90       23.7 / 26.9   25.0 / 28.3       3 x 24, 576 + 36    45    24.2 / 18.9   25.6 / 18.8
+//   16 / 8 of 64           3 x 64, 320 + 36     140       26.6 / 18.8   28.0 / 20.6
+//   28 / 4 of 32           10 x 16, 304 + 36     28       34.7 / 24.3   36.4 / 25.0
+bool cohorts_pay(int64_t b, int64_t hn, int64_t gn, int64_t hd, int64_t max_ctx, int64_t cohort, int64_t element_size) {
+  if (cohort <= 1 || gn < 1) return false;
+  if (b * max_ctx * gn * hd * 2 * element_size > 192000000) return true;
+  const int64_t group = hn / gn, pairs = b * gn;
+  const bool pair_kernel = group <= 2 ? max_ctx <= 2048 : group <= 4 && max_ctx <= 1024 && pairs <= 512;
+  return hd == 64 && cohort * group > 64 && pairs >= 192 && !pair_kernel;
 }
 
 bool decode(const Tensor &out, const void *q, int64_t q_stride, const Pool &p, int64_t b, int64_t hn, const Decode &d,
@@ -243,7 +261,7 @@ OptTensor decode_step(const Tensor &query, const Tensor &key, const Tensor &valu
   const Decode asked{tables, lens, max_ctx, 0, cohort, shared, scale};
   const Rope rope(positions, cos, sin, in.b, p.hd, device);
   if (!rope.ok || !decode_fits(p, in.b, in.hn, asked, device)) return c10::nullopt;
-  if (cohort > 1 && !cohorts_pay(p, in.b, asked, query.element_size())) cohort = 1;
+  if (!cohorts_pay(in.b, in.hn, p.gn, p.hd, max_ctx, cohort, query.element_size())) cohort = 1;
   const Decode d{tables, lens, max_ctx, 0, cohort, shared, scale};
   const void *q = query.data_ptr();
   int64_t q_stride = row_stride4(query);
@@ -568,7 +586,7 @@ c10::optional<std::tuple<Tensor, Tensor>> decoder_layer(
   if (!rope.ok || !decode_fits(p, b, hn, dec, device) ||
       !rows16(p.k, p.sb, 1, es) || !rows16(p.v, p.sb, 1, es) || (p.sh * es) % 16 != 0 || (p.st * es) % 16 != 0)
     return c10::nullopt;
-  if (cohort > 1 && !cohorts_pay(p, b, dec, es)) cohort = 1;
+  if (!cohorts_pay(b, hn, p.gn, p.hd, max_ctx, cohort, es)) cohort = 1;
 
   ic_step_linear_call qkv = {}, proj = {}, up = {}, down = {};
   qkv.m = proj.m = up.m = down.m = (int)b;
@@ -824,6 +842,7 @@ bool advance(const Tensor &lens, const Tensor &tables, int64_t block_size, const
 // torch.OutOfMemoryError.  The GIL is given up for the call: a launch may wait on a full queue and an allocation on the
 // GPU, and other threads go on meanwhile.)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("cohorts_pay", &cohorts_pay);
   m.def("kv_append", torch::wrap_pybind_function_no_gil(kv_append));
   m.def("paged_decode", torch::wrap_pybind_function_no_gil(paged_decode));
   m.def("decode_step", torch::wrap_pybind_function_no_gil(decode_step));

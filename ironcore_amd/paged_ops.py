@@ -340,7 +340,7 @@ def cohorts_pay(k_pool: torch.Tensor, b: int, hn: int, max_context_len: int, coh
     measured: ``cohorts_pay`` in csrc/host_binding.cpp).  Cohorts that a decode call would refuse are left to it."""
     cohort_size = int(cohort_size)
     _, gn, _, hd = k_pool.shape
-    if cohort_size <= 1 or b * int(max_context_len) * gn * hd * 2 * k_pool.element_size() > 192000000:
+    if cohort_size <= 1 or _lib.host().cohorts_pay(b, hn, gn, hd, int(max_context_len), cohort_size, k_pool.element_size()):
         return True
     fits = (shared is not None and shared.dtype == torch.int32 and shared.numel() == -(-b // cohort_size)
             and shared.is_contiguous() and shared.device == k_pool.device
