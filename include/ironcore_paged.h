@@ -360,6 +360,9 @@ int ic_mask_pack(const uint8_t *mask, int64_t stride_seq, int64_t stride_head, i
  *                    chunk max_chunk_len rows, row_pitch >= max_chunk_len apart, and
  *                    sequence i is pool block i (uniform_context <= block_size,
  *                    any block size): a dense [b, s, gn, hd] tensor as a pool.
+ *                    With context_lens: no context is longer, 0 if the caller does not
+ *                    know (the block tables' width then bounds them).  It chooses
+ *                    between kernels and bounds nothing.
  *   row_pitch        with context_lens and block_tables, cu_seqlens_q and rows NULL:
  *                    chunks of max_chunk_len rows each, row_pitch >= max_chunk_len apart.
  *   positions, cos_table, sin_table, table_rows

@@ -315,12 +315,12 @@ ic_prefill_call prefill_call(const Tensor &out, const Tensor &query, const Pool 
 // A chunk of new tokens per sequence: append, then attend.  `bounds` int32 [b + 1] holds the bounds of the
 // packed chunks; chunks of unequal length come with the rows of the padded tensors they are (int64, any
 // placement), whose other rows are padding: slot -1, output zero.  The query is rotated inside the attention
-// kernel.
+// kernel.  `max_ctx`: no context is longer (0: not known).
 OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &value, const Tensor &k_pool,
                        const Tensor &v_pool, const Tensor &tables, const Tensor &lens, const Tensor &slots,
                        const OptTensor &bounds, const OptTensor &rows, int64_t longest, double scale,
                        const OptTensor &positions, const OptTensor &cos, const OptTensor &sin, int64_t device,
-                       int64_t stream) {
+                       int64_t stream, int64_t max_ctx) {
   const Pool p(k_pool, v_pool, device);
   if (!p.ok || !p.attends()) return c10::nullopt;
   const NewRows in(query, key, value, p, k_pool.scalar_type(), device);
@@ -354,6 +354,7 @@ OptTensor prefill_step(const Tensor &query, const Tensor &key, const Tensor &val
   c.block_tables = tables.data_ptr<int32_t>();
   c.block_table_stride = tables.stride(0);
   c.context_lens = lens.data_ptr<int32_t>();
+  c.uniform_context = (int)std::clamp<int64_t>(max_ctx, 0, INT_MAX);
   if (bounds.has_value())
     c.cu_seqlens_q = bounds->data_ptr<int32_t>();
   else
@@ -846,7 +847,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", torch::wrap_pybind_function_no_gil(kv_append));
   m.def("paged_decode", torch::wrap_pybind_function_no_gil(paged_decode));
   m.def("decode_step", torch::wrap_pybind_function_no_gil(decode_step));
-  m.def("prefill_step", torch::wrap_pybind_function_no_gil(prefill_step));
+  m.def("prefill_step", torch::wrap_pybind_function_no_gil(prefill_step), py::arg("query"), py::arg("key"), py::arg("value"),
+        py::arg("k_pool"), py::arg("v_pool"), py::arg("tables"), py::arg("lens"), py::arg("slots"), py::arg("bounds"),
+        py::arg("rows"), py::arg("longest"), py::arg("scale"), py::arg("positions"), py::arg("cos"), py::arg("sin"),
+        py::arg("device"), py::arg("stream"), py::arg("max_ctx") = 0);
   m.def("dense", torch::wrap_pybind_function_no_gil(dense));
   m.def("linear_rows", torch::wrap_pybind_function_no_gil(linear_rows));
   m.def("norm_rows", torch::wrap_pybind_function_no_gil(norm_rows));

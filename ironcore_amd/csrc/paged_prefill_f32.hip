@@ -549,17 +549,34 @@ int launch_hd(const PrefillKP &kp, int hd, dim3 grid, hipStream_t stream) {
 //           20 of 129, 12, dense                       1 200          5         24.6 / 26.6
 //           8 of 500, 16, dense without a mask         2 048         16         76.7 / 98.8
 //           12 of 117 behind up to 899, 64             3 072         32          165 / 172
+// and the sweeps of few tiles (paged but for the dense ones):
+//   hd 128  16 of 73, 16                               768          3         32.4 / 40.2
+//           9 of 40, 16, dense                         288          2         13.4 / 19.6
+//           15 of 129, 8, dense                        600          5         27.1 / 36.2
+//           14 of 200, 8                               784          7         54.7 / 56.7
+//           25 of 40 behind 150, 16                    800          6         80.6 / 73.4
+//           15 of 129 behind 140, 8                    600          9         67.3 / 63.3
+//           38 of 20 behind 250, 16                    608          9          160 / 70
+//   hd 64   16 of 73, 16                               768          3         20.6 / 25.3
+//           14 of 200, 8, dense                        784          7         21.9 / 25.5
+//           8 of 280, 8, dense                         576          9         25.9 / 23.1
+//           13 of 64 behind 210, 16                    416          9         36.3 / 27.0
 // Long sweeps split until the matrix units are busy either way, later under the causal rule over long chunks, whose
-// workgroups are of unequal length; short ones only while each block has a CU to itself.  (The tables' width stands
-// for the longest context, which the host does not know.)
+// workgroups are of unequal length; short ones only while each block has a CU to itself.  (The tables' width stands for the
+// longest context only where the caller does not say it: a table may have room for many more blocks.)
 bool takes_split(const PrefillArgs &a) {
   if (a.mask != nullptr || a.mask_bits != nullptr) return false;
   const bool one_block = a.block_tables == nullptr || a.block_table_stride == 1;
   if (!one_block && a.pool.block_size < 1) return false;
   const int64_t blocks = ((int64_t)a.max_chunk_len + 31) / 32 * a.hn * a.n_seqs;
-  const int64_t keys = a.context_lens == nullptr ? a.uniform_context : a.block_table_stride * a.pool.block_size;
-  if (keys < 10 * 32 - 31) return blocks <= device_cu_count();
-  return blocks <= (a.causal && a.max_chunk_len >= 300 ? 1700 : 800);
+  const int64_t cus = device_cu_count();
+  int64_t keys = a.uniform_context;
+  if (a.context_lens != nullptr) {
+    const int64_t width = a.block_table_stride * a.pool.block_size;
+    keys = keys > 0 && keys < width ? keys : width;
+  }
+  if (keys <= 7 * kF32BN) return blocks <= cus;
+  return blocks <= (a.causal && a.max_chunk_len >= 300 ? 53 : 25) * cus / 8;
 }
 
 }  // namespace

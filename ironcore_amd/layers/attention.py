@@ -351,9 +351,11 @@ class Attention(BaseModule):
             if out is not None:
                 return out
         elif here is not None and (rows is None or meta.cu_seqlens_q is not None):   # (rows come with their bounds)
+            known = getattr(meta, "max_context_len", 0)
             out = _lib.host().prefill_step(query, key, value, k_pool, v_pool, meta.block_tables, meta.context_lens,
                                            meta.slot_mapping, meta.cu_seqlens_q, rows, sq if rows is None else int(meta.max_chunk_len),
-                                           1.0 / self.scale_factor, *(rope or (None, None, None)), *here)
+                                           1.0 / self.scale_factor, *(rope or (None, None, None)), *here,
+                                           known if type(known) is int else 0)
             if out is not None:
                 return out
         if rotary_pos_emb is None:

@@ -68,3 +68,31 @@ def test_dense(gpu, hd, causal, b, s):
     for i in range(b):
         want = _attend(q[i], k[i], v[i], 0, causal, hd ** -0.5)
         assert ((out[i].double() - want).norm() / want.norm()).item() <= TOL
+
+
+@pytest.mark.parametrize("n,chunk,prefix", [(10, 73, 0), (12, 40, 150), (20, 129, 90)])
+def test_a_table_s_room_changes_nothing(gpu, n, chunk, prefix):
+    """The layer call knows its longest context: tables with reserved blocks take the same kernel, bit for bit, as
+    tables that end with the contexts (more workgroups than CUs, short sweeps: the one that does not split)."""
+    from ironcore_amd import config as ic_config
+    from ironcore_amd.layers import Attention, PagedAttentionMetadata
+    hn, gn, hd = 16, 16, 64
+    cfg = ic_config.MainConfig(model=ic_config.ModelConfig(d_model=hn * hd, num_attention_heads=hn, num_attention_groups=gn,
+                                                           head_dim=hd, dropout_attn=0.0, precision="fp32"),
+                               trainer=ic_config.TrainerConfig(use_flash_attn=False))
+    layer = Attention(cfg).to(gpu).eval()
+    g = torch.Generator().manual_seed(n)
+    blocks = -(-(prefix + chunk) // 16)
+    perm = torch.randperm(n * blocks, generator=g).view(n, blocks).to(torch.int32)
+    at = torch.arange(prefix, prefix + chunk)
+    slots = (perm[:, at // 16].long() * 16 + at % 16).reshape(-1).to(gpu)
+    q, k, v = (torch.randn(n, chunk, hn, hd, generator=g).to(gpu) for _ in range(3))
+    pools = [torch.randn(n * blocks, gn, 16, hd, generator=g).to(gpu) for _ in range(2)]
+    out = []
+    for room in (0, 64):
+        tables = torch.cat([perm, torch.zeros(n, room, dtype=torch.int32)], dim=1).to(gpu)
+        meta = PagedAttentionMetadata(block_tables=tables, slot_mapping=slots, max_context_len=prefix + chunk,
+                                      context_lens=torch.full((n,), prefix + chunk, dtype=torch.int32, device=gpu))
+        with torch.no_grad():
+            out.append(layer(q, k, v, None, kv_cache=tuple(t.clone() for t in pools), attn_metadata=meta))
+    assert torch.equal(*out)
