@@ -10,9 +10,11 @@ from __future__ import annotations
 
 import concurrent.futures
 import os
+import re
 import shutil
 import subprocess
 import sys
+import tempfile
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -69,13 +71,43 @@ PER_SOURCE_FLAGS = {"paged_prefill.hip": _VGPR_FORM, "paged_prefill_short.hip": 
                     "paged_prefill_f32.hip": _VGPR_FORM, "paged_decode_mfma.hip": _VGPR_FORM}
 
 
+# Sources whose kernels keep registers in scratch: their assembly is looked at, see masked_spills.
+_SPILLING = {"step_stack.hip"}
+
+
+def masked_spills(asm: str) -> list[str]:
+    """Labels of blocks that move registers to or from scratch and only then switch on the lanes that a branch had
+    switched off.  The compiler does that where a whole value is meant (it takes the block's start for the place behind
+    ``s_or_b64 exec``): the other lanes' part is then lost, and a kernel that counts on it ends wrong or never."""
+    found, kernel, label, moved = [], "", "", False
+    for line in asm.splitlines():
+        name = re.match(r"(\w+):|; (%bb\.\d+):|(\.LBB\w+):", line)
+        if name:
+            kernel, label, moved = name[1] or kernel, name[2] or name[3] or "entry", False
+        elif re.match(r"\ts_\w+ exec, exec|\ts_mov_b64 exec|\ts_\w+_saveexec", line):
+            if moved and line.startswith("\ts_or_b64 exec, exec"):
+                found.append(f"{kernel} {label}")
+            moved = False
+        elif "Folded" in line and "scratch_" in line:
+            moved = True
+    return found
+
+
 def _compile(src: str, extra: list[str]) -> Path:
     obj = OBJ_DIR / (src + ".o")
-    cmd = [_hipcc(), *HIPCC_FLAGS, *PER_SOURCE_FLAGS.get(src, []), *extra, "-c", str(CSRC / src),
-           "-o", str(obj)]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed on {src}:\n{res.stdout}\n{res.stderr}")
+    with tempfile.TemporaryDirectory(dir=OBJ_DIR) as temps:
+        out = Path(temps) / obj.name
+        cmd = [_hipcc(), *HIPCC_FLAGS, *PER_SOURCE_FLAGS.get(src, []), *extra, "-c", str(CSRC / src), "-o", str(out)]
+        if src in _SPILLING:
+            cmd.append("-save-temps=obj")
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        if res.returncode != 0:
+            raise RuntimeError(f"hipcc failed on {src}:\n{res.stdout}\n{res.stderr}")
+        if src in _SPILLING:
+            (asm,) = Path(temps).glob("*-gfx950.s")
+            if found := masked_spills(asm.read_text()):
+                raise RuntimeError(f"{src}: registers go to scratch before all lanes are on again, in {found}")
+        os.replace(out, obj)
     noise = "is not a recognized feature for this target"
     warn = "\n".join(line for line in res.stderr.splitlines() if noise not in line)
     if warn.strip():

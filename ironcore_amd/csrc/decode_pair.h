@@ -46,11 +46,13 @@ __device__ __forceinline__ int walk_pair(const DecodeKP &p, const char *k_pool, 
   const int tiles = (ctx + BS - 1) / BS;
   const int mine = __builtin_amdgcn_readfirstlane(tiles > wave ? (tiles - wave + kPairWaves - 1) / kPairWaves : 0);
   rows.early();
-  // lane r: byte offset of this wave's tile of round r, and the tile's number in the pool
+  // lane r: byte offset of this wave's tile of round r, and the tile's number in the pool (lanes past the last round: the last
+  // one's).  Nothing here depends on the lane's number but its operands: behind a branch of some lanes the compiler has put
+  // registers into scratch before it switched the other lanes on again, and a wave without tiles then lost its lanes' numbers.
   int64_t tile_off = 0;
   int tile_id = -1;
-  if (lane < mine) {
-    const int tile = wave + lane * kPairWaves;
+  if (mine > 0) {
+    const int tile = wave + (lane < mine ? lane : mine - 1) * kPairWaves;
     const int blk = tile / p.tiles_per_block;
     int64_t phys = p.block_tables[seq * p.bt_stride + blk];
     // A corrupt table entry must not become an out-of-pool address.

@@ -159,8 +159,8 @@ struct StackRows {
   __device__ __forceinline__ Vec16 key(int j) const { return take16(p, at(j, p.q_cols + kvh * HD)); }
   __device__ __forceinline__ Vec16 value(int j) const { return take16(p, at(j, p.q_cols + p.kv_cols + kvh * HD)); }
   __device__ __forceinline__ void early() {
-    if (lane < p.m) slot = p.slots[lane];
-    if (slot >= p.num_slots) slot = -1;
+    slot = p.slots[lane < p.m ? lane : 0];
+    if (lane >= p.m || slot >= p.num_slots) slot = -1;
   }
   __device__ __forceinline__ void queries(Vec16 *qreg) {
     uint64_t w[GT + 2][2];
