@@ -25,6 +25,7 @@
  *    class (asked once, see ic_decode_occupancy_queries) and whether a
  *    variant's dynamic-LDS limit has been raised.  All of it is written
  *    once and read with atomics.
+ *  - Host memory the library owns: the word of ic_step_status.
  *  - Device memory the library owns: one array of IC_STATIC_SCRATCH_BYTES
  *    (32 MiB), part of the code object, so every process that loads the
  *    library holds it on each GPU it uses, whether or not it ever calls
@@ -572,6 +573,11 @@ int ic_step_linear(const ic_step_linear_call *call, void *stream);
  *   workspace  ic_step_stack_workspace_bytes(call) bytes, 256-byte aligned (0: unsupported).
  *   workgroups  0: one to a CU.  draw: nonzero deals the work by a counter, as the launch does
  *          by itself when other work keeps its workgroups from starting together.
+ *   max_polls, status  a wait for another workgroup's results is given up after so many polls (0: 4 194 304,
+ *          seconds; met only if a part of the launch stopped).  The launch then ends all the same: rows of out and
+ *          norm_out that needed those results hold NaNs, no row that came of them is appended (rows of the step may be
+ *          missing from the pools, none is wrong), and *status, if not NULL, is set to 1.  It is never cleared
+ *          here; device or pinned host memory that lives until the launch has ended, such as ic_step_status().
  */
 #define IC_STEP_STACK_LAYERS 16
 #define IC_STEP_STACK_ROWS 16
@@ -606,9 +612,18 @@ typedef struct ic_step_stack_call {
   int dtype, workgroups, draw;
   void *workspace;
   size_t workspace_bytes;
+  int32_t *status;
+  int max_polls;
 } ic_step_stack_call;
 size_t ic_step_stack_workspace_bytes(const ic_step_stack_call *call);
 int ic_step_stack(const ic_step_stack_call *call, void *stream);
+
+/*
+ * A word for `status` that launches in flight may write at any time: pinned host memory, one for the process, allocated
+ * and cleared by the first call and never freed (NULL: not to be had).  The library neither reads it nor hands it to a
+ * launch by itself.  Any host thread, also while a stream is capturing.
+ */
+int32_t *ic_step_status(void);
 
 /*
  * The append of a step's chunks in one launch: ic_kv_append, or with cos_table and

@@ -17,6 +17,7 @@ LIB_PATH = Path(__file__).resolve().parent / "lib" / "libironcore_paged.so"
 HOST_PATH = LIB_PATH.parent / "_host.so"
 
 IC_OK = 0
+IC_ERR_LAUNCH = -5
 IC_DTYPE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 # Call descriptors, field by field as in the header (tests hold them to it).
@@ -38,7 +39,7 @@ _FIELDS = {
         ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("block_tables", c_void_p),
         ("block_table_stride", c_int64), ("context_lens slot_mapping positions cos_table sin_table", c_void_p),
         ("table_rows", c_int64), ("block_size max_context_len", c_int), ("scale", c_float), ("dtype workgroups draw", c_int),
-        ("workspace", c_void_p), ("workspace_bytes", c_size_t)),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t), ("status", c_void_p), ("max_polls", c_int)),
     "ic_append_call": (
         ("k_new v_new", c_void_p), ("new_stride_token", c_int64), ("k_pool v_pool", c_void_p),
         ("pool_stride_block pool_stride_head pool_stride_token num_blocks", c_int64), ("slot_mapping", c_void_p),
@@ -145,6 +146,7 @@ SIGNATURES = {
     "ic_step_linear": (c_int, [c_void_p, c_void_p]),    # call descriptor, stream
     "ic_step_stack_workspace_bytes": (c_size_t, [c_void_p]),   # call descriptor
     "ic_step_stack": (c_int, [c_void_p, c_void_p]),     # call descriptor, stream
+    "ic_step_status": (c_void_p, []),
     "ic_append_chunks": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_paged_decode_append": (c_int, [c_void_p, c_void_p]),   # call descriptor, stream
     "ic_greedy_workspace_bytes": (c_size_t, [c_int, c_int]),   # rows, n

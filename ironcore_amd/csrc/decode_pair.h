@@ -24,8 +24,8 @@ struct PairShared {
 };
 
 // Leaves the waves' sums in `s` and returns the number of tiles; the caller's barrier comes next.  `rows` hands over the query rows and, with kNew, the
-// step's new rows: the slots, a lane a row, the pair's own row as it is stored, any other row by key(j) and value(j), all in
-// the lane's chunk.  kLate: the queries (and the own row) are asked for once the first two tiles are on their way.
+// step's new rows: the slots, a lane a row, the pair's own row as it is stored (if it is sound()), any other row by key(j) and
+// value(j), all in the lane's chunk.  kLate: the queries (and the own row) are asked for once the first two tiles are on their way.
 template <class E, int HD, int GT, class Rows>
 __device__ __forceinline__ int walk_pair(const DecodeKP &p, const char *k_pool, const char *v_pool, int seq, int kvh,
                                          int thread, PairShared<HD, GT> &s, Rows &rows) {
@@ -155,7 +155,7 @@ __device__ __forceinline__ int walk_pair(const DecodeKP &p, const char *k_pool, 
     // the last wave has the fewest tiles; K from its first row of lanes, V from the second
     const int64_t to = ((int64_t)__builtin_amdgcn_readlane((uint32_t)((uint64_t)rows.slot >> 32), seq) << 32) |
                        (uint32_t)__builtin_amdgcn_readlane((uint32_t)rows.slot, seq);
-    if (wave == kPairWaves - 1 && to >= 0 && rowg < 2) {
+    if (wave == kPairWaves - 1 && to >= 0 && rows.sound() && rowg < 2) {
       const int64_t blk = (uint64_t)to / (uint32_t)(p.tiles_per_block * BS);
       const int64_t at = blk * p.stride_block + kvh * p.stride_head + (to - blk * p.tiles_per_block * BS) * p.stride_token;
       Vec16 own;  // (word by word: a choice between two members would put `rows` into scratch)

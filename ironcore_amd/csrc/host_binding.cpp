@@ -20,6 +20,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 
 #include "../../include/ironcore_paged.h"
@@ -698,6 +699,13 @@ bool stack_takes(at::ScalarType type, int64_t b, int64_t d, int64_t f, int64_t h
   return stack_pays(type, b, d, f, hn / gn, hd, max_ctx, d * columns * (int64_t)c10::elementSize(type));
 }
 
+// Where launches say that they gave up a wait (ic_step_stack), and whether one has since the last time this was asked.
+std::atomic<int32_t *> step_status{nullptr};
+bool step_given_up() {
+  int32_t *const word = step_status.load(std::memory_order_acquire);
+  return word != nullptr && __atomic_load_n(word, __ATOMIC_RELAXED) != 0 && __atomic_exchange_n(word, 0, __ATOMIC_RELAXED) != 0;
+}
+
 OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor>> &w,
                         const std::vector<std::tuple<Norm, Norm>> &norms, const Norm &last, int64_t hn, int64_t gn,
                         int64_t hd, int64_t act, const std::vector<std::tuple<Tensor, Tensor>> &pools, const Tensor &tables,
@@ -759,6 +767,8 @@ OptTensor decoder_stack(const Tensor &x, const std::vector<std::vector<OptTensor
   c.context_lens = lens.data_ptr<int32_t>(), c.slot_mapping = slots.data_ptr<int64_t>();
   c.positions = rope.positions, c.cos_table = rope.cos, c.sin_table = rope.sin, c.table_rows = rope.rows;
   c.block_size = (int)first.bs, c.max_context_len = (int)max_ctx, c.scale = (float)scale, c.dtype = first.dtype;
+  c.status = ic_step_status();
+  step_status.store(c.status, std::memory_order_release);
   const size_t parts = (layers + IC_STEP_STACK_LAYERS - 1) / IC_STEP_STACK_LAYERS;
   Tensor in = x, out, ws;
   for (size_t part = 0, from = 0; part < parts; ++part) {
@@ -857,6 +867,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decoder_layer", torch::wrap_pybind_function_no_gil(decoder_layer));
   m.attr("STEP_ROWS") = IC_LINEAR_ROWS_MAX;
   m.def("stack_takes", &stack_takes);
+  m.def("step_given_up", &step_given_up);
   m.def("decoder_stack", torch::wrap_pybind_function_no_gil(decoder_stack));
   m.def("greedy", torch::wrap_pybind_function_no_gil(greedy));
   m.def("advance", torch::wrap_pybind_function_no_gil(advance));

@@ -1,6 +1,7 @@
 // C ABI: argument validation on the host, then dispatch to the kernel
 // launchers.  Nothing here allocates, synchronises or keeps state.
 #include <atomic>
+#include <cstring>
 
 #include "ic_internal.h"
 #include "../../include/ironcore_paged.h"
@@ -569,7 +570,7 @@ int ic_step_linear(const ic_step_linear_call *call, void *stream) {
 
 static int step_stack_sizes(const ic_step_stack_call &a) {
   if (a.num_layers < 0 || a.m < 0 || a.d <= 0 || a.f <= 0 || a.hn <= 0 || a.gn <= 0 || a.hd <= 0 || a.block_size <= 0 ||
-      a.workgroups < 0 || a.max_context_len < 0)
+      a.workgroups < 0 || a.max_context_len < 0 || a.max_polls < 0)
     return IC_ERR_BAD_SHAPE;
   if (!dtype_ok(a.dtype) || a.norm < IC_NORM_NONE || a.norm > IC_NORM_RMS || a.act < IC_ACT_NONE || a.act > IC_ACT_SWIGLU)
     return IC_ERR_UNSUPPORTED;
@@ -620,6 +621,19 @@ int ic_step_stack(const ic_step_stack_call *call, void *stream) {
       a.workspace_bytes < ic::step_stack_workspace_bytes(a))
     return IC_ERR_WORKSPACE;
   return ic::launch_step_stack(a, static_cast<hipStream_t>(stream));
+}
+
+int32_t *ic_step_status(void) {
+  static int32_t *const word = []() -> int32_t * {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (no part of a graph that this thread may be capturing)
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, 64, hipHostMallocDefault) != hipSuccess) p = nullptr, (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (p != nullptr) memset(p, 0, 64);
+    return static_cast<int32_t *>(p);
+  }();
+  return word;
 }
 
 int ic_paged_decode_append(const ic_decode_append_call *call, void *stream) {

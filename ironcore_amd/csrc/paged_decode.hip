@@ -348,6 +348,7 @@ struct PairRows {
     return rotate_chunk<E>(k, n.cos_table + at, n.sin_table + at);
   }
   __device__ __forceinline__ Vec16 value(int j) const { return load16(n.v_new + j * n.new_stride_bytes + new_at()); }
+  __device__ __forceinline__ bool sound() const { return true; }
   __device__ __forceinline__ void early() {
     if constexpr (APPEND) {
       if (lane < p.n_seqs) slot = n.slots[lane];

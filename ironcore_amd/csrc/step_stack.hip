@@ -17,8 +17,9 @@
 //    workgroup r takes the tasks r, r + workgroups, ...  If they do not within kMeetTicks (other streams hold CUs), tasks
 //    are drawn from a counter: a task waits for tasks with lower numbers only, those are drawn before it by workgroups that
 //    are running, and of the tasks drawn and not finished the lowest waits for nothing.  Either way is chosen once, by one
-//    word.  (A ticket each time costs: 3.7 us from task to task over all CUs, 2.3 without.)  A wait that lasts for kGiveUp polls
-//    all the same (seconds) ends the launch with NaNs.
+//    word.  (A ticket each time costs: 3.7 us from task to task over all CUs, 2.3 without.)  A wait that lasts for kMaxPolls
+//    polls all the same (seconds) is given up: the words that it lacks are NaNs and make NaNs of what comes of them.  That is
+//    known everywhere (kGaveUp) before any such word is handed on, and a row of K or V that may be one is not appended.
 //
 // Bound by the hand-over: from the last result of a phase to its arrival in all workgroups 1.5-2 us (past the L2s), five
 // times a layer and once more for the splits of the down-projection, then 0.8-2 us for the phase itself; the launches
@@ -40,7 +41,7 @@ namespace {
 
 constexpr uint32_t kMissing = 0xffffffffu;
 constexpr uint64_t kMeetTicks = 3000;                    // of the 100 MHz counter
-constexpr uint32_t kGiveUp = 1u << 22;
+constexpr int kMaxPolls = 1 << 22;  // of a wait, unless the call says otherwise
 
 enum Phase { kQkv = 0, kAttend = 1, kProj = 2, kUp = 3, kDown = 4, kPhases = 5 };
 
@@ -68,6 +69,8 @@ struct StackKP {
   const float *cos_table, *sin_table;
   int64_t num_slots, table_rows;
   int gn, hd, must_draw;
+  uint32_t poll_mask, max_polls;
+  int32_t *status;
 };
 static_assert(sizeof(StackKP) <= 4096, "kernel arguments");
 
@@ -108,9 +111,16 @@ __device__ __forceinline__ void publish(char *at, float a, float b) {
 // A pause between two polls; true: give the wait up.
 __device__ __forceinline__ bool pause(const StackKP &p, uint32_t &polls) {
   __builtin_amdgcn_s_sleep(1);
-  if ((++polls & 1023) != 0) return false;
-  if (polls >= kGiveUp) __hip_atomic_store(p.control + kGaveUp, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return peek(p.control + kGaveUp) != 0;
+  if ((++polls & p.poll_mask) != 0) return false;
+  const __attribute__((address_space(4))) StackKP *rare = (const __attribute__((address_space(4))) StackKP *)layer_args();
+  asm volatile("" : "+s"(rare));  // (read here only: as arguments they would be kept in registers throughout)
+  if (polls >= rare->max_polls) {
+    int32_t *const status = rare->status;
+    __hip_atomic_store(rare->control + kGaveUp, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (status != nullptr) __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // before what this workgroup hands on from now
+  }
+  return peek(rare->control + kGaveUp) != 0;
 }
 
 // Two neighbouring values that a lane needs: as they are, and waited for (plain: a tensor from before the launch).
@@ -158,6 +168,8 @@ struct StackRows {
   }
   __device__ __forceinline__ Vec16 key(int j) const { return take16(p, at(j, p.q_cols + kvh * HD)); }
   __device__ __forceinline__ Vec16 value(int j) const { return take16(p, at(j, p.q_cols + p.kv_cols + kvh * HD)); }
+  // Whether the pair's own row, which is there, may be appended.
+  __device__ __forceinline__ bool sound() const { return peek(p.control + kGaveUp) == 0; }
   __device__ __forceinline__ void early() {
     slot = p.slots[lane < p.m ? lane : 0];
     if (lane >= p.m || slot >= p.num_slots) slot = -1;
@@ -885,6 +897,8 @@ int launch_step_stack(const ic_step_stack_call &a, hipStream_t stream) {
   kp.cos_table = a.cos_table, kp.sin_table = a.sin_table, kp.table_rows = a.table_rows;
   kp.num_slots = a.num_blocks * a.block_size;
   kp.gn = a.gn, kp.hd = a.hd, kp.must_draw = a.draw;
+  kp.max_polls = (uint32_t)(a.max_polls > 0 ? a.max_polls : kMaxPolls), kp.status = a.status;
+  kp.poll_mask = kp.max_polls < 1024 ? 0 : 1023;
   const int64_t pieces = (int64_t)step_stack_workspace_bytes(a) / 16;
   const int64_t fill = (pieces + kFillThreads - 1) / kFillThreads, most = 4 * (int64_t)device_cu_count();
   hipLaunchKernelGGL(step_stack_fill_kernel, dim3((unsigned)(fill < most ? fill : most)), dim3(kFillThreads), 0, stream,

@@ -307,6 +307,14 @@ def _step_plan(model, d):
     return None if last is None or None in layers or not layers else (layers, last)
 
 
+def _check_steps(host) -> None:
+    """Raises if a decode step whose launches have ended gave up (ic_step_stack): its logits are NaN, and rows of it are
+    missing from its cache.  Reads a word of host memory; nothing is waited for."""
+    if host.step_given_up():
+        raise _lib.PagedLibraryError("ic_step_stack", _lib.IC_ERR_LAUNCH, "an earlier decode step gave up waiting for a part "
+                                     "of its launch; its logits are NaN and its cache lacks rows")
+
+
 def _untouched_by_anyone() -> bool:
     module = torch.nn.modules.module
     return not (module._global_forward_hooks or module._global_forward_pre_hooks or module._global_backward_hooks
@@ -429,6 +437,7 @@ class LanguageModel(BaseModule):
                 or torch.overrides.has_torch_function_unary(x) or torch.compiler.is_compiling() or torch.jit.is_tracing()):
             return None
         host = _lib.host()
+        _check_steps(host)
         if x.shape[0] > host.STEP_ROWS:   # (more than any of the calls takes: nothing is gathered for them)
             return None
         plan = _step_plan(self, x.shape[-1])
@@ -565,8 +574,12 @@ def generate(model: LanguageModel, input_ids: torch.Tensor, max_new_tokens: int,
             finished |= nxt.squeeze(1) == eos_token_id
         tokens = torch.cat([tokens, nxt], dim=1)
         step_input = nxt
-        if eos_token_id is not None and bool(finished.all()):
-            break
+        if eos_token_id is not None:
+            ended = bool(finished.all())
+            if finished.is_cuda:
+                _check_steps(_lib.host())
+            if ended:
+                break
     if own_cache:
         for sid in seq_ids:
             kv_cache.free_sequence(sid)
@@ -679,8 +692,11 @@ def _generate_graphed(model, input_ids, max_new_tokens, block_size, eos_token_id
         for i in range(max_new_tokens - 2):
             graph.replay()
             steps_run += 1
-            if eos_token_id is not None and i % 8 == 7 and bool(finished.all()):
-                break
+            if eos_token_id is not None and i % 8 == 7:
+                ended = bool(finished.all())
+                _check_steps(_lib.host())
+                if ended:
+                    break
     kv_cache.advance(seq_ids, steps_run)
     n = steps_run + 1
     if eos_token_id is not None:

@@ -202,6 +202,27 @@ def test_nan_and_infinity_pass_through(gpu):
     assert torch.equal(out[0], clean[0]) and torch.equal(out[3], clean[3])
 
 
+@pytest.mark.parametrize("over", [dict(), dict(workgroups=37), dict(draw=1)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[2], SHAPES[3]], ids=lambda s: "-".join(map(str, s[:6])))
+def test_a_wait_that_is_given_up(gpu, dtype, shape, over):
+    """With one poll to a wait the launch ends, says so, and appends nothing that is wrong: outputs are the right ones or
+    NaN, the pools' rows the right ones or the old ones."""
+    c, weights, x, pools = _case(gpu, dtype, *shape)
+    out, normed, after = _run(gpu, dtype, c, weights, x, pools, **over)
+    status = torch.zeros(1, dtype=torch.int32, device=gpu)
+    _run(gpu, dtype, c, weights, x, pools, status=status.data_ptr(), **over)
+    assert status.item() == 0
+    lost_out, lost_normed, lost_after = _run(gpu, dtype, c, weights, x, pools, status=status.data_ptr(), max_polls=1, **over)
+    assert status.item() == 1
+    for got, want in ((lost_out, out), (lost_normed, normed)):
+        assert got.isnan().any() and bool((got.isnan() | (got == want)).all())
+    assert bool((lost_normed.isnan().all(1) | (lost_normed == normed).all(1)).all())
+    for pair, right, before in zip(lost_after, after, pools):
+        for got, want, old in zip(pair, right, before):
+            assert bool(((got == want) | (got == old.to(gpu))).all())
+
+
 def _model(gpu, dtype, layers):
     from ironcore_amd import config as ic_config
     from ironcore_amd import generation
@@ -256,3 +277,16 @@ def test_model_of_two_parts_two_streams_and_a_graph(gpu, monkeypatch):
     for t in threads:
         t.join()
     assert torch.equal(got[0], want) and torch.equal(got[1], want)
+
+
+def test_a_step_that_gave_up_is_raised(gpu):
+    """The next step of the process raises what an earlier one's launch has left in the status word, once."""
+    from ironcore_amd import generation
+    model = _model(gpu, torch.float32, 2)
+    ids = torch.randint(0, 500, (3, 20), generator=torch.Generator().manual_seed(1)).to(gpu)
+    want = generation.generate(model, ids, 4)
+    torch.cuda.synchronize()
+    ctypes.c_int32.from_address(_lib.load().ic_step_status()).value = 1
+    with pytest.raises(_lib.PagedLibraryError, match="gave up"):
+        generation.generate(model, ids, 4)
+    assert torch.equal(generation.generate(model, ids, 4, eos_token_id=511), want)
