@@ -1,5 +1,6 @@
 // C ABI: argument validation on the host, then dispatch to the kernel
-// launchers.  Nothing here allocates, synchronises or keeps state.
+// launchers.  Nothing here synchronises or keeps state, and nothing but
+// ic_step_status allocates.
 #include <atomic>
 #include <cstring>
 
@@ -593,8 +594,11 @@ int ic_step_stack(const ic_step_stack_call *call, void *stream) {
   if (const int rc = step_stack_sizes(a); rc != IC_OK) return rc;
   if (a.m == 0 || a.num_layers == 0) return IC_OK;
   const int es = ic::elem_size(a.dtype);
-  if (a.num_blocks <= 0 || a.num_blocks * (a.block_size / 16) >= (int64_t)1 << 31 || a.pool_stride_block <= 0 ||
-      a.pool_stride_head <= 0 || a.pool_stride_token <= 0 ||
+  if (const int rc = check_pool(a.pool_stride_block, a.pool_stride_head, a.pool_stride_token, a.gn, a.hd, a.block_size,
+                                a.num_blocks, es))
+    return rc;
+  if (a.pool_stride_token >= ((int64_t)1 << 32) / (16 * es)) return IC_ERR_UNSUPPORTED;  // (32-bit offsets in a tile of 16 tokens)
+  if (a.num_blocks * (a.block_size / 16) >= (int64_t)1 << 31 ||
       a.block_table_stride < ((int64_t)a.max_context_len + a.block_size - 1) / a.block_size)
     return IC_ERR_BAD_SHAPE;
   if (!a.layers || !a.x || (!a.out && a.norm == IC_NORM_NONE) || (a.norm != IC_NORM_NONE && (!a.norm_weight || !a.norm_out)) ||
@@ -602,8 +606,7 @@ int ic_step_stack(const ic_step_stack_call *call, void *stream) {
       (a.cos_table && (!a.positions || a.table_rows <= 0)))
     return IC_ERR_NULL_POINTER;
   bool whole = aligned16(a.x) && aligned16(a.out) && aligned16(a.norm_out) && aligned16(a.norm_weight) &&
-               aligned16(a.norm_bias) && stride16(a.pool_stride_block, es) && stride16(a.pool_stride_head, es) &&
-               stride16(a.pool_stride_token, es);
+               aligned16(a.norm_bias);
   for (int i = 0; i < a.num_layers; ++i) {
     const ic_step_layer &l = a.layers[i];
     if (!l.input_norm_weight || !l.q_weight || !l.kv_weight || !l.proj_weight || !l.post_norm_weight || !l.up_weight ||
