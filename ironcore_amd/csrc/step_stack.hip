@@ -482,8 +482,9 @@ struct Stack {
     }
   }
 
-  // The wave's sums of the tile, [row of x][column] in LDS.
-  __device__ __forceinline__ void multiply_block(const Words<1> (&wv)[S][KR], const Vec16 (&xv)[S]) const {
+  // The wave's sums of the tile, [row of x][column] in LDS, over its first `used` steps (those past the end of a column hold
+  // other rows' weights: with zeros of x they add nothing, but a NaN if a weight is infinite).
+  __device__ __forceinline__ void multiply_block(const Words<1> (&wv)[S][KR], const Vec16 (&xv)[S], int used) const {
     float *const sums = sh.sum[wave];
     f32x4_t acc[NB][1];
 #pragma unroll
@@ -491,11 +492,13 @@ struct Stack {
     if (few) {
       if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int i = 0; i < S; ++i)
+        for (int i = 0; i < S; ++i) {
+          if (i >= used) break;
 #pragma unroll
           for (int r = 0; r < KR; ++r)
             acc[0][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(__builtin_bit_cast(float, wv[i][r].w[0]),
                                                            __builtin_bit_cast(float, xv[i].w[r]), acc[0][0], 0, 0, 0);
+        }
         // lane (c, g): columns 4 * (c / 4) + r of row c % 4, the k of lane group g
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -510,6 +513,7 @@ struct Stack {
     }
 #pragma unroll
     for (int i = 0; i < S; ++i) {
+      if (i >= used) break;
       const Vec16 x[1] = {xv[i]};
       multiply<M, 1, NB>(wv[i], x, acc);
     }
@@ -597,11 +601,11 @@ struct Stack {
     barrier();  // (the rows of x go where the weights are)
     // ---- the product -----------------------------------------------------------------------------
     Vec16 xv[S];
-    take_rows(PHASE == kQkv ? hidden : mine_words + (PHASE == kProj ? p.at_att : PHASE == kUp ? p.at_mid : p.at_act),
-              PHASE == kProj ? p.q_cols : PHASE == kDown ? p.f : p.d, t.split, PHASE == kQkv && plain, slot, xv, last ? residual : nullptr,
+    const int k = PHASE == kProj ? p.q_cols : PHASE == kDown ? p.f : p.d;
+    take_rows(PHASE == kQkv ? hidden : mine_words + (PHASE == kProj ? p.at_att : PHASE == kUp ? p.at_mid : p.at_act), k, t.split, PHASE == kQkv && plain, slot, xv, last ? residual : nullptr,
               res_word);
     if constexpr (kNormed) norm_rows(xv, slot, shifted, centered, eps);
-    multiply_block(wv, xv);
+    multiply_block(wv, xv, (k * ES / 64 - first_step(t.split, wave) + kStepWaves - 1) / kStepWaves);
     barrier();
     if (!mine) return;
     float2 v = total(row, at);

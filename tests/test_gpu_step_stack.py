@@ -202,6 +202,21 @@ def test_nan_and_infinity_pass_through(gpu):
     assert torch.equal(out[0], clean[0]) and torch.equal(out[3], clean[3])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m", [4, 5])
+def test_infinite_weights(gpu, dtype, m):
+    """Infinities in the last row of a matrix whose rows do not fill a task's steps: infinite keys where they belong."""
+    c, weights, x, pools = _case(gpu, dtype, m, 512, 512, 8, 8, 64, GELU, NORM_LAYER, False, tuple(range(17, 17 + m)), layers=1)
+    weights[0]["kv"][511, 3] = float("inf")
+    weights[0]["kv"][511, 70] = -float("inf")
+    _, _, [(keys, _)] = _run(gpu, dtype, c, weights, x, pools)
+    last = _norm(x.double(), NORM_LAYER, weights[0]["n1"].double(), weights[0]["n1b"].double(), 1e-5)[:, 511]
+    for i, slot in enumerate(c["slots"].tolist()):
+        row = keys[slot // 16, :, slot % 16].cpu().float()
+        assert row[0, 3] == float("inf") * last[i].sign() and row[1, 6] == -float("inf") * last[i].sign()
+        assert row.isfinite().sum() == row.numel() - 2
+
+
 @pytest.mark.parametrize("over", [dict(), dict(workgroups=37), dict(draw=1)], ids=str)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[2], SHAPES[3]], ids=lambda s: "-".join(map(str, s[:6])))
