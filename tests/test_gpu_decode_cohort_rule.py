@@ -46,6 +46,12 @@ def test_as_without_cohorts(gpu, dtype, shape):
     assert off.item() <= 4 * {torch.bfloat16: 2 ** -9, torch.float16: 2 ** -12}[dtype]
 
 
+@pytest.mark.parametrize("shape", [(5, 16, 28, 4, 64, 576, 36), (2, 16, 64, 8, 64, 320, 20),   # read once: the line for head dim 64
+                                   (2, 16, 28, 4, 64, 576, 36)], ids=lambda s: "-".join(map(str, s)))
+def test_many_query_rows_of_head_dim_64(gpu, shape):
+    test_as_without_cohorts(gpu, torch.bfloat16, shape)
+
+
 def test_cohorts_that_do_not_fit_are_refused(gpu):
     with pytest.raises(ValueError):
         _call(gpu, torch.bfloat16, 2, 4, 4, 4, 64, 32, 20, True, torch.zeros(3, dtype=torch.int32, device=gpu))

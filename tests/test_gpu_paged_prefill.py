@@ -101,7 +101,8 @@ def test_prefill_block_sizes_that_are_no_power_of_two(gpu, block):
 @pytest.mark.parametrize("prefix,chunk", [(0, 1), (0, 17), (0, 128), (5, 64), (100, 33), (64, 129), (300, 200),
                                           (1000, 256), (63, 65), (31, 300)])
 def test_prefill_fp32_prefix_chunk_shapes(gpu, prefix, chunk):
-    """fp32 pools: 32-token K/V tiles, 128-row query tiles, every product and sum in fp32."""
+    """fp32 pools: 32-token K/V tiles, every product and sum in fp32; grids this small take 32 rows to a workgroup and split
+    the keys over its waves (the kernel with 128 rows: test_gpu_prefill_f32_whole.py)."""
     wl = workloads.make_prefill_workload(2, 4, 4, 128, prefix, prefix, chunk, chunk, dtype=torch.float32,
                                          seed=prefix + chunk)
     _check(wl, gpu)

@@ -44,7 +44,7 @@ def _turn(x, cos, sin):  # [m, heads, hd], [m, 1, hd / 2]
 
 def _oracle(c, layers, x, pools):
     """(last norm's output, pools) in float64."""
-    m, hn, gn, hd = c["m"], c["hn"], c["gn"], c["hd"]
+    m, hn, gn, hd, bs = c["m"], c["hn"], c["gn"], c["hd"], c["block"]
     for w, (kp, vp) in zip(layers, pools):
         n = _norm(x, c["norm"], w["n1"], w["n1b"], 1e-5)
         q = (n @ w["q"] + w["qb"]).view(m, hn, hd)
@@ -54,12 +54,12 @@ def _oracle(c, layers, x, pools):
             q, k = _turn(q, cos, sin), _turn(k, cos, sin)
         for i, slot in enumerate(c["slots"].tolist()):
             if slot >= 0:
-                kp[slot // 16, :, slot % 16], vp[slot // 16, :, slot % 16] = k[i], v[i]
+                kp[slot // bs, :, slot % bs], vp[slot // bs, :, slot % bs] = k[i], v[i]
         att = torch.zeros(m, hn, hd, dtype=torch.float64)
         for i, ctx in enumerate(c["ctx"]):
             if ctx == 0:
                 continue
-            blocks = c["tables"][i, :(ctx + 15) // 16].long()
+            blocks = c["tables"][i, :(ctx + bs - 1) // bs].long()
             kk = kp[blocks].permute(0, 2, 1, 3).reshape(-1, gn, hd)[:ctx].repeat_interleave(hn // gn, 1)
             vv = vp[blocks].permute(0, 2, 1, 3).reshape(-1, gn, hd)[:ctx].repeat_interleave(hn // gn, 1)
             p = torch.softmax(torch.einsum("hd,thd->ht", q[i], kk) * c["scale"], -1)
@@ -70,7 +70,7 @@ def _oracle(c, layers, x, pools):
     return x, _norm(x, c["norm"], c["last"].double().cpu(), None, 1e-5)
 
 
-def _case(gpu, dtype, m, d, f, hn, gn, hd, act, norm, rope, contexts, seed=0, layers=2):
+def _case(gpu, dtype, m, d, f, hn, gn, hd, act, norm, rope, contexts, seed=0, layers=2, block=16):
     g = torch.Generator().manual_seed(seed)
 
     def rand(*shape, std=1.0):
@@ -85,28 +85,31 @@ def _case(gpu, dtype, m, d, f, hn, gn, hd, act, norm, rope, contexts, seed=0, la
         if norm == NORM_LAYER:
             w.update(n1b=rand(d, std=0.1), n2b=rand(d, std=0.1))
         weights.append(w)
-    n_blocks = sum((c + 15) // 16 for c in contexts) + 1
+    held = [(c + block - 1) // block for c in contexts]
+    n_blocks = sum(held) + 1
     perm = torch.randperm(n_blocks, generator=g).tolist()
-    tables = torch.zeros(m, max((c + 15) // 16 for c in contexts) + 1, dtype=torch.int32)
+    tables = torch.zeros(m, max(held) + 1, dtype=torch.int32)
     slots = []
     for i, c in enumerate(contexts):
-        for j in range((c + 15) // 16):
+        for j in range(held[i]):
             tables[i, j] = perm.pop()
-        slots.append(int(tables[i, (c - 1) // 16]) * 16 + (c - 1) % 16 if c > 0 else -1)
+        slots.append(int(tables[i, (c - 1) // block]) * block + (c - 1) % block if c > 0 else -1)
     angles = torch.rand(max(contexts) + 1, hd // 2, generator=g) * 6
     c = {"m": m, "d": d, "f": f, "hn": hn, "gn": gn, "hd": hd, "act": act, "norm": norm, "rope": rope, "ctx": list(contexts),
          "tables": tables, "slots": torch.tensor(slots), "positions": torch.tensor([max(n - 1, 0) for n in contexts], dtype=torch.int32),
-         "cos": angles.cos().to(gpu), "sin": angles.sin().to(gpu), "scale": hd ** -0.5, "last": (1 + rand(d, std=0.1)).to(gpu)}
+         "cos": angles.cos().to(gpu), "sin": angles.sin().to(gpu), "scale": hd ** -0.5, "block": block, "last": (1 + rand(d, std=0.1)).to(gpu)}
     x = rand(m, d)
-    pools = [(rand(n_blocks, gn, 16, hd), rand(n_blocks, gn, 16, hd)) for _ in range(layers)]
+    pools = [(rand(n_blocks, gn, block, hd), rand(n_blocks, gn, block, hd)) for _ in range(layers)]
     return c, weights, x, pools
 
 
-def _run(gpu, dtype, c, weights, x, pools, **over):
-    """(out, norm_out, pools) of the library's call."""
+def _run(gpu, dtype, c, weights, x, pools, tokens_first=False, **over):
+    """(out, norm_out, pools) of the library's call; ``tokens_first``: a block's tokens are its outer rows in the pools."""
     lib = _lib.load()
     keep = [{k: None if t is None else t.to(gpu) for k, t in w.items()} for w in weights]
     on = [tuple(t.to(gpu) for t in kv) for kv in pools]
+    if tokens_first:
+        on = [tuple(t.transpose(1, 2).contiguous().transpose(1, 2) for t in kv) for kv in on]
     table = (_lib.STRUCTS["ic_step_layer"] * len(weights))()
     ptr = lambda t: None if t is None else t.data_ptr()
     for row, w, (k, v) in zip(table, keep, on):
@@ -129,7 +132,7 @@ def _run(gpu, dtype, c, weights, x, pools, **over):
         pool_stride_token=pool.stride(2), num_blocks=pool.shape[0], block_tables=meta[0].data_ptr(),
         block_table_stride=meta[0].stride(0), context_lens=meta[1].data_ptr(), slot_mapping=meta[2].data_ptr(),
         positions=meta[3].data_ptr() if c["rope"] else None, cos_table=c["cos"].data_ptr() if c["rope"] else None,
-        sin_table=c["sin"].data_ptr() if c["rope"] else None, table_rows=c["cos"].shape[0], block_size=16,
+        sin_table=c["sin"].data_ptr() if c["rope"] else None, table_rows=c["cos"].shape[0], block_size=c["block"],
         max_context_len=max(c["ctx"]), scale=c["scale"], dtype=_lib.dtype_code(dtype), **over)
     need = lib.ic_step_stack_workspace_bytes(ctypes.byref(call))
     assert need > 0
@@ -172,6 +175,34 @@ def test_against_float64(gpu, dtype, shape):
                 assert _close(got, t, TOL[dtype]), over
         if first is None:
             first = (out, normed)
+        assert torch.equal(out, first[0]) and torch.equal(normed, first[1]), over
+
+
+MORE = [  # m, d, f, hn, gn, hd, act, norm, rope, contexts; block size
+    ((4, 256, 512, 16, 16, 64, GELU, NORM_LAYER, False, (200, 3, 64, 31)), 32),      # an output projection in parts (fp32)
+    ((3, 512, 576, 16, 16, 128, SWIGLU, NORM_RMS, True, (40, 129, 16)), 48),         # ... and in 16 bits
+    ((7, 768, 1024, 12, 4, 64, SILU, NORM_LAYER, True, (511, 512, 513, 128, 127, 1, 257)), 64),   # three heads to a KV head
+    ((2, 384, 384, 6, 2, 64, RELU, NORM_RMS, False, (96, 97)), 16),
+    ((3, 512, 512, 8, 8, 64, GELU, NORM_LAYER, True, (1024, 2047, 2048)), 16),       # up to 16 tiles a wave
+    ((16, 128, 128, 2, 2, 64, GLU, NORM_LAYER, False, (2048,) * 8 + tuple(1900 + 17 * i for i in range(8))), 48),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape,block", MORE, ids=lambda v: "-".join(map(str, v[:6])) if isinstance(v, tuple) else str(v))
+def test_projections_groups_blocks_and_long_contexts(gpu, dtype, shape, block):
+    c, weights, x, pools = _case(gpu, dtype, *shape, block=block)
+    wide = [(k.double(), v.double()) for k, v in pools]
+    want = _oracle(c, [{k: None if t is None else t.double() for k, t in w.items()} for w in weights], x.double(), wide)
+    first = None
+    for over in (dict(), dict(tokens_first=True), dict(draw=1, workgroups=61)):
+        out, normed, after = _run(gpu, dtype, c, weights, x, pools, **over)
+        for got, true in zip((out, normed), want):
+            assert _close(got, true, TOL[dtype]), over
+        for pair, true in zip(after, wide):
+            for got, t in zip(pair, true):
+                assert _close(got, t, TOL[dtype]), over
+        first = first or (out, normed)
         assert torch.equal(out, first[0]) and torch.equal(normed, first[1]), over
 
 
