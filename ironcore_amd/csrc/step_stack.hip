@@ -515,7 +515,13 @@ struct Stack {
     for (int i = 0; i < S; ++i) {
       if (i >= used) break;
       const Vec16 x[1] = {xv[i]};
-      multiply<M, 1, NB>(wv[i], x, acc);
+      if constexpr (sizeof(T) == 4) {  // (a step's own sum: one chain over all would round as often as it has products)
+        f32x4_t step[NB][1] = {{{0.f, 0.f, 0.f, 0.f}}};
+        multiply<M, 1, NB>(wv[i], x, step);
+        acc[0][0] += step[0][0];
+      } else {
+        multiply<M, 1, NB>(wv[i], x, acc);
+      }
     }
     float *to = sums + c * PITCH + g * 4 * NB;
 #pragma unroll

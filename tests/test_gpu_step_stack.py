@@ -206,6 +206,32 @@ def test_projections_groups_blocks_and_long_contexts(gpu, dtype, shape, block):
         assert torch.equal(out, first[0]) and torch.equal(normed, first[1]), over
 
 
+@pytest.mark.parametrize("m", [4, 5, 16])   # the two forms of the product
+def test_fp32_rounds_no_more_than_the_layers_own_launches(gpu, m):
+    """Distance to float64 of the last norm, over four draws: not above that of a call per layer."""
+    host, off, dtype = _lib.host(), [0.0, 0.0], torch.float32
+    for seed in range(4):
+        c, weights, x, pools = _case(gpu, dtype, m, 768, 3072, 12, 12, 64, GELU, NORM_LAYER, False,
+                                     tuple(60 + 11 * i for i in range(m)), seed=seed)
+        wide = [(k.double(), v.double()) for k, v in pools]
+        want = _oracle(c, [{k: None if t is None else t.double() for k, t in w.items()} for w in weights], x.double(), wide)[1]
+        _, normed, _ = _run(gpu, dtype, c, weights, x, pools)
+        w = [{k: None if t is None else t.to(gpu) for k, t in layer.items()} for layer in weights]
+        hidden = x.to(gpu).view(m, 1, 768)
+        here = _lib.here(hidden)
+        n = host.norm_rows(hidden, w[0]["n1"], w[0]["n1b"], NORM_LAYER, 1e-5, *here)
+        meta = (c["tables"].to(gpu), torch.tensor(c["ctx"], dtype=torch.int32, device=gpu), c["slots"].to(gpu), max(c["ctx"]))
+        for i, layer in enumerate(w):
+            after = (w[i + 1]["n1"], w[i + 1]["n1b"]) if i + 1 < len(w) else (c["last"], None)
+            hidden, n = host.decoder_layer(
+                hidden, n, [layer[k] for k in ("q", "qb", "kv", "kvb", "o", "ob", "n2", "n2b", "up", "upb", "down", "downb")] + [*after],
+                12, 12, 64, GELU, NORM_LAYER, 1e-6, NORM_LAYER, 1e-5, False, *(t.to(gpu) for t in pools[i]), *meta, c["scale"], 1,
+                None, None, None, None, *here)
+        for j, got in enumerate((normed, n.view(m, 768))):
+            off[j] += ((got.double().cpu() - want).norm() / want.norm()).item()
+    assert off[0] <= off[1]
+
+
 def test_rows_that_see_each_other(gpu):
     """Two tokens of one sequence as rows of a step, and blocks that two rows share."""
     c, weights, x, pools = _case(gpu, torch.float32, 4, 128, 256, 2, 2, 64, GELU, NORM_LAYER, False, (40, 40, 17, 17))
