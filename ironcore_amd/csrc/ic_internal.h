@@ -149,6 +149,7 @@ struct PrefillArgs {
   int q_rows = 0;  // rows of q and out
   // Equal sequences: context_lens, cu_seqlens_q and block_tables may be null; then every context has
   // uniform_context keys, every chunk max_chunk_len rows, row_pitch rows apart, and sequence i is pool block i.
+  // With context_lens: no context is longer than uniform_context (0: not known), which only chooses between kernels.
   int64_t row_pitch = 0;
   int uniform_context = 0;
   // Rotary embedding of the query rows as they are loaded (nullptr = none): row r of q uses table row
