@@ -631,7 +631,7 @@ int32_t *ic_step_status(void) {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (no part of a graph that this thread may be capturing)
     if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
     void *p = nullptr;
-    if (hipHostMalloc(&p, 64, hipHostMallocDefault) != hipSuccess) p = nullptr, (void)hipGetLastError();
+    if (hipHostMalloc(&p, 64, hipHostMallocPortable) != hipSuccess) p = nullptr, (void)hipGetLastError();
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (p != nullptr) memset(p, 0, 64);
     return static_cast<int32_t *>(p);
